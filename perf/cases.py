@@ -151,3 +151,81 @@ def tolerance(case):
     smallest calls) a few of the bf16 roundings on the way go the other way: up to 2e-4 in the 2-norm, and 7e-3 of the
     larger of the value and the root mean square (one bf16 step of a slot's value).  Four times that."""
     return {"rel": 8e-4, "max": 3e-2}
+
+
+_VALUES = [0.0, 0.5, 1.0, 1.5, 2.0, 3.0, 4.0, 6.0, -0.0, -0.5, -1.0, -1.5, -2.0, -3.0, -4.0, -6.0]
+
+
+def _weights64(w, scales, e):
+    """Expert e's matrix [N, K] in 64 bits from the packed layout: 1 KB blocks of 16 rows x 128 values in the order
+    (32-value group, row), and scale tiles of 32 rows x 8 groups in the order (group % 4, row % 16, group / 4, row / 16)."""
+    N, kb = w.shape[1:]
+    codes = w[e].view(N // 16, kb // 64, 4, 16, 16).permute(0, 3, 1, 2, 4).reshape(N, kb)
+    codes = torch.stack([codes & 15, codes >> 4], dim=-1).reshape(N, kb // 16, 32)
+    s = scales[e * N:(e + 1) * N].reshape(N // 32, -1, 4, 16, 2, 2).permute(0, 5, 3, 1, 4, 2).reshape(N, -1)[:, :kb // 16]
+    table = torch.tensor(_VALUES, dtype=torch.float64, device=w.device)
+    return torch.ldexp(table[codes.long()], (s.int() - 127)[..., None]).reshape(N, 2 * kb)
+
+
+def _mxfp4(x):
+    """x rounded to MXFP4: blocks of 32 share a power of two, 2 ** (floor(log2(largest)) - 2); ties go to even codes."""
+    b = x.reshape(x.shape[0], -1, 32)
+    exponent = torch.frexp(b.abs().amax(-1, keepdim=True))[1] - 3
+    a = torch.ldexp(b.abs(), -exponent)
+    step = torch.where(a < 2, 0.5, torch.where(a < 4, 1.0, 2.0)).double()
+    return torch.ldexp((torch.round(a / step) * step).clamp(max=6.0) * torch.sign(b), exponent).reshape(x.shape)
+
+
+def _bf16_activations(case):
+    """The smallest calls keep the activations in bf16, all others round them to MXFP4: part of what the call computes."""
+    pairs = case["tokens"] * case["k"]
+    hidden = (case["H"] + 511) // 512 * 512
+    few = min(pairs, case["E"]) * (hidden // 256) < 512 and pairs <= 8 * case["E"]
+    return 8 * pairs <= case["E"] or few
+
+
+def _routing64(case, logits):
+    if case["router"] == "grouped":
+        p = torch.sigmoid(logits.double())
+        groups = p.view(p.shape[0], 8, -1)
+        best = groups.topk(2, dim=-1).values.sum(-1).topk(4, dim=-1).indices
+        keep = torch.zeros(groups.shape[:2], dtype=torch.bool, device=p.device).scatter_(1, best, True)
+        p = groups.masked_fill(~keep[..., None], -1.0).view(p.shape)
+    else:
+        p = torch.softmax(logits.double(), dim=-1)
+    w, ids = p.topk(case["k"], dim=-1)
+    return w / w.sum(-1, keepdim=True), ids
+
+
+def exact(case, seed):
+    """The layer in 64 bits, expert by expert, with the roundings that define it: activations and intermediate to MXFP4
+    (the intermediate to bf16 before) unless the call keeps them in bf16; nothing is rounded after the second product."""
+    state = prepare(case, seed)
+    opts, hidden, w1, w2 = state["opts"], state["hidden"], state["w1"], state["w2"]
+    if "logits" in state:
+        topk_w, topk_ids = _routing64(case, state["logits"])
+    else:
+        topk_w, topk_ids = state["topk_w"].double(), state["topk_ids"].long()
+    H, inter, local = case["H"], w1.shape[1] // 2, w1.shape[0]
+    quantise = (lambda v: v) if _bf16_activations(case) else _mxfp4
+    x = quantise(torch.nn.functional.pad(hidden.double(), (0, w1.shape[2] * 2 - H)))
+    out = torch.zeros(case["tokens"], H, dtype=torch.float64, device=x.device)
+    first = int(opts["expert_mask"].argmax()) if "expert_mask" in opts else 0
+    for e in range(local):
+        tok, slot = torch.nonzero(topk_ids == first + e, as_tuple=True)
+        if not len(tok):
+            continue
+        y = x[tok] @ _weights64(w1, opts["w1_scale"], e).T
+        if case["bias"]:
+            y = y + opts["bias1"][e].double()
+        gate, up = y[:, :inter], y[:, inter:]
+        if case["swiglu"]:
+            gate, up = gate.clamp(max=7.0), up.clamp(-7.0, 7.0) + 1.0
+            a = gate * torch.sigmoid(1.702 * gate) * up
+        else:
+            a = gate * torch.sigmoid(gate) * up
+        z = quantise(a.to(torch.bfloat16).double()) @ _weights64(w2, opts["w2_scale"], e).T
+        if case["bias"]:
+            z = z + opts["bias2"][e].double()
+        out.index_add_(0, tok, z[:, :H] * topk_w[tok, slot, None])
+    return (out, topk_w, topk_ids.int()) if "logits" in state else out
