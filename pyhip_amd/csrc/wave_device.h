@@ -1,0 +1,26 @@
+// Scans and reductions over the 64 lanes of a wave in the vector ALU.  A shuffle is an LDS operation with its latency
+// (about 100 cycles, six of them in a row for a wave-wide result); a DPP move rides in the instruction that uses it.
+#pragma once
+#include "common.h"
+
+// the value `v` of the lane that the DPP control selects, `old` in the lanes that it leaves out
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ u32 dpp_u32(u32 old, u32 v)
+{
+    return (u32)__builtin_amdgcn_update_dpp((int)old, (int)v, CTRL, ROW_MASK, 0xF, false);
+}
+#define DPP_ROW_SHR(n) (0x110 + (n))
+#define DPP_ROW_BCAST15 0x142
+#define DPP_ROW_BCAST31 0x143
+
+// inclusive prefix sum over the lanes: inside the rows of 16, then rows 0 and 2 into 1 and 3, then the lower half into the upper
+__device__ __forceinline__ u32 wave_scan_add(u32 v)
+{
+    v += dpp_u32<DPP_ROW_SHR(1), 0xF>(0, v);
+    v += dpp_u32<DPP_ROW_SHR(2), 0xF>(0, v);
+    v += dpp_u32<DPP_ROW_SHR(4), 0xF>(0, v);
+    v += dpp_u32<DPP_ROW_SHR(8), 0xF>(0, v);
+    v += dpp_u32<DPP_ROW_BCAST15, 0xA>(0, v);
+    v += dpp_u32<DPP_ROW_BCAST31, 0xC>(0, v);
+    return v;
+}

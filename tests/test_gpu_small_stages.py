@@ -43,3 +43,35 @@ def test_topk_reduce_edges(T, k, H, mode, f32):
                                                     _lib.current_stream()))
     want = torch.from_numpy(ref)
     assert torch.equal(out.cpu(), want if f32 else want.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("T,k", [(1, 1), (63, 1), (64, 1), (65, 1), (31, 8), (129, 8), (255, 4), (1025, 1), (256, 8)])
+@pytest.mark.parametrize("E,masked", [(1, False), (8, False), (63, True), (256, True), (1040, False)])
+def test_single_workgroup_sort_edges(T, k, E, masked):
+    """One wave with pairs, two, all sixteen with one or two groups each; fewer experts than lanes, more than threads:
+    the positions an expert-by-expert walk on the CPU gives."""
+    from pyhip_amd.moe_sorting import moe_sorting
+    rng = np.random.default_rng(T * 1000 + E)
+    ids = rng.integers(0, E, (T, k)).astype(np.int32)
+    w = rng.random((T, k), dtype=np.float32)
+    mask = (rng.random(E) < 0.7).astype(np.int32) if masked else None
+    bm = 32
+    so, sw, se = [], [], []
+    local = 0
+    for e in range(E):
+        if mask is not None and not mask[e]:
+            continue
+        t, s = np.nonzero(ids == e)
+        fill = -len(t) % bm
+        so += [(int(b) << 24) | int(a) for a, b in zip(t, s)] + [(k << 24) | T] * fill
+        sw += list(w[t, s]) + [0.0] * fill
+        se += [local] * ((len(t) + fill) // bm)
+        local += 1
+    print("sort", T, k, E, masked, flush=True)
+    got = moe_sorting(torch.from_numpy(ids).cuda(), torch.from_numpy(w).cuda(), E, 256, torch.bfloat16, bm,
+                      None if mask is None else torch.from_numpy(mask).cuda(), alloc_moe_out=False)
+    n = int(got[3][0])
+    assert n == len(so) and int(got[3][1]) == T
+    assert (got[0].cpu().numpy().view(np.uint32)[:n] == np.array(so, np.uint32)).all()
+    assert (got[1].cpu().numpy()[:n] == np.array(sw, np.float32)).all()
+    assert (got[2].cpu().numpy().view(np.uint32)[:n // bm] == np.array(se, np.uint32)).all()
