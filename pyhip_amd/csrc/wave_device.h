@@ -24,3 +24,20 @@ __device__ __forceinline__ u32 wave_scan_add(u32 v)
     v += dpp_u32<DPP_ROW_BCAST31, 0xC>(0, v);
     return v;
 }
+
+// maximum over the lanes (fmaxf's: a NaN loses against a number), the same in every lane
+__device__ __forceinline__ float wave_max_dpp(float f)
+{
+    auto step = [&](auto C, auto M) __attribute__((always_inline)) {
+        const u32 v = __builtin_bit_cast(u32, f);
+        f = fmaxf(f, __builtin_bit_cast(float, dpp_u32<decltype(C)::value, decltype(M)::value>(v, v)));
+    };
+    using Rows = std::integral_constant<int, 0xF>;
+    step(std::integral_constant<int, DPP_ROW_SHR(1)>{}, Rows{});
+    step(std::integral_constant<int, DPP_ROW_SHR(2)>{}, Rows{});
+    step(std::integral_constant<int, DPP_ROW_SHR(4)>{}, Rows{});
+    step(std::integral_constant<int, DPP_ROW_SHR(8)>{}, Rows{});
+    step(std::integral_constant<int, DPP_ROW_BCAST15>{}, std::integral_constant<int, 0xA>{});
+    step(std::integral_constant<int, DPP_ROW_BCAST31>{}, std::integral_constant<int, 0xC>{});
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(u32, f), WAVE - 1));
+}

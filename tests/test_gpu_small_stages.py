@@ -75,3 +75,29 @@ def test_single_workgroup_sort_edges(T, k, E, masked):
     assert (got[0].cpu().numpy().view(np.uint32)[:n] == np.array(so, np.uint32)).all()
     assert (got[1].cpu().numpy()[:n] == np.array(sw, np.float32)).all()
     assert (got[2].cpu().numpy().view(np.uint32)[:n // bm] == np.array(se, np.uint32)).all()
+
+
+@pytest.mark.parametrize("E", [64, 128, 256, 512])
+@pytest.mark.parametrize("grouped", [False, True])
+def test_router_ties_and_missing_scores(E, grouped):
+    """Equal scores go to the lower expert, minus infinity ranks last: the picks of a stable descending sort."""
+    from pyhip_amd.routing import fused_topk, grouped_topk
+    g = torch.Generator().manual_seed(E)
+    T, k = 37, 8
+    x = torch.randint(-3, 4, (T, E), generator=g).float()          # seven distinct scores: ties everywhere
+    x[0] = 0.0
+    x[1, :E - 1] = float("-inf")
+    x[2, ::2] = float("-inf")
+    x[3] = torch.arange(E).float().flip(0) / 64
+    s = torch.sigmoid(x) if grouped else torch.softmax(x, dim=-1)
+    if grouped:
+        best = s.view(T, 8, -1).topk(2, dim=-1).values.sum(-1)
+        groups = torch.sort(best, dim=-1, descending=True, stable=True).indices[:, :4]
+        on = torch.zeros(T, 8, dtype=torch.bool).scatter_(1, groups, True)
+        s = s.masked_fill(~on.repeat_interleave(E // 8, dim=1), float("-inf"))
+    want = torch.sort(s, dim=-1, descending=True, stable=True).indices[:, :k]
+    print("router", E, grouped, flush=True)
+    dev = x.cuda()
+    hidden = torch.zeros(T, 64, dtype=torch.bfloat16, device="cuda")
+    got = grouped_topk(dev, k, True, 8, 4) if grouped else fused_topk(hidden, dev, k, True)
+    assert torch.equal(got[1].cpu().long(), want)
