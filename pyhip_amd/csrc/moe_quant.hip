@@ -22,17 +22,18 @@ extern "C" __global__ void __launch_bounds__(QUANT_THREADS) moe_act_quant_mxfp4_
 extern "C" int64_t pyhip_moe_act_scale_stride(int K) { return ((int64_t)K + 511) / 512 * 16; }
 
 int pyhip_make_quant_args(const char* name, const void* x_bf16, int64_t row_stride_elems, int64_t rows, int K,
-                          uint8_t* q, uint8_t* scales, const uint32_t* rows_limit, QuantArgs* out)
+                          uint8_t* q, uint8_t* scales, const uint32_t* rows_limit, QuantArgs* out, int x_cols)
 {
     PYHIP_REQUIRE(x_bf16 && q && scales, "%s: null pointer", name);
     PYHIP_REQUIRE(K > 0 && K % 32 == 0, "%s: K=%d must be a positive multiple of 32", name, K);
-    PYHIP_REQUIRE(row_stride_elems >= K && row_stride_elems % 8 == 0,
+    PYHIP_REQUIRE(x_cols >= 0 && x_cols <= K && x_cols % 32 == 0, "%s: %d of %d columns given (a multiple of 32)", name, x_cols, K);
+    PYHIP_REQUIRE(row_stride_elems >= (x_cols ? x_cols : K) && row_stride_elems % 8 == 0,
                   "%s: row stride %lld must be >= K and a multiple of 8 elements", name, (long long)row_stride_elems);
     PYHIP_REQUIRE(((uintptr_t)x_bf16 % 16) == 0 && ((uintptr_t)q % 16) == 0 && ((uintptr_t)scales % 4) == 0,
                   "%s: pointers must be 16-byte aligned", name);
     out->x = (const uint16_t*)x_bf16; out->ldx = (long long)row_stride_elems; out->q = q; out->s = scales;
     out->rows = rows > 0 ? (long long)rows : 0; out->K = K; out->SK = (int)pyhip_moe_act_scale_stride(K);
-    out->rows_limit = rows_limit;
+    out->rows_limit = rows_limit; out->x_cols = x_cols;
     PYHIP_REQUIRE(out->rows * out->SK < (1ll << 40), "%s: too many rows", name);
     return PYHIP_OK;
 }

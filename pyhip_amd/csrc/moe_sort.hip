@@ -644,6 +644,24 @@ extern "C" int pyhip_moe_sorting(const int32_t* topk_ids, const float* topk_weig
                         workspace, workspace_bytes, qa, RouteArgs{}, stream);
 }
 
+// pyhip_moe_sorting_quant with activations of x_cols columns (a multiple of 32; 0: K), zeros from there up to K
+int pyhip_sorting_quant_cols(const int32_t* topk_ids, const float* topk_weights, int tokens, int topk,
+                                       int experts, int block_size, const int32_t* expert_mask,
+                                       const int32_t* num_local_tokens, uint32_t* sorted_ids, float* sorted_weights,
+                                       uint32_t* sorted_expert_ids, uint32_t* num_valid_ids, uint32_t* schedule,
+                                       void* workspace, int64_t workspace_bytes, const void* x_bf16,
+                                       int64_t row_stride_elems, int64_t rows, int K, uint8_t* q, uint8_t* scales,
+                                       int x_cols, hipStream_t stream)
+{
+    QuantArgs qa;
+    int rc = pyhip_make_quant_args("moe_sorting_quant", x_bf16, row_stride_elems, rows, K, q, scales, nullptr, &qa, x_cols);
+    if(rc)
+        return rc;
+    return sorting_impl(topk_ids, topk_weights, tokens, topk, experts, block_size, expert_mask, num_local_tokens,
+                        sorted_ids, sorted_weights, sorted_expert_ids, num_valid_ids, schedule, nullptr, 0, workspace,
+                        workspace_bytes, qa, RouteArgs{}, stream);
+}
+
 extern "C" int pyhip_moe_sorting_quant(const int32_t* topk_ids, const float* topk_weights, int tokens, int topk,
                                        int experts, int block_size, const int32_t* expert_mask,
                                        const int32_t* num_local_tokens, uint32_t* sorted_ids, float* sorted_weights,
@@ -652,13 +670,9 @@ extern "C" int pyhip_moe_sorting_quant(const int32_t* topk_ids, const float* top
                                        int64_t row_stride_elems, int64_t rows, int K, uint8_t* q, uint8_t* scales,
                                        hipStream_t stream)
 {
-    QuantArgs qa;
-    int rc = pyhip_make_quant_args("moe_sorting_quant", x_bf16, row_stride_elems, rows, K, q, scales, nullptr, &qa);
-    if(rc)
-        return rc;
-    return sorting_impl(topk_ids, topk_weights, tokens, topk, experts, block_size, expert_mask, num_local_tokens,
-                        sorted_ids, sorted_weights, sorted_expert_ids, num_valid_ids, schedule, nullptr, 0, workspace,
-                        workspace_bytes, qa, RouteArgs{}, stream);
+    return pyhip_sorting_quant_cols(topk_ids, topk_weights, tokens, topk, experts, block_size, expert_mask, num_local_tokens,
+                                    sorted_ids, sorted_weights, sorted_expert_ids, num_valid_ids, schedule, workspace,
+                                    workspace_bytes, x_bf16, row_stride_elems, rows, K, q, scales, 0, stream);
 }
 
 int pyhip_check_router(const char* name, const void* logits, const void* w, const void* ids, int tokens, int experts,

@@ -12,6 +12,7 @@ struct QuantArgs
     long long rows;            // 0: nothing to do
     int K, SK;
     const u32* rows_limit;     // device scalar or null
+    int x_cols;                // columns x has, a multiple of 32 (0: K); the rest up to K is quantised as the zeros it stands for
 };
 
 // One thread per 32-element block (id = row * SK + block; blocks past K are padding); 16 consecutive threads own
@@ -29,7 +30,12 @@ __device__ __forceinline__ void act_quant_block(const QuantArgs& a, long long id
     if(row >= rows)                                      // whole 16-thread groups leave together
         return;
     u32 e8 = 0;
-    if(j * 32 < a.K)
+    if(a.x_cols && j * 32 >= a.x_cols)
+    {
+        if(j * 32 < a.K)
+            *(uint4*)(a.q + row * (long long)(a.K / 2) + (long long)j * 16) = make_uint4(0, 0, 0, 0);
+    }
+    else if(j * 32 < a.K)
     {
         const uint4* src = (const uint4*)(a.x + row * a.ldx + (long long)j * 32);
         uint4 v0 = src[0], v1 = src[1], v2 = src[2], v3 = src[3];
@@ -57,4 +63,4 @@ __device__ __forceinline__ void act_quant_block(const QuantArgs& a, long long id
 
 // argument checks and the filled-in struct, shared by the entry points that quantise
 int pyhip_make_quant_args(const char* name, const void* x_bf16, int64_t row_stride_elems, int64_t rows, int K,
-                          uint8_t* q, uint8_t* scales, const uint32_t* rows_limit, QuantArgs* out);
+                          uint8_t* q, uint8_t* scales, const uint32_t* rows_limit, QuantArgs* out, int x_cols = 0);

@@ -193,9 +193,7 @@ def fused_moe(
     # returned at the true width.  The MXFP4-activation GEMMs are told the pads and leave the weights' padding unfetched.
     _require(0 <= hidden_pad < w1u.shape[2] * 2 and 0 <= intermediate_pad < w1u.shape[1] // 2, "bad hidden_pad / intermediate_pad")
     narrow = hidden_pad > 0 and hidden_states.shape[1] == w1u.shape[2] * 2 - hidden_pad
-    if narrow:
-        hidden_states = torch.nn.functional.pad(hidden_states, (0, hidden_pad))
-    T, H = hidden_states.shape
+    T, H = hidden_states.shape[0], w1u.shape[2] * 2 if narrow else hidden_states.shape[1]
     _require(topk_ids.dim() == 2 and topk_ids.shape[0] == T and tuple(topk_weight.shape) == tuple(topk_ids.shape),
              "topk_ids / topk_weight must be [tokens, topk]")
     k = topk_ids.shape[1]
@@ -254,7 +252,17 @@ def fused_moe(
         _require(not w4a16 and bm in (16, 128, 288) and not lds_tile,
                  "topk_reduce='last_arriver' needs the MXFP4-activation path and a row block of 16, 128 or 288")
 
-    if not return_parts and stage_events is None and not atomic and not lds_tile and not arriver:
+    one_call = not return_parts and stage_events is None and not atomic and not lds_tile and not arriver
+    cols = 0
+    if narrow:
+        # the one-call path quantises activations at the true width as they are: whole 32-column blocks, rows that lie
+        # one after the other and start on 16 bytes (anything else is widened into a buffer of its own first)
+        cols = H - hidden_pad
+        if not (one_call and not w4a16 and cols % 32 == 0 and hidden_states.stride(1) == 1 and hidden_states.stride(0) >= cols
+                and hidden_states.stride(0) % 8 == 0 and hidden_states.data_ptr() % 16 == 0):
+            cols = 0
+            hidden_states = torch.nn.functional.pad(hidden_states, (0, hidden_pad))
+    if one_call:
         # the whole layer in one library call, intermediates in one workspace: two allocations and one foreign call
         # per layer instead of a dozen of each (the host side is what bounds small layers when they are not replayed
         # from a graph)
@@ -265,7 +273,7 @@ def fused_moe(
         ws_bytes = lib.pyhip_moe_forward_workspace_bytes(T, k, global_E, H, I, bm, 1 if w4a16 else 0)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         out = torch.empty(T, H, dtype=out_dtype, device=dev)
-        rc = lib.pyhip_moe_forward(_lib.dptr(x), x.stride(0), _lib.dptr(w1u), _lib.dptr(w1s), _lib.dptr(w2u),
+        rc = lib.pyhip_moe_forward_cols(_lib.dptr(x), x.stride(0), cols, _lib.dptr(w1u), _lib.dptr(w1s), _lib.dptr(w2u),
                                    _lib.dptr(w2s), _lib.dptr(bias1), _lib.dptr(bias2), _lib.dptr(topk_ids),
                                    _lib.dptr(topk_weight), _lib.dptr(expert_mask), _lib.dptr(num_local_tokens),
                                    _lib.dptr(out), 1 if out_dtype == torch.float32 else 0, T, k, global_E, H, I,

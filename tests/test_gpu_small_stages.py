@@ -101,3 +101,34 @@ def test_router_ties_and_missing_scores(E, grouped):
     hidden = torch.zeros(T, 64, dtype=torch.bfloat16, device="cuda")
     got = grouped_topk(dev, k, True, 8, 4) if grouped else fused_topk(hidden, dev, k, True)
     assert torch.equal(got[1].cpu().long(), want)
+
+
+@pytest.mark.parametrize("T", [5, 65, 600])
+@pytest.mark.parametrize("form", ["contiguous", "row_stride", "odd_stride", "misaligned", "expanded", "transposed"])
+def test_true_width_activations(T, form):
+    """A padded layer called with activations at the true width, in every form they may come in, against the same
+    values widened by the caller: the same bits, and the widened shape's result cut to the true width."""
+    import cases
+    from pyhip_amd import fused_moe
+    L = cases.make_layer("gptoss_s", T, seed=5, bias=True)
+    w1, w1s, w2, w2s, b1, b2, hp, ip = cases.padded_device_weights(L)
+    tw, ti = torch.from_numpy(L.topk_w).cuda(), torch.from_numpy(L.topk_ids).cuda()
+    x, H = L.hidden.cuda(), L.H
+    if form == "row_stride":
+        x = torch.nn.functional.pad(x, (0, 8), value=float("nan"))[:, :H]
+    elif form == "odd_stride":
+        x = torch.nn.functional.pad(x, (0, 3), value=float("nan"))[:, :H]
+    elif form == "misaligned":
+        buf = torch.empty(T * H + 1, dtype=x.dtype, device="cuda")
+        buf[1:] = x.flatten()
+        x = buf[1:].view(T, H)
+    elif form == "expanded":
+        x = x[:1].expand(T, H)
+    elif form == "transposed":
+        x = x.t().contiguous().t()
+    kw = dict(w1_scale=w1s, w2_scale=w2s, bias1=b1, bias2=b2, hidden_pad=hp, intermediate_pad=ip)
+    for method in ("auto", "a4w4", "w4a16"):
+        print("true width", T, form, method, flush=True)
+        got = fused_moe(x, w1, w2, tw, ti, method=method, **kw)
+        wide = fused_moe(torch.nn.functional.pad(x, (0, hp)), w1, w2, tw, ti, method=method, **kw)
+        assert got.shape == (T, H) and torch.equal(got, wide[:, :H])
