@@ -83,10 +83,11 @@ def check(rc, what=""):
 
 
 def dptr(t):
-    """device pointer of a torch tensor (or None)"""
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    """device pointer of a torch tensor (or None), for a ``c_void_p`` parameter"""
+    return None if t is None else t.data_ptr()
 
 
 def current_stream():
+    """the current torch stream's handle, without the Stream object that ``torch.cuda.current_stream()`` builds"""
     import torch
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
