@@ -82,12 +82,25 @@ def check(rc, what=""):
         raise PyhipError("%s failed (code %d): %s" % (what or "pyhip_moe call", rc, msg))
 
 
-def dptr(t):
-    """device pointer of a torch tensor (or None), for a ``c_void_p`` parameter"""
+def addr(t):
+    """device address of a torch tensor (or None) as a plain integer, the cheapest form of a pointer: only for functions
+    whose ``argtypes`` say ``c_void_p``, as those of ``load()`` do (ctypes cuts an integer to 32 bits without them)"""
     return None if t is None else t.data_ptr()
 
 
-def current_stream():
-    """the current torch stream's handle, without the Stream object that ``torch.cuda.current_stream()`` builds"""
+def stream_handle():
+    """the current torch stream's handle as an integer, without the Stream object that ``torch.cuda.current_stream()``
+    builds; for the same functions as ``addr``"""
     import torch
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+
+
+def dptr(t):
+    """device pointer of a torch tensor (or None) as a ``c_void_p``: also right for functions without ``argtypes`` and
+    among the arguments of a ``co_module.Kernel``, where an integer is a 32-bit int"""
+    return None if t is None else ctypes.c_void_p(t.data_ptr())
+
+
+def current_stream():
+    """``stream_handle()`` as a ``c_void_p``"""
+    return ctypes.c_void_p(stream_handle())

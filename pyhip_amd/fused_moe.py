@@ -128,8 +128,8 @@ def act_quant_mxfp4(x, rows_limit=None):
     sk = lib.pyhip_moe_act_scale_stride(K)
     q = torch.empty(rows, K // 2, dtype=torch.uint8, device=x.device)
     s = torch.empty(rows, sk, dtype=torch.uint8, device=x.device)
-    rc = lib.pyhip_moe_act_quant_mxfp4(_lib.dptr(x), x.stride(0), rows, K, _lib.dptr(q), _lib.dptr(s),
-                                       _lib.dptr(rows_limit), _lib.current_stream())
+    rc = lib.pyhip_moe_act_quant_mxfp4(_lib.addr(x), x.stride(0), rows, K, _lib.addr(q), _lib.addr(s),
+                                       _lib.addr(rows_limit), _lib.stream_handle())
     _lib.check(rc, "act_quant_mxfp4")
     return q, s
 
@@ -284,12 +284,12 @@ def fused_moe(
             x = x.contiguous()
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         out = torch.empty(T, H, dtype=out_dtype, device=dev)
-        rc = lib.pyhip_moe_forward_cols(_lib.dptr(x), x.stride(0), cols, _lib.dptr(w1u), _lib.dptr(w1s), _lib.dptr(w2u),
-                                   _lib.dptr(w2s), _lib.dptr(bias1), _lib.dptr(bias2), _lib.dptr(topk_ids),
-                                   _lib.dptr(topk_weight), _lib.dptr(expert_mask), _lib.dptr(num_local_tokens),
-                                   _lib.dptr(out), 1 if out_dtype == torch.float32 else 0, T, k, global_E, H, I,
+        rc = lib.pyhip_moe_forward_cols(_lib.addr(x), x.stride(0), cols, _lib.addr(w1u), _lib.addr(w1s), _lib.addr(w2u),
+                                   _lib.addr(w2s), _lib.addr(bias1), _lib.addr(bias2), _lib.addr(topk_ids),
+                                   _lib.addr(topk_weight), _lib.addr(expert_mask), _lib.addr(num_local_tokens),
+                                   _lib.addr(out), 1 if out_dtype == torch.float32 else 0, T, k, global_E, H, I,
                                    hidden_pad, intermediate_pad, bm, 1 if w4a16 else 0, splitk, act, limit,
-                                   _lib.dptr(ws), ws_bytes, _lib.current_stream())
+                                   _lib.addr(ws), ws_bytes, _lib.stream_handle())
         _lib.check(rc, "moe_forward")
         return out[:, : H - hidden_pad] if narrow else out
 
@@ -303,27 +303,27 @@ def fused_moe(
     sorted_ids, sorted_w, sorted_e, num_valid, _, sched = res[:6]
     ev = _mark("sort", ev)
     n_blk = sorted_e.numel()
-    stream = _lib.current_stream()
+    stream = _lib.stream_handle()
 
     def _reduce(out3, out):
         # slots the sort dropped (ids outside [0, E), masked experts, tokens past the local count) were never
         # written by the down GEMM: the reduction reads the routing and leaves them out
-        return lib.pyhip_moe_topk_reduce_routed(_lib.dptr(out3), _lib.dptr(out), T, k, H,
-                                                1 if out_dtype == torch.float32 else 0, _lib.dptr(topk_ids), global_E,
-                                                _lib.dptr(expert_mask), _lib.dptr(num_local_tokens), stream)
+        return lib.pyhip_moe_topk_reduce_routed(_lib.addr(out3), _lib.addr(out), T, k, H,
+                                                1 if out_dtype == torch.float32 else 0, _lib.addr(topk_ids), global_E,
+                                                _lib.addr(expert_mask), _lib.addr(num_local_tokens), stream)
 
     if w4a16:
         hs = hidden_states.contiguous()
         a2 = torch.empty(n_blk * bm, I, dtype=torch.bfloat16, device=dev)
-        rc = lib.pyhip_moe_gemm1_w4a16(_lib.dptr(hs), _lib.dptr(w1u), _lib.dptr(w1s), _lib.dptr(bias1),
-                                       _lib.dptr(sorted_ids), _lib.dptr(sorted_e), _lib.dptr(num_valid),
-                                       _lib.dptr(a2), T, k, global_E, H, I, bm, n_blk, splitk, act, limit, stream)
+        rc = lib.pyhip_moe_gemm1_w4a16(_lib.addr(hs), _lib.addr(w1u), _lib.addr(w1s), _lib.addr(bias1),
+                                       _lib.addr(sorted_ids), _lib.addr(sorted_e), _lib.addr(num_valid),
+                                       _lib.addr(a2), T, k, global_E, H, I, bm, n_blk, splitk, act, limit, stream)
         _lib.check(rc, "moe_gemm1_w4a16")
         ev = _mark("gemm1", ev)
         out3 = torch.empty(T, k, H, dtype=torch.bfloat16, device=dev)
-        rc = lib.pyhip_moe_gemm2_w4a16(_lib.dptr(a2), _lib.dptr(w2u), _lib.dptr(w2s), _lib.dptr(bias2),
-                                       _lib.dptr(sorted_ids), _lib.dptr(sorted_w), _lib.dptr(sorted_e),
-                                       _lib.dptr(num_valid), _lib.dptr(out3), T, k, global_E, H, I, bm, n_blk, splitk, stream)
+        rc = lib.pyhip_moe_gemm2_w4a16(_lib.addr(a2), _lib.addr(w2u), _lib.addr(w2s), _lib.addr(bias2),
+                                       _lib.addr(sorted_ids), _lib.addr(sorted_w), _lib.addr(sorted_e),
+                                       _lib.addr(num_valid), _lib.addr(out3), T, k, global_E, H, I, bm, n_blk, splitk, stream)
         _lib.check(rc, "moe_gemm2_w4a16")
         ev = _mark("gemm2", ev)
         out = torch.empty(T, H, dtype=out_dtype, device=dev)
@@ -343,25 +343,25 @@ def fused_moe(
     a2_q = torch.empty(n_blk * bm, I // 2, dtype=torch.uint8, device=dev)
     a2_s = torch.empty(n_blk * bm, lib.pyhip_moe_act_scale_stride(I), dtype=torch.uint8, device=dev)
     if lds_tile:
-        rc = lib.pyhip_moe_gemm1_mxfp4_lds(_lib.dptr(a1_q), _lib.dptr(a1_s), _lib.dptr(w1u), _lib.dptr(w1s),
-                                           _lib.dptr(bias1), _lib.dptr(sorted_ids), _lib.dptr(sorted_e),
-                                           _lib.dptr(num_valid), _lib.dptr(sched), _lib.dptr(a2), _lib.dptr(a2_q),
-                                           _lib.dptr(a2_s), T, k, global_E, H, I, n_blk, act, limit, stream)
+        rc = lib.pyhip_moe_gemm1_mxfp4_lds(_lib.addr(a1_q), _lib.addr(a1_s), _lib.addr(w1u), _lib.addr(w1s),
+                                           _lib.addr(bias1), _lib.addr(sorted_ids), _lib.addr(sorted_e),
+                                           _lib.addr(num_valid), _lib.addr(sched), _lib.addr(a2), _lib.addr(a2_q),
+                                           _lib.addr(a2_s), T, k, global_E, H, I, n_blk, act, limit, stream)
     else:
-        rc = lib.pyhip_moe_gemm1_mxfp4(_lib.dptr(a1_q), _lib.dptr(a1_s), _lib.dptr(w1u), _lib.dptr(w1s),
-                                       _lib.dptr(bias1), _lib.dptr(sorted_ids), _lib.dptr(sorted_e),
-                                       _lib.dptr(num_valid), _lib.dptr(sched), _lib.dptr(a2), _lib.dptr(a2_q),
-                                       _lib.dptr(a2_s), T, k, global_E, H, I, hidden_pad, intermediate_pad, bm, n_blk,
+        rc = lib.pyhip_moe_gemm1_mxfp4(_lib.addr(a1_q), _lib.addr(a1_s), _lib.addr(w1u), _lib.addr(w1s),
+                                       _lib.addr(bias1), _lib.addr(sorted_ids), _lib.addr(sorted_e),
+                                       _lib.addr(num_valid), _lib.addr(sched), _lib.addr(a2), _lib.addr(a2_q),
+                                       _lib.addr(a2_s), T, k, global_E, H, I, hidden_pad, intermediate_pad, bm, n_blk,
                                        act, limit, stream)
     _lib.check(rc, "moe_gemm1_mxfp4")
     ev = _mark("gemm1", ev)
     if atomic:
         out3 = None
         out = torch.empty(T, H, dtype=out_dtype, device=dev)
-        _lib.check(lib.pyhip_moe_zero_fill(_lib.dptr(out), out.numel() * 2, stream), "moe_zero_fill")
-        rc = lib.pyhip_moe_gemm2_mxfp4_atomic(_lib.dptr(a2_q), _lib.dptr(a2_s), _lib.dptr(w2u), _lib.dptr(w2s),
-                                              _lib.dptr(bias2), _lib.dptr(sorted_ids), _lib.dptr(sorted_w),
-                                              _lib.dptr(sorted_e), _lib.dptr(num_valid), _lib.dptr(sched), _lib.dptr(out),
+        _lib.check(lib.pyhip_moe_zero_fill(_lib.addr(out), out.numel() * 2, stream), "moe_zero_fill")
+        rc = lib.pyhip_moe_gemm2_mxfp4_atomic(_lib.addr(a2_q), _lib.addr(a2_s), _lib.addr(w2u), _lib.addr(w2s),
+                                              _lib.addr(bias2), _lib.addr(sorted_ids), _lib.addr(sorted_w),
+                                              _lib.addr(sorted_e), _lib.addr(num_valid), _lib.addr(sched), _lib.addr(out),
                                               T, k, global_E, H, I, bm, n_blk, stream)
         _lib.check(rc, "moe_gemm2_mxfp4_atomic")
         _mark("gemm2", ev)
@@ -370,25 +370,25 @@ def fused_moe(
         out3 = torch.empty(T, k, H, dtype=torch.bfloat16, device=dev)
         out = torch.empty(T, H, dtype=out_dtype, device=dev)
         arrive = torch.empty(T * (H // 256), dtype=torch.int32, device=dev)
-        rc = lib.pyhip_moe_gemm2_mxfp4_reduce(_lib.dptr(a2_q), _lib.dptr(a2_s), _lib.dptr(w2u), _lib.dptr(w2s),
-                                              _lib.dptr(bias2), _lib.dptr(sorted_ids), _lib.dptr(sorted_w),
-                                              _lib.dptr(sorted_e), _lib.dptr(num_valid), _lib.dptr(sched), _lib.dptr(out3),
-                                              _lib.dptr(topk_ids), _lib.dptr(expert_mask), _lib.dptr(num_local_tokens),
-                                              _lib.dptr(arrive), _lib.dptr(out), 1 if out_dtype == torch.float32 else 0,
+        rc = lib.pyhip_moe_gemm2_mxfp4_reduce(_lib.addr(a2_q), _lib.addr(a2_s), _lib.addr(w2u), _lib.addr(w2s),
+                                              _lib.addr(bias2), _lib.addr(sorted_ids), _lib.addr(sorted_w),
+                                              _lib.addr(sorted_e), _lib.addr(num_valid), _lib.addr(sched), _lib.addr(out3),
+                                              _lib.addr(topk_ids), _lib.addr(expert_mask), _lib.addr(num_local_tokens),
+                                              _lib.addr(arrive), _lib.addr(out), 1 if out_dtype == torch.float32 else 0,
                                               T, k, global_E, H, I, bm, n_blk, stream)
         _lib.check(rc, "moe_gemm2_mxfp4_reduce")
         _mark("gemm2", ev)
     else:
         out3 = torch.empty(T, k, H, dtype=torch.bfloat16, device=dev)
         if lds_tile:
-            rc = lib.pyhip_moe_gemm2_mxfp4_lds(_lib.dptr(a2_q), _lib.dptr(a2_s), _lib.dptr(w2u), _lib.dptr(w2s),
-                                               _lib.dptr(bias2), _lib.dptr(sorted_ids), _lib.dptr(sorted_w),
-                                               _lib.dptr(sorted_e), _lib.dptr(num_valid), _lib.dptr(sched),
-                                               _lib.dptr(out3), T, k, global_E, H, I, n_blk, stream)
+            rc = lib.pyhip_moe_gemm2_mxfp4_lds(_lib.addr(a2_q), _lib.addr(a2_s), _lib.addr(w2u), _lib.addr(w2s),
+                                               _lib.addr(bias2), _lib.addr(sorted_ids), _lib.addr(sorted_w),
+                                               _lib.addr(sorted_e), _lib.addr(num_valid), _lib.addr(sched),
+                                               _lib.addr(out3), T, k, global_E, H, I, n_blk, stream)
         else:
-            rc = lib.pyhip_moe_gemm2_mxfp4(_lib.dptr(a2_q), _lib.dptr(a2_s), _lib.dptr(w2u), _lib.dptr(w2s),
-                                           _lib.dptr(bias2), _lib.dptr(sorted_ids), _lib.dptr(sorted_w),
-                                           _lib.dptr(sorted_e), _lib.dptr(num_valid), _lib.dptr(sched), _lib.dptr(out3),
+            rc = lib.pyhip_moe_gemm2_mxfp4(_lib.addr(a2_q), _lib.addr(a2_s), _lib.addr(w2u), _lib.addr(w2s),
+                                           _lib.addr(bias2), _lib.addr(sorted_ids), _lib.addr(sorted_w),
+                                           _lib.addr(sorted_e), _lib.addr(num_valid), _lib.addr(sched), _lib.addr(out3),
                                            T, k, global_E, H, I, hidden_pad, intermediate_pad, bm, n_blk, stream)
         _lib.check(rc, "moe_gemm2_mxfp4")
         ev = _mark("gemm2", ev)
@@ -448,12 +448,12 @@ def fused_moe_routed(hidden_states, w1, w2, gating_output, topk, renormalize=Tru
     out = torch.empty(T, H, dtype=out_dtype, device=dev)
     tw = torch.empty(T, topk, dtype=torch.float32, device=dev)
     ti = torch.empty(T, topk, dtype=torch.int32, device=dev)
-    rc = lib.pyhip_moe_forward_routed(_lib.dptr(x), x.stride(0), _lib.dptr(w1u), _lib.dptr(w1s), _lib.dptr(w2u),
-                                      _lib.dptr(w2s), _lib.dptr(bias1), _lib.dptr(bias2), _lib.dptr(g),
-                                      int(num_expert_group), int(topk_group), 1 if renormalize else 0, _lib.dptr(ti),
-                                      _lib.dptr(tw), _lib.dptr(expert_mask), _lib.dptr(num_local_tokens), _lib.dptr(out),
+    rc = lib.pyhip_moe_forward_routed(_lib.addr(x), x.stride(0), _lib.addr(w1u), _lib.addr(w1s), _lib.addr(w2u),
+                                      _lib.addr(w2s), _lib.addr(bias1), _lib.addr(bias2), _lib.addr(g),
+                                      int(num_expert_group), int(topk_group), 1 if renormalize else 0, _lib.addr(ti),
+                                      _lib.addr(tw), _lib.addr(expert_mask), _lib.addr(num_local_tokens), _lib.addr(out),
                                       1 if out_dtype == torch.float32 else 0, T, topk, global_E, H, I, int(hidden_pad),
-                                      int(intermediate_pad), bm, 1 if w4a16 else 0, splitk, act, limit, _lib.dptr(ws),
-                                      ws_bytes, _lib.current_stream())
+                                      int(intermediate_pad), bm, 1 if w4a16 else 0, splitk, act, limit, _lib.addr(ws),
+                                      ws_bytes, _lib.stream_handle())
     _lib.check(rc, "moe_forward_routed")
     return (out, tw, ti) if return_routing else out

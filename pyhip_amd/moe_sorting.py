@@ -54,20 +54,20 @@ def moe_sorting(topk_ids, topk_weights, num_experts, model_dim, moebuf_dtype, bl
         q = torch.empty(rows, K // 2, dtype=torch.uint8, device=dev)
         s = torch.empty(rows, lib.pyhip_moe_act_scale_stride(K), dtype=torch.uint8, device=dev)
         rc = lib.pyhip_moe_sorting_quant(
-            _lib.dptr(topk_ids), _lib.dptr(topk_weights), T, k, num_experts, block_size,
-            _lib.dptr(expert_mask), _lib.dptr(num_local_tokens),
-            _lib.dptr(sorted_ids), _lib.dptr(sorted_w), _lib.dptr(sorted_e), _lib.dptr(num_valid), _lib.dptr(sched),
-            _lib.dptr(ws), ws_bytes, _lib.dptr(x), x.stride(0), rows, K, _lib.dptr(q), _lib.dptr(s),
-            _lib.current_stream())
+            _lib.addr(topk_ids), _lib.addr(topk_weights), T, k, num_experts, block_size,
+            _lib.addr(expert_mask), _lib.addr(num_local_tokens),
+            _lib.addr(sorted_ids), _lib.addr(sorted_w), _lib.addr(sorted_e), _lib.addr(num_valid), _lib.addr(sched),
+            _lib.addr(ws), ws_bytes, _lib.addr(x), x.stride(0), rows, K, _lib.addr(q), _lib.addr(s),
+            _lib.stream_handle())
         _lib.check(rc, "moe_sorting_quant")
         extra = ((q, s),)
     else:
         rc = lib.pyhip_moe_sorting(
-            _lib.dptr(topk_ids), _lib.dptr(topk_weights), T, k, num_experts, block_size,
-            _lib.dptr(expert_mask), _lib.dptr(num_local_tokens),
-            _lib.dptr(sorted_ids), _lib.dptr(sorted_w), _lib.dptr(sorted_e), _lib.dptr(num_valid), _lib.dptr(sched),
-            _lib.dptr(moe_out), 0 if moe_out is None else moe_out.numel() * moe_out.element_size(),
-            _lib.dptr(ws), ws_bytes, _lib.current_stream())
+            _lib.addr(topk_ids), _lib.addr(topk_weights), T, k, num_experts, block_size,
+            _lib.addr(expert_mask), _lib.addr(num_local_tokens),
+            _lib.addr(sorted_ids), _lib.addr(sorted_w), _lib.addr(sorted_e), _lib.addr(num_valid), _lib.addr(sched),
+            _lib.addr(moe_out), 0 if moe_out is None else moe_out.numel() * moe_out.element_size(),
+            _lib.addr(ws), ws_bytes, _lib.stream_handle())
         _lib.check(rc, "moe_sorting")
     if return_schedule:
         return (sorted_ids, sorted_w, sorted_e, num_valid, moe_out, sched) + extra

@@ -35,8 +35,8 @@ def fused_topk(hidden_states, gating_output, topk, renormalize=True):
     g = _scores(gating_output, True)
     w = torch.empty(T, topk, dtype=torch.float32, device=g.device)
     ids = torch.empty(T, topk, dtype=torch.int32, device=g.device)
-    _lib.check(lib.pyhip_moe_topk_softmax(_lib.dptr(g), T, g.shape[1], topk, 1 if renormalize else 0, _lib.dptr(w),
-                                          _lib.dptr(ids), _lib.current_stream()), "topk_softmax")
+    _lib.check(lib.pyhip_moe_topk_softmax(_lib.addr(g), T, g.shape[1], topk, 1 if renormalize else 0, _lib.addr(w),
+                                          _lib.addr(ids), _lib.stream_handle()), "topk_softmax")
     return w, ids
 
 
@@ -47,9 +47,9 @@ def grouped_topk(gating_output, topk, renormalize=True, num_expert_group=8, topk
     g = _scores(gating_output, False)
     w = torch.empty(T, topk, dtype=torch.float32, device=g.device)
     ids = torch.empty(T, topk, dtype=torch.int32, device=g.device)
-    _lib.check(lib.pyhip_moe_topk_grouped_sigmoid(_lib.dptr(g), T, E, topk, num_expert_group, topk_group,
-                                                  1 if renormalize else 0, _lib.dptr(w), _lib.dptr(ids),
-                                                  _lib.current_stream()), "topk_grouped_sigmoid")
+    _lib.check(lib.pyhip_moe_topk_grouped_sigmoid(_lib.addr(g), T, E, topk, num_expert_group, topk_group,
+                                                  1 if renormalize else 0, _lib.addr(w), _lib.addr(ids),
+                                                  _lib.stream_handle()), "topk_grouped_sigmoid")
     return w, ids
 
 
