@@ -31,8 +31,7 @@ class GemmArgs(ctypes.Structure):
 
 class QuantArgs(ctypes.Structure):
     """argument of moe_act_quant_mxfp4_kernel (pyhip_amd/csrc/quant_device.h)"""
-    _fields_ = [("x", _P), ("ldx", _L), ("q", _P), ("s", _P), ("rows", _L), ("K", _I), ("SK", _I), ("rows_limit", _P),
-                ("x_cols", _I)]
+    _fields_ = [("x", _P), ("ldx", _L), ("q", _P), ("s", _P), ("rows", _L), ("K", _I), ("SK", _I), ("rows_limit", _P)]
 
 
 class ReduceRouting(ctypes.Structure):

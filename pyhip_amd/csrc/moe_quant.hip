@@ -33,7 +33,7 @@ int pyhip_make_quant_args(const char* name, const void* x_bf16, int64_t row_stri
                   "%s: pointers must be 16-byte aligned", name);
     out->x = (const uint16_t*)x_bf16; out->ldx = (long long)row_stride_elems; out->q = q; out->s = scales;
     out->rows = rows > 0 ? (long long)rows : 0; out->K = K; out->SK = (int)pyhip_moe_act_scale_stride(K);
-    out->rows_limit = rows_limit; out->x_cols = x_cols;
+    out->rows_limit = rows_limit;
     PYHIP_REQUIRE(out->rows * out->SK < (1ll << 40), "%s: too many rows", name);
     return PYHIP_OK;
 }

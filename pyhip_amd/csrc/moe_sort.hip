@@ -270,19 +270,11 @@ __device__ __forceinline__ void write_schedule(const SortArgs& a, const u32* off
 // ---------------------------------------------------------------------------------------------
 // single workgroup: everything in one launch (up to SMALL_GROUPS * 64 pairs per wave)
 // LDS: whist[SMALL_WAVES][E] | tot[E] | off[E] | lid[E] | scratch[2*SMALL_WAVES]
-// Workgroups past the first quantise activations (qa.rows > 0): the input quantisation of the MXFP4-activation
-// path depends on nothing the sort computes, and carrying it in this launch saves a dispatch.
 // NE > 0: the workgroup first routes the tokens itself (a wave per token, tokens dealt round-robin to its 16 waves;
 // the step before the sort, aiter.fused_topk at tests/contrib/moe/test_fused_moe.py:38,87, costs no launch of its own).
 template <int NE, bool GROUPED>
-__global__ void __launch_bounds__(SMALL_THREADS) moe_sort_small_kernel(SortArgs a, QuantArgs qa, RouteArgs ra)
+__device__ __forceinline__ void sort_small(const SortArgs& a, const RouteArgs& ra, u32* lds)
 {
-    if(blockIdx.x > 0)
-    {
-        act_quant_block(qa, (long long)(blockIdx.x - 1) * SMALL_THREADS + threadIdx.x);
-        return;
-    }
-    extern __shared__ u32 lds[];
     u32* whist   = lds;
     u32* tot     = whist + SMALL_WAVES * a.E;
     u32* off     = tot + a.E;
@@ -359,6 +351,28 @@ __global__ void __launch_bounds__(SMALL_THREADS) moe_sort_small_kernel(SortArgs 
     wp.scatter(a, whist + wave * a.E, off, beg, end);
 }
 
+// Workgroups past the first quantise activations (qa.rows > 0): the input quantisation of the MXFP4-activation
+// path depends on nothing the sort computes, and carrying it in this launch saves a dispatch.
+template <int NE, bool GROUPED>
+__global__ void __launch_bounds__(SMALL_THREADS) moe_sort_small_kernel(SortArgs a, QuantArgs qa, RouteArgs ra)
+{
+    extern __shared__ u32 lds[];
+    if(blockIdx.x > 0)
+        act_quant_block(qa, (long long)(blockIdx.x - 1) * SMALL_THREADS + threadIdx.x);
+    else
+        sort_small<NE, GROUPED>(a, ra, lds);
+}
+
+// the same for activations that have x_cols columns: a kernel of its own, so that the others keep their arguments
+extern "C" __global__ void __launch_bounds__(SMALL_THREADS) moe_sort_small_cols_kernel(SortArgs a, QuantArgs qa, int x_cols)
+{
+    extern __shared__ u32 lds[];
+    if(blockIdx.x > 0)
+        act_quant_block(qa, (long long)(blockIdx.x - 1) * SMALL_THREADS + threadIdx.x, x_cols);
+    else
+        sort_small<0, false>(a, RouteArgs{}, lds);
+}
+
 // ---------------------------------------------------------------------------------------------
 // large inputs, launch 1 of 3: per-workgroup histogram -> ws[g][E]; padding entries everywhere
 extern "C" __global__ void __launch_bounds__(SORT_THREADS) moe_sort_hist_kernel(SortArgs a)
@@ -386,16 +400,8 @@ extern "C" __global__ void __launch_bounds__(SORT_THREADS) moe_sort_hist_kernel(
 
 // launch 2 of 3 (one workgroup): ws[g][e] -> exclusive prefix over g; offsets; tables
 // LDS: tot[E] | off[E] | lid[E] | scratch
-// Workgroups past the first quantise activations, as in the single-workgroup sort: the scan is one workgroup
-// of serial work during which the rest of the GPU would idle.
-extern "C" __global__ void __launch_bounds__(SMALL_THREADS) moe_sort_scan_kernel(SortArgs a, QuantArgs qa)
+__device__ __forceinline__ void sort_scan(const SortArgs& a, u32* lds)
 {
-    if(blockIdx.x > 0)
-    {
-        act_quant_block(qa, (long long)(blockIdx.x - 1) * SMALL_THREADS + threadIdx.x);
-        return;
-    }
-    extern __shared__ u32 lds[];
     u32* tot     = lds;
     u32* off     = tot + a.E;
     u32* lid     = off + a.E;
@@ -427,6 +433,25 @@ extern "C" __global__ void __launch_bounds__(SMALL_THREADS) moe_sort_scan_kernel
         g_off[e] = off[e];
     fill_blocks(a, tot, off, lid, padded_total, T);
     write_schedule(a, off, lid, padded_total);
+}
+
+// Workgroups past the first quantise activations, as in the single-workgroup sort: the scan is one workgroup
+// of serial work during which the rest of the GPU would idle.
+extern "C" __global__ void __launch_bounds__(SMALL_THREADS) moe_sort_scan_kernel(SortArgs a, QuantArgs qa)
+{
+    extern __shared__ u32 lds[];
+    if(blockIdx.x > 0)
+        act_quant_block(qa, (long long)(blockIdx.x - 1) * SMALL_THREADS + threadIdx.x);
+    else
+        sort_scan(a, lds);
+}
+extern "C" __global__ void __launch_bounds__(SMALL_THREADS) moe_sort_scan_cols_kernel(SortArgs a, QuantArgs qa, int x_cols)
+{
+    extern __shared__ u32 lds[];
+    if(blockIdx.x > 0)
+        act_quant_block(qa, (long long)(blockIdx.x - 1) * SMALL_THREADS + threadIdx.x, x_cols);
+    else
+        sort_scan(a, lds);
 }
 
 // launch 3 of 3: scatter.  LDS: whist[SORT_WAVES][E]
@@ -558,7 +583,7 @@ static int sorting_impl(const int32_t* topk_ids, const float* topk_weights, int 
                         const int32_t* num_local_tokens, uint32_t* sorted_ids, float* sorted_weights,
                         uint32_t* sorted_expert_ids, uint32_t* num_valid_ids, uint32_t* schedule,
                         void* moe_out, int64_t moe_out_bytes, void* workspace, int64_t workspace_bytes,
-                        QuantArgs qa, RouteArgs ra, hipStream_t stream)
+                        QuantArgs qa, RouteArgs ra, hipStream_t stream, int x_cols = 0)
 {
     PYHIP_REQUIRE(topk_ids && topk_weights && sorted_ids && sorted_weights && sorted_expert_ids && num_valid_ids,
                   "moe_sorting: null pointer");
@@ -609,21 +634,28 @@ static int sorting_impl(const int32_t* topk_ids, const float* topk_weights, int 
         if(lds > 64 * 1024)
         {
             PYHIP_REQUIRE(!ra.gating, "moe_sorting: the routing sort handles at most %d experts", ROUTE_SORT_MAX_EXPERTS);
-            hipError_t e = hipFuncSetAttribute((const void*)moe_sort_small_kernel<0, false>,
+            hipError_t e = hipFuncSetAttribute(x_cols ? (const void*)moe_sort_small_cols_kernel
+                                                      : (const void*)moe_sort_small_kernel<0, false>,
                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
             PYHIP_REQUIRE(e == hipSuccess, "moe_sorting: cannot reserve %zu B of LDS", lds);
         }
         if(ra.gating)
             return launch_routing_sort(a, qa, ra, qblocks, lds, stream);
-        hipLaunchKernelGGL((moe_sort_small_kernel<0, false>), dim3(1 + qblocks), dim3(SMALL_THREADS), lds, stream, a, qa, ra);
+        if(x_cols)
+            hipLaunchKernelGGL(moe_sort_small_cols_kernel, dim3(1 + qblocks), dim3(SMALL_THREADS), lds, stream, a, qa, x_cols);
+        else
+            hipLaunchKernelGGL((moe_sort_small_kernel<0, false>), dim3(1 + qblocks), dim3(SMALL_THREADS), lds, stream, a, qa, ra);
         PYHIP_CHECK_LAUNCH("moe_sort_small_kernel");
         return PYHIP_OK;
     }
     a.G = sort_groups(pairs);
     hipLaunchKernelGGL(moe_sort_hist_kernel, dim3(a.G), dim3(SORT_THREADS), (size_t)experts * 4, stream, a);
     PYHIP_CHECK_LAUNCH("moe_sort_hist_kernel");
-    hipLaunchKernelGGL(moe_sort_scan_kernel, dim3(1 + qblocks), dim3(SMALL_THREADS),
-                       ((size_t)3 * experts + 2 * SMALL_WAVES + 2) * 4, stream, a, qa);
+    const size_t scan_lds = ((size_t)3 * experts + 2 * SMALL_WAVES + 2) * 4;
+    if(x_cols)
+        hipLaunchKernelGGL(moe_sort_scan_cols_kernel, dim3(1 + qblocks), dim3(SMALL_THREADS), scan_lds, stream, a, qa, x_cols);
+    else
+        hipLaunchKernelGGL(moe_sort_scan_kernel, dim3(1 + qblocks), dim3(SMALL_THREADS), scan_lds, stream, a, qa);
     PYHIP_CHECK_LAUNCH("moe_sort_scan_kernel");
     hipLaunchKernelGGL(moe_sort_scatter_kernel, dim3(a.G), dim3(SORT_THREADS), (size_t)SORT_WAVES * experts * 4,
                        stream, a);
@@ -659,7 +691,7 @@ int pyhip_sorting_quant_cols(const int32_t* topk_ids, const float* topk_weights,
         return rc;
     return sorting_impl(topk_ids, topk_weights, tokens, topk, experts, block_size, expert_mask, num_local_tokens,
                         sorted_ids, sorted_weights, sorted_expert_ids, num_valid_ids, schedule, nullptr, 0, workspace,
-                        workspace_bytes, qa, RouteArgs{}, stream);
+                        workspace_bytes, qa, RouteArgs{}, stream, x_cols);
 }
 
 extern "C" int pyhip_moe_sorting_quant(const int32_t* topk_ids, const float* topk_weights, int tokens, int topk,

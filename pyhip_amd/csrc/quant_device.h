@@ -12,12 +12,14 @@ struct QuantArgs
     long long rows;            // 0: nothing to do
     int K, SK;
     const u32* rows_limit;     // device scalar or null
-    int x_cols;                // columns x has, a multiple of 32 (0: K); the rest up to K is quantised as the zeros it stands for
 };
+// callers with a launcher of their own pack this struct for the kernels of the code objects (co_module.py mirrors it)
+static_assert(sizeof(QuantArgs) == 56, "QuantArgs is part of the kernels' interface");
 
 // One thread per 32-element block (id = row * SK + block; blocks past K are padding); 16 consecutive threads own
 // one 16-byte scale group, so ids must be handed out in multiples of 16 per wave.
-__device__ __forceinline__ void act_quant_block(const QuantArgs& a, long long id)
+// x_cols: columns x has, a multiple of 32 (0: K); the rest up to K is quantised as the zeros it stands for.
+__device__ __forceinline__ void act_quant_block(const QuantArgs& a, long long id, int x_cols = 0)
 {
     long long rows = a.rows;
     if(a.rows_limit)
@@ -30,7 +32,7 @@ __device__ __forceinline__ void act_quant_block(const QuantArgs& a, long long id
     if(row >= rows)                                      // whole 16-thread groups leave together
         return;
     u32 e8 = 0;
-    if(a.x_cols && j * 32 >= a.x_cols)
+    if(x_cols && j * 32 >= x_cols)
     {
         if(j * 32 < a.K)
             *(uint4*)(a.q + row * (long long)(a.K / 2) + (long long)j * 16) = make_uint4(0, 0, 0, 0);
