@@ -105,17 +105,26 @@ def pick_w4a16(tokens, topk, experts, hidden):
     return bool(_lib.load().pyhip_moe_pick_w4a16(tokens, topk, experts, hidden))
 
 
-@functools.lru_cache(maxsize=512, typed=True)
 def _plan(tokens, topk, experts, hidden, inter, method, block_m):
     """(bf16 activations?, row block, workspace bytes) of a layer call: a function of its sizes and options alone, so a
     program's few call shapes ask the library once each instead of three times a call (``method`` and ``block_m`` as
-    given by the caller).  Small layers are bound by the host: with this, checks whose messages are put together only when they
-    fail, and raw stream and data pointers, the tiny layer at 64 tokens went from 29.1 to 22.7 us a call."""
+    given by the caller).  Only plain integers are remembered: whatever else converts to one may not be hashable (a numpy
+    array) or may change its value and stay the same key (a tensor is hashed by identity).
+    With this, checks whose messages are put together only when they fail, and raw stream and data pointers, the
+    tiny layer at 64 tokens went from 29.1 to 22.7 us a call."""
+    plain = type(topk) is int and (block_m is None or type(block_m) is int)
+    return (_remembered_plan if plain else _ask_plan)(tokens, topk, experts, hidden, inter, method, block_m)
+
+
+def _ask_plan(tokens, topk, experts, hidden, inter, method, block_m):
     w4a16 = method == "w4a16" or (method != "a4w4" and pick_w4a16(tokens, topk, experts, hidden))
     bm = block_m if block_m is not None else pick_block_m(tokens, topk, experts, hidden, w4a16)
     if w4a16:
         bm = min(bm, 64)
     return w4a16, bm, _lib.load().pyhip_moe_forward_workspace_bytes(tokens, topk, experts, hidden, inter, bm, 1 if w4a16 else 0)
+
+
+_remembered_plan = functools.lru_cache(maxsize=512)(_ask_plan)
 
 
 def act_quant_mxfp4(x, rows_limit=None):

@@ -1,6 +1,9 @@
 """CPU checks of the host side of a layer call: pointers, and what the remembered sizes accept."""
 import ctypes
+import sys
 
+import numpy as np
+import pytest
 import torch
 
 from pyhip_amd import _lib, co_module
@@ -17,3 +20,24 @@ def test_pointers_keep_all_their_bits_outside_declared_argtypes():
     same.restype = ctypes.c_void_p
     assert same(p, 0, 1) == x.data_ptr()
     assert _lib.dptr(None) is None and _lib.addr(None) is None and _lib.addr(x) == x.data_ptr()
+
+
+@pytest.mark.parametrize("method", ["a4w4", "w4a16", "auto"])
+def test_row_block_of_any_integer_type(method):
+    """a row block that converts to an integer is taken as one, and by its value at the time of the call"""
+    import pyhip_amd.fused_moe  # noqa: F401
+    plan = sys.modules["pyhip_amd.fused_moe"]._plan
+    sizes = (300, 2, 8, 1024, 512, method)
+    for bm in (16, 32, 64):
+        want = plan(*sizes, bm)
+        for v in (np.int64(bm), np.array(bm), torch.tensor(bm)):
+            got = plan(*sizes, v)
+            assert (got[0], int(got[1]), got[2]) == want
+    t = torch.tensor(16)
+    plan(*sizes, t)
+    t.fill_(64)
+    assert plan(*sizes, t)[2] == plan(*sizes, 64)[2]
+    assert plan(300, np.array(2), *sizes[2:], 16) == plan(*sizes, 16)
+    for v in (32.0, "32"):
+        with pytest.raises((TypeError, ctypes.ArgumentError)):
+            plan(*sizes, v)
