@@ -19,14 +19,15 @@ struct ReduceRouting
 // One wave per (token, 64 pieces of 16 bytes): everything about the routing is then the same for the whole wave.  Lanes
 // 0..7 fetch the ids of eight slots, one ballot says which of them count, and the loop over slots branches on scalar
 // bits, so a slot that was dropped costs neither a load nor an addition.  (One thread per piece that read its token's
-// ids and mask entries for itself issued sixteen loads, one after the other, for every eight of data: the bound at
-// decode sizes, where the kernel is a chain of latencies, and under expert parallelism, where most slots are dropped.)
-// Without an expert mask or a local token count nearly every slot counts: its data is fetched together with the ids
-// instead of after them (the rows exist in memory whether they were written or not; what a dropped one holds is
-// not looked at).
-// Bound: HBM at prefill sizes, latency at decode sizes.  Whole layer, before -> after: DeepSeek-V3 shape, one of eight expert-parallel
-// ranks, 4001 tokens 251.7 -> 239.0 us; Mixtral shape, 4096 tokens 777.5 -> 773.3 us, 1 token 39.05 -> 38.71 us; Qwen3 shape,
-// 64 tokens 104.3 -> 103.8 us; no difference at 8192 tokens of the DeepSeek-V3 shape (6.3 TB/s before).
+// ids and mask entries for itself issued sixteen loads, one after the other, for every eight of data.)
+// The ids always come before the data.  Fetching the data of every slot along with them saves a latency where nothing is
+// dropped, but a caller may drop slots by their ids alone, without a mask: an expert-parallel rank of eight then read
+// eight times what it needs.
+// Bound: HBM at prefill sizes, latency at decode sizes.  This kernel alone, us, the thread-per-piece kernel / data along with
+// the ids / ids first (k slots of H bf16):
+//   k = 8, H = 7168, 4001 tokens, one slot in eight kept: by ids 44.5 / 83.2 / 29.7, by a mask 53.7 / 29.4 / 30.3
+//   the same, all kept: 87.2 / 84.2 / 85.1; 8192 tokens 181.0 / 170.7 / 172.7 (6.1 TB/s); 16 tokens 4.4 / 4.4 / 4.3
+//   k = 2, H = 4096, all kept: 4001 tokens 21.4 / 18.2 / 19.7; 1024 tokens 8.0 / 6.7 / 7.4; 1 token 4.2 / 4.3 / 4.3
 template <bool OUT_F32, bool ROUTED>
 __global__ void __launch_bounds__(256)
     moe_topk_reduce_kernel(const uint4* __restrict__ in, void* __restrict__ out, long long T, int k, int H8,
@@ -45,8 +46,7 @@ __global__ void __launch_bounds__(256)
     const u32 step_t = step / chunks, step_c = step - step_t * chunks;
     long long t = first / chunks;
     u32 ch      = first - (u32)t * chunks;
-    const bool ask_first = ROUTED && (rt.expert_mask || rt.num_local_tok);
-    long long T_local    = T;
+    long long T_local = T;
     if(ROUTED && rt.num_local_tok)
     {
         const long long lim = (long long)*rt.num_local_tok;
@@ -62,18 +62,16 @@ __global__ void __launch_bounds__(256)
         {
             const int n = k - s0 < 8 ? k - s0 : 8;
             u32 on      = (1u << n) - 1u;           // slots that count, the same in every lane
-            int e       = -1;
-            if(ROUTED && lane < n && t < T_local)
-                e = rt.topk_ids[t * k + s0 + lane];
-            if(ROUTED && ask_first)
-                on = (u32)__ballot(moe_pair_is_kept(e, rt.experts, rt.expert_mask));
+            if(ROUTED)
+            {
+                const int e = lane < n && t < T_local ? rt.topk_ids[t * k + s0 + lane] : -1;
+                on          = (u32)__ballot(moe_pair_is_kept(e, rt.experts, rt.expert_mask));
+            }
             v4i v[8];
 #pragma unroll
             for(int j = 0; j < 8; j++)
                 if((on >> j) & 1u)
                     v[j] = __builtin_nontemporal_load((const v4i*)(p + (long long)(s0 + j) * H8));
-            if(ROUTED && !ask_first)
-                on = (u32)__ballot(moe_pair_is_kept(e, rt.experts, nullptr));
 #pragma unroll
             for(int j = 0; j < 8; j++)
             {
