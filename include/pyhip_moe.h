@@ -18,7 +18,8 @@ extern "C" {
 
 typedef void* pyhip_stream_t; /* hipStream_t */
 
-/* ABI revision of this header. */
+/* ABI revision of this header: raised when an entry point is added, taken away or changed, and when an argument struct
+ * of a shipped code object's kernels is.  10: pyhip_moe_forward_cols. */
 int pyhip_moe_abi_version(void);
 
 /* Message of the last failed call on this thread (replaces the Python exception text of

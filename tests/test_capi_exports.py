@@ -2,6 +2,7 @@
 include/pyhip_moe.h declares, the ctypes table covers exactly those symbols, and the argument
 checks reject bad input without touching a GPU."""
 import ctypes
+import hashlib
 import os
 import re
 
@@ -18,6 +19,13 @@ def _declared():
     return sorted(set(re.findall(r"\b(pyhip_moe_\w+)\s*\(", text)))
 
 
+def _prototypes_digest():
+    """of the header without its comments and its spacing: names and types of every entry point"""
+    text = open(os.path.join(ROOT, "include", "pyhip_moe.h")).read()
+    text = re.sub(r"/\*.*?\*/|//[^\n]*", "", text, flags=re.S)
+    return hashlib.sha256("".join(text.split()).encode()).hexdigest()[:16]
+
+
 def test_library_exports_every_declared_symbol():
     lib = _lib.load()
     names = _declared()
@@ -25,7 +33,8 @@ def test_library_exports_every_declared_symbol():
     for n in names:
         assert hasattr(lib, n), n
     assert sorted(_lib.SIGNATURES) == names
-    assert lib.pyhip_moe_abi_version() == 9
+    # an entry point added, taken away or changed raises the version
+    assert (lib.pyhip_moe_abi_version(), len(names), _prototypes_digest()) == (10, 34, "5673cd6383ed6c66")
 
 
 def test_size_helpers():
@@ -65,6 +74,33 @@ def test_argument_errors_are_reported():
     # the tile with both operands through LDS only exists with the sort's schedule
     rc = lib.pyhip_moe_gemm1_mxfp4_lds(one, one, one, one, None, one, one, one, None, one, None, None, 4, 2, 8, 1024, 1024, 4, 0, 0.0, None)
     assert rc == 1 and b"schedule missing" in lib.pyhip_moe_last_error()
+
+
+def test_true_width_arguments_are_checked():
+    """pyhip_moe_forward_cols: hidden_cols is 0 or exactly the true width, whole blocks of 32, MXFP4 activations only"""
+    lib = _lib.load()
+    p = ctypes.c_void_p(256)
+    T, k, E, H, inter, bm = 4, 2, 8, 1024, 512, 16
+
+    def call(cols, stride, pad, a16=0):
+        ws = lib.pyhip_moe_forward_workspace_bytes(T, k, E, H, inter, bm, a16)
+        rc = lib.pyhip_moe_forward_cols(p, stride, cols, p, p, p, p, None, None, p, p, None, None, p, 0, T, k, E, H, inter,
+                                        pad, 0, bm, a16, 0, 0, 0.0, p, ws, None)
+        return rc, lib.pyhip_moe_last_error()
+
+    for cols, stride, pad, a16 in ((960, 960, 96, 0), (960, 960, 0, 0), (1008, 1008, 16, 0), (928, 1024, 96, 1)):
+        rc, msg = call(cols, stride, pad, a16)
+        assert rc == 1 and b"hidden_cols" in msg, (cols, stride, pad, a16, msg)
+    rc, msg = call(928, 928, 96, 1)
+    assert rc == 1 and b"contiguous rows" in msg
+    rc, msg = call(-32, 1024, 1056)
+    assert rc == 1 and b"columns given" in msg
+    rc, msg = call(928, 920, 96)
+    assert rc == 1 and b"row stride" in msg
+    rc, msg = call(0, 928, 96)                          # rows at the padded width are longer than that
+    assert rc == 1 and b"row stride" in msg
+    rc, msg = call(928, 932, 96)                        # rows that do not start on 16 bytes
+    assert rc == 1 and b"row stride" in msg
 
 
 def test_missing_library_fails_loudly(monkeypatch):
