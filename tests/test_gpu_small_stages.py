@@ -132,3 +132,36 @@ def test_true_width_activations(T, form):
         got = fused_moe(x, w1, w2, tw, ti, method=method, **kw)
         wide = fused_moe(torch.nn.functional.pad(x, (0, hp)), w1, w2, tw, ti, method=method, **kw)
         assert got.shape == (T, H) and torch.equal(got, wide[:, :H])
+
+
+@pytest.mark.parametrize("T", [5, 65, 600])
+@pytest.mark.parametrize("option", ["mask", "many_experts", "local", "f32"])
+def test_true_width_activations_with_options(T, option):
+    """True-width rows of a padded layer under an expert mask (also over so many experts that the sort needs more than
+    64 KB of LDS), a local token count and fp32 output: the bits of the same call with the rows widened by the caller."""
+    import cases
+    from pyhip_amd import fused_moe
+    L = cases.make_layer("gptoss_s", T, seed=6, bias=True)
+    w1, w1s, w2, w2s, b1, b2, hp, ip = cases.padded_device_weights(L)
+    tw, ti = torch.from_numpy(L.topk_w).cuda(), torch.from_numpy(L.topk_ids).cuda()
+    x = L.hidden.cuda()
+    kw = dict(w1_scale=w1s, w2_scale=w2s, bias1=b1, bias2=b2, hidden_pad=hp, intermediate_pad=ip, method="a4w4")
+    if option in ("mask", "many_experts"):
+        # this rank's 16 experts among 48 or 1040: every third or sixty-fifth id
+        step = 3 if option == "mask" else 65
+        mask = torch.zeros(L.E * step, dtype=torch.int32)
+        mask[::step] = 1
+        kw["expert_mask"] = mask.cuda()
+        ti = ti * step
+        ti[:, 1] += 1                                  # a slot of experts that live elsewhere
+    elif option == "local":
+        kw["num_local_tokens"] = torch.tensor([T * 2 // 3], dtype=torch.int32, device="cuda")
+        x = x.clone()
+        x[T * 2 // 3:] = float("nan")                  # rows past the count are not looked at
+    else:
+        kw["dtype"] = torch.float32
+    print("true width", T, option, flush=True)
+    got = fused_moe(x, w1, w2, tw, ti, **kw)
+    wide = fused_moe(torch.nn.functional.pad(x, (0, hp)), w1, w2, tw, ti, **kw)
+    assert got.dtype == (torch.float32 if option == "f32" else torch.bfloat16) and torch.isfinite(got.float()).all()
+    assert got.shape == (T, L.H) and torch.equal(got, wide[:, :L.H]) and got.float().abs().sum() > 0
