@@ -20,14 +20,20 @@ struct ReduceRouting
 // 0..7 fetch the ids of eight slots, one ballot says which of them count, and the loop over slots branches on scalar
 // bits, so a slot that was dropped costs neither a load nor an addition.  (One thread per piece that read its token's
 // ids and mask entries for itself issued sixteen loads, one after the other, for every eight of data.)
-// The ids always come before the data.  Fetching the data of every slot along with them saves a latency where nothing is
-// dropped, but a caller may drop slots by their ids alone, without a mask: an expert-parallel rank of eight then read
-// eight times what it needs.
+// Without a mask or a local token count nearly every slot counts as a rule, and its data could be fetched along with the
+// ids (the rows exist in memory whether they were written or not; what a dropped one holds is not looked at).  But a
+// caller may drop slots by their ids alone, and an expert-parallel rank of eight that does then reads eight times what
+// it needs.  So only calls of up to ALONG_PIECES (4 MiB), where reading every slot takes less than asking first, do.
 // Bound: HBM at prefill sizes, latency at decode sizes.  This kernel alone, us, the thread-per-piece kernel / data along with
 // the ids / ids first (k slots of H bf16):
-//   k = 8, H = 7168, 4001 tokens, one slot in eight kept: by ids 44.5 / 83.2 / 29.7, by a mask 53.7 / 29.4 / 30.3
-//   the same, all kept: 87.2 / 84.2 / 85.1; 8192 tokens 181.0 / 170.7 / 172.7 (6.1 TB/s); 16 tokens 4.4 / 4.4 / 4.3
-//   k = 2, H = 4096, all kept: 4001 tokens 21.4 / 18.2 / 19.7; 1024 tokens 8.0 / 6.7 / 7.4; 1 token 4.2 / 4.3 / 4.3
+//   k = 8, H = 7168, 4001 tokens, one slot in eight kept: by ids 44.5 / 83.2 / 29.7, by a mask 53.7 / - / 30.3
+//     all kept: 87.2 / 84.2 / 85.1; 8192 tokens 181.0 / 170.7 / 172.7 (6.1 TB/s)
+//     32 tokens (3.5 MiB): all kept 4.27 / 3.87 / 3.87, one in eight 3.78 / 3.71 / 3.58
+//     64 tokens (7 MiB): all kept 4.57 / 4.18 / 4.18, one in eight 3.79 / 3.99 / 3.56
+//   k = 2, H = 4096, 256 tokens (4 MiB): all kept 3.97 / 3.84 / 4.28, half 3.72 / 3.78 / 3.98
+//     512 tokens: all kept 5.42 / 4.58 / 5.04; 4001 tokens 21.4 / 18.2 / 19.7
+// In the layer, where the ids come from memory rather than a cache, asking first costs decode sizes 0.1-0.35 us.
+#define ALONG_PIECES (1 << 18)
 template <bool OUT_F32, bool ROUTED>
 __global__ void __launch_bounds__(256)
     moe_topk_reduce_kernel(const uint4* __restrict__ in, void* __restrict__ out, long long T, int k, int H8,
@@ -46,7 +52,8 @@ __global__ void __launch_bounds__(256)
     const u32 step_t = step / chunks, step_c = step - step_t * chunks;
     long long t = first / chunks;
     u32 ch      = first - (u32)t * chunks;
-    long long T_local = T;
+    const bool ask_first = ROUTED && (rt.expert_mask || rt.num_local_tok || T * k * H8 > ALONG_PIECES);
+    long long T_local    = T;
     if(ROUTED && rt.num_local_tok)
     {
         const long long lim = (long long)*rt.num_local_tok;
@@ -62,16 +69,18 @@ __global__ void __launch_bounds__(256)
         {
             const int n = k - s0 < 8 ? k - s0 : 8;
             u32 on      = (1u << n) - 1u;           // slots that count, the same in every lane
-            if(ROUTED)
-            {
-                const int e = lane < n && t < T_local ? rt.topk_ids[t * k + s0 + lane] : -1;
-                on          = (u32)__ballot(moe_pair_is_kept(e, rt.experts, rt.expert_mask));
-            }
+            int e       = -1;
+            if(ROUTED && lane < n && t < T_local)
+                e = rt.topk_ids[t * k + s0 + lane];
+            if(ROUTED && ask_first)
+                on = (u32)__ballot(moe_pair_is_kept(e, rt.experts, rt.expert_mask));
             v4i v[8];
 #pragma unroll
             for(int j = 0; j < 8; j++)
                 if((on >> j) & 1u)
                     v[j] = __builtin_nontemporal_load((const v4i*)(p + (long long)(s0 + j) * H8));
+            if(ROUTED && !ask_first)
+                on = (u32)__ballot(moe_pair_is_kept(e, rt.experts, nullptr));
 #pragma unroll
             for(int j = 0; j < 8; j++)
             {
