@@ -325,11 +325,11 @@ int pyhip_moe_forward(const void* hidden_bf16, int64_t hidden_row_stride, const 
 /* The same with MXFP4 activations and hidden states [tokens, hidden_cols] at the layer's true width: hidden_cols = hidden -
  * hidden_pad, a multiple of 32 (0: the padded width, as above), hidden_row_stride >= hidden_cols and a multiple of 8. */
 int pyhip_moe_forward_cols(const void* hidden_bf16, int64_t hidden_row_stride, int hidden_cols, const uint8_t* w1, const uint8_t* w1_scale,
-                      const uint8_t* w2, const uint8_t* w2_scale, const void* bias1_bf16, const void* bias2_bf16,
-                      const int32_t* topk_ids, const float* topk_weights, const int32_t* expert_mask,
-                      const int32_t* num_local_tokens, void* out, int out_is_f32, int tokens, int topk, int experts,
-                      int hidden, int inter, int hidden_pad, int inter_pad, int block_m, int w4a16, int split_k,
-                      int activation, float swiglu_limit, void* workspace, int64_t workspace_bytes, pyhip_stream_t stream);
+                           const uint8_t* w2, const uint8_t* w2_scale, const void* bias1_bf16, const void* bias2_bf16,
+                           const int32_t* topk_ids, const float* topk_weights, const int32_t* expert_mask,
+                           const int32_t* num_local_tokens, void* out, int out_is_f32, int tokens, int topk, int experts,
+                           int hidden, int inter, int hidden_pad, int inter_pad, int block_m, int w4a16, int split_k,
+                           int activation, float swiglu_limit, void* workspace, int64_t workspace_bytes, pyhip_stream_t stream);
 
 /* pyhip_moe_forward with the router inside the call: gating f32 [tokens, experts] in (n_group / topk_group /
  * renormalize as for pyhip_moe_route_sorting), the picks out in topk_ids / topk_weights next to the layer output.

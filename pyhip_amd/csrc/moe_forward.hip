@@ -287,13 +287,13 @@ extern "C" int pyhip_moe_forward(const void* hidden_bf16, int64_t hidden_row_str
 // quantisation reads them as they are.  Widening them first was a launch and a pass over memory of its own in front of the
 // layer: gpt-oss shape (2880 of 3072 columns), before -> after, 16 tokens 126.3 -> 121.7 us, 4096 tokens 543.3 -> 524.7 us.
 extern "C" int pyhip_moe_forward_cols(const void* hidden_bf16, int64_t hidden_row_stride, int hidden_cols, const uint8_t* w1,
-                                 const uint8_t* w1_scale, const uint8_t* w2, const uint8_t* w2_scale,
-                                 const void* bias1_bf16, const void* bias2_bf16, const int32_t* topk_ids,
-                                 const float* topk_weights, const int32_t* expert_mask,
-                                 const int32_t* num_local_tokens, void* out, int out_is_f32, int tokens, int topk,
-                                 int experts, int hidden, int inter, int hidden_pad, int inter_pad, int block_m,
-                                 int w4a16, int split_k, int activation, float swiglu_limit, void* workspace,
-                                 int64_t workspace_bytes, hipStream_t stream)
+                                      const uint8_t* w1_scale, const uint8_t* w2, const uint8_t* w2_scale,
+                                      const void* bias1_bf16, const void* bias2_bf16, const int32_t* topk_ids,
+                                      const float* topk_weights, const int32_t* expert_mask,
+                                      const int32_t* num_local_tokens, void* out, int out_is_f32, int tokens, int topk,
+                                      int experts, int hidden, int inter, int hidden_pad, int inter_pad, int block_m,
+                                      int w4a16, int split_k, int activation, float swiglu_limit, void* workspace,
+                                      int64_t workspace_bytes, hipStream_t stream)
 {
     return forward_impl(hidden_bf16, hidden_row_stride, hidden_cols, w1, w1_scale, w2, w2_scale, bias1_bf16, bias2_bf16, Router{},
                         const_cast<int32_t*>(topk_ids), const_cast<float*>(topk_weights), expert_mask, num_local_tokens,

@@ -211,8 +211,9 @@ def fused_moe(
     _require(w1u.dim() == 3 and w2u.dim() == 3, "w1 [E, 2*inter, hidden/2] and w2 [E, hidden, inter/2] expected")
     # hidden_pad / intermediate_pad: the weights arrive zero-padded to the kernels' tile multiples and the last
     # hidden_pad (intermediate_pad) channels are padding.  The activations may come at the padded width (the
-    # reference's convention) or at the true width, in which case they are widened here and the result is
-    # returned at the true width.  The MXFP4-activation GEMMs are told the pads and leave the weights' padding unfetched.
+    # reference's convention) or at the true width, in which case the result is returned at the true width too; the input
+    # quantisation then fills in the padding's zeros, or the rows are widened first where it cannot take them (below).
+    # The MXFP4-activation GEMMs are told the pads and leave the weights' padding unfetched.
     _require(0 <= hidden_pad < w1u.shape[2] * 2 and 0 <= intermediate_pad < w1u.shape[1] // 2, "bad hidden_pad / intermediate_pad")
     narrow = hidden_pad > 0 and hidden_states.shape[1] == w1u.shape[2] * 2 - hidden_pad
     T, H = hidden_states.shape[0], w1u.shape[2] * 2 if narrow else hidden_states.shape[1]
@@ -294,11 +295,11 @@ def fused_moe(
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         out = torch.empty(T, H, dtype=out_dtype, device=dev)
         rc = lib.pyhip_moe_forward_cols(_lib.addr(x), x.stride(0), cols, _lib.addr(w1u), _lib.addr(w1s), _lib.addr(w2u),
-                                   _lib.addr(w2s), _lib.addr(bias1), _lib.addr(bias2), _lib.addr(topk_ids),
-                                   _lib.addr(topk_weight), _lib.addr(expert_mask), _lib.addr(num_local_tokens),
-                                   _lib.addr(out), 1 if out_dtype == torch.float32 else 0, T, k, global_E, H, I,
-                                   hidden_pad, intermediate_pad, bm, 1 if w4a16 else 0, splitk, act, limit,
-                                   _lib.addr(ws), ws_bytes, _lib.stream_handle())
+                                        _lib.addr(w2s), _lib.addr(bias1), _lib.addr(bias2), _lib.addr(topk_ids),
+                                        _lib.addr(topk_weight), _lib.addr(expert_mask), _lib.addr(num_local_tokens),
+                                        _lib.addr(out), 1 if out_dtype == torch.float32 else 0, T, k, global_E, H, I,
+                                        hidden_pad, intermediate_pad, bm, 1 if w4a16 else 0, splitk, act, limit,
+                                        _lib.addr(ws), ws_bytes, _lib.stream_handle())
         _lib.check(rc, "moe_forward")
         return out[:, : H - hidden_pad] if narrow else out
 
