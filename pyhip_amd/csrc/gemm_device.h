@@ -227,21 +227,23 @@ __device__ __forceinline__ void vm_load_b32(int& dst, int voff, v4i rsrc, int so
 // which neither tracks nor preserves it around inline assembly (it says so when asked to).  These helpers are sound
 // as long as the compiler's own code never uses M0 in these kernels (on gfx9 LDS instructions do not need it);
 // tests/test_build_checks.py checks on the generated code that nothing outside the inline assembly names M0.
-template <int IMM, int LDS_IMM, bool NT = false>
+// (WS: wait states beyond the one that M0 needs, for kernels whose descriptors the compiler reads back from vector registers
+// right before: the hazard that vm_dma_b32_fresh_sgprs describes)
+template <int IMM, int LDS_IMM, bool NT = false, int WS = 0>
 __device__ __forceinline__ void vm_dma_b128(int voff, v4i rsrc, int soff, u32 lds_base)
 {
     if(NT)      // streamed once: the line is the first to go when the L2 needs room
-        asm volatile("s_add_u32 m0, %3, %5\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen offset:%4 nt lds"
-                     ::"v"(voff), "s"(rsrc), "s"(soff), "s"(lds_base), "n"(IMM), "n"(LDS_IMM - IMM) : "memory", "scc");
+        asm volatile("s_add_u32 m0, %3, %5\n\ts_nop %6\n\tbuffer_load_dwordx4 %0, %1, %2 offen offset:%4 nt lds"
+                     ::"v"(voff), "s"(rsrc), "s"(soff), "s"(lds_base), "n"(IMM), "n"(LDS_IMM - IMM), "n"(WS) : "memory", "scc");
     else
-        asm volatile("s_add_u32 m0, %3, %5\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen offset:%4 lds"
-                     ::"v"(voff), "s"(rsrc), "s"(soff), "s"(lds_base), "n"(IMM), "n"(LDS_IMM - IMM) : "memory", "scc");
+        asm volatile("s_add_u32 m0, %3, %5\n\ts_nop %6\n\tbuffer_load_dwordx4 %0, %1, %2 offen offset:%4 lds"
+                     ::"v"(voff), "s"(rsrc), "s"(soff), "s"(lds_base), "n"(IMM), "n"(LDS_IMM - IMM), "n"(WS) : "memory", "scc");
 }
-template <int IMM, int LDS_IMM>
+template <int IMM, int LDS_IMM, int WS = 0>
 __device__ __forceinline__ void vm_dma_b32(int voff, v4i rsrc, int soff, u32 lds_base)
 {
-    asm volatile("s_add_u32 m0, %3, %5\n\ts_nop 0\n\tbuffer_load_dword %0, %1, %2 offen offset:%4 lds"
-                 ::"v"(voff), "s"(rsrc), "s"(soff), "s"(lds_base), "n"(IMM), "n"(LDS_IMM - IMM) : "memory", "scc");
+    asm volatile("s_add_u32 m0, %3, %5\n\ts_nop %6\n\tbuffer_load_dword %0, %1, %2 offen offset:%4 lds"
+                 ::"v"(voff), "s"(rsrc), "s"(soff), "s"(lds_base), "n"(IMM), "n"(LDS_IMM - IMM), "n"(WS) : "memory", "scc");
 }
 // The same for descriptors that were just made uniform with v_readfirstlane: a vector-memory instruction must not
 // read a scalar register earlier than 5 wait states after a vector instruction wrote it, and the compiler does
@@ -250,6 +252,14 @@ __device__ __forceinline__ void vm_dma_b32_fresh_sgprs(int voff, v4i rsrc, u32 l
 {
     asm volatile("s_nop 4\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds"
                  ::"v"(voff), "s"(rsrc), "s"(lds_base) : "memory");
+}
+// ... by lanes 0..31 only (the other lanes write nothing): 128 bytes at lds_base
+__device__ __forceinline__ void vm_dma_b32_low_half(int voff, v4i rsrc, u32 lds_base)
+{
+    u64 saved;
+    asm volatile("s_mov_b64 %0, exec\n\ts_mov_b32 exec_hi, 0\n\ts_mov_b32 m0, %3\n\ts_nop 4\n\t"
+                 "buffer_load_dword %1, %2, 0 offen lds\n\ts_mov_b64 exec, %0"
+                 : "=&s"(saved) : "v"(voff), "s"(rsrc), "s"(lds_base) : "memory");
 }
 __device__ __forceinline__ u32 lds_addr_of(const void* p)
 {
@@ -288,6 +298,14 @@ __device__ __forceinline__ void transpose4x4_rows(u32 (&x)[4])
     t = __builtin_amdgcn_permlane16_swap(x[2], x[3], false, false); x[2] = t.x; x[3] = t.y;
 }
 
+// the lane number, computed where it stands: what is derived from it is not kept in a register across the K loop
+__device__ __forceinline__ int fresh_lane()
+{
+    int zero = 0;
+    asm volatile("" : "+s"(zero));
+    return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
+}
+
 struct TileId
 {
     int m_blk, nt, e;   // row block, weight tile, (local) expert; all wave-uniform
@@ -306,8 +324,8 @@ __device__ __forceinline__ void gemm_zero_acc(v4f* xacc = nullptr)
         for(int i = 0; i < (16 * MT - 256) / 4; i++)
             xacc[i] = (v4f){0.f, 0.f, 0.f, 0.f};
 }
-// the four accumulators of row group MTI, plus bias when the instance has one (bias4(j) = the address of the lane's
-// four bf16 biases of weight row group j; re-read per row group to keep the epilogue's register need small)
+// the four accumulators of row group MTI, plus bias when the instance has one (bias4(j) = the lane's four bf16 biases of
+// weight row group j)
 template <int MT, int MTI, bool BIAS, typename B>
 __device__ __forceinline__ void gemm_fetch_row(v4f (&row)[4], B bias4, const v4f* xacc)
 {
@@ -319,7 +337,7 @@ __device__ __forceinline__ void gemm_fetch_row(v4f (&row)[4], B bias4, const v4f
             row[j] = (v4f){acc_fixed_read<a0>(), acc_fixed_read<a0 + 1>(), acc_fixed_read<a0 + 2>(), acc_fixed_read<a0 + 3>()};
         if constexpr(BIAS)
         {
-            const uint2 b = *(const uint2*)bias4(j);
+            const uint2 b = bias4(j);
             row[j][0] += bf16_bits_to_f32((uint16_t)b.x);
             row[j][1] += bf16_bits_to_f32((uint16_t)(b.x >> 16));
             row[j][2] += bf16_bits_to_f32((uint16_t)b.y);
@@ -327,20 +345,32 @@ __device__ __forceinline__ void gemm_fetch_row(v4f (&row)[4], B bias4, const v4f
         }
     });
 }
-// e, nt: (local) expert and weight tile; row0: sorted position of the wave's first row; wcol: which 64 (stage 1: 32 + 32)
+// nt: weight tile; row0: sorted position of the wave's first row; wcol: which 64 (stage 1: 32 + 32)
 // of the tile's weight rows the wave owns; meta: the sorted ids of the wave's rows, their routing weights mpad words
 // further; ma: how many of the wave's row groups hold real rows (a prefix; may be <= 0).  BIAS: the layer has biases
-// (the kernel branches once per tile between the two instances).
+// (the kernel branches once per tile between the two instances); bias4(j): the lane's four bf16 biases (kb * 4 .. + 3) of the
+// wave's weight row group j, asked for once per tile by the tall tiles and once per row group by the others.
 //
 // With one wave per SIMD (the tiles above 128 rows) nothing else runs while a wave is in its epilogue, so the row groups
 // are taken two at a time and everything up to the stores is one stretch of code without branches: the second group's
 // accumulator reads, conversions and lane exchanges fill the latencies of the first one's (the transcendental pipeline,
 // the exchanges).  The tiles up to 128 rows have two or more waves per SIMD for that, and no registers for a second group.
-template <int STAGE, int MT, int ACT, bool ATOMIC, bool BIAS>
-__device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, int e, int nt, int row0, int wcol, const u32* meta, int mpad,
-                                              int ma, int r, int kb, const v4f* xacc = nullptr)
+template <int STAGE, int MT, int ACT, bool ATOMIC, bool BIAS, typename B>
+__device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, int nt, int row0, int wcol, const u32* meta, int mpad,
+                                              int ma, int r, int kb, B bias4, const v4f* xacc = nullptr)
 {
     constexpr int PAIR = MT > 8 ? 2 : 1;
+    uint2 bz4[4];
+    if constexpr(BIAS && PAIR == 2)
+#pragma unroll
+        for(int j = 0; j < 4; j++)
+            bz4[j] = bias4(j);
+    auto bz = [&](int j) __attribute__((always_inline)) -> uint2 {
+        if constexpr(BIAS && PAIR == 2)
+            return bz4[j];
+        else
+            return bias4(j);
+    };
     const int I = g.N / 2;   // stage 1 only
     if(STAGE == 1)
     {
@@ -349,9 +379,6 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, int e, int nt, 
         typedef unsigned v2u __attribute__((ext_vector_type(2)));
         uint16_t* out = (uint16_t*)g.out;
         const int chw = nt * 128 + wcol * 32;
-        auto bz = [&](int j) __attribute__((always_inline)) {
-            return g.bias + (size_t)e * g.N + (j >> 1) * I + chw + (j & 1) * 16 + kb * 4;
-        };
         // after the swap: lane rows 0..3 hold channel offsets 0, 16, 8, 24
         const int ch_out = chw + (kb & 1) * 16 + (kb >> 1) * 8;
         const int blk = nt * 4 + wcol, jb = blk & 15;              // scale byte: see moe_quant.hip
@@ -430,7 +457,6 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, int e, int nt, 
         // four lane rows gives every lane 16 consecutive channels: 32 B stores, 128 B contiguous per row.
         uint16_t* out = (uint16_t*)g.out;
         const int chw = nt * 256 + wcol * 64;
-        auto bz = [&](int j) __attribute__((always_inline)) { return g.bias + (size_t)e * g.N + chw + j * 16 + kb * 4; };
         const int lane_col  = chw + kb * 16;
         const u32 row_bytes = (u32)g.N * 2u;
         static_for<(MT + PAIR - 1) / PAIR>([&](auto GI) __attribute__((always_inline)) {
@@ -482,7 +508,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, int e, int nt, 
                 {
                     // (plain stores: marked non-temporal they cost the down GEMM 5 % and the reduction, which then finds
                     // nothing of out3 in the last-level cache, another 4 %)
-                    const u32 orow = tok * (u32)g.topk + slot;              // row of out3 [tokens * topk, N]
+                    const u32 orow = __umul24(tok, (u32)g.topk) + slot;     // row of out3 [tokens * topk, N]
                     uint4* dst = (uint4*)((unsigned long long)(out + lane_col) + (unsigned long long)orow * row_bytes);
                     dst[0]     = make_uint4(lo[q][0], hi[q][0], lo[q][1], hi[q][1]);
                     dst[1]     = make_uint4(lo[q][2], hi[q][2], lo[q][3], hi[q][3]);

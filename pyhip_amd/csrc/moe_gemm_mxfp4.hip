@@ -83,6 +83,7 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
     constexpr int SCHED_E = TALL ? 0 : MT == 1 ? SCHED_E_MAX_16 : SCHED_E_MAX;
     __shared__ u32 lds_pre[SCHED_E + 1];      // the schedule: row blocks before every expert (and their total),
     __shared__ u32 lds_lid[SCHED_E + 1];      //   local id of every expert
+    __shared__ __attribute__((aligned(16))) u32 lds_bias[4][32];   // the tile's biases, 64 bf16 per wave
     __shared__ u32 lds_tab[TALL ? 1 : 128];   // the workgroup's next 64 tiles, decoded (the 288-row tile keeps them in registers)
 
     const int tid  = threadIdx.x;
@@ -265,26 +266,36 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
         const int n   = __builtin_popcountll(__ballot(ok));
         return n < 1 ? 1 : n;
     };
+    // The arguments again, from the kernel's argument segment: what only a tile's boundary needs (output pointers, biases, sizes)
+    // is loaded there, instead of living in scalar registers across the K loop, which has none to spare: the descriptors
+    // of the pipeline alone take 24, and what does not fit is parked in vector registers and read back a lane at a time.
+    auto args_again = [&]() __attribute__((always_inline)) -> const GemmArgs* {
+        unsigned long long p = (unsigned long long)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(p));              // (opaque: the loads stay where they are written)
+        return (const GemmArgs*)(const __attribute__((address_space(4))) GemmArgs*)p;
+    };
+
     // ids: the tile's sorted ids, either in LDS (meta buffer) or in global memory
     auto setup_load = [&](const TileId& t, const u32* ids) __attribute__((always_inline)) {
-        const size_t sc_tile = (size_t)(g.SC / 8) * 256;           // bytes of one 32-row scale tile
+        const GemmArgs& ga   = *args_again();
+        const size_t sc_tile = (size_t)(ga.SC / 8) * 256;          // bytes of one 32-row scale tile
         if(STAGE == 1)
         {
 #pragma unroll
             for(int h = 0; h < 2; h++)
             {
-                const size_t row = (size_t)t.e * g.N + h * I + t.nt * 128 + wave * 32;
-                const bool real  = t.nt * 128 + wave * 32 < I - g.n_pad;       // (rows of padding: nothing to fetch)
-                wrs[h]           = make_rsrc(g.w + row * Kb, real ? (u32)(32 * Kb) : 0u);
-                wsrs[h]          = make_rsrc(g.w_s + (row / 32) * sc_tile, real ? (u32)sc_tile : 0u);
+                const size_t row = (size_t)t.e * ga.N + h * I + t.nt * 128 + wave * 32;
+                const bool real  = t.nt * 128 + wave * 32 < I - ga.n_pad;       // (rows of padding: nothing to fetch)
+                wrs[h]           = make_rsrc(ga.w + row * Kb, real ? (u32)(32 * Kb) : 0u);
+                wsrs[h]          = make_rsrc(ga.w_s + (row / 32) * sc_tile, real ? (u32)sc_tile : 0u);
             }
         }
         else
         {
-            const size_t row = (size_t)t.e * g.N + t.nt * 256 + wave * 64;
-            const bool real  = t.nt * 256 + wave * 64 < g.N - g.n_pad;
-            wrs[0] = wrs[1] = make_rsrc(g.w + row * Kb, real ? (u32)(64 * Kb) : 0u);
-            wsrs[0] = wsrs[1] = make_rsrc(g.w_s + (row / 32) * sc_tile, real ? (u32)(2 * sc_tile) : 0u);
+            const size_t row = (size_t)t.e * ga.N + t.nt * 256 + wave * 64;
+            const bool real  = t.nt * 256 + wave * 64 < ga.N - ga.n_pad;
+            wrs[0] = wrs[1] = make_rsrc(ga.w + row * Kb, real ? (u32)(64 * Kb) : 0u);
+            wsrs[0] = wsrs[1] = make_rsrc(ga.w_s + (row / 32) * sc_tile, real ? (u32)(2 * sc_tile) : 0u);
         }
         // (all the reads first, from a clamped position and without a branch between them: one LDS round trip instead of
         // one per slot)
@@ -353,14 +364,49 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
     // accumulators and epilogue: gemm_device.h
     v4f xacc[TALL ? MT - ACC_SPILL_MT0 : 1];      // the accumulator tiles beyond the accumulation registers (288-row tile)
     auto zero_acc = [&]() __attribute__((always_inline)) { gemm_zero_acc<MT>(xacc); };
+    // Biases: each wave brings the 64 bf16 of its weight rows (stage 1: 32 gate, then 32 up) to its own 128 bytes of LDS, by
+    // DMA in the tile's first K-group, ahead of the schedule like the sorted ids, so the waits of that K-group cover it.
+    // (Read from global memory in the epilogue, every row group waited for a round trip, and the first one for all of
+    // the next tile's prefetches: vector-memory operations complete in order.  gpt-oss shape, 4096 tokens, 160-row tile, clocks
+    // of an epilogue, before -> after: gate_up 19950 -> 10170, down 15250 -> 5850.)
+    auto bias_row  = [&](const TileId& t) __attribute__((always_inline)) -> int { return STAGE == 1 ? t.nt * 128 + wave * 32 : t.nt * 256 + wave * 64; };
+    auto bias_lane = [&](int c, int N) __attribute__((always_inline)) -> int { return STAGE == 1 && c >= 32 ? N / 2 + c - 32 : c; };
+    auto fetch_bias = [&](const TileId& t) __attribute__((always_inline)) {
+        const GemmArgs& ga = *args_again();
+        if(ga.bias && ((unsigned long long)ga.bias & 3) == 0)
+            vm_dma_b32_low_half(bias_lane((fresh_lane() & 31) * 2, ga.N) * 2,
+                                uni4(make_rsrc(ga.bias + (size_t)t.e * ga.N + bias_row(t), (u32)ga.N * 2)), uni(lds_addr_of(lds_bias[wave])));
+    };
     // free_lds: the LDS stage that the tile's last K-group has just finished reading (stage 3 keeps a list there)
     auto epilogue = [&](const TileId& t, const u32* meta, int ma_t, uint8_t* free_lds) __attribute__((always_inline)) {
-        if(g.bias)
-            gemm_epilogue<STAGE, MT, ACT, ATOMIC, true>(g, t.e, t.nt, t.m_blk * BM, wave, meta, MPAD, ma_t, r, kb, xacc);
-        else
-            gemm_epilogue<STAGE, MT, ACT, ATOMIC, false>(g, t.e, t.nt, t.m_blk * BM, wave, meta, MPAD, ma_t, r, kb, xacc);
         if constexpr(STAGE == 3)
+        {
+            // (an option that was built to be measured: its registers are spoken for, the biases come from global memory)
+            auto bias4 = [&](int j) __attribute__((always_inline)) -> uint2 {
+                return *(const uint2*)(g.bias + (size_t)t.e * g.N + bias_row(t) + j * 16 + kb * 4);
+            };
+            if(g.bias)
+                gemm_epilogue<STAGE, MT, ACT, ATOMIC, true>(g, t.nt, t.m_blk * BM, wave, meta, MPAD, ma_t, r, kb, bias4, xacc);
+            else
+                gemm_epilogue<STAGE, MT, ACT, ATOMIC, false>(g, t.nt, t.m_blk * BM, wave, meta, MPAD, ma_t, r, kb, bias4, xacc);
             gemm_arrive_reduce<MT>(g, t.nt, meta, ma_t, (u32*)free_lds);
+        }
+        else
+        {
+            auto bias4 = [&](int j) __attribute__((always_inline)) -> uint2 { return *(const uint2*)&lds_bias[wave][j * 8 + kb * 2]; };
+            const GemmArgs& ga = *args_again();
+            if(ga.bias)
+            {
+                if((unsigned long long)ga.bias & 3)      // (only element-aligned: fetch_bias left them to ordinary loads)
+                {
+                    const int c = fresh_lane();
+                    ((uint16_t*)lds_bias[wave])[c] = ga.bias[(size_t)t.e * ga.N + bias_row(t) + bias_lane(c, ga.N)];
+                }
+                gemm_epilogue<STAGE, MT, ACT, ATOMIC, true>(ga, t.nt, t.m_blk * BM, wave, meta, MPAD, ma_t, r, kb, bias4, xacc);
+            }
+            else
+                gemm_epilogue<STAGE, MT, ACT, ATOMIC, false>(ga, t.nt, t.m_blk * BM, wave, meta, MPAD, ma_t, r, kb, bias4, xacc);
+        }
     };
 
     // ---------------------------------------------------------------- pipeline
@@ -377,6 +423,7 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
     // at 128 rows: gpt-oss shape, 4096 tokens, layer 0.573 against 0.597 ms; Mixtral shape, 512 tokens, 0.216 against
     // 0.224 ms).
     constexpr bool SPREAD = MT > 8;
+    constexpr int WS = STAGE == 3 ? 4 : 0;        // see vm_dma_b128
     // the last GUARDED row groups of a tall tile are jumped over when they hold no real rows (mfma_row_group_guarded)
     constexpr int GUARDED = MT == 18 ? 2 : MT > 8 ? 3 : 0;
     using VS = VmSchedule<MA, NPF, SPREAD ? 2 : 1>;
@@ -409,10 +456,10 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
             if constexpr(sub < 4)
             {
                 constexpr int imm = (sub * SLOTS + 4 * i) * 1024;
-                vm_dma_b128<sub * 64, imm>(a_off[i], ars, kpre * 256, slot_base(II{}, std::integral_constant<int, imm>{}, lds_a[ts]));
+                vm_dma_b128<sub * 64, imm, false, WS>(a_off[i], ars, kpre * 256, slot_base(II{}, std::integral_constant<int, imm>{}, lds_a[ts]));
             }
             else
-                vm_dma_b32<0, 4 * i * 256>(as_off[i], asrs, kpre * 16, slot_base(II{}, std::integral_constant<int, 4 * i * 256>{}, lds_s[ts]));
+                vm_dma_b32<0, 4 * i * 256, WS>(as_off[i], asrs, kpre * 16, slot_base(II{}, std::integral_constant<int, 4 * i * 256>{}, lds_s[ts]));
         }
         else
         {
@@ -487,6 +534,8 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
         // finished before the barrier that ends this tile's first K-group: the fetch waits for the second K-group)
         if(ks == (TALL ? 1 : 0) && nxt.valid)
             dma_meta(nxt, mb_nxt);
+        if(STAGE != 3 && ks == 0)
+            fetch_bias(cur);
         using TS = std::integral_constant<int, p ^ 1>;
         // The activation operand of a row group and its scale dword (one per 16-row group and K-group, op_sel picks the
         // K-step's byte) are read RA row groups ahead of the MFMAs that consume them, across K-step boundaries, through

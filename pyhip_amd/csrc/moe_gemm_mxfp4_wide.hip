@@ -254,12 +254,17 @@ __global__ void __launch_bounds__(WIDE_THREADS) moe_gemm_mxfp4_wide_kernel(GemmA
     // accumulators and epilogue: gemm_device.h (a wave's rows start wr * 128 rows into the tile)
     auto zero_acc = [&]() __attribute__((always_inline)) { gemm_zero_acc<MT>(); };
     auto epilogue = [&](const TileId& t, const u32* meta, int ma_t) __attribute__((always_inline)) {
+        // (biases from global memory: this tile has neither the LDS nor the registers for a copy)
+        auto bias4 = [&](int j) __attribute__((always_inline)) -> uint2 {
+            const int row = STAGE == 1 ? (j >> 1) * (g.N / 2) + t.nt * 128 + wc * 32 + (j & 1) * 16 : t.nt * 256 + wc * 64 + j * 16;
+            return *(const uint2*)(g.bias + (size_t)t.e * g.N + row + kb * 4);
+        };
         if(g.bias)
-            gemm_epilogue<STAGE, MT, ACT, false, true>(g, t.e, t.nt, t.m_blk * BM + wr * MT * 16, wc, meta + wr * MT * 16, MPAD,
-                                                        ma_t - wr * MT, r, kb);
+            gemm_epilogue<STAGE, MT, ACT, false, true>(g, t.nt, t.m_blk * BM + wr * MT * 16, wc, meta + wr * MT * 16, MPAD,
+                                                        ma_t - wr * MT, r, kb, bias4);
         else
-            gemm_epilogue<STAGE, MT, ACT, false, false>(g, t.e, t.nt, t.m_blk * BM + wr * MT * 16, wc, meta + wr * MT * 16, MPAD,
-                                                         ma_t - wr * MT, r, kb);
+            gemm_epilogue<STAGE, MT, ACT, false, false>(g, t.nt, t.m_blk * BM + wr * MT * 16, wc, meta + wr * MT * 16, MPAD,
+                                                         ma_t - wr * MT, r, kb, bias4);
     };
 
     // ---------------------------------------------------------------- pipeline
