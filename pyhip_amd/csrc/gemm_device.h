@@ -208,18 +208,27 @@ __device__ __forceinline__ v4i make_rsrc(const void* p, u32 bytes)
     return (v4i){(int)(u32)a, (int)((a >> 32) & 0xFFFFu), (int)bytes, 0x00020000};
 }
 // address = rsrc.base + voff + soff + IMM (IMM < 4096); only voff + IMM is range-checked
-template <int IMM = 0, bool NT = false>
+// (WS: wait states ahead of the operation, for kernels whose descriptors the compiler reads back from vector registers right
+// before it: the hazard that vm_dma_b32_fresh_sgprs describes)
+template <int IMM = 0, bool NT = false, int WS = 0>
 __device__ __forceinline__ void vm_load_b128(v4i& dst, int voff, v4i rsrc, int soff)
 {
-    if(NT)      // streamed once: the line is the first to go when the L2 needs room
+    if constexpr(WS > 0 && NT)
+        asm volatile("s_nop %5\n\tbuffer_load_dwordx4 %0, %1, %2, %3 offen offset:%4 nt" : "=v"(dst) : "v"(voff), "s"(rsrc), "s"(soff), "n"(IMM), "n"(WS) : "memory");
+    else if constexpr(WS > 0)
+        asm volatile("s_nop %5\n\tbuffer_load_dwordx4 %0, %1, %2, %3 offen offset:%4" : "=v"(dst) : "v"(voff), "s"(rsrc), "s"(soff), "n"(IMM), "n"(WS) : "memory");
+    else if(NT)      // streamed once: the line is the first to go when the L2 needs room
         asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen offset:%4 nt" : "=v"(dst) : "v"(voff), "s"(rsrc), "s"(soff), "n"(IMM) : "memory");
     else
         asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen offset:%4" : "=v"(dst) : "v"(voff), "s"(rsrc), "s"(soff), "n"(IMM) : "memory");
 }
-template <int IMM = 0>
+template <int IMM = 0, int WS = 0>
 __device__ __forceinline__ void vm_load_b32(int& dst, int voff, v4i rsrc, int soff)
 {
-    asm volatile("buffer_load_dword %0, %1, %2, %3 offen offset:%4" : "=v"(dst) : "v"(voff), "s"(rsrc), "s"(soff), "n"(IMM) : "memory");
+    if constexpr(WS > 0)
+        asm volatile("s_nop %5\n\tbuffer_load_dword %0, %1, %2, %3 offen offset:%4" : "=v"(dst) : "v"(voff), "s"(rsrc), "s"(soff), "n"(IMM), "n"(WS) : "memory");
+    else
+        asm volatile("buffer_load_dword %0, %1, %2, %3 offen offset:%4" : "=v"(dst) : "v"(voff), "s"(rsrc), "s"(soff), "n"(IMM) : "memory");
 }
 // global -> LDS without passing through registers: lane i's bytes land at lds_base + LDS_IMM + i * size.
 // (The hardware adds the instruction's immediate offset to the LDS address as well as to the global one, so
@@ -227,8 +236,7 @@ __device__ __forceinline__ void vm_load_b32(int& dst, int voff, v4i rsrc, int so
 // which neither tracks nor preserves it around inline assembly (it says so when asked to).  These helpers are sound
 // as long as the compiler's own code never uses M0 in these kernels (on gfx9 LDS instructions do not need it);
 // tests/test_build_checks.py checks on the generated code that nothing outside the inline assembly names M0.
-// (WS: wait states beyond the one that M0 needs, for kernels whose descriptors the compiler reads back from vector registers
-// right before: the hazard that vm_dma_b32_fresh_sgprs describes)
+// (WS: as above, beyond the one wait state that M0 needs)
 template <int IMM, int LDS_IMM, bool NT = false, int WS = 0>
 __device__ __forceinline__ void vm_dma_b128(int voff, v4i rsrc, int soff, u32 lds_base)
 {
@@ -282,20 +290,6 @@ __device__ __forceinline__ void wait_vmcnt_barrier()
 {
     // own DMA writes complete (all but the N youngest VMEM ops), own LDS reads complete, then meet
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
-}
-
-// 4x4 transpose of dwords across the four 16-lane rows of a wave: in: x[j] of lane row kb;
-// out: x[c] of lane row q holds what x[q] of lane row c held.  (permlane32_swap exchanges lanes
-// 32..63 of its first operand with lanes 0..31 of its second; permlane16_swap exchanges the odd
-// 16-lane rows of its first operand with the even rows of its second.)
-__device__ __forceinline__ void transpose4x4_rows(u32 (&x)[4])
-{
-    typedef unsigned v2u __attribute__((ext_vector_type(2)));
-    v2u t;
-    t = __builtin_amdgcn_permlane32_swap(x[0], x[2], false, false); x[0] = t.x; x[2] = t.y;
-    t = __builtin_amdgcn_permlane32_swap(x[1], x[3], false, false); x[1] = t.x; x[3] = t.y;
-    t = __builtin_amdgcn_permlane16_swap(x[0], x[1], false, false); x[0] = t.x; x[1] = t.y;
-    t = __builtin_amdgcn_permlane16_swap(x[2], x[3], false, false); x[2] = t.x; x[3] = t.y;
 }
 
 // the lane number, computed where it stands: what is derived from it is not kept in a register across the K loop
@@ -372,6 +366,31 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, int nt, int row
             return bias4(j);
     };
     const int I = g.N / 2;   // stage 1 only
+    // sorted ids (and, for the down GEMM, routing weights) of the rows of the pair at row group m0; the tall tiles read the next
+    // pair's from LDS along with them
+    u32 ids_ahead[PAIR], rws_ahead[PAIR];
+    auto read_ids = [&](int m0) __attribute__((always_inline)) {
+#pragma unroll
+        for(int q = 0; q < PAIR; q++)
+        {
+            const int m  = m0 + q < MT ? m0 + q : MT - 1;
+            ids_ahead[q] = meta[m * 16 + r];
+            if constexpr(STAGE != 1)
+                rws_ahead[q] = meta[mpad + m * 16 + r];
+        }
+    };
+    auto take_ids = [&](int m0, u32 (&ids)[PAIR], u32 (&rws)[PAIR]) __attribute__((always_inline)) {
+        if(PAIR == 1 || m0 == 0)
+            read_ids(m0);
+#pragma unroll
+        for(int q = 0; q < PAIR; q++)
+        {
+            ids[q] = ids_ahead[q];
+            rws[q] = STAGE != 1 ? rws_ahead[q] : 0u;
+        }
+        if(PAIR == 2 && m0 + PAIR < MT)
+            read_ids(m0 + PAIR);
+    };
     if(STAGE == 1)
     {
         // lane (r, kb) holds channels j*16 + kb*4 .. +3 (j = 0, 1) of row r.  After one permlane16 swap per
@@ -388,15 +407,17 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, int nt, int row
             constexpr int NP = m0 + PAIR <= MT ? PAIR : MT - m0;       // row groups of this pair
             uint4 o[NP];
             u32 q4[NP], e8[NP];
+            bool ok[NP];
+            u32 ids[PAIR], rws[PAIR];
+            take_ids(m0, ids, rws);
 #pragma unroll
             for(int q = 0; q < NP; q++)
-                o[q] = make_uint4(0u, 0u, 0u, 0u);                // row groups that hold only padding store zeros
+            {
+                o[q]  = make_uint4(0u, 0u, 0u, 0u);
+                ok[q] = m0 < ma && (int)(ids[q] >> 24) < g.topk;      // padding rows store zeros
+            }
             if(m0 < ma)                                           // (a pair leaves together: a padding group next to a real one computes)
             {
-                u32 ids[NP];
-#pragma unroll
-                for(int q = 0; q < NP; q++)
-                    ids[q] = meta[(m0 + q) * 16 + r];
                 static_for<NP>([&](auto Q) __attribute__((always_inline)) {
                     constexpr int q = decltype(Q)::value, mt = m0 + q;
                     v4f row[4];
@@ -415,8 +436,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, int nt, int row
                     v2u t0 = __builtin_amdgcn_permlane16_swap(d[0][0], d[1][0], false, false);
                     v2u t1 = __builtin_amdgcn_permlane16_swap(d[0][1], d[1][1], false, false);
                     // even lane rows: x = (kb, j0), y = (kb+1, j0); odd lane rows: x = (kb-1, j1), y = (kb, j1)
-                    const bool ok = (int)(ids[q] >> 24) < g.topk;          // padding rows store zeros
-                    o[q] = make_uint4(ok ? t0.x : 0u, ok ? t1.x : 0u, ok ? t0.y : 0u, ok ? t1.y : 0u);
+                    o[q] = make_uint4(t0.x, t1.x, t0.y, t1.y);
                 });
             }
             // the wave's 32 channels of a row are exactly one MX block (8 channels in each of the four lane rows): block
@@ -433,7 +453,8 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, int nt, int row
                     v2u s32 = __builtin_amdgcn_permlane32_swap(am, am, false, false);
                     am      = s32.x > s32.y ? s32.x : s32.y;
                     e8[q]   = mx_scale_byte(am);
-                    q4[q]   = cvt8(o[q], mx_inv_scale(e8[q]));
+                    q4[q]   = ok[q] ? cvt8(o[q], e8[q]) : 0u;
+                    e8[q]   = ok[q] ? e8[q] : 0u;
                 }
 #pragma unroll
                 for(int q = 0; q < NP; q++)
@@ -447,45 +468,44 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, int nt, int row
             if(out)
 #pragma unroll
                 for(int q = 0; q < NP; q++)
-                    *(uint4*)(out + (size_t)(row0 + (m0 + q) * 16 + r) * I + ch_out) = o[q];
+                    *(uint4*)(out + (size_t)(row0 + (m0 + q) * 16 + r) * I + ch_out) =
+                        ok[q] ? o[q] : make_uint4(0u, 0u, 0u, 0u);
             __builtin_amdgcn_sched_barrier(0);      // a pair of row groups at a time: keeps the temporaries few
         });
     }
     else
     {
-        // lane (r, kb) holds channels j*16 + kb*4 .. +3 (j = 0..3) of row r.  A 4x4 transpose across the
-        // four lane rows gives every lane 16 consecutive channels: 32 B stores, 128 B contiguous per row.
+        // lane (r, kb) holds channels j*16 + kb*4 .. +3 (j = 0..3) of row r.  One permlane16 swap per packed dword, between
+        // j = 0, 1 and between j = 2, 3, gives every lane 8 consecutive channels of the wave's lower and 8 of its upper 32:
+        // two 16 B stores, each of which writes 64 contiguous bytes per row.  (A 4x4 transpose that gives a lane 16
+        // consecutive channels costs twice the swaps, and each of its stores writes every other 16 bytes of 128.)
+        typedef unsigned v2u __attribute__((ext_vector_type(2)));
         uint16_t* out = (uint16_t*)g.out;
         const int chw = nt * 256 + wcol * 64;
-        const int lane_col  = chw + kb * 16;
+        const int lane_col  = chw + (kb & 1) * 16 + (kb >> 1) * 8;      // lane rows 0..3: channel offsets 0, 16, 8, 24
         const u32 row_bytes = (u32)g.N * 2u;
         static_for<(MT + PAIR - 1) / PAIR>([&](auto GI) __attribute__((always_inline)) {
             constexpr int m0 = decltype(GI)::value * PAIR;
             constexpr int NP = m0 + PAIR <= MT ? PAIR : MT - m0;
             if(m0 >= ma)
                 return;
-            u32 ids[NP], rws[NP];
-#pragma unroll
-            for(int q = 0; q < NP; q++)
-            {
-                ids[q] = meta[(m0 + q) * 16 + r];
-                rws[q] = meta[mpad + (m0 + q) * 16 + r];
-            }
-            u32 lo[NP][4], hi[NP][4];
+            u32 ids[PAIR], rws[PAIR];
+            take_ids(m0, ids, rws);
+            uint4 d[NP][2];                       // channels lane_col .. + 7 and lane_col + 32 .. + 39
             static_for<NP>([&](auto Q) __attribute__((always_inline)) {
                 constexpr int q = decltype(Q)::value, mt = m0 + q;
                 v4f row[4];
                 gemm_fetch_row<MT, mt, BIAS>(row, bz, xacc);
                 const float rw = __builtin_bit_cast(float, rws[q]);
 #pragma unroll
-                for(int j = 0; j < 4; j++)
+                for(int h = 0; h < 2; h++)
                 {
-                    lo[q][j] = pack_bf16x2(row[j][0] * rw, row[j][1] * rw);
-                    hi[q][j] = pack_bf16x2(row[j][2] * rw, row[j][3] * rw);
+                    v2u t0 = __builtin_amdgcn_permlane16_swap(pack_bf16x2(row[2 * h][0] * rw, row[2 * h][1] * rw),
+                                                              pack_bf16x2(row[2 * h + 1][0] * rw, row[2 * h + 1][1] * rw), false, false);
+                    v2u t1 = __builtin_amdgcn_permlane16_swap(pack_bf16x2(row[2 * h][2] * rw, row[2 * h][3] * rw),
+                                                              pack_bf16x2(row[2 * h + 1][2] * rw, row[2 * h + 1][3] * rw), false, false);
+                    d[q][h] = make_uint4(t0.x, t1.x, t0.y, t1.y);
                 }
-                transpose4x4_rows(lo[q]);
-                transpose4x4_rows(hi[q]);
-                // lane row c now holds channels c*16 + i*4 .. +3 in (lo[i], hi[i])
             });
 #pragma unroll
             for(int q = 0; q < NP; q++)
@@ -499,29 +519,32 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, int nt, int row
                     // atomic store of that scope
                     const u32 orow               = tok * (u32)g.topk + slot;
                     const unsigned long long dst = (unsigned long long)(out + lane_col) + (unsigned long long)orow * row_bytes;
-                    const v4i d0 = {(int)lo[q][0], (int)hi[q][0], (int)lo[q][1], (int)hi[q][1]};
-                    const v4i d1 = {(int)lo[q][2], (int)hi[q][2], (int)lo[q][3], (int)hi[q][3]};
-                    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\tglobal_store_dwordx4 %0, %2, off offset:16 sc1"
+                    const v4i d0 = __builtin_bit_cast(v4i, d[q][0]), d1 = __builtin_bit_cast(v4i, d[q][1]);
+                    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\tglobal_store_dwordx4 %0, %2, off offset:64 sc1"
                                  ::"v"(dst), "v"(d0), "v"(d1) : "memory");
                 }
                 if(ok && !ATOMIC && STAGE != 3)
                 {
                     // (plain stores: marked non-temporal they cost the down GEMM 5 % and the reduction, which then finds
                     // nothing of out3 in the last-level cache, another 4 %)
+                    // (the address space is named: a pointer made from an integer is a generic one, whose stores count as LDS
+                    // operations as well, and the next LDS read then waits for them)
                     const u32 orow = __umul24(tok, (u32)g.topk) + slot;     // row of out3 [tokens * topk, N]
-                    uint4* dst = (uint4*)((unsigned long long)(out + lane_col) + (unsigned long long)orow * row_bytes);
-                    dst[0]     = make_uint4(lo[q][0], hi[q][0], lo[q][1], hi[q][1]);
-                    dst[1]     = make_uint4(lo[q][2], hi[q][2], lo[q][3], hi[q][3]);
+                    auto* dst      = (__attribute__((address_space(1))) v4i*)((unsigned long long)(out + lane_col) + (unsigned long long)orow * row_bytes);
+                    dst[0]         = __builtin_bit_cast(v4i, d[q][0]);
+                    dst[4]         = __builtin_bit_cast(v4i, d[q][1]);
                 }
                 if(ok && ATOMIC)
                 {
                     typedef short v2s __attribute__((ext_vector_type(2)));
                     auto* dst = (__attribute__((address_space(1))) v2s*)((unsigned long long)(out + lane_col) + (unsigned long long)tok * row_bytes);
 #pragma unroll
-                    for(int c = 0; c < 4; c++)
+                    for(int h = 0; h < 2; h++)
                     {
-                        __builtin_amdgcn_global_atomic_fadd_v2bf16(dst + 2 * c, __builtin_bit_cast(v2s, lo[q][c]));
-                        __builtin_amdgcn_global_atomic_fadd_v2bf16(dst + 2 * c + 1, __builtin_bit_cast(v2s, hi[q][c]));
+                        __builtin_amdgcn_global_atomic_fadd_v2bf16(dst + 16 * h, __builtin_bit_cast(v2s, d[q][h].x));
+                        __builtin_amdgcn_global_atomic_fadd_v2bf16(dst + 16 * h + 1, __builtin_bit_cast(v2s, d[q][h].y));
+                        __builtin_amdgcn_global_atomic_fadd_v2bf16(dst + 16 * h + 2, __builtin_bit_cast(v2s, d[q][h].z));
+                        __builtin_amdgcn_global_atomic_fadd_v2bf16(dst + 16 * h + 3, __builtin_bit_cast(v2s, d[q][h].w));
                     }
                 }
             }

@@ -73,6 +73,7 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
     // operations that bring the next tile's sorted ids are issued once per tile, ahead of a K-group's schedule, and are
     // not counted: an operation the counts do not know of only makes a wait cover more than it must.
     constexpr int NPF = 5 * NA + 4;
+    constexpr int WS  = STAGE == 3 ? 4 : 0;   // wait states before a vector-memory operation, see vm_load_b128
     // one LDS stage = the activation tile of a whole K-group (4 K-steps of 128) + its scales
     __shared__ __attribute__((aligned(16))) uint8_t lds_a0[4 * SLOTS * 1024];
     __shared__ __attribute__((aligned(16))) uint8_t lds_a1[4 * SLOTS * 1024];
@@ -93,6 +94,17 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
     const int Kb = g.K / 2;
     const int KS = g.K / 512;
     const int I  = g.N / 2;   // stage 1 only
+
+    // The arguments again, from the kernel's argument segment: what only a tile's boundary needs (output pointers, biases, sizes)
+    // is loaded there, instead of living in scalar registers across the K loop, which has none to spare: the descriptors
+    // of the pipeline alone take 24, and what does not fit is parked in vector registers and read back a lane at a time.
+    auto args_again = [&]() __attribute__((always_inline)) -> const GemmArgs* {
+        if constexpr(STAGE == 3)
+            return &g;
+        unsigned long long p = (unsigned long long)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(p));              // (opaque: the loads stay where they are written)
+        return (const GemmArgs*)(const __attribute__((address_space(4))) GemmArgs*)p;
+    };
 
     // ---- tile iterator.  With a schedule the grid is persistent.  All tiles, ordered expert -> weight tile -> row
     // block (the row blocks that share a weight tile next to each other), form one list; it is cut into 8 equal
@@ -193,20 +205,21 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
             }
             else
             {
+                const GemmArgs& ga = *args_again();
                 auto pre_u = [&](int i) __attribute__((always_inline)) -> u32 {
                     typedef const __attribute__((address_space(4))) u32* sched_ptr;    // scalar loads
-                    return TALL ? ((sched_ptr)(unsigned long long)g.sched)[i] : uni(lds_pre[i]);
+                    return TALL ? ((sched_ptr)(unsigned long long)ga.sched)[i] : uni(lds_pre[i]);
                 };
                 if(ei < 0)
                     ei = 0;
-                while(q >= pre_u(ei + 1) * (u32)g.n_tiles)
+                while(q >= pre_u(ei + 1) * (u32)ga.n_tiles)
                     ei++;
                 const u32 p0    = pre_u(ei);
                 const u32 nb    = pre_u(ei + 1) - p0;
-                const u32 local = q - p0 * (u32)g.n_tiles;
+                const u32 local = q - p0 * (u32)ga.n_tiles;
                 t.nt            = (int)(local / nb);
                 t.m_blk         = (int)(p0 + (local - (u32)t.nt * nb));
-                t.e             = (int)(TALL ? pre_u(g.E + 1 + ei) : uni(lds_lid[ei]));
+                t.e             = (int)(TALL ? pre_u(ga.E + 1 + ei) : uni(lds_lid[ei]));
             }
             q += qstride;
         }
@@ -244,8 +257,7 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
     const int rd_a      = r * 64 + ((kb ^ ((r >> 1) & 3)) * 16);   // operand read offset inside a 1 KB block
     const int rd_s      = (r * 4 + kb) * 4;                  // scale dword read offset inside a 256 B block
     auto setup_null = [&]() __attribute__((always_inline)) {
-        wrs[0] = wrs[1] = make_rsrc(g.w, 0);
-        wsrs[0] = wsrs[1] = make_rsrc(g.w_s, 0);
+        wrs[0] = wrs[1] = wsrs[0] = wsrs[1] = make_rsrc(nullptr, 0);
 #pragma unroll
         for(int i = 0; i < NA; i++)
             a_off[i] = as_off[i] = (int)0xFFFF0000u;
@@ -266,15 +278,6 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
         const int n   = __builtin_popcountll(__ballot(ok));
         return n < 1 ? 1 : n;
     };
-    // The arguments again, from the kernel's argument segment: what only a tile's boundary needs (output pointers, biases, sizes)
-    // is loaded there, instead of living in scalar registers across the K loop, which has none to spare: the descriptors
-    // of the pipeline alone take 24, and what does not fit is parked in vector registers and read back a lane at a time.
-    auto args_again = [&]() __attribute__((always_inline)) -> const GemmArgs* {
-        unsigned long long p = (unsigned long long)__builtin_amdgcn_kernarg_segment_ptr();
-        asm volatile("" : "+s"(p));              // (opaque: the loads stay where they are written)
-        return (const GemmArgs*)(const __attribute__((address_space(4))) GemmArgs*)p;
-    };
-
     // ids: the tile's sorted ids, either in LDS (meta buffer) or in global memory
     auto setup_load = [&](const TileId& t, const u32* ids) __attribute__((always_inline)) {
         const GemmArgs& ga   = *args_again();
@@ -352,10 +355,10 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
         if constexpr(MT <= 2)
         {
             const int away = kt * 128 + kb * 32 >= k_real ? (int)0x80000000u : 0;
-            vm_load_b128<0, NT>(wf[u][j], w_voff[j & 1] + away, wrs[j >> 1], kt * 1024 + (j >> 1) * w_half);
+            vm_load_b128<0, NT, WS>(wf[u][j], w_voff[j & 1] + away, wrs[j >> 1], kt * 1024 + (j >> 1) * w_half);
         }
         else
-            vm_load_b128<0, NT>(wf[u][j], w_voff[j & 1], wrs[j >> 1], kt * 1024 + (j >> 1) * w_half);
+            vm_load_b128<0, NT, WS>(wf[u][j], w_voff[j & 1], wrs[j >> 1], kt * 1024 + (j >> 1) * w_half);
     };
     auto load_wtiles = [&](auto U, int kt) __attribute__((always_inline)) {
         static_for<4>([&](auto J) __attribute__((always_inline)) { load_wtile(U, J, kt); });
@@ -423,7 +426,6 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
     // at 128 rows: gpt-oss shape, 4096 tokens, layer 0.573 against 0.597 ms; Mixtral shape, 512 tokens, 0.216 against
     // 0.224 ms).
     constexpr bool SPREAD = MT > 8;
-    constexpr int WS = STAGE == 3 ? 4 : 0;        // see vm_dma_b128
     // the last GUARDED row groups of a tall tile are jumped over when they hold no real rows (mfma_row_group_guarded)
     constexpr int GUARDED = MT == 18 ? 2 : MT > 8 ? 3 : 0;
     using VS = VmSchedule<MA, NPF, SPREAD ? 2 : 1>;
@@ -432,15 +434,16 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
     // sorted ids and routing weights of a tile's rows -> LDS meta buffer `buf` (DMA, 64 rows per operation, spread over
     // the four waves)
     auto dma_meta = [&](const TileId& t, int buf) __attribute__((always_inline)) {
-        const v4i rid = make_rsrc(g.sorted_ids + (size_t)t.m_blk * BM, BM * 4);
-        const v4i rwt = make_rsrc(g.sorted_w + (size_t)t.m_blk * BM, BM * 4);
+        const GemmArgs& ga = *args_again();
+        const v4i rid = make_rsrc(ga.sorted_ids + (size_t)t.m_blk * BM, BM * 4);
+        const v4i rwt = make_rsrc(ga.sorted_w + (size_t)t.m_blk * BM, BM * 4);
 #pragma unroll
         for(int i = 0; i < NM; i++)
         {
             const int o    = wave + 4 * i;               // op index: [0, NID) ids, [NID, 2*NID) weights, beyond: nothing
             const bool wts = o >= NID;
             const int oo   = wts ? o - NID : o;
-            if(o < 2 * NID && (!wts || g.sorted_w != nullptr))
+            if(o < 2 * NID && (!wts || STAGE != 1))
                 vm_dma_b32_fresh_sgprs((oo * 64 + lane) * 4, uni4(wts ? rwt : rid),
                                        uni(lds_addr_of(&lds_meta[buf][(wts ? MPAD : 0) + oo * 64])));
         }
@@ -464,7 +467,7 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
         else
         {
             constexpr int h = (k - 5 * NA) / 2, c = (k - 5 * NA) % 2;
-            vm_load_b32<0>(w_sc[ts][h * 2 + c], lane * 4 + c * 256, wsrs[h], kpre * 512 + h * ws_half);
+            vm_load_b32<0, WS>(w_sc[ts][h * 2 + c], lane * 4 + c * 256, wsrs[h], kpre * 512 + h * ws_half);
         }
     };
     // the vector-memory operations of gap G of row group N (see VmSchedule)

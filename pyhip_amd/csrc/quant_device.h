@@ -47,12 +47,11 @@ __device__ __forceinline__ void act_quant_block(const QuantArgs& a, long long id
         am = amax15(am, v2.x); am = amax15(am, v2.y); am = amax15(am, v2.z); am = amax15(am, v2.w);
         am = amax15(am, v3.x); am = amax15(am, v3.y); am = amax15(am, v3.z); am = amax15(am, v3.w);
         e8        = mx_scale_byte(am);
-        float mul = mx_inv_scale(e8);
         uint4 o;
-        o.x = cvt8(v0, mul);
-        o.y = cvt8(v1, mul);
-        o.z = cvt8(v2, mul);
-        o.w = cvt8(v3, mul);
+        o.x = cvt8(v0, e8);
+        o.y = cvt8(v1, e8);
+        o.z = cvt8(v2, e8);
+        o.w = cvt8(v3, e8);
         *(uint4*)(a.q + row * (long long)(a.K / 2) + (long long)j * 16) = o;
     }
     // 4x4 byte transpose of the 16 scales of this group through lane shuffles
