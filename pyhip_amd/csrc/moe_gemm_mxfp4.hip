@@ -591,11 +591,16 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
                 }
                 else
                 static_for<4>([&](auto J) __attribute__((always_inline)) {
-                    constexpr int j = decltype(J)::value;
+                    constexpr int j = decltype(J)::value;          // the gap; the weight row group is w
+                    // (to and fro: the first MFMA of a row group takes the weight tile of the last one before it, so that one
+                    // operand changes from MFMA to MFMA and not both.  What toggles costs power, and power is what bounds these
+                    // kernels: the MFMA stream alone sustains 1.7 % more, the whole pattern of the 288-row tile 0.8 % (weights
+                    // from HBM) to 2.6 % (from the L2).)
+                    constexpr int w = n & 1 ? 3 - j : j;
                     v4f* xa = nullptr;
-                    if constexpr(acc_in_vgprs<MT, mt>() && j == 3)
+                    if constexpr(acc_in_vgprs<MT, mt>() && w == 3)
                         xa = &xacc[mt - ACC_SPILL_MT0];
-                    mfma_one<u, mt, MT, j>(wf[u][j], af, w_sc[p][(j >> 1) * 2 + (u >> 1)], asc, xa);
+                    mfma_one<u, mt, MT, w>(wf[u][w], af, w_sc[p][(w >> 1) * 2 + (u >> 1)], asc, xa);
                     if constexpr(SPREAD)
                     {
                         __builtin_amdgcn_sched_barrier(0);
