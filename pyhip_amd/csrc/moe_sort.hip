@@ -11,8 +11,8 @@
 //   expert_offset[e] + (#pairs of e in earlier workgroups) + (#pairs of e in earlier waves of this
 //   workgroup) + (#pairs of e earlier in this wave's chunk).
 //
-// Three launches for large inputs (histogram -> scan -> scatter) and one single-workgroup
-// launch for small inputs.
+// Small inputs: one launch of a single workgroup.  Middle sizes: one launch of several workgroups, each of which counts all
+// pairs for itself (moe_sort_count_kernel).  Large inputs: three launches (histogram -> scan -> scatter).
 #include "common.h"
 #include "quant_device.h"
 #include "router_device.h"
@@ -374,6 +374,138 @@ extern "C" __global__ void __launch_bounds__(SMALL_THREADS) moe_sort_small_cols_
 }
 
 // ---------------------------------------------------------------------------------------------
+// Middle sizes, one launch: workgroup g writes the pairs of its own chunk and finds out where they go by itself.  It counts ALL
+// pairs, those before its chunk and those behind it apart, in LDS, so nothing passes between workgroups.  That reads the ids
+// once per workgroup instead of twice in all, from the L2 as a rule, and replaces two dependent launches and their gaps, which
+// is where the time of the three-launch sort goes.  Kernel times, us, the three launches (gaps between them not counted) / this one:
+//   256 experts, top-8:  2400 pairs 14.5 / 8.5; 8192: 15.2 / 9.0; 16384: 15.4 / 9.8; 65536: 20.7 / 14.6; 131072: 26.8 / 21.9; 262144: 39.5 / 37.0
+//   8 experts, top-2:    4096 pairs 11.3 / 5.9; 16384: 13.0 / 7.5; 65536: 17.3 / 12.3
+//   128 experts, top-8, Zipf: 8192 pairs 13.3 / 7.3; 65536: 18.8 / 13.6; 131072: 24.3 / 21.1; 262144: 36.6 / 37.3
+// Beyond COUNT_PAIRS_MAX the reads grow with the square of the pairs and the three launches win (524288 pairs: 101-121 us here).
+// At 2048 pairs the single workgroup takes 9.6 us with 256 experts, this 8.1; below about 1500 pairs it is the faster one.
+// At least COUNT_WGS_MIN workgroups, because the padding entries are theirs to write as well (2400 pairs: 10.7 us with three).
+// The counters come in COUNT_COPIES, a lane's copy next to its neighbour's: with few experts, or under a router that prefers some,
+// many lanes of a wave count the same expert at once, and equal addresses are served one after the other (16384 pairs of 8 experts:
+// 8.4 us with one copy, 7.5 with four; 131072 Zipf pairs: 28.2 / 21.1).
+// LDS: whist[SMALL_WAVES][E] | before[E][COUNT_COPIES] | behind[E][COUNT_COPIES] | tot[E] | off[E] | lid[E] | scratch[2*SMALL_WAVES]
+#define COUNT_PAIRS_MAX (1 << 17)
+#define COUNT_WGS_MIN 16
+#define COUNT_COPIES 4
+#define COUNT_GROUPS 1                                      // groups of 64 pairs a wave places
+#define COUNT_CHUNK (SMALL_WAVES * COUNT_GROUPS * WAVE)     // pairs a workgroup places
+__device__ __forceinline__ void sort_count(const SortArgs& a, u32* lds)
+{
+    u32* whist   = lds;
+    u32* before  = whist + SMALL_WAVES * a.E;
+    u32* behind  = before + COUNT_COPIES * a.E;
+    u32* tot     = behind + COUNT_COPIES * a.E;
+    u32* off     = tot + a.E;
+    u32* lid     = off + a.E;
+    u32* scratch = lid + a.E;
+    const int T     = sort_tokens(a);
+    const int pairs = T * a.k;
+    const int wave  = threadIdx.x / WAVE;
+    const int beg_g = min(pairs, (int)blockIdx.x * COUNT_CHUNK), end_g = min(pairs, beg_g + COUNT_CHUNK);
+    const int beg   = min(pairs, beg_g + wave * COUNT_GROUPS * WAVE), end = min(pairs, beg + COUNT_GROUPS * WAVE);
+
+    WavePairs<COUNT_GROUPS> wp;
+    wp.load(a, beg, end, true);
+    for(int i = threadIdx.x; i < (SMALL_WAVES + 2 * COUNT_COPIES) * a.E; i += SMALL_THREADS)
+        whist[i] = 0;                                       // (before and behind follow)
+    __syncthreads();
+    // every pair outside the chunk, by its id alone (an expert that is masked is left out as a whole below); four ids at a
+    // time where the array allows it, eight such loads in flight (the chunk's bounds are multiples of four)
+    const int copy = threadIdx.x % COUNT_COPIES;
+    auto count = [&](int e, int i) __attribute__((always_inline)) {
+        if((u32)e < (u32)a.E && (i < beg_g || i >= end_g))
+            atomicAdd((i < beg_g ? before : behind) + e * COUNT_COPIES + copy, 1u);
+    };
+    int done = 0;
+    if(((unsigned long long)a.topk_ids & 15) == 0)
+    {
+        const int n4 = pairs / 4;
+        for(int i0 = 0; i0 < n4; i0 += SMALL_THREADS * 8)
+        {
+            int4 v[8];
+#pragma unroll
+            for(int j = 0; j < 8; j++)
+            {
+                const int i = i0 + j * SMALL_THREADS + (int)threadIdx.x;
+                v[j]        = i < n4 ? ((const int4*)a.topk_ids)[i] : make_int4(-1, -1, -1, -1);
+            }
+#pragma unroll
+            for(int j = 0; j < 8; j++)
+            {
+                const int i = 4 * (i0 + j * SMALL_THREADS + (int)threadIdx.x);
+                count(v[j].x, i);
+                count(v[j].y, i);
+                count(v[j].z, i);
+                count(v[j].w, i);
+            }
+        }
+        done = n4 * 4;
+    }
+    for(int i = done + (int)threadIdx.x; i < pairs; i += SMALL_THREADS)
+        count(a.topk_ids[i], i);
+    wp.match(a, beg, end);
+    wp.hist_private(whist + wave * a.E);
+    __syncthreads();
+    for(int e = threadIdx.x; e < a.E; e += SMALL_THREADS)
+    {
+        u32 run = 0, rest = 0;
+#pragma unroll
+        for(int c = 0; c < COUNT_COPIES; c++)
+        {
+            run += before[e * COUNT_COPIES + c];
+            rest += behind[e * COUNT_COPIES + c];
+        }
+#pragma unroll
+        for(int w = 0; w < SMALL_WAVES; w++)
+        {
+            const u32 c        = whist[w * a.E + e];
+            whist[w * a.E + e] = run;
+            run += c;
+        }
+        tot[e] = moe_pair_is_kept(e, a.E, a.expert_mask) ? run + rest : 0u;
+    }
+    __syncthreads();
+    const u32 padded_total = expert_offsets(a, tot, off, lid, scratch);
+    wp.scatter(a, whist + wave * a.E, off, beg, end);
+    // the padding entries: those behind an expert's rows by the workgroup that the expert falls to, those behind everything by
+    // all of them
+    const u32 pad_id = ((u32)a.k << 24) | ((u32)T & 0xFFFFFFu);
+    for(int e = (int)blockIdx.x + wave * a.G; e < a.E; e += SMALL_WAVES * a.G)
+    {
+        const u32 first = off[e] + tot[e], last = off[e] + (tot[e] + a.Bm - 1) / a.Bm * a.Bm;
+        for(u32 p = first + lane_id(); p < last; p += WAVE)
+        {
+            a.sorted_ids[p] = pad_id;
+            a.sorted_w[p]   = 0.f;
+        }
+    }
+    for(u32 p = padded_total + blockIdx.x * SMALL_THREADS + threadIdx.x; p < (u32)a.n_blk * (u32)a.Bm; p += a.G * SMALL_THREADS)
+    {
+        a.sorted_ids[p] = pad_id;
+        a.sorted_w[p]   = 0.f;
+    }
+    if(blockIdx.x == 0)
+    {
+        fill_blocks(a, tot, off, lid, padded_total, T);
+        write_schedule(a, off, lid, padded_total);
+    }
+}
+
+// workgroups past the a.G of the sort quantise activations, as in the single-workgroup sort
+extern "C" __global__ void __launch_bounds__(SMALL_THREADS) moe_sort_count_kernel(SortArgs a, QuantArgs qa, int x_cols)
+{
+    extern __shared__ u32 lds[];
+    if((int)blockIdx.x >= a.G)
+        act_quant_block(qa, (long long)((int)blockIdx.x - a.G) * SMALL_THREADS + threadIdx.x, x_cols);
+    else
+        sort_count(a, lds);
+}
+
+// ---------------------------------------------------------------------------------------------
 // large inputs, launch 1 of 3: per-workgroup histogram -> ws[g][E]; padding entries everywhere
 extern "C" __global__ void __launch_bounds__(SORT_THREADS) moe_sort_hist_kernel(SortArgs a)
 {
@@ -646,6 +778,17 @@ static int sorting_impl(const int32_t* topk_ids, const float* topk_weights, int 
         else
             hipLaunchKernelGGL((moe_sort_small_kernel<0, false>), dim3(1 + qblocks), dim3(SMALL_THREADS), lds, stream, a, qa, ra);
         PYHIP_CHECK_LAUNCH("moe_sort_small_kernel");
+        return PYHIP_OK;
+    }
+    // one launch while counting everything in every workgroup costs less than the two launches it saves, and while the counters
+    // fit the LDS that a kernel gets without asking (606 experts)
+    const size_t count_lds = ((size_t)(SMALL_WAVES + 2 * COUNT_COPIES + 3) * experts + 2 * SMALL_WAVES + 2) * 4;
+    if(pairs <= COUNT_PAIRS_MAX && count_lds <= 64 * 1024)
+    {
+        a.G = (int)((pairs + COUNT_CHUNK - 1) / COUNT_CHUNK);
+        a.G = a.G > COUNT_WGS_MIN ? a.G : COUNT_WGS_MIN;
+        hipLaunchKernelGGL(moe_sort_count_kernel, dim3(a.G + qblocks), dim3(SMALL_THREADS), count_lds, stream, a, qa, x_cols);
+        PYHIP_CHECK_LAUNCH("moe_sort_count_kernel");
         return PYHIP_OK;
     }
     a.G = sort_groups(pairs);
