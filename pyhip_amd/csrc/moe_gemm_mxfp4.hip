@@ -107,12 +107,18 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
     };
 
     // ---- tile iterator.  With a schedule the grid is persistent.  All tiles, ordered expert -> weight tile -> row
-    // block (the row blocks that share a weight tile next to each other), form one list; it is cut into 8 equal
-    // runs, one per XCD, so every XCD (its own L2) gets the same number of tiles however unevenly the router loads
-    // the experts, and an expert's data still meets in one L2 (two where a cut falls inside an expert).  Workgroup w
-    // serves XCD w % 8 (the hardware deals consecutive workgroup ids round-robin to the XCDs) and walks that XCD's
-    // run with stride gridDim/8.
+    // block (the row blocks that share a weight tile next to each other), form one list, of which every XCD (its own L2) gets
+    // the same number of tiles however unevenly the router loads the experts.  Workgroup w serves XCD w % 8 (the hardware
+    // deals consecutive workgroup ids round-robin to the XCDs) and walks that XCD's share with stride gridDim/8.
+    // A share is one run of the list, so that an expert's data meets in one L2 (two where a cut falls inside an expert), or,
+    // in the tiles of 128 rows and more, up to eight pieces of at least 64 tiles, dealt round-robin.  A busy expert's tiles are
+    // bound by their MFMAs and a quiet one's by its weights, so where the busy experts of a layer are neighbours, equal runs
+    // leave some XCDs with the long tiles and all of the others waiting for memory at once (Qwen3 shape with the Zipf router,
+    // 2048 tokens: layer 410.7 us in runs, 396.8 in pieces; even routers the same in both).  With fewer than 32 experts a
+    // share is about one of them, and cutting it costs (Mixtral shape, 4096 tokens: 767.5 / 773.6); the smaller tiles are
+    // bound by the weights in any case (decode sizes 0.2-0.6 % slower in pieces).
     // Without a schedule (or when K has a single K-group): one tile per workgroup, weight tile fastest.
+    constexpr bool PIECES = MT >= 8;
     const bool persistent = g.sched != nullptr;
     const int xcd         = blockIdx.x & 7;
     const u32 qstride     = gridDim.x >> 3;
@@ -146,12 +152,18 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
     u32 tab_blk = 0xFFFFFFFFu, tab_nte = 0;       // lane i: row block and weight tile | expert << 16
     int tab_i   = 0;                              // next entry; 64: the table is used up
     int ei      = -1;                             // beyond the table: cursor into the expert list (q only grows)
+    // place i of the XCD's share -> tile
+    u32 piece    = 1;
+    auto tile_of = [&](u32 i) __attribute__((always_inline)) -> u32 {
+        return PIECES ? (i / piece * 8u + (u32)xcd) * piece + i % piece : (u32)xcd * piece + i;
+    };
     auto build_table = [&]() __attribute__((always_inline)) {
-        const u32 qi = q + (u32)lane * qstride;
-        tab_blk      = 0xFFFFFFFFu;
-        tab_nte      = 0;
-        if(qi < q_end && qi >= q)                 // (qi >= q: no wrap-around)
+        const u32 place = q + (u32)lane * qstride;
+        tab_blk         = 0xFFFFFFFFu;
+        tab_nte         = 0;
+        if(place < q_end && place >= q)           // (place >= q: no wrap-around)
         {
+            const u32 qi = tile_of(place);
             int lo = 0, hi = g.E - 1;             // first expert whose tiles end beyond qi
             while(lo < hi)
             {
@@ -178,13 +190,14 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
     if(persistent)
     {
         const u32 tiles = uni(sched_pre(g.E)) * (u32)g.n_tiles;
-        const u32 chunk = (tiles + 7u) >> 3;
+        const u32 pieces = !PIECES || g.E < 32 || tiles < 1024u ? 1u : tiles > 4096u ? 8u : tiles / 512u;
+        piece            = (tiles + 8u * pieces - 1u) / (8u * pieces);
+        const u32 last   = ((pieces - 1u) * 8u + (u32)xcd) * piece;       // where the last piece starts, the only one that can be short
+        q_end            = (pieces - 1u) * piece + (last >= tiles ? 0u : tiles - last < piece ? tiles - last : piece);
         // (Every workgroup of the launch takes part, also when the last round of an XCD's run is nearly empty.  Letting only
         // as many take part as make the rounds even (113 tiles on 96 workgroups: 57 with two tiles each) was measured and is
         // slower everywhere: DeepSeek-V3 shape at 16 tokens 0.379 -> 0.412 ms, Mixtral shape at 4096 tokens 0.790 -> 0.831 ms.
         // More workgroups keep more loads in flight, and that is worth more than even rounds.)
-        q += (u32)xcd * chunk;
-        q_end = (u32)(xcd + 1) * chunk < tiles ? (u32)(xcd + 1) * chunk : tiles;
         if(q < q_end)
             build_table();
     }
@@ -206,17 +219,18 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
             else
             {
                 const GemmArgs& ga = *args_again();
+                const u32 tile     = tile_of(q);
                 auto pre_u = [&](int i) __attribute__((always_inline)) -> u32 {
                     typedef const __attribute__((address_space(4))) u32* sched_ptr;    // scalar loads
                     return TALL ? ((sched_ptr)(unsigned long long)ga.sched)[i] : uni(lds_pre[i]);
                 };
                 if(ei < 0)
                     ei = 0;
-                while(q >= pre_u(ei + 1) * (u32)ga.n_tiles)
+                while(tile >= pre_u(ei + 1) * (u32)ga.n_tiles)
                     ei++;
                 const u32 p0    = pre_u(ei);
                 const u32 nb    = pre_u(ei + 1) - p0;
-                const u32 local = q - p0 * (u32)ga.n_tiles;
+                const u32 local = tile - p0 * (u32)ga.n_tiles;
                 t.nt            = (int)(local / nb);
                 t.m_blk         = (int)(p0 + (local - (u32)t.nt * nb));
                 t.e             = (int)(TALL ? pre_u(ga.E + 1 + ei) : uni(lds_lid[ei]));
