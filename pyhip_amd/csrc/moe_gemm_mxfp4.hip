@@ -111,10 +111,12 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
     // the same number of tiles however unevenly the router loads the experts.  Workgroup w serves XCD w % 8 (the hardware
     // deals consecutive workgroup ids round-robin to the XCDs) and walks that XCD's share with stride gridDim/8.
     // A share is one run of the list, so that an expert's data meets in one L2 (two where a cut falls inside an expert), or,
-    // in the tiles of 128 rows and more, up to eight pieces of at least 64 tiles, dealt round-robin.  A busy expert's tiles are
-    // bound by their MFMAs and a quiet one's by its weights, so where the busy experts of a layer are neighbours, equal runs
-    // leave some XCDs with the long tiles and all of the others waiting for memory at once (Qwen3 shape with the Zipf router,
-    // 2048 tokens: layer 410.7 us in runs, 396.8 in pieces; even routers the same in both).  With fewer than 32 experts a
+    // in the tiles of 128 rows and more, up to eight pieces of at least 64 tiles, dealt round-robin, of which every XCD starts
+    // with another one.  A busy expert's tiles are bound by their MFMAs and a quiet one's by its weights: where the busy
+    // experts are neighbours, equal runs give some XCDs only long tiles, and pieces in the same order have all XCDs multiply
+    // first and wait for memory together afterwards.  Layer, us, runs / pieces from the first on / each XCD from its own:
+    // Qwen3 shape, Zipf router, 2048 tokens (160 rows) 410.7 / 396.8 / 382, 2400 (128 rows) 416 / 420 / 400; 160 experts, top-6,
+    // 5120 x 1536, Zipf, 4000 tokens 583 / 602 / 562; gpt-oss shape, 4700 tokens 602 / 573 / 571.  With fewer than 32 experts a
     // share is about one of them, and cutting it costs (Mixtral shape, 4096 tokens: 767.5 / 773.6); the smaller tiles are
     // bound by the weights in any case (decode sizes 0.2-0.6 % slower in pieces).
     // Without a schedule (or when K has a single K-group): one tile per workgroup, weight tile fastest.
@@ -151,11 +153,15 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
     // large calls have, are decoded one at a time with uniform reads of the schedule.)
     u32 tab_blk = 0xFFFFFFFFu, tab_nte = 0;       // lane i: row block and weight tile | expert << 16
     int tab_i   = 0;                              // next entry; 64: the table is used up
-    int ei      = -1;                             // beyond the table: cursor into the expert list (q only grows)
-    // place i of the XCD's share -> tile
-    u32 piece    = 1;
+    int ei      = -1;                             // beyond the table: cursor into the expert list
+    // place i of the XCD's share -> tile.  The pieces are walked in the list's order from piece `turn` on, and after the last
+    // piece, whose places end at `wrap`, from the first one.
+    u32 piece = 1, turn = 0, wrap = 0;
     auto tile_of = [&](u32 i) __attribute__((always_inline)) -> u32 {
-        return PIECES ? (i / piece * 8u + (u32)xcd) * piece + i % piece : (u32)xcd * piece + i;
+        if(!PIECES)
+            return (u32)xcd * piece + i;
+        const u32 j = i < wrap ? i + turn * piece : i - wrap;
+        return (j / piece * 8u + (u32)xcd) * piece + j % piece;
     };
     auto build_table = [&]() __attribute__((always_inline)) {
         const u32 place = q + (u32)lane * qstride;
@@ -194,6 +200,8 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
         piece            = (tiles + 8u * pieces - 1u) / (8u * pieces);
         const u32 last   = ((pieces - 1u) * 8u + (u32)xcd) * piece;       // where the last piece starts, the only one that can be short
         q_end            = (pieces - 1u) * piece + (last >= tiles ? 0u : tiles - last < piece ? tiles - last : piece);
+        turn             = (u32)xcd * pieces / 8u;
+        wrap             = q_end - turn * piece;
         // (Every workgroup of the launch takes part, also when the last round of an XCD's run is nearly empty.  Letting only
         // as many take part as make the rounds even (113 tiles on 96 workgroups: 57 with two tiles each) was measured and is
         // slower everywhere: DeepSeek-V3 shape at 16 tokens 0.379 -> 0.412 ms, Mixtral shape at 4096 tokens 0.790 -> 0.831 ms.
@@ -224,7 +232,7 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
                     typedef const __attribute__((address_space(4))) u32* sched_ptr;    // scalar loads
                     return TALL ? ((sched_ptr)(unsigned long long)ga.sched)[i] : uni(lds_pre[i]);
                 };
-                if(ei < 0)
+                if(ei < 0 || tile < pre_u(ei) * (u32)ga.n_tiles)      // (the walk starts over at the first piece)
                     ei = 0;
                 while(tile >= pre_u(ei + 1) * (u32)ga.n_tiles)
                     ei++;
