@@ -104,6 +104,12 @@ extern "C" int pyhip_moe_pick_block_m(int64_t tokens, int topk, int experts, int
         for(int bm = 16; bm <= 64; bm *= 2)
             if(2 * est <= bm)
                 return bm;
+        // one block of 64 rows holds an expert as long as few experts have more than that (layer, us, 64 / 128 rows; 16 experts,
+        // top-2, 4096 x 3584: 34 rows per expert 79.0 / 83.0, 48: 80.7 / 84.5, 56: 100.2 / 87.0; Mixtral shape: 40: 147.9 / 155.5,
+        // 48: 149.7 / 158.8, 56: 170.6 / 163.5; under a Zipf router the 16 experts 34: 102.8 / 99.5, 40: 104.2 / 101.4,
+        // 48: 104.3 / 111.1, and 8 experts of 5120 x 2048 44.9 / 50.2, 45.5 / 51.9, 47.1 / 50.7)
+        if(!w4a16 && est <= 50)
+            return 64;
     }
     else
     {
