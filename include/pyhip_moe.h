@@ -91,7 +91,7 @@ int pyhip_moe_sorting_quant(const int32_t* topk_ids, const float* topk_weights, 
  * src/contrib/fused_moe.py:283).  gating f32 [tokens, experts]; n_group = 0 selects pyhip_moe_topk_softmax's
  * router, n_group > 0 pyhip_moe_topk_grouped_sigmoid's; the picks are written to topk_weight / topk_ids (both
  * required: the top-k reduction and the caller read them) and sorted as pyhip_moe_sorting does.  x_bf16 (may be
- * NULL) .. scales: the input quantisation of pyhip_moe_sorting_quant.  Up to 64 tokens (and 512 experts, a power of
+ * NULL) .. scales: the input quantisation of pyhip_moe_sorting_quant.  Up to 7 tokens (and 512 experts, a power of
  * two times 64) all of it is ONE launch: the sort's single workgroup routes the tokens itself; larger inputs take
  * the router's own launch first.  Same results either way.  experts must be a multiple of 64. */
 int pyhip_moe_route_sorting(const float* gating, int tokens, int topk, int experts, int n_group, int topk_group,

@@ -685,8 +685,14 @@ extern "C" int64_t pyhip_moe_sorting_workspace_bytes(int64_t tokens, int topk, i
 
 extern "C" int64_t pyhip_moe_schedule_words(int experts) { return 2ll * experts + 1; }
 
-// most tokens / experts the single-workgroup sort routes itself; beyond, the router gets a launch of its own
-#define ROUTE_SORT_MAX_TOKENS 64
+// Most tokens / experts the single-workgroup sort routes itself; beyond, the router gets a launch of its own, a wave per token.
+// One workgroup routes a token per wave at a time on one CU, so its router grows with the tokens, while a launch costs the same
+// for any number.  Router + sort, kernel times, us, one launch / two, and a small layer around them (1024 x 512), us a call:
+//   256 experts, grouped: 4 tokens 11.2 / 10.8, 25.4 / 24.8; 8: 11.3 / 10.9, 31.3 / 30.7; 16: 13.3 / 11.3, 38.9 / 36.5;
+//     32: 18.6 / 11.6, 52.5 / 45.5; 64: 29.5 / 12.1, 72.3 / 55.0
+//   128 experts, softmax: 4 tokens 9.1 / 9.0, 23.4 / 23.6; 8: 9.3 / 9.2, 29.0 / 28.1; 64: 20.2 / 10.4, 48.0 / 37.3
+//   64 experts, softmax: 4 tokens 7.9 / 8.1, 21.6 / 23.5; 8: 8.6 / 8.4, 25.2 / 24.1; 64: 15.7 / 9.4, 38.1 / 30.4
+#define ROUTE_SORT_MAX_TOKENS 7
 #define ROUTE_SORT_MAX_EXPERTS 512
 
 static int launch_routing_sort(const SortArgs& a, const QuantArgs& qa, const RouteArgs& ra, unsigned qblocks, size_t lds,

@@ -420,7 +420,7 @@ def fused_moe_routed(hidden_states, w1, w2, gating_output, topk, renormalize=Tru
                      block_size_M=None, num_local_tokens=None, dtype=None, bias1=None, bias2=None, splitk=0,
                      method="auto", swiglu_limit=None, return_routing=False, hidden_pad=0, intermediate_pad=0):
     """``fused_topk`` (or ``grouped_topk`` when ``num_expert_group > 0``) followed by ``fused_moe``, as the reference's
-    callers chain them (tests/contrib/moe/test_fused_moe.py:38-60), in one library call: for up to 64 tokens the
+    callers chain them (tests/contrib/moe/test_fused_moe.py:38-60), in one library call: for up to 7 tokens the
     router runs inside the sort's launch.  ``gating_output`` f32 [T, E], E a multiple of 64 (use ``fused_topk`` +
     ``fused_moe`` otherwise).  ``hidden_pad`` / ``intermediate_pad`` as for ``fused_moe``, with the activations at the
     padded width.  -> out, or (out, topk_weights, topk_ids) with ``return_routing``."""
