@@ -36,6 +36,9 @@ int pyhip_sorting_quant_cols(const int32_t*, const float*, int, int, int, int, c
                              float*, uint32_t*, uint32_t*, uint32_t*, void*, int64_t, const void*, int64_t, int64_t, int,
                              uint8_t*, uint8_t*, int, hipStream_t);
 
+int pyhip_w4a16_token_top2(const void*, const uint8_t*, const uint8_t*, const void*, const int32_t*, const float*, const int32_t*,
+                           const int32_t*, void*, int, int, int, int, int, int, hipStream_t);
+
 namespace {
 struct Carve
 {
@@ -221,6 +224,11 @@ static int forward_impl(const void* hidden_bf16, int64_t hidden_row_stride, int 
         rc = pyhip_moe_gemm1_w4a16_token(hidden_bf16, w1, w1_scale, bias1_bf16, topk_ids, expert_mask, num_local_tokens,
                                          ws + l.a2, topk, experts, hidden, inter, split_k, activation, swiglu_limit, stream);
         if(rc)
+            return rc;
+        // both slots of a top-2 token in one workgroup: the down GEMM writes the layer's output
+        rc = pyhip_w4a16_token_top2(ws + l.a2, w2, w2_scale, bias2_bf16, topk_ids, topk_weights, expert_mask, num_local_tokens,
+                                    out, out_is_f32, topk, experts, hidden, inter, split_k, stream);
+        if(rc >= 0)
             return rc;
         rc = pyhip_moe_gemm2_w4a16_token(ws + l.a2, w2, w2_scale, bias2_bf16, topk_ids, topk_weights, expert_mask,
                                          num_local_tokens, out3, topk, experts, hidden, inter, split_k, stream);

@@ -44,6 +44,7 @@ struct W4A16Args
     const int* expert_mask   = nullptr;   // [experts] or null
     const int* num_local_tok = nullptr;   // device scalar or null: 0 = the token is not this rank's
     int experts              = 0;
+    int out_f32              = 0;         // token kernel that also sums the slots: the type of its output
 };
 
 // 32 e2m1 values (4 dwords) times 2^(scale byte - 127) -> four MFMA operands of 8 bf16
@@ -323,6 +324,184 @@ __global__ void __launch_bounds__(SPLIT >= 16 ? 1024 : W4A16_THREADS) moe_gemm_w
     }
 }
 
+// The down GEMM of a single token whose workgroups hold both slots of a top-2 layer: the token's output is then complete in
+// the workgroup, so it sums the slots and writes the layer's output, and the reduction's launch is left out.  A wave's row groups are
+// RG / 2 groups of 16 weight rows of either slot's expert, so the grid, the K split and what a wave keeps in flight are
+// those of moe_gemm_w4a16_kernel<2, 1, SPLIT> (whose tiles are twice as wide and one slot deep), and so is the arithmetic: partial
+// sums of the same K-steps in the same order, a slot's value rounded to bf16 after its routing weight, slots added in order in
+// fp32.  Bound: latency.  Kernel times, us, down GEMM + reduction / this: Mixtral shape (sixteen waves) 12.7 + 4.1 / 13.1, tiny
+// layer (four waves) 4.0 + 3.4 / 3.4; the layer 38.5 / 37.0 and 17.6 / 15.8.
+template <int SPLIT>
+__global__ void __launch_bounds__(SPLIT == 32 ? 1024 : W4A16_THREADS) moe_gemm_w4a16_top2_kernel(W4A16Args g)
+{
+    constexpr int NW = SPLIT == 32 ? 16 : SPLIT;
+    constexpr int NR = SPLIT == 32 ? 1 : 2;       // row groups of 16 weight rows
+    // K-steps of weights in flight.  Sixteen waves leave a wave 128 registers: there the two activation rows, which all lanes of a
+    // lane row and all waves share, sit in LDS (in registers, with two K-steps of weights: 16.6 us at the Mixtral shape; two to
+    // four K-steps 13.0-13.4, five 14.0, seven 16.3)
+    constexpr bool ROWS_IN_LDS = SPLIT == 32;
+    constexpr int NB           = ROWS_IN_LDS ? 3 : 2;
+    extern __shared__ __attribute__((aligned(16))) float red[];   // the two rows, later the partial sums
+    const int tid = threadIdx.x, lane = tid % WAVE;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    const int r = lane & 15, kb = lane >> 4;
+    const int ch0 = blockIdx.x * (16 * NR);
+    bool on[2];
+    int e[2];
+    const bool here = !(g.num_local_tok && *g.num_local_tok < 1);
+#pragma unroll
+    for(int s = 0; s < 2; s++)
+    {
+        const int eg = g.token_ids[s];
+        on[s]        = here && moe_pair_is_kept(eg, g.experts, g.expert_mask);
+        e[s]         = eg;
+        if(on[s] && g.expert_mask)            // local id: the experts this rank holds before this one
+        {
+            e[s] = 0;
+            for(int i0 = 0; i0 < eg; i0 += WAVE)
+                e[s] += __builtin_popcountll(__ballot(i0 + lane < eg && g.expert_mask[i0 + lane] != 0));
+        }
+        e[s] = __builtin_amdgcn_readfirstlane(e[s]);
+    }
+    const bool any = on[0] || on[1];
+    if(any)
+    {
+        // a slot that does not take part repeats the other one's fetches; what it computes is not used
+        const int es[2] = {on[0] ? e[0] : e[1], on[1] ? e[1] : e[0]};
+        const int Kb = g.K / 2, KT = g.K / 128;
+        const size_t sc_tile = (size_t)(g.SC / 8) * 256;
+        const uint8_t* wp[2][NR];
+        const uint8_t* sp[2][NR];
+        const uint16_t* ap[2];
+        v4f acc[2][NR];
+        const int half = (ch0 / 16) & 1;      // which 16-row half of the 32-row scale tile the first row group is
+#pragma unroll
+        for(int s = 0; s < 2; s++)
+        {
+            ap[s] = g.a + (size_t)((on[s] ? s : 1 - s) * 16) * g.K + kb * 32;
+#pragma unroll
+            for(int j = 0; j < NR; j++)
+            {
+                const size_t row = (size_t)es[s] * g.N + ch0 + j * 16;
+                wp[s][j]         = g.w + row * Kb + lane * 16;
+                sp[s][j]         = g.w_s + (row / 32) * sc_tile + lane * 4;
+                acc[s][j]        = (v4f){0.f, 0.f, 0.f, 0.f};
+            }
+        }
+        v4i wf[NB][2][NR], af[ROWS_IN_LDS ? 1 : NB][2][4];
+        u32 wsc[NB][2][NR];
+        auto load_step = [&](auto BB, int kt) __attribute__((always_inline)) {
+            constexpr int b = decltype(BB)::value;
+#pragma unroll
+            for(int s = 0; s < 2; s++)
+            {
+#pragma unroll
+                for(int j = 0; j < NR; j++)
+                {
+                    wsc[b][s][j] = *(const u32*)(sp[s][j] + (size_t)(kt >> 1) * 256);
+                    wf[b][s][j]  = __builtin_nontemporal_load((const v4i*)(wp[s][j] + (size_t)kt * 1024));
+                }
+                if constexpr(!ROWS_IN_LDS)
+#pragma unroll
+                    for(int i = 0; i < 4; i++)
+                        af[b][s][i] = *(const v4i*)(ap[s] + kt * 128 + i * 8);
+            }
+        };
+        auto step = [&](auto BB, int kt) __attribute__((always_inline)) {
+            constexpr int b = decltype(BB)::value, ab = ROWS_IN_LDS ? 0 : b;
+            if constexpr(ROWS_IN_LDS)
+#pragma unroll
+                for(int s = 0; s < 2; s++)
+#pragma unroll
+                    for(int i = 0; i < 4; i++)
+                        af[0][s][i] = *(const v4i*)((const uint16_t*)red + s * g.K + kt * 128 + kb * 32 + i * 8);
+#pragma unroll
+            for(int s = 0; s < 2; s++)
+#pragma unroll
+                for(int j = 0; j < NR; j++)
+                {
+                    const u32 sb = (wsc[b][s][j] >> (8 * ((kt & 1) * 2 + ((half + j) & 1)))) & 0xFFu;
+                    v8bf wq[4];
+                    expand_fp4(wf[b][s][j], sb, wq);
+#pragma unroll
+                    for(int i = 0; i < 4; i++)
+                        acc[s][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wq[i], __builtin_bit_cast(v8bf, af[ab][s][i]), acc[s][j], 0, 0, 0);
+                }
+            if(kt + NB * NW < KT)
+                load_step(BB, kt + NB * NW);
+        };
+        // (the rows are asked for first: behind the weights they would arrive after them)
+        constexpr int RP = ROWS_IN_LDS ? 4 : 1;       // 16-byte pieces of the two rows a thread brings (K <= 16384)
+        const int pieces = g.K / 8;                   // ... of one row
+        uint4 piece[RP];
+        if constexpr(ROWS_IN_LDS)
+#pragma unroll
+            for(int q = 0; q < RP; q++)
+            {
+                const int i = tid + q * (NW * WAVE), s = i >= pieces ? 1 : 0;
+                piece[q]    = make_uint4(0u, 0u, 0u, 0u);
+                if(i < 2 * pieces)
+                    piece[q] = ((const uint4*)(g.a + (size_t)((on[s] ? s : 1 - s) * 16) * g.K))[i - s * pieces];
+            }
+        static_for<NB>([&](auto BB) __attribute__((always_inline)) {
+            const int kt = wave + decltype(BB)::value * NW;
+            if(kt < KT)
+                load_step(BB, kt);
+        });
+        if constexpr(ROWS_IN_LDS)
+        {
+#pragma unroll
+            for(int q = 0; q < RP; q++)
+                if(tid + q * (NW * WAVE) < 2 * pieces)
+                    ((uint4*)red)[tid + q * (NW * WAVE)] = piece[q];
+            __syncthreads();
+        }
+        for(int kt0 = wave; kt0 < KT; kt0 += NB * NW)
+            static_for<NB>([&](auto BB) __attribute__((always_inline)) {
+                const int kt = kt0 + decltype(BB)::value * NW;
+                if(kt < KT)
+                    step(BB, kt);
+            });
+        if constexpr(ROWS_IN_LDS)
+            __syncthreads();                  // (every wave has read the rows)
+#pragma unroll
+        for(int s = 0; s < 2; s++)
+#pragma unroll
+            for(int j = 0; j < NR; j++)
+                *(v4f*)&red[(((wave * 2 + s) * NR + j) * WAVE + lane) * 4] = acc[s][j];
+    }
+    __syncthreads();
+    // wave j finishes row group j of both slots; the token is column 0 of the products
+    if(wave >= NR || r != 0)
+        return;
+    const int j = wave, ch = ch0 + j * 16 + kb * 4;
+    float out[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for(int s = 0; s < 2; s++)
+    {
+        if(!on[s])
+            continue;
+        v4f sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for(int w = 0; w < NW; w++)
+            sum += *(const v4f*)&red[(((w * 2 + s) * NR + j) * WAVE + lane) * 4];
+        if(g.bias)
+#pragma unroll
+            for(int i = 0; i < 4; i++)
+                sum[i] += bf16_bits_to_f32(g.bias[(size_t)e[s] * g.N + ch + i]);
+        const float rw = g.token_w[s];
+        const u32 lo = pack_bf16x2(sum[0] * rw, sum[1] * rw), hi = pack_bf16x2(sum[2] * rw, sum[3] * rw);
+        out[0] += bf16_bits_to_f32(lo & 0xFFFFu);
+        out[1] += bf16_bits_to_f32(lo >> 16);
+        out[2] += bf16_bits_to_f32(hi & 0xFFFFu);
+        out[3] += bf16_bits_to_f32(hi >> 16);
+    }
+    if(g.out_f32)
+        *(float4*)((float*)g.out + ch) = make_float4(out[0], out[1], out[2], out[3]);
+    else
+        *(uint2*)(g.out + ch) = make_uint2(pack_bf16x2(out[0], out[1]), pack_bf16x2(out[2], out[3]));
+}
+
 // split_k: 0 = decide here, 1 = never, 4 / 16 = always that many waves per 64-row tile, 32 = sixteen waves per 32-row
 // tile with three K-steps in flight (down GEMM; the gate_up GEMM takes 16 instead)
 template <int STAGE>
@@ -470,6 +649,45 @@ extern "C" int pyhip_moe_gemm2_w4a16_token(const void* a2_bf16, const uint8_t* w
     g.token_ids = topk_ids; g.token_w = topk_weights; g.expert_mask = expert_mask; g.num_local_tok = num_local_tokens;
     g.experts = experts;
     return launch_w4a16<2>(g, 16, topk, topk, experts, split_k, stream);
+}
+
+// The down GEMM of a top-2 token together with the sum over its slots: out [hidden], bf16 or fp32.  -1 when the launch is not
+// one that it serves (another top-k, a K split that was asked for and that it does not have): the caller then takes
+// pyhip_moe_gemm2_w4a16_token and the reduction, which compute the same bits.
+int pyhip_w4a16_token_top2(const void* a2_bf16, const uint8_t* w2, const uint8_t* w2_scale, const void* bias2_bf16,
+                           const int32_t* topk_ids, const float* topk_weights, const int32_t* expert_mask,
+                           const int32_t* num_local_tokens, void* out, int out_is_f32, int topk, int experts, int hidden,
+                           int inter, int split_k, hipStream_t stream)
+{
+    if(topk != 2 || hidden % 256 != 0 || inter % 512 != 0 || (split_k != 0 && split_k != 4 && split_k != 32))
+        return -1;
+    PYHIP_REQUIRE(((uintptr_t)a2_bf16 % 16) == 0 && ((uintptr_t)w2 % 16) == 0 && ((uintptr_t)w2_scale % 4) == 0 &&
+                      ((uintptr_t)out % 16) == 0,
+                  "moe_gemm2_w4a16_token: unaligned pointer");
+    // the split that launch_w4a16 takes for this launch (two blocks of hidden / 256 tiles)
+    int split = split_k;
+    if(split == 0 && 2 * (hidden / 256) >= 2048)
+        return -1;
+    if(split == 0)
+        split = (2 * (hidden / 256) * 4 < 256 && inter >= 8192) ? 32 : 4;
+    // (sixteen waves: a K-step for each, and the two rows in the LDS that a kernel gets without asking)
+    if(split == 32 && (inter < 2048 || inter > 16384))
+        return -1;
+    const size_t sums = (split == 32 ? 16 * 2 : 4 * 4) * WAVE * 16, rows = split == 32 ? (size_t)inter * 4 : 0;
+    const size_t lds  = sums > rows ? sums : rows;
+    W4A16Args g;
+    g.a = (const uint16_t*)a2_bf16; g.w = w2; g.w_s = w2_scale; g.bias = (const uint16_t*)bias2_bf16;
+    g.sorted_ids = nullptr; g.sorted_w = nullptr; g.sorted_e = nullptr; g.num_valid = nullptr;
+    g.out = (uint16_t*)out; g.T = 1; g.topk = topk; g.K = inter; g.N = hidden; g.SC = (inter / 32 + 7) / 8 * 8; g.n_tiles = 0;
+    g.act = make_gated_act(0, 0.f);
+    g.token_ids = topk_ids; g.token_w = topk_weights; g.expert_mask = expert_mask; g.num_local_tok = num_local_tokens;
+    g.experts = experts; g.out_f32 = out_is_f32;
+    if(split == 32)
+        hipLaunchKernelGGL((moe_gemm_w4a16_top2_kernel<32>), dim3(hidden / 16), dim3(1024), lds, stream, g);
+    else
+        hipLaunchKernelGGL((moe_gemm_w4a16_top2_kernel<4>), dim3(hidden / 32), dim3(W4A16_THREADS), lds, stream, g);
+    PYHIP_CHECK_LAUNCH("moe_gemm_w4a16_top2_kernel");
+    return PYHIP_OK;
 }
 
 extern "C" int pyhip_moe_gemm2_w4a16(const void* a2_bf16, const uint8_t* w2, const uint8_t* w2_scale,
