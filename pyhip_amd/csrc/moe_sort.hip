@@ -252,7 +252,7 @@ __device__ __forceinline__ void fill_blocks(const SortArgs& a, const u32* tot, c
 //   sched[e], e = 0..E   : number of row blocks of the experts before e (sched[E] = all row blocks); the row blocks
 //                          of expert e are sched[e] .. sched[e+1]-1
 //   sched[E + 1 + e]     : local id of expert e (its index among the unmasked experts)
-// A GEMM orders its tiles expert -> weight tile -> row block and cuts that list into 8 equal runs, one per XCD
+// A GEMM orders its tiles expert -> weight tile -> row block and cuts that list into 8 equal shares, one per XCD
 // (moe_gemm_mxfp4.hip), so the XCDs get the same number of tiles however unevenly the router loads the experts.
 __device__ __forceinline__ void write_schedule(const SortArgs& a, const u32* off, const u32* lid, u32 padded_total)
 {
