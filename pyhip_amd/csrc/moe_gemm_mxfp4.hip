@@ -424,8 +424,11 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
             {
                 if((unsigned long long)ga.bias & 3)      // (only element-aligned: fetch_bias left them to ordinary loads)
                 {
-                    const int c = fresh_lane();
-                    ((uint16_t*)lds_bias[wave])[c] = ga.bias[(size_t)t.e * ga.N + bias_row(t) + bias_lane(c, ga.N)];
+                    // a dword at a time, the type that the array has and is read as: nothing keeps the reads below behind
+                    // a store of another type
+                    const int c       = fresh_lane() & 31;
+                    const uint16_t* b = ga.bias + (size_t)t.e * ga.N + bias_row(t) + bias_lane(c * 2, ga.N);
+                    lds_bias[wave][c] = (u32)b[0] | (u32)b[1] << 16;
                 }
                 gemm_epilogue<STAGE, MT, ACT, ATOMIC, true>(ga, t.nt, t.m_blk * BM, wave, meta, MPAD, ma_t, r, kb, bias4, xacc);
             }

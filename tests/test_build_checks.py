@@ -93,6 +93,15 @@ def test_compiler_never_uses_m0(gemm_asm):
         assert hand, name
 
 
+def test_lds_is_written_in_the_dwords_it_is_read_in(four_wave_asm):
+    """The four-wave kernels' LDS arrays are dwords and are read as such.  A 16-bit store into them (the biases of a tensor that
+    is only element-aligned went that way) is of a type that the compiler may move behind those reads."""
+    _, kernels = four_wave_asm
+    for name, body in kernels:
+        narrow = [line for line in _instructions(body) if re.match(r"ds_write_b(?:8|16)\b", line)]
+        assert not narrow, (name, narrow)
+
+
 def _instructions(body):
     for line in body.split("\n"):
         code = line.split(";")[0].strip()
