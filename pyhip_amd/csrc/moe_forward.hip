@@ -107,11 +107,18 @@ extern "C" int pyhip_moe_pick_block_m(int64_t tokens, int topk, int experts, int
         for(int bm = 16; bm <= 64; bm *= 2)
             if(2 * est <= bm)
                 return bm;
-        // one block of 64 rows holds an expert as long as few experts have more than that (layer, us, 64 / 128 rows; 16 experts,
-        // top-2, 4096 x 3584: 34 rows per expert 79.0 / 83.0, 48: 80.7 / 84.5, 56: 100.2 / 87.0; Mixtral shape: 40: 147.9 / 155.5,
-        // 48: 149.7 / 158.8, 56: 170.6 / 163.5; under a Zipf router the 16 experts 34: 102.8 / 99.5, 40: 104.2 / 101.4,
-        // 48: 104.3 / 111.1, and 8 experts of 5120 x 2048 44.9 / 50.2, 45.5 / 51.9, 47.1 / 50.7)
-        if(!w4a16 && est <= 50)
+        // One block of 64 rows holds an expert as long as few experts have more than that, which the mean tells with up to 16
+        // experts and up to 44 rows.  Layer, us, 64 / 128 rows, by rows per expert (even router; Zipf router, two seeds):
+        //    8 experts, 4096 x 14336:  34: 145 / 153; 171 / 167, 170 / 168      40: 154 / 162; 171 / 169, 170 / 170
+        //                              48: 156 / 163; 176 / 176, 175 / 175      50: 169 / 164; 180 / 176, 178 / 174
+        //   12 experts, 5120 x 2048:   34: 48.5 / 51.5; 56.0 / 64.2, 56.0 / 63.6   42: 50.2 / 53.0; 57.4 / 65.0, 57.3 / 64.5
+        //                              48: 51.0 / 54.3; 74.1 / 66.2, 75.8 / 65.8
+        //   16 experts, 4096 x 3584:   34: 77.0 / 82.1; 98.9 / 99.6, 99.9 / 98.6   40: 79.0 / 84.5; 101 / 98.5, 102 / 101
+        //                              44: 78.7 / 83.6; 102 / 110, 101 / 98.5      50: 87.1 / 84.5; 105 / 111, 106 / 110
+        //   28 experts, 2048 x 4096:   34: 81.4 / 86.1; 101 / 91.3, 102 / 91.5     46: 82.6 / 87.4; 103 / 92.0, 105 / 89.2
+        // (5-7 % under even routers against 3 % at most under Zipf ones; with more experts, or nearer to 64 rows, the busy ones
+        // need a second block and cost up to 17 %)
+        if(!w4a16 && experts <= 16 && est <= 44)
             return 64;
     }
     else

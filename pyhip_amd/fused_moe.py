@@ -78,7 +78,7 @@ def _shuffled_u8(w):
 def pick_block_m(tokens, topk, experts, hidden=0, w4a16=False):
     """M-tile (= sort block size), from the expected rows per expert ``est = tokens * topk / experts``: 16 rows below 4,
     32 below 12, 64 up to 32, 128 above (layers with fewer than 32 experts: the smallest of 16 / 32 / 64 that holds
-    twice ``est``).  Every extra row block of an expert streams the expert's weights once more,
+    twice ``est``, and 64 up to 44 with at most 16 experts).  Every extra row block of an expert streams the expert's weights once more,
     routing is uneven enough that a tile of just the mean size overflows for about half of the experts, and the rows a
     larger tile leaves empty fetch nothing (DS-V3 shape: T = 1024: 64-row tiles 1.20 ms against 1.27 ms with 32;
     T = 2048: 128-row tiles 1.27 ms against 1.39 ms with 64).  The ladder sits one step above "twice the mean" at decode
