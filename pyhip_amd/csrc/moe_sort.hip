@@ -381,7 +381,8 @@ extern "C" __global__ void __launch_bounds__(SMALL_THREADS) moe_sort_small_cols_
 //   256 experts, top-8:  2400 pairs 14.5 / 8.5; 8192: 15.2 / 9.0; 16384: 15.4 / 9.8; 65536: 20.7 / 14.6; 131072: 26.8 / 21.9; 262144: 39.5 / 37.0
 //   8 experts, top-2:    4096 pairs 11.3 / 5.9; 16384: 13.0 / 7.5; 65536: 17.3 / 12.3
 //   128 experts, top-8, Zipf: 8192 pairs 13.3 / 7.3; 65536: 18.8 / 13.6; 131072: 24.3 / 21.1; 262144: 36.6 / 37.3
-// Beyond COUNT_PAIRS_MAX the reads grow with the square of the pairs and the three launches win (524288 pairs: 101-121 us here).
+// The reads grow with the square of the pairs: at twice COUNT_PAIRS_MAX the two tie, beyond that the three launches win (524288
+// pairs: 101-121 us here).
 // At 2048 pairs the single workgroup takes 9.6 us with 256 experts, this 8.1; below about 1500 pairs it is the faster one.
 // At least COUNT_WGS_MIN workgroups, because the padding entries are theirs to write as well (2400 pairs: 10.7 us with three).
 // The counters come in COUNT_COPIES, a lane's copy next to its neighbour's: with few experts, or under a router that prefers some,
@@ -762,7 +763,7 @@ static int sorting_impl(const int32_t* topk_ids, const float* topk_weights, int 
                            (unsigned char*)moe_out + n16 * 16, ntail);
         PYHIP_CHECK_LAUNCH("moe_zero_kernel");
     }
-    // workgroups that quantise, riding on the single-workgroup launch of either path
+    // workgroups that quantise ride on the sort's one launch, or on the scan's where there are three
     const long long qwork = qa.rows * qa.SK;
     PYHIP_REQUIRE((qwork + SMALL_THREADS - 1) / SMALL_THREADS < (1ll << 31) - 1, "moe_sorting: too many rows to quantise");
     const unsigned qblocks = (unsigned)((qwork + SMALL_THREADS - 1) / SMALL_THREADS);
@@ -787,7 +788,7 @@ static int sorting_impl(const int32_t* topk_ids, const float* topk_weights, int 
         return PYHIP_OK;
     }
     // one launch while counting everything in every workgroup costs less than the two launches it saves, and while the counters
-    // fit the LDS that a kernel gets without asking (606 experts)
+    // fit the LDS that a kernel gets without asking (605 experts: 65476 bytes)
     const size_t count_lds = ((size_t)(SMALL_WAVES + 2 * COUNT_COPIES + 3) * experts + 2 * SMALL_WAVES + 2) * 4;
     if(pairs <= COUNT_PAIRS_MAX && count_lds <= 64 * 1024)
     {

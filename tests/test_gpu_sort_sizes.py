@@ -12,8 +12,9 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("T,k,E,Bm,offset,masked", [
     (2049, 1, 8, 16, 0, False),            # one pair more than the single workgroup takes; a last group of one
     (683, 3, 12, 32, 1, True),             # pairs no multiple of four, ids that start 4 bytes into 16
-    (1024, 8, 606, 64, 0, False),          # most experts that the counters have LDS for
-    (1024, 8, 607, 64, 0, True),           # three launches for one expert more
+    (1024, 8, 605, 64, 0, False),          # most experts that the counters have LDS for
+    (1024, 8, 605, 64, 2, True),
+    (1024, 8, 606, 64, 0, True),           # three launches for one expert more
     (16384, 8, 64, 160, 0, True),          # most pairs of the one launch: every workgroup's chunk is full
     (16384, 8, 64, 160, 3, False),
     (131073, 1, 16, 288, 0, False),        # three launches for one pair more
