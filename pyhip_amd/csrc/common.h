@@ -125,8 +125,8 @@ __device__ __forceinline__ u32 amax15_fold(u32 w)
 }
 
 // eight bf16 (one uint4) over the block's power of two -> eight e2m1 codes in one dword.  The instruction takes its scale as an
-// exponent byte and divides exactly: the same codes as scaling in fp32 and converting from there (all 65536 bf16 values against
-// all scale bytes 0..253, infinities and NaNs included), in 4 instructions instead of 20.
+// exponent byte and divides exactly: the same codes as scaling in fp32 and converting from there, in 4 instructions instead of 20.
+// Infinities and NaNs become 6 of their sign, as they did there.
 __device__ __forceinline__ u32 cvt8(uint4 v, u32 e8)
 {
     const float scale = __builtin_bit_cast(float, e8 << 23);
