@@ -326,11 +326,15 @@ __global__ void __launch_bounds__(SPLIT >= 16 ? 1024 : W4A16_THREADS) moe_gemm_w
 
 // The down GEMM of a single token whose workgroups hold both slots of a top-2 layer: the token's output is then complete in
 // the workgroup, so it sums the slots and writes the layer's output, and the reduction's launch is left out.  A wave's row groups are
-// RG / 2 groups of 16 weight rows of either slot's expert, so the grid, the K split and what a wave keeps in flight are
-// those of moe_gemm_w4a16_kernel<2, 1, SPLIT> (whose tiles are twice as wide and one slot deep), and so is the arithmetic: partial
+// NR groups of 16 weight rows of either slot's expert, so the grid and the K split are those of
+// moe_gemm_w4a16_kernel<2, 1, SPLIT> (whose tiles are twice as wide and one slot deep), and so is the arithmetic: partial
 // sums of the same K-steps in the same order, a slot's value rounded to bf16 after its routing weight, slots added in order in
 // fp32.  Bound: latency.  Kernel times, us, down GEMM + reduction / this: Mixtral shape (sixteen waves) 12.7 + 4.1 / 13.1, tiny
 // layer (four waves) 4.0 + 3.4 / 3.4; the layer 38.5 / 37.0 and 17.6 / 15.8.
+// Four waves keep two K-steps in flight, one fewer than moe_gemm_w4a16_kernel does.  Layer, us, two launches / this / this with
+// three K-steps (hidden x inter): 1024 x 512 20.3 / 16.4 / 16.7; 2048 x 1024 20.2 / 17.4 / 16.8; 4096 x 3584 20.5 / 17.5 / 17.2;
+// 4096 x 7168 28.0 / 26.7 / 26.4; 5120 x 7168 31.0 / 31.2 / 28.7 (30.1-31.1 / 28.9-31.3 / 28.7-29.1); 7168 x 2048 21.3 / 18.9 / 19.0;
+// 8192 x 14336 68.3 / 66.4 / 66.1; 16384 x 4096 43.7 / 41.4 / 41.9.
 template <int SPLIT>
 __global__ void __launch_bounds__(SPLIT == 32 ? 1024 : W4A16_THREADS) moe_gemm_w4a16_top2_kernel(W4A16Args g)
 {
@@ -502,8 +506,23 @@ __global__ void __launch_bounds__(SPLIT == 32 ? 1024 : W4A16_THREADS) moe_gemm_w
         *(uint2*)(g.out + ch) = make_uint2(pack_bf16x2(out[0], out[1]), pack_bf16x2(out[2], out[3]));
 }
 
-// split_k: 0 = decide here, 1 = never, 4 / 16 = always that many waves per 64-row tile, 32 = sixteen waves per 32-row
-// tile with three K-steps in flight (down GEMM; the gate_up GEMM takes 16 instead)
+// The K split of a launch of `tiles` tiles of 256 weight rows.  split_k: 0 = decide here, 1 = never, 4 / 16 = always that many
+// waves per 64-row tile, 32 = sixteen waves per 32-row tile with three K-steps in flight (down GEMM; the gate_up GEMM takes 16
+// instead)
+static int w4a16_split(int stage, int block_m, int64_t tiles, int K, int split_k)
+{
+    if(split_k == 0 && tiles < 2048)
+        // sixteen waves when the four-way split would still start fewer workgroups than there are CUs and the K loop
+        // is long enough to matter (Mixtral shape, one token: the layer 54.0 -> 49.7 us; forced onto the gate_up GEMM as well,
+        // which already starts 896 workgroups there, 57.5 us)
+        // (the down GEMM then takes the sixteen-wave split on 32-row tiles with three K-steps in flight, split 32:
+        // Mixtral shape, one token, the down GEMM 16.9 -> see the measurements in the kernel's comment)
+        return (tiles * 4 < 256 && K >= 8192 && block_m == 16) ? (stage == 2 ? 32 : 16) : 4;
+    if(stage == 1 && split_k == 32)       // (the 32-row tile exists for the down GEMM: gate_up takes sixteen waves, or four)
+        return K >= 2048 ? 16 : 4;
+    return split_k == 1 ? 0 : split_k;
+}
+
 template <int STAGE>
 static int launch_w4a16(W4A16Args g, int block_m, int64_t n_blk, int64_t rows, int experts, int split_k,
                         hipStream_t stream)
@@ -512,16 +531,7 @@ static int launch_w4a16(W4A16Args g, int block_m, int64_t n_blk, int64_t rows, i
     int64_t blocks = rows < n_blk ? rows : n_blk;
     if(experts + rows / block_m < blocks)
         blocks = experts + rows / block_m;
-    int split = split_k == 1 ? 0 : split_k;
-    if(STAGE == 1 && split == 32)       // (the 32-row tile exists for the down GEMM: gate_up takes sixteen waves, or four)
-        split = g.K >= 2048 ? 16 : 4;
-    if(split_k == 0 && blocks * g.n_tiles < 2048)
-        // sixteen waves when the four-way split would still start fewer workgroups than there are CUs and the K loop
-        // is long enough to matter (Mixtral shape, one token: the layer 54.0 -> 49.7 us; forced onto the gate_up GEMM as well,
-        // which already starts 896 workgroups there, 57.5 us)
-        // (the down GEMM then takes the sixteen-wave split on 32-row tiles with three K-steps in flight, split 32:
-        // Mixtral shape, one token, the down GEMM 16.9 -> see the measurements in the kernel's comment)
-        split = (blocks * g.n_tiles * 4 < 256 && g.K >= 8192 && block_m == 16) ? (STAGE == 2 ? 32 : 16) : 4;
+    const int split = w4a16_split(STAGE, block_m, blocks * g.n_tiles, g.K, split_k);
     // (sixteen waves of a workgroup share the register file four to a SIMD: 128 registers each, which only the 16-row
     // tile fits into; and every wave needs a K-step of its own)
     if(split >= 16 && (g.K < 2048 || block_m != 16))
@@ -659,20 +669,16 @@ int pyhip_w4a16_token_top2(const void* a2_bf16, const uint8_t* w2, const uint8_t
                            const int32_t* num_local_tokens, void* out, int out_is_f32, int topk, int experts, int hidden,
                            int inter, int split_k, hipStream_t stream)
 {
-    if(topk != 2 || hidden % 256 != 0 || inter % 512 != 0 || (split_k != 0 && split_k != 4 && split_k != 32))
+    if(topk != 2 || hidden % 256 != 0 || inter % 512 != 0)
+        return -1;
+    // the split of the launch that this one replaces: a 16-row block for either slot
+    const int split = w4a16_split(2, 16, 2 * (hidden / 256), inter, split_k);
+    // (sixteen waves: a K-step for each, and the two rows in the LDS that a kernel gets without asking)
+    if((split != 4 && split != 32) || (split == 32 && (inter < 2048 || inter > 16384)))
         return -1;
     PYHIP_REQUIRE(((uintptr_t)a2_bf16 % 16) == 0 && ((uintptr_t)w2 % 16) == 0 && ((uintptr_t)w2_scale % 4) == 0 &&
                       ((uintptr_t)out % 16) == 0,
                   "moe_gemm2_w4a16_token: unaligned pointer");
-    // the split that launch_w4a16 takes for this launch (two blocks of hidden / 256 tiles)
-    int split = split_k;
-    if(split == 0 && 2 * (hidden / 256) >= 2048)
-        return -1;
-    if(split == 0)
-        split = (2 * (hidden / 256) * 4 < 256 && inter >= 8192) ? 32 : 4;
-    // (sixteen waves: a K-step for each, and the two rows in the LDS that a kernel gets without asking)
-    if(split == 32 && (inter < 2048 || inter > 16384))
-        return -1;
     const size_t sums = (split == 32 ? 16 * 2 : 4 * 4) * WAVE * 16, rows = split == 32 ? (size_t)inter * 4 : 0;
     const size_t lds  = sums > rows ? sums : rows;
     W4A16Args g;
