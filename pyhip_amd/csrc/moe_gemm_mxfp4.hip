@@ -116,9 +116,15 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
     // experts are neighbours, equal runs give some XCDs only long tiles, and pieces in the same order have all XCDs multiply
     // first and wait for memory together afterwards.  Layer, us, runs / pieces from the first on / each XCD from its own:
     // Qwen3 shape, Zipf router, 2048 tokens (160 rows) 410.7 / 396.8 / 382, 2400 (128 rows) 416 / 420 / 400; 160 experts, top-6,
-    // 5120 x 1536, Zipf, 4000 tokens 583 / 602 / 562; gpt-oss shape, 4700 tokens 602 / 573 / 571.  With fewer than 32 experts a
-    // share is about one of them, and cutting it costs (Mixtral shape, 4096 tokens: 767.5 / 773.6); the smaller tiles are
-    // bound by the weights in any case (decode sizes 0.2-0.6 % slower in pieces).
+    // 5120 x 1536, Zipf, 4000 tokens 583 / 602 / 562; gpt-oss shape, 4700 tokens 602 / 573 / 571.  Even routers pay for it where
+    // experts have several full blocks (runs / pieces: 128 experts, 4096 x 1536, 4096 tokens 508 / 516; 96 experts, 4096 x 2048,
+    // 8192 tokens 1057 / 1063; 32 experts, 2880 x 2880, 4700 tokens 340 / 350) and the rule cannot see which it has.  In layers of
+    // fewer than 32 experts, where a share is about one expert, what pieces lose there is as much as they gain under Zipf ones
+    // (4096 x 3584, even router, Zipf router: 12 experts, 4096 tokens 406.8 / 410.2; 16, 8192 tokens 433.2 / 435.9, 460.2 / 446.5;
+    // 24, 8192 tokens 797.4 / 813.7, 851.1 / 837.5; 32, 8192 tokens 836.0 / 830.3, 869.4 / 854.6).
+    // The count is the layer's, also on a rank that holds few of them: 8 of 64 254.8 / 248.9, 358.2 / 353.6; 12 of 96 (4096 x
+    // 2048) 180.7 / 180.7, 210.0 / 205.5; 16 of 64 433.7 / 437.4 (ranges overlap), 265.1 / 259.6.  The smaller tiles are bound by the
+    // weights in any case (decode sizes 0.2-0.6 % slower in pieces).
     // Without a schedule (or when K has a single K-group): one tile per workgroup, weight tile fastest.
     constexpr bool PIECES = MT >= 8;
     const bool persistent = g.sched != nullptr;
@@ -619,8 +625,8 @@ __global__ void __launch_bounds__(GEMM_THREADS, (MT > 8 ? 1 : 2)) moe_gemm_mxfp4
                     constexpr int j = decltype(J)::value;          // the gap; the weight row group is w
                     // (to and fro: the first MFMA of a row group takes the weight tile of the last one before it, so that one
                     // operand changes from MFMA to MFMA and not both.  What toggles costs power, and power is what bounds these
-                    // kernels: the MFMA stream alone sustains 1.7 % more, the whole pattern of the 288-row tile 0.8 % (weights
-                    // from HBM) to 2.6 % (from the L2).)
+                    // kernels at prefill sizes: layer, us, before -> after, Mixtral shape, 4096 tokens 767.5 -> 763.0; DeepSeek-V3
+                    // shape, 8192 tokens 1921.9 -> 1914.2.)
                     constexpr int w = n & 1 ? 3 - j : j;
                     v4f* xa = nullptr;
                     if constexpr(acc_in_vgprs<MT, mt>() && w == 3)

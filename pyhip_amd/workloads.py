@@ -115,13 +115,16 @@ def algorithmic_work(shape, tokens, topk_ids):
 
 def xcd_tile_counts(shape, topk_ids, block_m, pad=0):
     """gate_up tiles per XCD for a routing: under the grouped GEMMs' schedule (the list expert -> weight tile -> row
-    block cut into 8 equal runs) and, for comparison, with whole experts dealt to the XCDs round-robin (e % 8)"""
+    block, of which each XCD gets one run or, in tiles of 128 rows and more and layers of 32 and more experts, up to
+    eight pieces dealt round-robin) and, for comparison, with whole experts dealt to the XCDs round-robin (e % 8)"""
     cfg = SHAPES[shape] if isinstance(shape, str) else shape
     cnt = torch.bincount(topk_ids.flatten().long().clamp(0, cfg["E"] - 1), minlength=cfg["E"]).cpu()
     nb = (cnt + block_m - 1) // block_m
     n_tiles = (cfg["I"] + pad + 127) // 128
     total = int(nb.sum()) * n_tiles
-    chunk = (total + 7) // 8
-    return dict(equal_runs=[min(chunk, max(0, total - x * chunk)) for x in range(8)],
+    pieces = 1 if block_m < 128 or cfg["E"] < 32 or total < 1024 else min(8, total // 512)
+    size = -(-total // (8 * pieces))
+    return dict(equal_shares=[sum(min(size, max(0, total - (8 * p + x) * size)) for p in range(pieces)) for x in range(8)],
+                pieces=pieces,
                 experts_round_robin=[int(nb[x::8].sum()) * n_tiles for x in range(8)],
                 rows_per_expert_max=int(cnt.max()), rows_per_expert_median=int(cnt.median()))

@@ -22,7 +22,7 @@ def _arguments(name):
             for k in meta["amdhsa.kernels"]}
 
 
-SORT, QUANT, ROUTE = 104, 56, 40       # SortArgs, QuantArgs, RouteArgs
+SORT, QUANT, ROUTE, W4A16 = 104, 56, 40, 152       # SortArgs, QuantArgs, RouteArgs, W4A16Args
 
 
 def test_quantiser_struct():
@@ -36,6 +36,13 @@ def test_sort_structs():
     assert len(routed) == 9 and all(v == [SORT, QUANT, ROUTE] for v in routed.values())
     assert got["moe_sort_hist_kernel"] == [SORT] and got["moe_sort_scatter_kernel"] == [SORT]
     assert got["moe_sort_scan_kernel"] == [SORT, QUANT]
+    assert got["moe_sort_count_kernel"] == got["moe_sort_small_cols_kernel"] == got["moe_sort_scan_cols_kernel"] == [SORT, QUANT, 4]
+
+
+def test_bf16_activation_struct():
+    got = _arguments("moe_gemm_w4a16")
+    assert sum("moe_gemm_w4a16_top2_kernel" in k for k in got) == 2 and len(got) == 17
+    assert all(v == [W4A16] for v in got.values())
 
 
 def test_mirrored_structs():

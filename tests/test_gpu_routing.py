@@ -79,10 +79,11 @@ def test_routed_layer_end_to_end():
     assert (a - b).abs().max().item() <= 1e-4 * rms          # only the fp32 routing weights differ
 
 
-@pytest.mark.parametrize("T,router,method", [(1, "grouped", "w4a16"), (16, "grouped", "auto"), (64, "softmax", "a4w4"),
-                                             (65, "softmax", "a4w4"), (300, "grouped", "a4w4")])
+@pytest.mark.parametrize("T,router,method", [(1, "grouped", "w4a16"), (7, "softmax", "a4w4"), (8, "softmax", "a4w4"),
+                                             (16, "grouped", "auto"), (64, "softmax", "a4w4"), (65, "softmax", "a4w4"),
+                                             (300, "grouped", "a4w4")])
 def test_router_inside_the_layer_call(T, router, method):
-    """fused_moe_routed (router + sort + GEMMs + reduce behind one library call; up to 64 tokens the sort's own
+    """fused_moe_routed (router + sort + GEMMs + reduce behind one library call; up to 7 tokens the sort's own
     workgroup routes the tokens, beyond that the router has its launch) gives, bit for bit, the picks of the
     stand-alone router and the output of fused_moe on those picks."""
     import cases
