@@ -54,6 +54,12 @@ SIGNATURES = {
     "pyhip_moe_topk_reduce_routed": (_I, [_P, _P, _L, _I, _I, _I, _P, _I, _P, _P, _P]),
 }
 
+#: what fused_moe.py calls and the header does not declare: the layer call as one block of arguments
+INTERNAL = {
+    "pyhip_layer_forward": (_I, [_c.c_char_p, _P]),
+    "pyhip_layer_takes_cols": (_I, [_L, _I, _I, _I, _I, _I, _I, _I]),
+}
+
 _lib = None
 
 
@@ -69,7 +75,7 @@ def load():
                 "%s is missing: build it with `python -m pyhip_amd.build` (needs hipcc); "
                 "there is no fallback path" % LIB_PATH)
         lib = ctypes.CDLL(LIB_PATH)
-        for name, (res, args) in SIGNATURES.items():
+        for name, (res, args) in [*SIGNATURES.items(), *INTERNAL.items()]:
             fn = getattr(lib, name)
             fn.restype, fn.argtypes = res, args
         _lib = lib
@@ -86,6 +92,11 @@ def addr(t):
     """device address of a torch tensor (or None) as a plain integer, the cheapest form of a pointer: only for functions
     whose ``argtypes`` say ``c_void_p``, as those of ``load()`` do (ctypes cuts an integer to 32 bits without them)"""
     return None if t is None else t.data_ptr()
+
+
+def address(t):
+    """the same for a packed block of arguments, where None is 0"""
+    return 0 if t is None else t.data_ptr()
 
 
 def stream_handle():

@@ -3,6 +3,7 @@
 // step by step (the reference's operator, src/contrib/fused_moe.py:128-576, allocates its intermediates with torch
 // and launches its kernels one by one from Python); the choice of kernel family and row block stays with the caller.
 #include "common.h"
+#include "moe_gemm_pairs.h"
 
 extern "C" {
 int64_t pyhip_moe_sorting_max_blocks(int64_t tokens, int topk, int experts, int block_size);
@@ -30,6 +31,8 @@ int pyhip_moe_route_sorting(const float*, int, int, int, int, int, int, int, con
                             int, uint8_t*, uint8_t*, hipStream_t);
 int pyhip_moe_topk_reduce_routed(const void*, void*, int64_t, int, int, int, const int32_t*, int, const int32_t*,
                                  const int32_t*, hipStream_t);
+int pyhip_moe_topk_softmax(const float*, int, int, int, int, float*, int32_t*, hipStream_t);
+int pyhip_moe_topk_grouped_sigmoid(const float*, int, int, int, int, int, int, float*, int32_t*, hipStream_t);
 }
 
 int pyhip_sorting_quant_cols(const int32_t*, const float*, int, int, int, int, const int32_t*, const int32_t*, uint32_t*,
@@ -195,14 +198,92 @@ struct Router
 };
 }   // namespace
 
+// Whether forward_pairs below serves the call
+static bool takes_pairs(int64_t tokens, int topk, int experts, int hidden, int inter, int block_m, int w4a16, int split_k)
+{
+    return w4a16 && block_m == 16 && hidden % 512 == 0 && inter % 512 == 0 && topk > 0 && experts <= 2048 &&
+           pyhip_pairs_served(tokens, topk, experts, hidden, inter, pyhip_moe_sorting_max_blocks(tokens, topk, experts, 16), split_k);
+}
+
+// The layer with bf16 activations and 16-row blocks (moe_gemm_pairs.hip).  Up to 64 pairs the kernels find their rows themselves
+// and the sort is left out; where pairs rarely share an expert the down GEMM sums the slots and the reduction is left out too: two
+// launches (with the router three) instead of four.  What that saves is the launch on the host (3.3 us each) and the latency chain of the stage
+// on the device (sort 4.5-5.5, reduction 3-5 us).
+static int forward_pairs(const void* hidden_bf16, int64_t row_stride, int hidden_cols, const uint8_t* w1, const uint8_t* w1_scale,
+                         const uint8_t* w2, const uint8_t* w2_scale, const void* bias1_bf16, const void* bias2_bf16,
+                         const Router& router, int32_t* topk_ids, float* topk_weights, const int32_t* expert_mask,
+                         const int32_t* num_local_tokens, void* out, int out_is_f32, int tokens, int topk, int experts,
+                         int hidden, int inter, int hidden_pad, int inter_pad, int split_k, int activation, float swiglu_limit,
+                         const Layout& l, uint8_t* ws, hipStream_t stream)
+{
+    const bool unsorted = (int64_t)tokens * topk <= PAIRS_UNSORTED_MAX;
+    uint32_t* s_ids     = (uint32_t*)(ws + l.sorted_ids);
+    float* s_w          = (float*)(ws + l.sorted_w);
+    uint32_t *s_e = (uint32_t*)(ws + l.sorted_e), *n_valid = (uint32_t*)(ws + l.num_valid), *sched = (uint32_t*)(ws + l.sched);
+    int rc = PYHIP_OK;
+    if(router.gating && unsorted)
+        rc = router.n_group > 0 ? pyhip_moe_topk_grouped_sigmoid(router.gating, tokens, experts, topk, router.n_group, router.topk_group,
+                                                                 router.renormalize, topk_weights, topk_ids, stream)
+                                : pyhip_moe_topk_softmax(router.gating, tokens, experts, topk, router.renormalize, topk_weights, topk_ids, stream);
+    else if(router.gating)
+        rc = pyhip_moe_route_sorting(router.gating, tokens, topk, experts, router.n_group, router.topk_group, router.renormalize, 16,
+                                     expert_mask, num_local_tokens, topk_weights, topk_ids, s_ids, s_w, s_e, n_valid, sched,
+                                     ws + l.sort_ws, l.sort_ws_bytes, nullptr, 0, tokens, hidden, nullptr, nullptr, stream);
+    else if(!unsorted)
+        rc = pyhip_moe_sorting(topk_ids, topk_weights, tokens, topk, experts, 16, expert_mask, num_local_tokens, s_ids, s_w, s_e,
+                               n_valid, sched, nullptr, 0, ws + l.sort_ws, l.sort_ws_bytes, stream);
+    if(rc)
+        return rc;
+    PairArgs g;
+    if(unsorted)
+    {
+        g.ids = topk_ids; g.weights = topk_weights; g.mask = expert_mask; g.local_tok = num_local_tokens;
+    }
+    else
+    {
+        g.sorted_ids = s_ids; g.sorted_w = s_w; g.sorted_e = s_e; g.num_valid = n_valid;
+    }
+    g.T = tokens; g.topk = topk; g.experts = experts;
+    PairArgs up = g, down = g;
+    up.a = (const uint16_t*)hidden_bf16; up.w = w1; up.w_s = w1_scale; up.bias = (const uint16_t*)bias1_bf16;
+    up.out = ws + l.a2; up.K = hidden; up.N = 2 * inter;
+    up.a_pitch = (int)row_stride; up.k_real = hidden_cols ? hidden_cols : hidden - hidden_pad; up.n_pad = inter_pad;
+    down.a = (const uint16_t*)(ws + l.a2); down.w = w2; down.w_s = w2_scale; down.bias = (const uint16_t*)bias2_bf16;
+    down.out = out; down.out_f32 = out_is_f32; down.K = inter; down.N = hidden;
+    down.a_pitch = inter; down.k_real = inter - inter_pad; down.n_pad = hidden_pad;
+    // (the kernel that sums a top-2 token's slots on sixteen waves reads the rows of a2 where the single-token entry points put them)
+    const bool top2 = tokens == 1 && topk == 2;
+    up.row_step = down.row_step = top2 ? 16 : 1;
+    rc = pyhip_pairs_gate_up(up, tokens, l.n_blk, split_k, activation, swiglu_limit, stream);
+    if(rc)
+        return rc;
+    if(top2)
+    {
+        rc = pyhip_w4a16_token_top2(ws + l.a2, w2, w2_scale, bias2_bf16, topk_ids, topk_weights, expert_mask, num_local_tokens,
+                                    out, out_is_f32, topk, experts, hidden, inter, split_k, stream);
+        if(rc >= 0)
+            return rc;
+    }
+    rc = pyhip_pairs_down_sum(down, l.rows2, l.n_blk, split_k, stream);
+    if(rc >= 0)
+        return rc;
+    down.out = ws + l.out3;
+    rc       = pyhip_pairs_down(down, l.rows2, l.n_blk, split_k, stream);
+    if(rc)
+        return rc;
+    return pyhip_moe_topk_reduce_routed(ws + l.out3, out, tokens, topk, hidden, out_is_f32, topk_ids, experts, expert_mask,
+                                        num_local_tokens, stream);
+}
+
 // hidden_cols = 0: the hidden states are at the padded width; otherwise they have hidden_cols columns, and the input
-// quantisation fills in the zeros of the padding
+// quantisation fills in the zeros of the padding (bf16 activations: the GEMM does, and only where bf16_cols allows it)
 static int forward_impl(const void* hidden_bf16, int64_t hidden_row_stride, int hidden_cols, const uint8_t* w1, const uint8_t* w1_scale,
                         const uint8_t* w2, const uint8_t* w2_scale, const void* bias1_bf16, const void* bias2_bf16,
                         const Router& router, int32_t* topk_ids, float* topk_weights, const int32_t* expert_mask,
                         const int32_t* num_local_tokens, void* out, int out_is_f32, int tokens, int topk, int experts,
                         int hidden, int inter, int hidden_pad, int inter_pad, int block_m, int w4a16, int split_k,
-                        int activation, float swiglu_limit, void* workspace, int64_t workspace_bytes, hipStream_t stream)
+                        int activation, float swiglu_limit, void* workspace, int64_t workspace_bytes, hipStream_t stream,
+                        bool bf16_cols = false)
 {
     PYHIP_REQUIRE(hidden_bf16 && w1 && w1_scale && w2 && w2_scale && topk_ids && topk_weights && out,
                   "moe_forward: null pointer");
@@ -210,8 +291,11 @@ static int forward_impl(const void* hidden_bf16, int64_t hidden_row_stride, int 
     PYHIP_REQUIRE(block_m == 16 || block_m == 32 || block_m == 64 ||
                       ((block_m == 128 || block_m == 160 || block_m == 192 || block_m == 256 || block_m == 288) && !w4a16),
                   "moe_forward: block_m=%d (16/32/64, and 128/160/192/256/288 with MXFP4 activations)", block_m);
-    PYHIP_REQUIRE(!w4a16 || hidden_row_stride == hidden, "moe_forward: the bf16-activation kernels need contiguous rows");
-    PYHIP_REQUIRE(hidden_cols == 0 || (!w4a16 && !router.gating && hidden_cols == hidden - hidden_pad && hidden_cols % 32 == 0),
+    const bool pairs = takes_pairs(tokens, topk, experts, hidden, inter, block_m, w4a16, split_k);
+    bf16_cols        = bf16_cols && pairs && hidden_cols > 0 && hidden_row_stride >= hidden_cols && hidden_row_stride % 8 == 0 &&
+                hidden_row_stride < (1 << 24);
+    PYHIP_REQUIRE(!w4a16 || hidden_row_stride == hidden || bf16_cols, "moe_forward: the bf16-activation kernels need contiguous rows");
+    PYHIP_REQUIRE(hidden_cols == 0 || ((!w4a16 || bf16_cols) && !router.gating && hidden_cols == hidden - hidden_pad && hidden_cols % 32 == 0),
                   "moe_forward: hidden_cols=%d (0, or hidden - hidden_pad, a multiple of 32, with MXFP4 activations)", hidden_cols);
     const Layout l = make_layout(tokens, topk, experts, hidden, inter, block_m, w4a16);
     PYHIP_REQUIRE(workspace && workspace_bytes >= l.total && ((uintptr_t)workspace % 256) == 0,
@@ -225,6 +309,10 @@ static int forward_impl(const void* hidden_bf16, int64_t hidden_row_stride, int 
     uint32_t* sched   = (uint32_t*)(ws + l.sched);
     void* out3        = ws + l.out3;
     int rc;
+    if(pairs)
+        return forward_pairs(hidden_bf16, hidden_row_stride, hidden_cols, w1, w1_scale, w2, w2_scale, bias1_bf16, bias2_bf16, router,
+                             topk_ids, topk_weights, expert_mask, num_local_tokens, out, out_is_f32, tokens, topk, experts, hidden,
+                             inter, hidden_pad, inter_pad, split_k, activation, swiglu_limit, l, ws, stream);
     if(w4a16 && tokens == 1 && !router.gating)
     {
         // a single token with bf16 activations: no sort; the GEMMs read the routing themselves, one block per slot
@@ -341,4 +429,34 @@ extern "C" int pyhip_moe_forward_routed(const void* hidden_bf16, int64_t hidden_
                         topk_weights, expert_mask, num_local_tokens, out, out_is_f32, tokens, topk, experts, hidden, inter,
                         hidden_pad, inter_pad, block_m, w4a16, split_k, activation, swiglu_limit, workspace, workspace_bytes,
                         stream);
+}
+
+// The layer call of pyhip_amd/fused_moe.py in one argument, a block that the caller packs (24 pointers and sizes cost ctypes longer
+// one by one).  Also the only entry point that takes hidden states at the true width with bf16 activations
+// (pyhip_layer_takes_cols).
+struct LayerCall
+{
+    const void *x, *w1, *w1_scale, *w2, *w2_scale, *bias1, *bias2, *gating, *topk_ids, *topk_weights, *expert_mask, *num_local_tokens;
+    void *out, *workspace;
+    int64_t row_stride, workspace_bytes;
+    int cols, out_f32, tokens, topk, experts, hidden, inter, hidden_pad, inter_pad, block_m, w4a16, split_k, activation;
+    int n_group, topk_group, renormalize;
+    float swiglu_limit;
+};
+static_assert(sizeof(LayerCall) == 200, "packed by pyhip_amd/fused_moe.py");
+
+extern "C" int pyhip_layer_forward(const LayerCall* c, hipStream_t stream)
+{
+    Router r;
+    r.gating = (const float*)c->gating; r.n_group = c->n_group; r.topk_group = c->topk_group; r.renormalize = c->renormalize;
+    return forward_impl(c->x, c->row_stride, c->cols, (const uint8_t*)c->w1, (const uint8_t*)c->w1_scale, (const uint8_t*)c->w2,
+                        (const uint8_t*)c->w2_scale, c->bias1, c->bias2, r, (int32_t*)c->topk_ids, (float*)c->topk_weights,
+                        (const int32_t*)c->expert_mask, (const int32_t*)c->num_local_tokens, c->out, c->out_f32, c->tokens, c->topk,
+                        c->experts, c->hidden, c->inter, c->hidden_pad, c->inter_pad, c->block_m, c->w4a16, c->split_k, c->activation,
+                        c->swiglu_limit, c->workspace, c->workspace_bytes, stream, true);
+}
+
+extern "C" int pyhip_layer_takes_cols(int64_t tokens, int topk, int experts, int hidden, int inter, int block_m, int w4a16, int split_k)
+{
+    return !w4a16 || takes_pairs(tokens, topk, experts, hidden, inter, block_m, w4a16, split_k);
 }

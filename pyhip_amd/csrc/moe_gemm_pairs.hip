@@ -1,0 +1,488 @@
+// The layer call's GEMMs with bf16 activations and 16-row blocks: few tokens, so the call is a weight stream and a chain of
+// launches.  The arithmetic (and with it every bit of the result) is that of moe_gemm_w4a16.hip, whose entry points serve callers
+// that run the stages one by one; what is different is what a call of 20-100 us spends beside its weights:
+//   * Up to 64 pairs (token, slot) there is no sort: every wave reads the routing, a pair to a lane, and finds its block's
+//     expert and rows with a few ballots (find_block).
+//   * Activations come at their own row pitch and width, and neither the padding rows nor the padding columns of the weights
+//     are fetched (raw buffer loads: a lane or a row group that has nothing to fetch is out of its descriptor's range).
+//   * Where nearly every pair has an expert of its own, the down GEMM goes by token instead of by expert: a workgroup holds
+//     all of a token's slots for 16 or 32 output channels, so it sums them and no reduction follows.
+// Bound: the weight stream from about 40 us on, the launches and their latency chains below.  Layer call, us, sort + moe_gemm_w4a16
+// kernels + reduction (padded layers: after a widening of the activations) / this: gpt-oss shape, 2 tokens 39.5 / 28.7, 5 tokens
+// 67.0 / 51.3 (bound at 6.9 TB/s: 38); 32 experts, top-1, 2144 x 3040, 3 tokens 36.7 / 18.4; 1024 x 512, 8 experts, 10 tokens 25.0 / 17.6;
+// Mixtral shape, 5 tokens 100.6 / 94.5, 29 tokens 129.9 / 124.1 (5.75 -> 6.0 TB/s).
+#include "w4a16_device.h"
+#include "moe_gemm_pairs.h"
+
+#define AUX_NT 2      // streamed once
+
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+__device__ __forceinline__ rsrc_t buffer_of(const void* p, u32 bytes)
+{
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
+}
+__device__ __forceinline__ v4i load16(rsrc_t b, int voff, int soff) { return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(b, voff, soff, 0)); }
+__device__ __forceinline__ v4i load16_nt(rsrc_t b, int voff, int soff) { return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(b, voff, soff, AUX_NT)); }
+__device__ __forceinline__ u32 load4(rsrc_t b, int voff, int soff) { return (u32)__builtin_amdgcn_raw_buffer_load_b32(b, voff, soff, 0); }
+#define NOWHERE ((int)0x80000000)      // an offset past every range; OR-ed, so two of them stay one
+
+// local id of an expert under a mask: the experts this rank holds before it
+__device__ __forceinline__ int local_expert(int e, const int* mask, int lane)
+{
+    if(!mask)
+        return e;
+    int n = 0;
+    for(int i0 = 0; i0 < e; i0 += WAVE)
+        n += __builtin_popcountll(__ballot(i0 + lane < e && mask[i0 + lane] != 0));
+    return __builtin_amdgcn_readfirstlane(n);
+}
+
+// Block m_blk of the unsorted call, or false.  Lane p holds pair p; lanes whose pairs share an expert are found by a ballot for each
+// bit of the expert number; every 16th of them, in pair order, starts a block, and blocks are numbered by the pair that starts them.
+// -> expert (local id) and, in lane r of each 16, the pair of the block's row r (-1: no row)
+__device__ __forceinline__ bool find_block(const PairArgs& g, int m_blk, int lane, int& e, int& pair)
+{
+    int n = g.T * g.topk;
+    if(g.local_tok)
+    {
+        const int lim = *g.local_tok;
+        n             = lim < 0 ? 0 : lim < g.T ? lim * g.topk : n;
+    }
+    const int id    = lane < n ? g.ids[lane] : -1;
+    const bool kept = moe_pair_is_kept(id, g.experts, g.mask);
+    u64 same        = __ballot(kept);
+    for(int b = 0; (g.experts - 1) >> b; b++)
+    {
+        const bool bit = (id >> b) & 1;
+        const u64 s    = __ballot(bit);
+        same &= bit ? s : ~s;
+    }
+    const u64 below  = (1ull << lane) - 1ull;
+    const bool start = kept && (__builtin_popcountll(same & below) & 15) == 0;
+    const u64 starts = __ballot(start);
+    const u64 hit    = __ballot(start && __builtin_popcountll(starts & below) == m_blk);
+    if(!hit)
+        return false;
+    const int lead = __builtin_ctzll(hit);
+    u64 rows = (u64)(u32)__builtin_amdgcn_readlane((int)same, lead) | (u64)(u32)__builtin_amdgcn_readlane((int)(same >> 32), lead) << 32;
+    rows &= ~((1ull << lead) - 1ull);
+    e    = local_expert(__builtin_amdgcn_readlane(id, lead), g.mask, lane);
+    pair = -1;
+    for(int i = 0; i < 16 && rows; i++, rows &= rows - 1ull)
+        pair = (lane & 15) == i ? __builtin_ctzll(rows) : pair;
+    return true;
+}
+
+// the lane's four biases of channels c .. c + 3 (element-aligned tensors: one by one)
+__device__ __forceinline__ uint2 load_bias4(const uint16_t* b)
+{
+    if(((unsigned long long)b & 7) == 0)
+        return *(const uint2*)b;
+    return make_uint2((u32)b[0] | (u32)b[1] << 16, (u32)b[2] | (u32)b[3] << 16);
+}
+__device__ __forceinline__ v4f add_bias4(v4f v, uint2 b)
+{
+    v[0] += bf16_bits_to_f32(b.x & 0xFFFFu);
+    v[1] += bf16_bits_to_f32(b.x >> 16);
+    v[2] += bf16_bits_to_f32(b.y & 0xFFFFu);
+    v[3] += bf16_bits_to_f32(b.y >> 16);
+    return v;
+}
+
+// STAGE 1 = gate_up (+ the gated activation), 2 = down (* routing weight).  SPLIT 0: a wave owns 64 weight rows over the whole K;
+// 4: the four waves share 64 weight rows, wave w takes K-steps w, w + 4, .. and the partial sums meet in LDS.
+// Three K-steps of operands are in flight; a register set is refilled as soon as its MFMAs are issued.
+template <int STAGE, int SPLIT>
+__global__ void __launch_bounds__(W4A16_THREADS) moe_gemm_pairs_kernel(PairArgs g)
+{
+    constexpr bool SPLITK = SPLIT != 0;
+    constexpr int NB = 3, KSTRIDE = SPLITK ? 4 : 1;
+    __shared__ float red[SPLITK ? 4 * 4 * WAVE * 4 : 1];          // [wave][row group][lane][4]
+    const int tid = threadIdx.x, lane = tid % WAVE;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    const int r = lane & 15, kb = lane >> 4;
+    const int m_blk = blockIdx.x / g.n_tiles, nt = blockIdx.x - m_blk * g.n_tiles;
+    const int Kb = g.K / 2, I = g.N / 2;
+    // first output channel of this wave's rows (stage 1: within the gate half; the up half is I further)
+    const int chbase = STAGE == 1 ? (SPLITK ? nt * 32 : nt * 128 + wave * 32) : (SPLITK ? nt * 64 : nt * 256 + wave * 64);
+    if(STAGE == 1 && chbase >= I - g.n_pad)      // (channels of padding: the down GEMM does not read them)
+        return;
+    // the block's expert, and for row r: the activation row, the output row, the routing weight
+    int e, arow = -1, orow = 0;
+    float rw = 0.f;
+    if(g.ids)
+    {
+        int pair;
+        if(!find_block(g, m_blk, lane, e, pair))
+            return;
+        if(pair >= 0)
+        {
+            arow = STAGE == 1 ? (int)((u32)pair / (u32)g.topk) : pair * g.row_step;
+            orow = STAGE == 1 ? pair * g.row_step : pair;
+            if(STAGE == 2)
+                rw = g.weights[pair];
+        }
+    }
+    else
+    {
+        // (all read together: the arrays are there for every block that is launched, whether or not it holds rows)
+        const int p  = m_blk * 16 + r;
+        const u32 id = g.sorted_ids[p], last = g.num_valid[0];
+        e            = __builtin_amdgcn_readfirstlane((int)g.sorted_e[m_blk]);
+        if(STAGE == 2)
+            rw = g.sorted_w[p];
+        if((u32)(m_blk * 16) >= last)
+            return;
+        const int tok = (int)(id & 0xFFFFFFu), slot = (int)(id >> 24);
+        if(slot < g.topk && tok < g.T)
+        {
+            arow = STAGE == 1 ? tok : p;
+            orow = STAGE == 1 ? p : tok * g.topk + slot;
+        }
+    }
+    // row group j = 0..3 (stage 1: 0, 1 gate rows, 2, 3 the matching up rows); two of them share a scale tile of 32 rows
+    const u32 sc_tile = (u32)(g.SC / 8) * 256u;
+    rsrc_t wb[4], sb[2];
+    auto row_of = [&](int j) __attribute__((always_inline)) -> u32 {
+        return (u32)e * (u32)g.N + (u32)(STAGE == 1 ? (j >> 1) * I + chbase + (j & 1) * 16 : chbase + j * 16);
+    };
+    auto is_real = [&](int j) __attribute__((always_inline)) -> bool {
+        return STAGE == 1 ? chbase + (j & 1) * 16 < I - g.n_pad : chbase + j * 16 < g.N - g.n_pad;
+    };
+#pragma unroll
+    for(int j = 0; j < 4; j++)
+        wb[j] = buffer_of(g.w + (size_t)row_of(j) * Kb, is_real(j) ? (u32)(16 * Kb) : 0u);
+#pragma unroll
+    for(int h = 0; h < 2; h++)
+        sb[h] = buffer_of(g.w_s + (size_t)(row_of(2 * h) / 32) * sc_tile, sc_tile);
+    const rsrc_t ab = buffer_of(g.a, g.a_bytes);
+    const int a_off = arow >= 0 ? arow * g.a_pitch * 2 + kb * 64 : NOWHERE;
+
+    v4f acc[4];
+#pragma unroll
+    for(int j = 0; j < 4; j++)
+        acc[j] = (v4f){0.f, 0.f, 0.f, 0.f};
+    const int KT = (g.k_real + 127) / 128;
+    v4i wf[NB][4], af[NB][4];
+    u32 wsc[NB][2];
+    auto load_step = [&](auto BB, int kt) __attribute__((always_inline)) {
+        constexpr int b = decltype(BB)::value;
+        const int away  = kt * 128 + kb * 32 >= g.k_real ? NOWHERE : 0;
+#pragma unroll
+        for(int h = 0; h < 2; h++)
+            wsc[b][h] = load4(sb[h], lane * 4, (kt >> 1) * 256);
+#pragma unroll
+        for(int j = 0; j < 4; j++)
+            wf[b][j] = load16_nt(wb[j], lane * 16 | away, kt * 1024);
+#pragma unroll
+        for(int i = 0; i < 4; i++)
+            af[b][i] = load16(ab, (a_off + i * 16) | away, kt * 256);
+    };
+    auto step = [&](auto BB, int kt) __attribute__((always_inline)) {
+        constexpr int b = decltype(BB)::value;
+#pragma unroll
+        for(int j = 0; j < 4; j++)
+        {
+            v8bf wq[4];
+            expand_fp4(wf[b][j], (wsc[b][j >> 1] >> (8 * ((kt & 1) * 2 + (j & 1)))) & 0xFFu, wq);
+#pragma unroll
+            for(int i = 0; i < 4; i++)
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wq[i], __builtin_bit_cast(v8bf, af[b][i]), acc[j], 0, 0, 0);
+        }
+        if(kt + NB * KSTRIDE < KT)
+            load_step(BB, kt + NB * KSTRIDE);
+    };
+    const int kt0 = SPLITK ? wave : 0;
+    static_for<NB>([&](auto BB) __attribute__((always_inline)) {
+        const int kt = kt0 + decltype(BB)::value * KSTRIDE;
+        if(kt < KT)
+            load_step(BB, kt);
+    });
+    for(int kb0 = kt0; kb0 < KT; kb0 += NB * KSTRIDE)
+        static_for<NB>([&](auto BB) __attribute__((always_inline)) {
+            const int kt = kb0 + decltype(BB)::value * KSTRIDE;
+            if(kt < KT)
+                step(BB, kt);
+        });
+
+    // ---- epilogue: lane (r, kb) holds channels kb*4 .. + 3 of row group j for row r.  Under the K split wave w finishes row
+    // group w (stage 1: gate group w and its up group, waves 0 and 1)
+    auto channel = [&](int j) __attribute__((always_inline)) -> int {
+        return (STAGE == 1 ? (j >> 1) * I + chbase + (j & 1) * 16 : chbase + j * 16) + kb * 4;
+    };
+    auto finish = [&](int j, v4f lo, v4f hi) __attribute__((always_inline)) {      // hi: stage 1, the up group
+        if(g.bias)
+        {
+            lo = add_bias4(lo, load_bias4(g.bias + (size_t)e * g.N + channel(j)));
+            if(STAGE == 1)
+                hi = add_bias4(hi, load_bias4(g.bias + (size_t)e * g.N + channel(j + 2)));
+        }
+        if(arow < 0)
+            return;
+        float v[4];
+#pragma unroll
+        for(int i = 0; i < 4; i++)
+            v[i] = STAGE == 1 ? gated_act_f32(g.act, lo[i], hi[i]) : lo[i] * rw;
+        *(uint2*)((uint16_t*)g.out + (size_t)orow * (STAGE == 1 ? I : g.N) + channel(j)) =
+            make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+    };
+    if constexpr(SPLITK)
+    {
+#pragma unroll
+        for(int j = 0; j < 4; j++)
+            *(v4f*)&red[((wave * 4 + j) * WAVE + lane) * 4] = acc[j];
+        __syncthreads();
+        if(STAGE == 1 && wave >= 2)
+            return;
+        auto sum_of = [&](int j) __attribute__((always_inline)) -> v4f {
+            v4f sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for(int w = 0; w < 4; w++)
+                sum += *(const v4f*)&red[((w * 4 + j) * WAVE + lane) * 4];
+            return sum;
+        };
+        finish(wave, sum_of(wave), STAGE == 1 ? sum_of(wave + 2) : (v4f){0.f, 0.f, 0.f, 0.f});
+    }
+    else
+#pragma unroll
+        for(int j = 0; j < (STAGE == 1 ? 2 : 4); j++)
+            finish(j, acc[j], acc[STAGE == 1 ? j + 2 : j]);
+}
+
+// The down GEMM by token, with the sum over the token's slots.  A workgroup owns NR groups of 16 output channels of one token;
+// its waves are four K splits (wave w: K-steps w, w + 4, ..) for each of up to four slots, SPW slots to a wave.  Partial sums, biases
+// and routing weights meet in LDS, where a thread per channel finishes slot after slot: the arithmetic and order of
+// moe_gemm_pairs_kernel<2, 4> and the reduction.
+template <int SPW, int NR>
+__global__ void __launch_bounds__(1024) moe_pairs_down_sum_kernel(PairArgs g)
+{
+    constexpr int NB = SPW == 1 ? 3 : 2;
+    __shared__ float red[8][4][NR * 16], bias_l[8][NR * 16], rw_l[8];
+    __shared__ int on_l[8];
+    const int tid = threadIdx.x, lane = tid % WAVE;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    const int w = wave & 3, q = wave >> 2, groups = blockDim.x / (4 * WAVE);
+    const int r = lane & 15, kb = lane >> 4;
+    const int t = blockIdx.x / g.n_tiles, ch0 = (blockIdx.x - t * g.n_tiles) * (16 * NR);
+    const int Kb = g.K / 2;
+    const u32 sc_tile = (u32)(g.SC / 8) * 256u;
+    const bool here   = !(g.local_tok && t >= *g.local_tok);
+    const rsrc_t ab   = buffer_of(g.a, g.a_bytes);
+    rsrc_t wb[SPW][NR], sb[SPW];
+    int a_off[SPW], e[SPW];
+    bool on[SPW], any = false;
+#pragma unroll
+    for(int i = 0; i < SPW; i++)
+    {
+        const int s = q + i * groups, pair = t * g.topk + s;
+        const int id = __builtin_amdgcn_readfirstlane(s < g.topk ? g.ids[pair] : -1);
+        on[i]        = __builtin_amdgcn_readfirstlane((int)(here && moe_pair_is_kept(id, g.experts, g.mask))) != 0;
+        e[i]         = on[i] ? local_expert(id, g.mask, lane) : 0;
+        any |= on[i];
+        const u32 row = (u32)e[i] * (u32)g.N + (u32)ch0;
+#pragma unroll
+        for(int j = 0; j < NR; j++)
+            wb[i][j] = buffer_of(g.w + (size_t)(row + j * 16) * Kb, on[i] && ch0 + j * 16 < g.N - g.n_pad ? (u32)(16 * Kb) : 0u);
+        sb[i]    = buffer_of(g.w_s + (size_t)(row / 32) * sc_tile, on[i] ? sc_tile : 0u);
+        a_off[i] = on[i] && r == 0 ? pair * g.row_step * g.a_pitch * 2 + kb * 64 : NOWHERE;      // (row 0 of the products is the token)
+    }
+    v4f acc[SPW][NR];
+#pragma unroll
+    for(int i = 0; i < SPW; i++)
+#pragma unroll
+        for(int j = 0; j < NR; j++)
+            acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
+    const int KT   = (g.k_real + 127) / 128;
+    const int half = NR == 1 ? (ch0 / 16) & 1 : 0;      // which half of the 32-row scale tile the first row group is
+    v4i wf[NB][SPW][NR], af[NB][SPW][4];
+    u32 wsc[NB][SPW];
+    auto load_step = [&](auto BB, int kt) __attribute__((always_inline)) {
+        constexpr int b = decltype(BB)::value;
+        const int away  = kt * 128 + kb * 32 >= g.k_real ? NOWHERE : 0;
+#pragma unroll
+        for(int i = 0; i < SPW; i++)
+        {
+            wsc[b][i] = load4(sb[i], lane * 4, (kt >> 1) * 256);
+#pragma unroll
+            for(int j = 0; j < NR; j++)
+                wf[b][i][j] = load16_nt(wb[i][j], lane * 16 | away, kt * 1024);
+#pragma unroll
+            for(int c = 0; c < 4; c++)
+                af[b][i][c] = load16(ab, (a_off[i] + c * 16) | away, kt * 256);
+        }
+    };
+    auto step = [&](auto BB, int kt) __attribute__((always_inline)) {
+        constexpr int b = decltype(BB)::value;
+#pragma unroll
+        for(int i = 0; i < SPW; i++)
+#pragma unroll
+            for(int j = 0; j < NR; j++)
+            {
+                v8bf wq[4];
+                expand_fp4(wf[b][i][j], (wsc[b][i] >> (8 * ((kt & 1) * 2 + half + j))) & 0xFFu, wq);
+#pragma unroll
+                for(int c = 0; c < 4; c++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wq[c], __builtin_bit_cast(v8bf, af[b][i][c]), acc[i][j], 0, 0, 0);
+            }
+        if(kt + NB * 4 < KT)
+            load_step(BB, kt + NB * 4);
+    };
+    if(any)
+    {
+        static_for<NB>([&](auto BB) __attribute__((always_inline)) {
+            const int kt = w + decltype(BB)::value * 4;
+            if(kt < KT)
+                load_step(BB, kt);
+        });
+        for(int kb0 = w; kb0 < KT; kb0 += NB * 4)
+            static_for<NB>([&](auto BB) __attribute__((always_inline)) {
+                const int kt = kb0 + decltype(BB)::value * 4;
+                if(kt < KT)
+                    step(BB, kt);
+            });
+    }
+#pragma unroll
+    for(int i = 0; i < SPW; i++)
+    {
+        const int s = q + i * groups;
+        if(s >= g.topk)
+            continue;
+        if(r == 0)
+#pragma unroll
+            for(int j = 0; j < NR; j++)
+                *(v4f*)&red[s][w][j * 16 + kb * 4] = acc[i][j];
+        if(w == 0)
+        {
+            if(lane == 0)
+            {
+                on_l[s] = on[i];
+                rw_l[s] = g.weights[t * g.topk + s];
+            }
+            if(g.bias && on[i] && lane < 16 * NR)
+                bias_l[s][lane] = bf16_bits_to_f32(g.bias[(size_t)e[i] * g.N + ch0 + lane]);
+        }
+    }
+    __syncthreads();
+    if(tid >= 16 * NR)
+        return;
+    float out = 0.f;
+    for(int s = 0; s < g.topk; s++)
+    {
+        if(!on_l[s])
+            continue;
+        float sum = 0.f;
+#pragma unroll
+        for(int p = 0; p < 4; p++)
+            sum += red[s][p][tid];
+        if(g.bias)
+            sum += bias_l[s][tid];
+        out += bf16_bits_to_f32(pack_bf16x2(sum * rw_l[s], 0.f) & 0xFFFFu);
+    }
+    const size_t at = (size_t)t * g.N + ch0 + tid;
+    if(g.out_f32)
+        ((float*)g.out)[at] = out;
+    else
+        ((uint16_t*)g.out)[at] = (uint16_t)pack_bf16x2(out, 0.f);
+}
+
+// the bound of the row blocks that hold rows, as the sorted entry points compute it: the K split depends on it
+static int64_t block_bound(int64_t rows, int64_t n_blk, int experts)
+{
+    const int64_t b = rows < n_blk ? rows : n_blk;
+    return experts + rows / 16 < b ? experts + rows / 16 : b;
+}
+
+bool pyhip_pairs_served(int64_t tokens, int topk, int experts, int hidden, int inter, int64_t n_blk, int split_k)
+{
+    const int64_t blocks = block_bound(tokens * topk, n_blk, experts);
+    const int s1 = w4a16_split(1, 16, blocks * (inter / 128), hidden, split_k), s2 = w4a16_split(2, 16, blocks * (hidden / 256), inter, split_k);
+    // (offsets into the activations are 32-bit and signed)
+    return (s1 == 0 || s1 == 4) && (s2 == 0 || s2 == 4 || (s2 == 32 && tokens == 1 && topk == 2 && inter >= 2048 && inter <= 16384)) &&      // (pyhip_w4a16_token_top2)
+          
+           (n_blk * 16 + tokens) * (int64_t)(hidden > inter ? hidden : inter) * 2 < (1ll << 31);
+}
+
+static int prepare(const char* name, PairArgs& g, int64_t rows, int64_t blocks, int64_t tiles)
+{
+    PYHIP_REQUIRE(g.a && g.w && g.w_s && g.out && (g.ids || (g.sorted_ids && g.sorted_e && g.num_valid)), "%s: null pointer", name);
+    PYHIP_REQUIRE(g.K > 0 && g.K % 512 == 0 && g.N > 0 && g.N % 256 == 0, "%s: K=%d must be a multiple of 512, N=%d of 256", name, g.K, g.N);
+    PYHIP_REQUIRE(g.T > 0 && g.topk > 0 && g.experts > 0 && (!g.ids || (int64_t)g.T * g.topk <= PAIRS_UNSORTED_MAX), "%s: bad sizes", name);
+    PYHIP_REQUIRE(g.k_real > 0 && g.k_real <= g.K && g.a_pitch >= (g.k_real + 31) / 32 * 32 && g.a_pitch % 8 == 0,
+                  "%s: %d of %d columns, rows of %d", name, g.k_real, g.K, g.a_pitch);
+    PYHIP_REQUIRE(((uintptr_t)g.a % 16) == 0 && ((uintptr_t)g.w % 16) == 0 && ((uintptr_t)g.w_s % 4) == 0 && ((uintptr_t)g.out % 8) == 0,
+                  "%s: unaligned pointer", name);
+    PYHIP_REQUIRE(rows * g.a_pitch * 2 < (1ll << 31) && blocks * tiles * 4 < (1ll << 31), "%s: too large", name);
+    g.SC      = (g.K / 32 + 7) / 8 * 8;
+    // (the last row need not be a whole pitch long)
+    g.a_bytes = (u32)(((rows - 1) * g.a_pitch + (g.k_real + 31) / 32 * 32) * 2);
+    return PYHIP_OK;
+}
+
+int pyhip_pairs_gate_up(PairArgs g, int64_t rows, int64_t n_blk, int split_k, int activation, float swiglu_limit, hipStream_t stream)
+{
+    PYHIP_REQUIRE(activation == 0 || (activation == 1 && swiglu_limit > 0.f),
+                  "moe_pairs_gate_up: activation=%d (0 SiLU, 1 SwiGLU with a positive limit)", activation);
+    const int64_t blocks = block_bound((int64_t)g.T * g.topk, n_blk, g.experts);
+    g.n_tiles            = g.N / 256;
+    const int split      = w4a16_split(1, 16, blocks * g.n_tiles, g.K, split_k);
+    const int rc         = prepare("moe_pairs_gate_up", g, rows, blocks, g.n_tiles);
+    if(rc)
+        return rc;
+    PYHIP_REQUIRE(split == 0 || split == 4, "moe_pairs_gate_up: split_k=%d", split_k);
+    g.act = make_gated_act(activation, swiglu_limit);
+    // (tiles whose channels are all padding are not launched)
+    const int tile = split ? 32 : 128;
+    g.n_tiles      = (g.N / 2 - g.n_pad + tile - 1) / tile;
+    const dim3 grid((unsigned)(blocks * g.n_tiles));
+    if(split)
+        hipLaunchKernelGGL((moe_gemm_pairs_kernel<1, 4>), grid, dim3(W4A16_THREADS), 0, stream, g);
+    else
+        hipLaunchKernelGGL((moe_gemm_pairs_kernel<1, 0>), grid, dim3(W4A16_THREADS), 0, stream, g);
+    PYHIP_CHECK_LAUNCH("moe_gemm_pairs_kernel");
+    return PYHIP_OK;
+}
+
+int pyhip_pairs_down(PairArgs g, int64_t rows, int64_t n_blk, int split_k, hipStream_t stream)
+{
+    const int64_t blocks = block_bound((int64_t)g.T * g.topk, n_blk, g.experts);
+    g.n_tiles            = g.N / 256;
+    const int split      = w4a16_split(2, 16, blocks * g.n_tiles, g.K, split_k);
+    const int rc         = prepare("moe_pairs_down", g, rows, blocks, g.n_tiles);
+    if(rc)
+        return rc;
+    PYHIP_REQUIRE(split == 0 || split == 4, "moe_pairs_down: split_k=%d", split_k);
+    if(split)
+        g.n_tiles *= 4;
+    const dim3 grid((unsigned)(blocks * g.n_tiles));
+    if(split)
+        hipLaunchKernelGGL((moe_gemm_pairs_kernel<2, 4>), grid, dim3(W4A16_THREADS), 0, stream, g);
+    else
+        hipLaunchKernelGGL((moe_gemm_pairs_kernel<2, 0>), grid, dim3(W4A16_THREADS), 0, stream, g);
+    PYHIP_CHECK_LAUNCH("moe_gemm_pairs_kernel");
+    return PYHIP_OK;
+}
+
+int pyhip_pairs_down_sum(PairArgs g, int64_t rows, int64_t n_blk, int split_k, hipStream_t stream)
+{
+    const int64_t pairs  = (int64_t)g.T * g.topk;
+    const int64_t blocks = block_bound(pairs, n_blk, g.experts);
+    // by token the weights of an expert are fetched for each of its pairs: only where pairs rarely share one
+    if(!g.ids || g.topk > 8 || (g.T > 1 && 8 * pairs > g.experts) || w4a16_split(2, 16, blocks * (g.N / 256), g.K, split_k) != 4)
+        return -1;
+    PYHIP_REQUIRE(((uintptr_t)g.out % 16) == 0, "moe_pairs_down_sum: unaligned pointer");
+    const int rc = prepare("moe_pairs_down_sum", g, rows, blocks, g.N / 64);
+    if(rc)
+        return rc;
+    const int groups = g.topk < 4 ? g.topk : 4;
+    const bool wide  = g.topk <= 4 && (int64_t)g.T * (g.N / 32) >= 512;
+    g.n_tiles        = g.N / (wide ? 32 : 16);
+    const dim3 grid((unsigned)(g.T * g.n_tiles)), block(groups * 4 * WAVE);
+    if(g.topk > 4)
+        hipLaunchKernelGGL((moe_pairs_down_sum_kernel<2, 1>), grid, block, 0, stream, g);
+    else if(wide)
+        hipLaunchKernelGGL((moe_pairs_down_sum_kernel<1, 2>), grid, block, 0, stream, g);
+    else
+        hipLaunchKernelGGL((moe_pairs_down_sum_kernel<1, 1>), grid, block, 0, stream, g);
+    PYHIP_CHECK_LAUNCH("moe_pairs_down_sum_kernel");
+    return PYHIP_OK;
+}

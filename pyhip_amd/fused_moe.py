@@ -14,6 +14,7 @@ reference runs for few tokens (src/contrib/moe.py:362-787); ``method="a4w4"`` fo
 ``method="auto"`` takes w4a16 for the very smallest calls (see ``pick_w4a16``) and a4w4 above.
 """
 import functools
+import struct
 
 import torch
 
@@ -125,6 +126,15 @@ def _ask_plan(tokens, topk, experts, hidden, inter, method, block_m):
 
 
 _remembered_plan = functools.lru_cache(maxsize=512)(_ask_plan)
+
+
+#: struct LayerCall of csrc/moe_forward.hip: pointers, row stride and workspace bytes, sizes and options, the SwiGLU limit
+_LAYER_CALL = struct.Struct("<14Q2q16if")
+
+
+@functools.lru_cache(maxsize=512)
+def _w4a16_takes_cols(tokens, topk, experts, hidden, inter, block_m, splitk):
+    return bool(_lib.load().pyhip_layer_takes_cols(tokens, topk, experts, hidden, inter, block_m, 1, splitk))
 
 
 def act_quant_mxfp4(x, rows_limit=None):
@@ -277,11 +287,13 @@ def fused_moe(
     one_call = not return_parts and stage_events is None and not atomic and not lds_tile and not arriver
     cols = 0
     if narrow:
-        # the one-call path quantises activations at the true width as they are: whole 32-column blocks, rows that lie
-        # one after the other and start on 16 bytes (anything else is widened into a buffer of its own first)
+        # the one-call path takes activations at the true width as they are (bf16 ones only in its 16-row blocks): whole
+        # 32-column blocks, rows that lie one after the other and start on 16 bytes (anything else is widened into a
+        # buffer of its own first)
         cols = H - hidden_pad
-        if not (one_call and not w4a16 and cols % 32 == 0 and hidden_states.stride(1) == 1 and hidden_states.stride(0) >= cols
-                and hidden_states.stride(0) % 8 == 0 and hidden_states.data_ptr() % 16 == 0):
+        if not (one_call and cols % 32 == 0 and hidden_states.stride(1) == 1 and hidden_states.stride(0) >= cols
+                and hidden_states.stride(0) % 8 == 0 and hidden_states.data_ptr() % 16 == 0
+                and (not w4a16 or (hidden_states.stride(0) < 1 << 24 and _w4a16_takes_cols(T, k, global_E, H, I, int(bm), int(splitk))))):
             cols = 0
             hidden_states = torch.nn.functional.pad(hidden_states, (0, hidden_pad))
     if one_call:
@@ -290,16 +302,16 @@ def fused_moe(
         # from a graph)
         x = hidden_states
         # the kernels read 16-byte pieces of a row: views with an odd row stride or base (a column slice) are copied
-        if x.stride(1) != 1 or (w4a16 and x.stride(0) != H) or x.stride(0) % 8 != 0 or x.data_ptr() % 16 != 0:
+        if x.stride(1) != 1 or (w4a16 and not cols and x.stride(0) != H) or x.stride(0) % 8 != 0 or x.data_ptr() % 16 != 0:
             x = x.contiguous()
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         out = torch.empty(T, H, dtype=out_dtype, device=dev)
-        rc = lib.pyhip_moe_forward_cols(_lib.addr(x), x.stride(0), cols, _lib.addr(w1u), _lib.addr(w1s), _lib.addr(w2u),
-                                        _lib.addr(w2s), _lib.addr(bias1), _lib.addr(bias2), _lib.addr(topk_ids),
-                                        _lib.addr(topk_weight), _lib.addr(expert_mask), _lib.addr(num_local_tokens),
-                                        _lib.addr(out), 1 if out_dtype == torch.float32 else 0, T, k, global_E, H, I,
-                                        hidden_pad, intermediate_pad, bm, 1 if w4a16 else 0, splitk, act, limit,
-                                        _lib.addr(ws), ws_bytes, _lib.stream_handle())
+        p = _lib.address
+        rc = lib.pyhip_layer_forward(
+            _LAYER_CALL.pack(x.data_ptr(), w1u.data_ptr(), w1s.data_ptr(), w2u.data_ptr(), w2s.data_ptr(), p(bias1), p(bias2), 0,
+                             topk_ids.data_ptr(), topk_weight.data_ptr(), p(expert_mask), p(num_local_tokens), out.data_ptr(),
+                             ws.data_ptr(), x.stride(0), ws_bytes, cols, out_dtype == torch.float32, T, k, global_E, H, I,
+                             hidden_pad, intermediate_pad, bm, w4a16, splitk, act, 0, 0, 0, limit), _lib.stream_handle())
         _lib.check(rc, "moe_forward")
         return out[:, : H - hidden_pad] if narrow else out
 
@@ -458,12 +470,12 @@ def fused_moe_routed(hidden_states, w1, w2, gating_output, topk, renormalize=Tru
     out = torch.empty(T, H, dtype=out_dtype, device=dev)
     tw = torch.empty(T, topk, dtype=torch.float32, device=dev)
     ti = torch.empty(T, topk, dtype=torch.int32, device=dev)
-    rc = lib.pyhip_moe_forward_routed(_lib.addr(x), x.stride(0), _lib.addr(w1u), _lib.addr(w1s), _lib.addr(w2u),
-                                      _lib.addr(w2s), _lib.addr(bias1), _lib.addr(bias2), _lib.addr(g),
-                                      int(num_expert_group), int(topk_group), 1 if renormalize else 0, _lib.addr(ti),
-                                      _lib.addr(tw), _lib.addr(expert_mask), _lib.addr(num_local_tokens), _lib.addr(out),
-                                      1 if out_dtype == torch.float32 else 0, T, topk, global_E, H, I, int(hidden_pad),
-                                      int(intermediate_pad), bm, 1 if w4a16 else 0, splitk, act, limit, _lib.addr(ws),
-                                      ws_bytes, _lib.stream_handle())
+    p = _lib.address
+    rc = lib.pyhip_layer_forward(
+        _LAYER_CALL.pack(x.data_ptr(), w1u.data_ptr(), w1s.data_ptr(), w2u.data_ptr(), w2s.data_ptr(), p(bias1), p(bias2),
+                         g.data_ptr(), ti.data_ptr(), tw.data_ptr(), p(expert_mask), p(num_local_tokens), out.data_ptr(),
+                         ws.data_ptr(), x.stride(0), ws_bytes, 0, out_dtype == torch.float32, T, topk, global_E, H, I,
+                         int(hidden_pad), int(intermediate_pad), bm, w4a16, splitk, act, int(num_expert_group), int(topk_group),
+                         bool(renormalize), limit), _lib.stream_handle())
     _lib.check(rc, "moe_forward_routed")
     return (out, tw, ti) if return_routing else out

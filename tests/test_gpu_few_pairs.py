@@ -1,0 +1,106 @@
+"""The layer call with bf16 activations and 16-row blocks (its own kernels, without a sort up to 64 pairs and without a reduction
+where pairs rarely share an expert) against the step-by-step path: the same arithmetic in the same order, so the same bits."""
+import pytest
+import torch
+
+import cases
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T,k,E,H,I,splitk", [
+    (1, 1, 8, 512, 512, 0),          # one pair; every K split has one K-step
+    (1, 4, 20, 1024, 2560, 0),       # a token's slots on four groups of waves, an uneven share of K-steps
+    (1, 4, 8, 16384, 512, 0),        # two row groups to a workgroup
+    (1, 6, 64, 512, 1024, 0),        # two slots for some waves, one for others
+    (1, 9, 16, 512, 512, 0),         # more slots than the summing kernel holds
+    (4, 1, 32, 512, 512, 0),         # summed by token
+    (4, 8, 256, 512, 512, 4),        # the most pairs that are summed by token in 256 experts
+    (5, 8, 256, 512, 512, 0),        # one token more
+    (64, 1, 8, 512, 512, 0),         # 64 pairs in 8 experts
+    (63, 1, 3, 512, 1024, 0),        # more than a block for an expert; an expert count that is no power of two
+    (64, 1, 1, 512, 512, 1),         # one expert, four full blocks, no K split
+    (8, 8, 16, 1024, 1536, 1),
+    (65, 1, 8, 512, 512, 0),         # one pair more: sorted
+    (13, 5, 8, 1536, 512, 0),        # sorted, an odd top-k
+    (40, 4, 16, 512, 1536, 1),       # sorted, no K split
+    (1, 2, 8, 512, 1024, 1),         # a top-2 token whose slots the reduction sums
+])
+def test_few_pairs_equal_the_stages(T, k, E, H, I, splitk):
+    from pyhip_amd import fused_moe
+    from pyhip_amd.enums import ActivationType
+    L = cases.make_layer("", T, seed=T * 7 + k, bias=True, E=E, k=min(k, E), H=H, I=I, router="softmax")
+    w1, w1s, w2, w2s = cases.device_weights(L)
+    g = torch.Generator().manual_seed(T + E)
+    ids = torch.from_numpy(L.topk_ids).clone()
+    if E > 1:
+        ids[0, 0] = ids[-1, -1]                       # an expert that two pairs share, also inside one token
+    hole = ids.clone()
+    hole[torch.rand(hole.shape, generator=g) < 0.3] = -1
+    hole[T // 2] = E                                  # a token that nobody serves
+    local = torch.tensor([T - 1], dtype=torch.int32, device="cuda")
+    mask = (torch.rand(E, generator=g) < 0.6).to(torch.int32)
+    mask[int(ids[0, 0])] = 1
+    keep = mask.bool().cuda()
+    s1, s2, b1, b2 = w1s.view(E, -1), w2s.view(E, -1), L.bias1.cuda() * 20, L.bias2.cuda() * 20
+    ma, mb = w1[keep].contiguous(), w2[keep].contiguous()
+    ma.is_shuffled = mb.is_shuffled = True
+    rank = dict(w1_scale=s1[keep].reshape(-1, w1s.shape[-1]).contiguous(), w2_scale=s2[keep].reshape(-1, w2s.shape[-1]).contiguous(),
+                bias1=b1[keep], bias2=b2[keep], expert_mask=mask.cuda())
+    whole = dict(w1_scale=w1s, w2_scale=w2s, bias1=b1, bias2=b2)
+    hidden, tw = L.hidden.cuda(), torch.from_numpy(L.topk_w).cuda()
+    for name, wa, wb, t, kw in (("plain", w1, w2, ids, whole), ("holes", w1, w2, hole, whole),
+                                ("no bias", w1, w2, ids, dict(whole, bias1=None, bias2=None)),
+                                ("mask", ma, mb, ids, rank), ("local", w1, w2, ids, dict(whole, num_local_tokens=local))):
+        for more in (dict(), dict(dtype=torch.float32, activation=ActivationType.Swiglu)):
+            print(f"few pairs T={T} k={L.k} E={E} H={H} I={I} {name} {sorted(more)}", flush=True)
+            kw2 = dict(kw, method="w4a16", block_size_M=16, splitk=splitk, **more)
+            want = fused_moe(hidden, wa, wb, tw, t.cuda(), return_parts=True, **kw2)[0]
+            for _ in range(2):
+                got = fused_moe(hidden, wa, wb, tw, t.cuda(), **kw2)
+                assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("T,H,I", [(1, 544, 544), (3, 1440, 1440), (1, 992, 32 * 47), (20, 1440, 1056), (30, 576, 1440)])
+@pytest.mark.parametrize("wide", [False, True])
+def test_few_pairs_leave_padding_alone(T, H, I, wide):
+    """Padded layers, activations at the true or the padded width.  The weights' padding is told, so it is not read: its rows and
+    columns are filled with ones here, and what the padded columns of the activations hold does not matter either."""
+    from pyhip_amd import fused_moe
+    L = cases.make_layer("", T, seed=H, bias=True, E=32, k=2, H=H, I=I, router="softmax")
+    w1, w1s, w2, w2s, b1, b2, hp, ip = cases.padded_device_weights(L)
+    tw, ti = torch.from_numpy(L.topk_w).cuda(), torch.from_numpy(L.topk_ids).cuda()
+    kw = dict(bias1=b1, bias2=b2, method="w4a16", block_size_M=16)
+    x = torch.nn.functional.pad(L.hidden.cuda(), (0, hp))
+    want = fused_moe(x, w1, w2, tw, ti, w1_scale=w1s, w2_scale=w2s, return_parts=True, **kw)[0]
+    # ones (code 2) in the padding rows of w2, in whole row groups of 16, and in the padding columns of both, in whole 1 KB blocks' groups of 32
+    f1, f2 = w1.clone(), w2.clone()
+    v1 = f1.view(32, -1, f1.shape[2] // 64, 4, 16, 16)      # [E, N / 16, K / 128, group of 32, row, byte]
+    v2 = f2.view(32, -1, f2.shape[2] // 64, 4, 16, 16)
+    for v, real in ((v1, H), (v2, I)):
+        for c in range(real, v.shape[2] * 128, 32):
+            v[:, :, c // 128, c % 128 // 32] = 0x22
+    f1.is_shuffled = f2.is_shuffled = True
+    if wide:
+        x[:, H:] = float("nan")
+    else:
+        x = x[:, :H]
+        x = torch.nn.functional.pad(x, (0, 8), value=float("nan"))[:, :H]
+    print("few pairs, padded", T, H, I, wide, flush=True)
+    got = fused_moe(x, f1, f2, tw, ti, w1_scale=w1s, w2_scale=w2s, hidden_pad=hp, intermediate_pad=ip, **kw)
+    assert torch.equal(got[:, :H], want[:, :H]) and (not wide or (got[:, H:] == 0).all())
+
+
+@pytest.mark.parametrize("T", [1, 4, 8, 9])
+@pytest.mark.parametrize("grouped", [False, True])
+def test_few_pairs_with_the_router(T, grouped):
+    from pyhip_amd import fused_moe, fused_moe_routed
+    L = cases.make_layer("", T, seed=T, E=256, k=8, H=512, I=512, router="softmax")
+    w1, w1s, w2, w2s = cases.device_weights(L)
+    logits = torch.randn(T, 256, generator=torch.Generator().manual_seed(T)).cuda()
+    kw = dict(w1_scale=w1s, w2_scale=w2s, method="w4a16", block_size_M=16)
+    print("few pairs, routed", T, grouped, flush=True)
+    out, tw, ti = fused_moe_routed(L.hidden.cuda(), w1, w2, logits, 8, return_routing=True,
+                                   **(dict(num_expert_group=8, topk_group=4) if grouped else {}), **kw)
+    want = fused_moe(L.hidden.cuda(), w1, w2, tw, ti, return_parts=True, **kw)[0]
+    assert torch.equal(out, want)
