@@ -251,9 +251,11 @@ static int forward_pairs(const void* hidden_bf16, int64_t row_stride, int hidden
     down.a = (const uint16_t*)(ws + l.a2); down.w = w2; down.w_s = w2_scale; down.bias = (const uint16_t*)bias2_bf16;
     down.out = out; down.out_f32 = out_is_f32; down.K = inter; down.N = hidden;
     down.a_pitch = inter; down.k_real = inter - inter_pad; down.n_pad = hidden_pad;
-    // (the kernel that sums a top-2 token's slots on sixteen waves reads the rows of a2 where the single-token entry points put them)
+    // (the kernels that sum a top-2 token's slots read the rows of a2 where the single-token entry points put them, and all of their
+    // columns)
     const bool top2 = tokens == 1 && topk == 2;
     up.row_step = down.row_step = top2 ? 16 : 1;
+    up.all_channels             = top2;
     rc = pyhip_pairs_gate_up(up, tokens, l.n_blk, split_k, activation, swiglu_limit, stream);
     if(rc)
         return rc;

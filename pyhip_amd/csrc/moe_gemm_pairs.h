@@ -24,6 +24,7 @@ struct PairArgs
     int a_pitch = 0, row_step = 1;
     int k_real = 0;                   // columns of the weights that are not padding ...
     int n_pad  = 0;                   // ... and rows of (each half of) an expert's matrix that are
+    int all_channels = 0;             // gate_up: channels of padding are written as well (zeros), for a reader that does not know of them
     int out_f32 = 0;                  // down that sums: the type of its output
     // filled in by the launchers
     int SC = 0, n_tiles = 0;

@@ -6,7 +6,7 @@
 //   * Activations come at their own row pitch and width, and neither the padding rows nor the padding columns of the weights
 //     are fetched (raw buffer loads: a lane or a row group that has nothing to fetch is out of its descriptor's range).
 //   * Where nearly every pair has an expert of its own, the down GEMM goes by token instead of by expert: a workgroup holds
-//     all of a token's slots for 16 or 32 output channels, so it sums them and no reduction follows.
+//     all of a token's slots for 16 to 64 output channels, so it sums them and no reduction follows.
 // Bound: the weight stream from about 40 us on, the launches and their latency chains below.  Layer call, us, sort + moe_gemm_w4a16
 // kernels + reduction (padded layers: after a widening of the activations) / this: gpt-oss shape, 2 tokens 39.5 / 28.7, 5 tokens
 // 67.0 / 51.3 (bound at 6.9 TB/s: 38); 32 experts, top-1, 2144 x 3040, 3 tokens 36.7 / 18.4; 1024 x 512, 8 experts, 10 tokens 25.0 / 17.6;
@@ -105,7 +105,7 @@ __global__ void __launch_bounds__(W4A16_THREADS) moe_gemm_pairs_kernel(PairArgs 
     const int Kb = g.K / 2, I = g.N / 2;
     // first output channel of this wave's rows (stage 1: within the gate half; the up half is I further)
     const int chbase = STAGE == 1 ? (SPLITK ? nt * 32 : nt * 128 + wave * 32) : (SPLITK ? nt * 64 : nt * 256 + wave * 64);
-    if(STAGE == 1 && chbase >= I - g.n_pad)      // (channels of padding: the down GEMM does not read them)
+    if(STAGE == 1 && chbase >= I - g.n_pad && !g.all_channels)      // (channels of padding: the down GEMM does not read them)
         return;
     // the block's expert, and for row r: the activation row, the output row, the routing weight
     int e, arow = -1, orow = 0;
@@ -249,16 +249,20 @@ __global__ void __launch_bounds__(W4A16_THREADS) moe_gemm_pairs_kernel(PairArgs 
             finish(j, acc[j], acc[STAGE == 1 ? j + 2 : j]);
 }
 
-// The down GEMM by token, with the sum over the token's slots.  A workgroup owns NR groups of 16 output channels of one token;
-// its waves are four K splits (wave w: K-steps w, w + 4, ..) for each of up to four slots, SPW slots to a wave.  Partial sums, biases
-// and routing weights meet in LDS, where a thread per channel finishes slot after slot: the arithmetic and order of
-// moe_gemm_pairs_kernel<2, 4> and the reduction.
-template <int SPW, int NR>
-__global__ void __launch_bounds__(1024) moe_pairs_down_sum_kernel(PairArgs g)
+// The down GEMM by token, with the sum over the token's slots.  A workgroup owns NR groups of 16 output channels of one token: groups
+// of four waves, a K split each (wave w: K-steps w, w + 4, ..), take the token's slots in turns, one after the other in one pipeline.
+// Partial sums, biases and routing weights meet in LDS, where a thread per channel finishes slot after slot: the arithmetic and
+// order of moe_gemm_pairs_kernel<2, 4> and the reduction.
+// Bound: the weight stream, less well fed than by expert (a wave brings the activations of one row for 1, 2 or 4 KB of weights),
+// against the reduction's launch.  Layer, us, down by expert + reduction / NR = 1 / 2 / 4: gpt-oss shape, 1 token 21.9 / 19.3 / 20.8 /
+// 24.0, 2 tokens 26.8 / 28.2 / 25.1 / 28.3, 4 tokens 41.7 / 50.3 / 43.1 / 40.5; DeepSeek-V3 shape, 1 token 37.2 / 39.8 / 35.3 / 38.7, 2 tokens
+// 61.2 / 71.0 / 61.9 / 58.9, 3 tokens 87.7 / 102 / 89.4 / 91.8, 4 tokens 111.5 / 128 / 115.6 / 111.2; 256 experts, top-1, 5120 x 1536,
+// 30 tokens 62.1 / 67.0 / 59.9 / 56.7.  (Sixteen waves, every slot on waves of its own: 113 us at 3 tokens of the DeepSeek-V3 shape.)
+template <int NR>
+__global__ void __launch_bounds__(512) moe_pairs_down_sum_kernel(PairArgs g)
 {
-    constexpr int NB = SPW == 1 ? 3 : 2;
+    constexpr int NB = NR == 4 ? 2 : 3;      // K-steps in flight
     __shared__ float red[8][4][NR * 16], bias_l[8][NR * 16], rw_l[8];
-    __shared__ int on_l[8];
     const int tid = threadIdx.x, lane = tid % WAVE;
     const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int w = wave & 3, q = wave >> 2, groups = blockDim.x / (4 * WAVE);
@@ -266,111 +270,131 @@ __global__ void __launch_bounds__(1024) moe_pairs_down_sum_kernel(PairArgs g)
     const int t = blockIdx.x / g.n_tiles, ch0 = (blockIdx.x - t * g.n_tiles) * (16 * NR);
     const int Kb = g.K / 2;
     const u32 sc_tile = (u32)(g.SC / 8) * 256u;
-    const bool here   = !(g.local_tok && t >= *g.local_tok);
-    const rsrc_t ab   = buffer_of(g.a, g.a_bytes);
-    rsrc_t wb[SPW][NR], sb[SPW];
-    int a_off[SPW], e[SPW];
-    bool on[SPW], any = false;
-#pragma unroll
-    for(int i = 0; i < SPW; i++)
+    // lane s: slot s's expert
+    const bool here = !(g.local_tok && t >= *g.local_tok);
+    const int id    = here && lane < g.topk ? g.ids[t * g.topk + lane] : -1;
+    const u32 on    = (u32)__ballot(moe_pair_is_kept(id, g.experts, g.mask));
+    u32 turn = 0;                         // this group's slots: in turns, of those that count
     {
-        const int s = q + i * groups, pair = t * g.topk + s;
-        const int id = __builtin_amdgcn_readfirstlane(s < g.topk ? g.ids[pair] : -1);
-        on[i]        = __builtin_amdgcn_readfirstlane((int)(here && moe_pair_is_kept(id, g.experts, g.mask))) != 0;
-        e[i]         = on[i] ? local_expert(id, g.mask, lane) : 0;
-        any |= on[i];
-        const u32 row = (u32)e[i] * (u32)g.N + (u32)ch0;
-#pragma unroll
-        for(int j = 0; j < NR; j++)
-            wb[i][j] = buffer_of(g.w + (size_t)(row + j * 16) * Kb, on[i] && ch0 + j * 16 < g.N - g.n_pad ? (u32)(16 * Kb) : 0u);
-        sb[i]    = buffer_of(g.w_s + (size_t)(row / 32) * sc_tile, on[i] ? sc_tile : 0u);
-        a_off[i] = on[i] && r == 0 ? pair * g.row_step * g.a_pitch * 2 + kb * 64 : NOWHERE;      // (row 0 of the products is the token)
+        int i = 0;
+        for(u32 rest = on; rest; rest &= rest - 1u, i++)
+            if(i % groups == q)
+                turn |= rest & -rest;
     }
-    v4f acc[SPW][NR];
-#pragma unroll
-    for(int i = 0; i < SPW; i++)
+    const rsrc_t ab = buffer_of(g.a, g.a_bytes);
+    const int KT = (g.k_real + 127) / 128, steps = (KT - w + 3) / 4;
+    const int half = NR == 1 ? (ch0 / 16) & 1 : 0;      // which half of the 32-row scale tile the first row group is
+    constexpr int NS = (NR + 1) / 2;      // scale tiles of 32 rows
+    rsrc_t wb[NR], sb[NS];
+    int a_off, lk = w, ls = 0;
+    u32 to_load = turn;
+    auto take_slot = [&]() __attribute__((always_inline)) {
+        ls = __builtin_ctz(to_load);
+        const int e   = local_expert(__builtin_amdgcn_readlane(id, ls), g.mask, lane);
+        const u32 row = (u32)e * (u32)g.N + (u32)ch0;
 #pragma unroll
         for(int j = 0; j < NR; j++)
-            acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
-    const int KT   = (g.k_real + 127) / 128;
-    const int half = NR == 1 ? (ch0 / 16) & 1 : 0;      // which half of the 32-row scale tile the first row group is
-    v4i wf[NB][SPW][NR], af[NB][SPW][4];
-    u32 wsc[NB][SPW];
-    auto load_step = [&](auto BB, int kt) __attribute__((always_inline)) {
+            wb[j] = buffer_of(g.w + (size_t)(row + j * 16) * Kb, ch0 + j * 16 < g.N - g.n_pad ? (u32)(16 * Kb) : 0u);
+#pragma unroll
+        for(int h = 0; h < NS; h++)
+            sb[h] = buffer_of(g.w_s + (size_t)(row / 32 + h) * sc_tile, sc_tile);
+        const int pair = t * g.topk + ls;
+        a_off = r == 0 ? pair * g.row_step * g.a_pitch * 2 + kb * 64 : NOWHERE;      // (row 0 of the products is the token)
+    };
+    v4f acc[NR];
+#pragma unroll
+    for(int j = 0; j < NR; j++)
+        acc[j] = (v4f){0.f, 0.f, 0.f, 0.f};
+    v4i wf[NB][NR], af[NB][4];
+    u32 wsc[NB][NS];
+    auto load_next = [&](auto BB) __attribute__((always_inline)) {
         constexpr int b = decltype(BB)::value;
-        const int away  = kt * 128 + kb * 32 >= g.k_real ? NOWHERE : 0;
+        if(!to_load)
+            return;
+        const int away = lk * 128 + kb * 32 >= g.k_real ? NOWHERE : 0;
 #pragma unroll
-        for(int i = 0; i < SPW; i++)
+        for(int h = 0; h < NS; h++)
+            wsc[b][h] = load4(sb[h], lane * 4, (lk >> 1) * 256);
+#pragma unroll
+        for(int j = 0; j < NR; j++)
+            wf[b][j] = load16_nt(wb[j], lane * 16 | away, lk * 1024);
+#pragma unroll
+        for(int c = 0; c < 4; c++)
+            af[b][c] = load16(ab, (a_off + c * 16) | away, lk * 256);
+        lk += 4;
+        if(lk >= KT)
         {
-            wsc[b][i] = load4(sb[i], lane * 4, (kt >> 1) * 256);
-#pragma unroll
-            for(int j = 0; j < NR; j++)
-                wf[b][i][j] = load16_nt(wb[i][j], lane * 16 | away, kt * 1024);
-#pragma unroll
-            for(int c = 0; c < 4; c++)
-                af[b][i][c] = load16(ab, (a_off[i] + c * 16) | away, kt * 256);
+            lk = w;
+            to_load &= to_load - 1u;
+            if(to_load)
+                take_slot();
         }
     };
-    auto step = [&](auto BB, int kt) __attribute__((always_inline)) {
-        constexpr int b = decltype(BB)::value;
-#pragma unroll
-        for(int i = 0; i < SPW; i++)
-#pragma unroll
-            for(int j = 0; j < NR; j++)
-            {
-                v8bf wq[4];
-                expand_fp4(wf[b][i][j], (wsc[b][i] >> (8 * ((kt & 1) * 2 + half + j))) & 0xFFu, wq);
-#pragma unroll
-                for(int c = 0; c < 4; c++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wq[c], __builtin_bit_cast(v8bf, af[b][i][c]), acc[i][j], 0, 0, 0);
-            }
-        if(kt + NB * 4 < KT)
-            load_step(BB, kt + NB * 4);
-    };
-    if(any)
+    if(turn && steps > 0)
     {
-        static_for<NB>([&](auto BB) __attribute__((always_inline)) {
-            const int kt = w + decltype(BB)::value * 4;
-            if(kt < KT)
-                load_step(BB, kt);
-        });
-        for(int kb0 = w; kb0 < KT; kb0 += NB * 4)
+        take_slot();
+        static_for<NB>([&](auto BB) __attribute__((always_inline)) { load_next(BB); });
+        u32 mine = turn;
+        int kt = w;
+        while(mine)
             static_for<NB>([&](auto BB) __attribute__((always_inline)) {
-                const int kt = kb0 + decltype(BB)::value * 4;
-                if(kt < KT)
-                    step(BB, kt);
+                constexpr int b = decltype(BB)::value;
+                if(!mine)
+                    return;
+#pragma unroll
+                for(int j = 0; j < NR; j++)
+                {
+                    v8bf wq[4];
+                    expand_fp4(wf[b][j], (wsc[b][j / 2] >> (8 * ((kt & 1) * 2 + half + (j & 1)))) & 0xFFu, wq);
+#pragma unroll
+                    for(int c = 0; c < 4; c++)
+                        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wq[c], __builtin_bit_cast(v8bf, af[b][c]), acc[j], 0, 0, 0);
+                }
+                load_next(BB);
+                kt += 4;
+                if(kt >= KT)
+                {
+                    kt = w;
+                    const int s = __builtin_ctz(mine);
+                    mine &= mine - 1u;
+#pragma unroll
+                    for(int j = 0; j < NR; j++)
+                    {
+                        if(r == 0)
+                            *(v4f*)&red[s][w][j * 16 + kb * 4] = acc[j];
+                        acc[j] = (v4f){0.f, 0.f, 0.f, 0.f};
+                    }
+                }
             });
     }
-#pragma unroll
-    for(int i = 0; i < SPW; i++)
-    {
-        const int s = q + i * groups;
-        if(s >= g.topk)
-            continue;
-        if(r == 0)
-#pragma unroll
-            for(int j = 0; j < NR; j++)
-                *(v4f*)&red[s][w][j * 16 + kb * 4] = acc[i][j];
-        if(w == 0)
+    else if(turn)
+        for(u32 m = turn; m; m &= m - 1u)      // (fewer K-steps than waves)
         {
-            if(lane == 0)
-            {
-                on_l[s] = on[i];
-                rw_l[s] = g.weights[t * g.topk + s];
-            }
-            if(g.bias && on[i] && lane < 16 * NR)
-                bias_l[s][lane] = bf16_bits_to_f32(g.bias[(size_t)e[i] * g.N + ch0 + lane]);
+            const int s = __builtin_ctz(m);
+            if(r == 0)
+#pragma unroll
+                for(int j = 0; j < NR; j++)
+                    *(v4f*)&red[s][w][j * 16 + kb * 4] = acc[j];
         }
-    }
+    // (asked for here and not at the start, where the wait for them would hold the weights up)
+    if(w == 0)
+        for(u32 m = turn; m; m &= m - 1u)
+        {
+            const int s = __builtin_ctz(m);
+            const int e = g.bias ? local_expert(__builtin_amdgcn_readlane(id, s), g.mask, lane) : 0;
+            if(lane == 0)
+                rw_l[s] = g.weights[t * g.topk + s];
+            if(g.bias && lane < 16 * NR)
+                bias_l[s][lane] = bf16_bits_to_f32(g.bias[(size_t)e * g.N + ch0 + lane]);
+        }
     __syncthreads();
     if(tid >= 16 * NR)
         return;
     float out = 0.f;
-    for(int s = 0; s < g.topk; s++)
+    for(u32 m = on; m; m &= m - 1u)
     {
-        if(!on_l[s])
-            continue;
-        float sum = 0.f;
+        const int s = __builtin_ctz(m);
+        float sum   = 0.f;
 #pragma unroll
         for(int p = 0; p < 4; p++)
             sum += red[s][p][tid];
@@ -432,7 +456,7 @@ int pyhip_pairs_gate_up(PairArgs g, int64_t rows, int64_t n_blk, int split_k, in
     g.act = make_gated_act(activation, swiglu_limit);
     // (tiles whose channels are all padding are not launched)
     const int tile = split ? 32 : 128;
-    g.n_tiles      = (g.N / 2 - g.n_pad + tile - 1) / tile;
+    g.n_tiles      = (g.N / 2 - (g.all_channels ? 0 : g.n_pad) + tile - 1) / tile;
     const dim3 grid((unsigned)(blocks * g.n_tiles));
     if(split)
         hipLaunchKernelGGL((moe_gemm_pairs_kernel<1, 4>), grid, dim3(W4A16_THREADS), 0, stream, g);
@@ -473,16 +497,17 @@ int pyhip_pairs_down_sum(PairArgs g, int64_t rows, int64_t n_blk, int split_k, h
     const int rc = prepare("moe_pairs_down_sum", g, rows, blocks, g.N / 64);
     if(rc)
         return rc;
-    const int groups = g.topk < 4 ? g.topk : 4;
-    const bool wide  = g.topk <= 4 && (int64_t)g.T * (g.N / 32) >= 512;
-    g.n_tiles        = g.N / (wide ? 32 : 16);
-    const dim3 grid((unsigned)(g.T * g.n_tiles)), block(groups * 4 * WAVE);
-    if(g.topk > 4)
-        hipLaunchKernelGGL((moe_pairs_down_sum_kernel<2, 1>), grid, block, 0, stream, g);
-    else if(wide)
-        hipLaunchKernelGGL((moe_pairs_down_sum_kernel<1, 2>), grid, block, 0, stream, g);
+    // as wide a tile as still gives half of the CUs a workgroup (and not, where a workgroup has many slots, every third CU a second one)
+    const int64_t at4 = (int64_t)g.T * (g.N / 64);
+    const int nr      = at4 >= 140 && !(g.topk > 4 && at4 > 256 && at4 < 400) ? 4 : at4 >= 80 ? 2 : 1;
+    g.n_tiles         = g.N / (16 * nr);
+    const dim3 grid((unsigned)(g.T * g.n_tiles)), block((g.topk > 1 ? 2 : 1) * 4 * WAVE);
+    if(nr == 4)
+        hipLaunchKernelGGL((moe_pairs_down_sum_kernel<4>), grid, block, 0, stream, g);
+    else if(nr == 2)
+        hipLaunchKernelGGL((moe_pairs_down_sum_kernel<2>), grid, block, 0, stream, g);
     else
-        hipLaunchKernelGGL((moe_pairs_down_sum_kernel<1, 1>), grid, block, 0, stream, g);
+        hipLaunchKernelGGL((moe_pairs_down_sum_kernel<1>), grid, block, 0, stream, g);
     PYHIP_CHECK_LAUNCH("moe_pairs_down_sum_kernel");
     return PYHIP_OK;
 }

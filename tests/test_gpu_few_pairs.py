@@ -8,11 +8,20 @@ import cases
 pytestmark = pytest.mark.gpu
 
 
+def _poison(T, k, E, H, I):
+    """the memory that the next call of these (padded) sizes gets as its workspace holds NaNs, in bf16 and in fp32"""
+    import sys
+    plan = sys.modules["pyhip_amd.fused_moe"]._plan
+    x = torch.empty(plan(T, k, E, H, I, "w4a16", 16)[2], dtype=torch.uint8, device="cuda")
+    x.fill_(255)
+
+
 @pytest.mark.parametrize("T,k,E,H,I,splitk", [
     (1, 1, 8, 512, 512, 0),          # one pair; every K split has one K-step
     (1, 4, 20, 1024, 2560, 0),       # a token's slots on four groups of waves, an uneven share of K-steps
-    (1, 4, 8, 16384, 512, 0),        # two row groups to a workgroup
-    (1, 6, 64, 512, 1024, 0),        # two slots for some waves, one for others
+    (1, 4, 8, 9216, 512, 0),         # four row groups to a workgroup, a K-step for each wave
+    (1, 5, 8, 5632, 1536, 0),        # two
+    (1, 6, 64, 512, 1024, 0),        # one; three slots for each group of waves
     (1, 9, 16, 512, 512, 0),         # more slots than the summing kernel holds
     (4, 1, 32, 512, 512, 0),         # summed by token
     (4, 8, 256, 512, 512, 4),        # the most pairs that are summed by token in 256 experts
@@ -57,11 +66,12 @@ def test_few_pairs_equal_the_stages(T, k, E, H, I, splitk):
             kw2 = dict(kw, method="w4a16", block_size_M=16, splitk=splitk, **more)
             want = fused_moe(hidden, wa, wb, tw, t.cuda(), return_parts=True, **kw2)[0]
             for _ in range(2):
+                _poison(T, L.k, E, H, I)
                 got = fused_moe(hidden, wa, wb, tw, t.cuda(), **kw2)
                 assert torch.equal(got, want)
 
 
-@pytest.mark.parametrize("T,H,I", [(1, 544, 544), (3, 1440, 1440), (1, 992, 32 * 47), (20, 1440, 1056), (30, 576, 1440)])
+@pytest.mark.parametrize("T,H,I", [(1, 544, 544), (1, 544, 8224), (3, 1440, 1440), (1, 992, 32 * 47), (20, 1440, 1056), (30, 576, 1440)])
 @pytest.mark.parametrize("wide", [False, True])
 def test_few_pairs_leave_padding_alone(T, H, I, wide):
     """Padded layers, activations at the true or the padded width.  The weights' padding is told, so it is not read: its rows and
@@ -87,6 +97,7 @@ def test_few_pairs_leave_padding_alone(T, H, I, wide):
         x = x[:, :H]
         x = torch.nn.functional.pad(x, (0, 8), value=float("nan"))[:, :H]
     print("few pairs, padded", T, H, I, wide, flush=True)
+    _poison(T, 2, 32, H + hp, I + ip)
     got = fused_moe(x, f1, f2, tw, ti, w1_scale=w1s, w2_scale=w2s, hidden_pad=hp, intermediate_pad=ip, **kw)
     assert torch.equal(got[:, :H], want[:, :H]) and (not wide or (got[:, H:] == 0).all())
 
