@@ -54,9 +54,10 @@ SIGNATURES = {
     "pyhip_moe_topk_reduce_routed": (_I, [_P, _P, _L, _I, _I, _I, _P, _I, _P, _P, _P]),
 }
 
-#: what fused_moe.py calls and the header does not declare: the layer call as one block of arguments
+#: what fused_moe.py calls and the header does not declare: the layer call as one block of arguments, and its choices
 INTERNAL = {
     "pyhip_layer_forward": (_I, [_c.c_char_p, _P]),
+    "pyhip_layer_block_m": (_I, [_L, _I, _I, _I, _I, _I]),
     "pyhip_layer_takes_cols": (_I, [_L, _I, _I, _I, _I, _I, _I, _I]),
 }
 

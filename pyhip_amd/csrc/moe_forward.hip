@@ -4,6 +4,7 @@
 // and launches its kernels one by one from Python); the choice of kernel family and row block stays with the caller.
 #include "common.h"
 #include "moe_gemm_pairs.h"
+#include <math.h>
 
 extern "C" {
 int64_t pyhip_moe_sorting_max_blocks(int64_t tokens, int topk, int experts, int block_size);
@@ -166,6 +167,73 @@ extern "C" int pyhip_moe_pick_block_m(int64_t tokens, int topk, int experts, int
             return 288;
     }
     return 128;
+}
+
+// Row blocks that hold an expert's rows, on average, when it gets a Poisson number of them with mean m
+static double expected_blocks(double m, int rows)
+{
+    if(m > 12.0 * rows)
+        return m / rows + 0.5;
+    double n = 1.0 - exp(-m);
+    for(int j = 1; j * rows < m + 5.0 * sqrt(m) + 1.0; j++)
+        n += 0.5 * erfc((j * rows + 0.5 - m) / sqrt(2.0 * m));
+    return n;
+}
+
+// What a launch of a tile height costs, us: a tile takes `start + step * K-groups`, `at_once` tiles run side by side (a launch of
+// fewer takes as long as one tile), and each further block of an expert costs `again` of the expert's weights in memory traffic (the rest it
+// finds in the L2).  Fitted to 490 random layers (8-256 experts, hidden 1024-7200, intermediate 512-14336, 16-8192 tokens, even and
+// Zipf routers, every height timed on each): the estimate of a call is within 8 % of its time (root mean square).
+struct TileCost
+{
+    int rows;
+    double start, step, at_once, again;
+};
+static const TileCost tile_costs[] = {{16, 1.2, 1.37, 1e9, 0.35}, {32, 1.5, 1.39, 1e9, 0.4},  {64, 3.3, 1.29, 334, 0.45},
+                                      {128, 4.5, 2.10, 307, 0.33}, {160, 5.8, 2.27, 284, 0.75}, {192, 6.8, 2.38, 271, 1.05},
+                                      {256, 8.6, 2.84, 276, 1.6},  {288, 9.8, 3.15, 273, 2.0}};
+
+// The tile height of an MXFP4-activation layer call whose sizes are known: the one of pyhip_moe_pick_block_m, which looks at the rows
+// per expert alone, unless that has fewer tiles in the gate_up GEMM than the chip has CUs and 64, 32 or 16 rows are estimated to
+// take 5 % less: lower tiles are more of them, and each is done sooner.  Layer, us: 8 experts, 1024 x 512, top-2, 493 tokens, 160 / 16 rows:
+// 30.2 / 23.7; 1024 tokens, 128 / 32: 30.2 / 27.1; 2208 x 1792, top-1, 446 tokens, 128 / 32: 36.5 / 27.2; 6176 x 512, Zipf, 371 tokens, 128 / 32:
+// 52.3 / 37.1.  Of 556 layers it moves 88, which take 16 % less then; two take more, by 2 and 3 %.
+// (With as many tiles as CUs and more the estimate would find other heights too, and is not good enough for it, nor does it know the
+// router: 64 rows instead of 128 cost up to 20 % between 33 and 60 rows per expert, 192 to 288 rows at hidden below 6144 save 14-23 % under
+// even routers and cost 6-18 % under Zipf ones.)
+extern "C" int pyhip_layer_block_m(int64_t tokens, int topk, int experts, int local_experts, int hidden, int inter)
+{
+    const int ladder = pyhip_moe_pick_block_m(tokens, topk, experts, hidden, 0);
+    if(tokens <= 0 || topk <= 0 || experts <= 0 || local_experts <= 0)
+        return ladder;
+    const double est = (double)tokens * topk / experts;
+    if(local_experts * expected_blocks(est, ladder) * (inter / 128) >= 256.0)
+        return ladder;
+    auto estimate = [&](const TileCost& c) {
+        const double hit = local_experts * (1.0 - exp(-est)), nb = local_experts * expected_blocks(est, c.rows);
+        // sort, reduction and the passes over the activations
+        double us = 12.0 + (double)tokens * (topk + 2) * hidden / 2.5e6;
+        for(int stage = 0; stage < 2; stage++)
+        {
+            const int n = stage ? hidden / 256 : inter / 128, groups = stage ? inter / 512 : hidden / 512;
+            const double run = (c.start + c.step * groups) * (nb * n > c.at_once ? nb * n / c.at_once : 1.0);
+            const double mem = (hit + c.again * (nb - hit)) * n * groups * (512.0 * 256.0 * 17.0 / 32.0) / 6.6e6;
+            us += sqrt(sqrt(run * run * run * run + mem * mem * mem * mem));
+        }
+        return us > 20.0 ? us : 20.0;       // (a call takes the host that long)
+    };
+    double best = 0.0;
+    for(const TileCost& c : tile_costs)
+        if(c.rows == ladder)
+            best = 0.95 * estimate(c);
+    int rows = ladder;
+    for(const TileCost& c : tile_costs)
+        if(c.rows < ladder && c.rows <= 64 && est <= 10.0 * c.rows && estimate(c) < best)      // (beyond ten blocks an expert: not measured)
+        {
+            best = estimate(c);
+            rows = c.rows;
+        }
+    return rows;
 }
 
 extern "C" int pyhip_moe_pick_w4a16(int64_t tokens, int topk, int experts, int hidden)

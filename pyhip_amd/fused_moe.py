@@ -106,7 +106,7 @@ def pick_w4a16(tokens, topk, experts, hidden):
     return bool(_lib.load().pyhip_moe_pick_w4a16(tokens, topk, experts, hidden))
 
 
-def _plan(tokens, topk, experts, hidden, inter, method, block_m):
+def _plan(tokens, topk, experts, hidden, inter, method, block_m, local_experts=None):
     """(bf16 activations?, row block, workspace bytes) of a layer call: a function of its sizes and options alone, so a
     program's few call shapes ask the library once each instead of three times a call (``method`` and ``block_m`` as
     given by the caller).  Only plain integers are remembered: whatever else converts to one may not be hashable (a numpy
@@ -114,12 +114,17 @@ def _plan(tokens, topk, experts, hidden, inter, method, block_m):
     With this, checks whose messages are put together only when they fail, and raw stream and data pointers, the
     tiny layer at 64 tokens went from 29.1 to 22.7 us a call."""
     plain = type(topk) is int and (block_m is None or type(block_m) is int)
-    return (_remembered_plan if plain else _ask_plan)(tokens, topk, experts, hidden, inter, method, block_m)
+    return (_remembered_plan if plain else _ask_plan)(tokens, topk, experts, hidden, inter, method, block_m, local_experts)
 
 
-def _ask_plan(tokens, topk, experts, hidden, inter, method, block_m):
+def _ask_plan(tokens, topk, experts, hidden, inter, method, block_m, local_experts=None):
     w4a16 = method == "w4a16" or (method != "a4w4" and pick_w4a16(tokens, topk, experts, hidden))
-    bm = block_m if block_m is not None else pick_block_m(tokens, topk, experts, hidden, w4a16)
+    if block_m is not None:
+        bm = block_m
+    elif w4a16:
+        bm = pick_block_m(tokens, topk, experts, hidden, True)
+    else:
+        bm = _lib.load().pyhip_layer_block_m(tokens, topk, experts, local_experts or experts, hidden, inter)
     if w4a16:
         bm = min(bm, 64)
     return w4a16, bm, _lib.load().pyhip_moe_forward_workspace_bytes(tokens, topk, experts, hidden, inter, bm, 1 if w4a16 else 0)
@@ -255,7 +260,7 @@ def fused_moe(
     if topk_weight.dtype != torch.float32 or not topk_weight.is_contiguous():
         topk_weight = topk_weight.to(torch.float32).contiguous()
     # "auto" (and the reference's "jit" / "gluon", which name its own back ends): see pick_w4a16
-    w4a16, bm, ws_bytes = _plan(T, k, global_E, H, I, method, block_size_M)
+    w4a16, bm, ws_bytes = _plan(T, k, global_E, H, I, method, block_size_M, E)
     if bias1 is not None:
         bias1 = bias1.to(torch.bfloat16).contiguous()
         _require(tuple(bias1.shape) == (E, 2 * I), "bias1 must be [E, 2*inter]")
@@ -458,7 +463,7 @@ def fused_moe_routed(hidden_states, w1, w2, gating_output, topk, renormalize=Tru
     dev = hidden_states.device
     if expert_mask is not None:
         expert_mask = expert_mask.to(device=dev, dtype=torch.int32).contiguous()
-    w4a16, bm, ws_bytes = _plan(T, topk, global_E, H, I, method, block_size_M)
+    w4a16, bm, ws_bytes = _plan(T, topk, global_E, H, I, method, block_size_M, E)
     if bias1 is not None:
         bias1 = bias1.to(torch.bfloat16).contiguous()
     if bias2 is not None:

@@ -1,0 +1,31 @@
+"""The tile height of a layer call whose sizes are known: a served one for any sizes, the ladder's where no other is clearly better."""
+import random
+
+import pytest
+
+from pyhip_amd import _lib
+
+
+@pytest.mark.parametrize("tokens,topk,experts,local,hidden,inter,want", [
+    (493, 2, 8, 8, 1024, 512, 16),           # few tiles: the ladder has 160 rows
+    (1024, 2, 8, 8, 1024, 512, 32),          # 128
+    (446, 1, 8, 8, 2560, 2048, 32),          # 128
+    # where the ladder stays
+    (4096, 2, 8, 8, 4096, 14336, 128), (4096, 4, 128, 128, 3072, 3072, 160), (2048, 8, 128, 128, 4096, 1536, 160),
+    (4001, 8, 256, 32, 7168, 2048, 160), (8192, 8, 256, 256, 7168, 2048, 288), (128, 8, 256, 256, 7168, 2048, 32),
+    (16, 4, 128, 128, 3072, 3072, 16), (64, 2, 8, 8, 1024, 512, 32),
+])
+def test_known_choices(tokens, topk, experts, local, hidden, inter, want):
+    assert _lib.load().pyhip_layer_block_m(tokens, topk, experts, local, hidden, inter) == want
+
+
+def test_any_sizes_get_a_served_height():
+    lib, rng = _lib.load(), random.Random(0)
+    served = {16, 32, 64, 128, 160, 192, 256, 288}
+    for _ in range(3000):
+        experts = rng.choice([1, 2, 3, 8, 60, 256, 2048, 5000])
+        a = (int(2 ** rng.uniform(0, 23)), rng.randint(1, 255), experts, rng.randint(1, experts), rng.randrange(512, 16897, 512),
+             rng.randrange(512, 16897, 512))
+        assert lib.pyhip_layer_block_m(*a) in served, a
+    for a in ((0, 2, 8, 8, 1024, 512), (64, 0, 8, 8, 1024, 512), (64, 2, 8, 0, 1024, 512)):
+        assert lib.pyhip_layer_block_m(*a) == lib.pyhip_moe_pick_block_m(a[0], a[1], a[2], a[4], 0)
