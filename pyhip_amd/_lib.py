@@ -5,8 +5,13 @@ There is no CPU fallback: if the library is missing, loading raises.
 import ctypes
 import os
 
+import torch
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libpyhip_moe.so")
+
+_current_device = torch.cuda.current_device
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)      # (a CPU-only torch has none)
 
 _c = ctypes
 _P, _I, _L, _F = _c.c_void_p, _c.c_int, _c.c_int64, _c.c_float
@@ -103,8 +108,7 @@ def address(t):
 def stream_handle():
     """the current torch stream's handle as an integer, without the Stream object that ``torch.cuda.current_stream()``
     builds; for the same functions as ``addr``"""
-    import torch
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    return _raw_stream(_current_device())
 
 
 def dptr(t):

@@ -37,6 +37,13 @@ def _require(cond, msg, exc=ValueError, *args):
         raise exc("fused_moe: " + (msg % tuple(tuple(a) if isinstance(a, torch.Size) else a for a in args) if args else msg))
 
 
+def _plain(t, dtype, device=None):
+    """``t`` as a contiguous tensor of that type (on that device), itself where it is one"""
+    if t.dtype == dtype and t.is_contiguous() and (device is None or t.device == device):
+        return t
+    return (t.to(dtype) if device is None else t.to(device=device, dtype=dtype)).contiguous()
+
+
 def _is_shuffled(w):
     """the reference's convention (src/contrib/fused_moe.py:198-206): an ``nn.Parameter`` counts as pre-shuffled
     (wrapping drops the attribute), otherwise the tensor attribute ``is_shuffled`` says so, default False"""
@@ -158,6 +165,32 @@ def act_quant_mxfp4(x, rows_limit=None):
     return q, s
 
 
+_ACTIVATIONS = (ActivationType.Silu, ActivationType.Swiglu)
+_SPLITS = (0, 1, 4, 16, 32)
+_OUT_DTYPES = (torch.bfloat16, torch.float32)
+_METHODS = ("auto", "a4w4", "w4a16", "jit", "gluon")
+_REDUCES = ("store", "atomic", "last_arriver")
+_STAGINGS = ("registers", "lds")
+
+
+def _refuse_options(hidden_states, activation, quant_type, doweight_stage1, w1_scale, w2_scale, a1_scale, a2_scale, splitk, out_dtype, method,
+                    topk_reduce, operand_staging):
+    """raises for the first of the options that ``fused_moe`` does not take"""
+    _require(activation in _ACTIVATIONS, "SiLU- or SwiGLU-gated experts only")
+    _require(quant_type == QuantType.per_1x32, "this operator is the MXFP4 (per_1x32) path")
+    _require(not doweight_stage1, "doweight_stage1 is not supported (the reference rejects it as well)")
+    _require(a1_scale is None and a2_scale is None, "activations are quantised dynamically: a1_scale / a2_scale must be None")
+    _require(splitk in _SPLITS, "splitk: 0 = automatic, 1 = off, 4 / 16 = split K over that many waves of a workgroup, "
+             "32 = sixteen waves on 32-row weight tiles in the down GEMM (w4a16 path only)")
+    _require(w1_scale is not None and w2_scale is not None, "w1_scale and w2_scale (e8m0, shuffled) are required")
+    _require(hidden_states.is_cuda and hidden_states.dtype == torch.bfloat16 and hidden_states.dim() == 2,
+             "hidden_states must be a bf16 matrix on the GPU", TypeError)
+    _require(out_dtype in _OUT_DTYPES, "dtype must be bfloat16 or float32", TypeError)
+    _require(method in _METHODS, "method=%r", ValueError, method)
+    _require(topk_reduce in _REDUCES, "topk_reduce=%r", ValueError, topk_reduce)
+    _require(operand_staging in _STAGINGS, "operand_staging=%r", ValueError, operand_staging)
+
+
 def fused_moe(
     hidden_states,
     w1,  # [E, inter_dim*2, dim/2]  gate rows then up rows
@@ -203,22 +236,16 @@ def fused_moe(
     src/contrib/moe_gemm_mxfp4.py:318-637) instead of the tiles that load weights straight into registers:
     bit-identical results, measured slower, never chosen automatically."""
     lib = _lib.load()
-    _require(activation in (ActivationType.Silu, ActivationType.Swiglu), "SiLU- or SwiGLU-gated experts only")
+    out_dtype = hidden_states.dtype if dtype is None else dtype
+    # everything at once; what is wrong is looked for when something is (a small call takes the host as long as the device)
+    if not (activation in _ACTIVATIONS and quant_type == QuantType.per_1x32 and not doweight_stage1 and a1_scale is None and a2_scale is None
+            and splitk in _SPLITS and w1_scale is not None and w2_scale is not None and hidden_states.is_cuda
+            and hidden_states.dtype == torch.bfloat16 and hidden_states.dim() == 2 and out_dtype in _OUT_DTYPES and method in _METHODS
+            and topk_reduce in _REDUCES and operand_staging in _STAGINGS):
+        _refuse_options(hidden_states, activation, quant_type, doweight_stage1, w1_scale, w2_scale, a1_scale, a2_scale, splitk, out_dtype,
+                        method, topk_reduce, operand_staging)
     act = 1 if activation == ActivationType.Swiglu else 0
     limit = float(swiglu_limit) if swiglu_limit else 7.0
-    _require(quant_type == QuantType.per_1x32, "this operator is the MXFP4 (per_1x32) path")
-    _require(not doweight_stage1, "doweight_stage1 is not supported (the reference rejects it as well)")
-    _require(a1_scale is None and a2_scale is None, "activations are quantised dynamically: a1_scale / a2_scale must be None")
-    _require(splitk in (0, 1, 4, 16, 32), "splitk: 0 = automatic, 1 = off, 4 / 16 = split K over that many waves of a workgroup, "
-             "32 = sixteen waves on 32-row weight tiles in the down GEMM (w4a16 path only)")
-    _require(w1_scale is not None and w2_scale is not None, "w1_scale and w2_scale (e8m0, shuffled) are required")
-    _require(hidden_states.is_cuda and hidden_states.dtype == torch.bfloat16 and hidden_states.dim() == 2,
-             "hidden_states must be a bf16 matrix on the GPU", TypeError)
-    out_dtype = hidden_states.dtype if dtype is None else dtype
-    _require(out_dtype in (torch.bfloat16, torch.float32), "dtype must be bfloat16 or float32", TypeError)
-    _require(method in ("auto", "a4w4", "w4a16", "jit", "gluon"), "method=%r", ValueError, method)
-    _require(topk_reduce in ("store", "atomic", "last_arriver"), "topk_reduce=%r", ValueError, topk_reduce)
-    _require(operand_staging in ("registers", "lds"), "operand_staging=%r", ValueError, operand_staging)
 
     # weights in the plain layout (no ``is_shuffled`` mark) are re-tiled once; the scales always come e8m0-shuffled,
     # as the reference passes them (tests/contrib/moe/test_moe.py:167-189)
@@ -229,16 +256,18 @@ def fused_moe(
     # reference's convention) or at the true width, in which case the result is returned at the true width too; the input
     # quantisation then fills in the padding's zeros, or the rows are widened first where it cannot take them (below).
     # The MXFP4-activation GEMMs are told the pads and leave the weights' padding unfetched.
-    _require(0 <= hidden_pad < w1u.shape[2] * 2 and 0 <= intermediate_pad < w1u.shape[1] // 2, "bad hidden_pad / intermediate_pad")
-    narrow = hidden_pad > 0 and hidden_states.shape[1] == w1u.shape[2] * 2 - hidden_pad
-    T, H = hidden_states.shape[0], w1u.shape[2] * 2 if narrow else hidden_states.shape[1]
-    _require(topk_ids.dim() == 2 and topk_ids.shape[0] == T and tuple(topk_weight.shape) == tuple(topk_ids.shape),
-             "topk_ids / topk_weight must be [tokens, topk]")
-    k = topk_ids.shape[1]
     E, N1, Hb = w1u.shape
     I = N1 // 2
-    _require(Hb * 2 == H and tuple(w2u.shape) == (E, H, I // 2), "shapes do not fit: hidden %s, w1 %s, w2 %s", ValueError,
-             H, w1u.shape, w2u.shape)
+    T, H = hidden_states.shape
+    _require(0 <= hidden_pad < Hb * 2 and 0 <= intermediate_pad < I, "bad hidden_pad / intermediate_pad")
+    narrow = hidden_pad > 0 and H == Hb * 2 - hidden_pad
+    if narrow:
+        H = Hb * 2
+    ids_shape = topk_ids.shape
+    _require(len(ids_shape) == 2 and ids_shape[0] == T and topk_weight.shape == ids_shape, "topk_ids / topk_weight must be [tokens, topk]")
+    k = ids_shape[1]
+    if Hb * 2 != H or w2u.shape != (E, H, I // 2):
+        _require(False, "shapes do not fit: hidden %s, w1 %s, w2 %s", ValueError, H, w1u.shape, w2u.shape)
     _require(w1u.is_contiguous() and w2u.is_contiguous() and w1s.is_contiguous() and w2s.is_contiguous(),
              "weights and scales must be contiguous")
     global_E = E if expert_mask is None else expert_mask.numel()
@@ -246,50 +275,34 @@ def fused_moe(
     if T == 0:
         return torch.zeros(0, H, dtype=out_dtype, device=dev)
 
-    def _mark(name, start=None):
-        if stage_events is None:
-            return None
-        ev = torch.cuda.Event(enable_timing=True)
-        ev.record()
-        if start is not None:
-            stage_events.append((name, start, ev))
-        return ev
-
-    if topk_ids.dtype != torch.int32 or not topk_ids.is_contiguous():
-        topk_ids = topk_ids.to(torch.int32).contiguous()
-    if topk_weight.dtype != torch.float32 or not topk_weight.is_contiguous():
-        topk_weight = topk_weight.to(torch.float32).contiguous()
+    topk_ids, topk_weight = _plain(topk_ids, torch.int32), _plain(topk_weight, torch.float32)
     # "auto" (and the reference's "jit" / "gluon", which name its own back ends): see pick_w4a16
     w4a16, bm, ws_bytes = _plan(T, k, global_E, H, I, method, block_size_M, E)
     if bias1 is not None:
-        bias1 = bias1.to(torch.bfloat16).contiguous()
-        _require(tuple(bias1.shape) == (E, 2 * I), "bias1 must be [E, 2*inter]")
+        bias1 = _plain(bias1, torch.bfloat16)
+        _require(bias1.shape == (E, N1), "bias1 must be [E, 2*inter]")
     if bias2 is not None:
-        bias2 = bias2.to(torch.bfloat16).contiguous()
-        _require(tuple(bias2.shape) == (E, H), "bias2 must be [E, hidden]")
+        bias2 = _plain(bias2, torch.bfloat16)
+        _require(bias2.shape == (E, H), "bias2 must be [E, hidden]")
 
     if expert_mask is not None:
-        expert_mask = expert_mask.to(device=dev, dtype=torch.int32).contiguous()
+        expert_mask = _plain(expert_mask, torch.int32, dev)
     if num_local_tokens is not None:
         _require(num_local_tokens.is_cuda and num_local_tokens.dtype == torch.int32,
                  "num_local_tokens must be an int32 scalar tensor on the GPU", TypeError)
 
-    lds_tile = operand_staging == "lds"
-    if lds_tile:
-        _require(not w4a16 and block_size_M in (None, 256) and topk_reduce == "store",
+    lds_tile = atomic = arriver = False
+    if topk_reduce != "store" or operand_staging != "registers":
+        lds_tile, atomic, arriver = operand_staging == "lds", topk_reduce == "atomic", topk_reduce == "last_arriver"
+        _require(not lds_tile or (not w4a16 and block_size_M in (None, 256) and topk_reduce == "store"),
                  "operand_staging='lds' needs the MXFP4-activation path, 256-row blocks and topk_reduce='store'")
-        bm = 256
-    atomic = topk_reduce == "atomic"
-    if atomic:
-        _require(not w4a16 and bm in (16, 128) and out_dtype == torch.bfloat16,
+        if lds_tile:
+            bm = 256
+        _require(not atomic or (not w4a16 and bm in (16, 128) and out_dtype == torch.bfloat16),
                  "topk_reduce='atomic' needs the MXFP4-activation path, a row block of 16 or 128 and bf16 output")
-
-    arriver = topk_reduce == "last_arriver"
-    if arriver:
-        _require(not w4a16 and bm in (16, 128, 288) and not lds_tile,
+        _require(not arriver or (not w4a16 and bm in (16, 128, 288) and not lds_tile),
                  "topk_reduce='last_arriver' needs the MXFP4-activation path and a row block of 16, 128 or 288")
-
-    one_call = not return_parts and stage_events is None and not atomic and not lds_tile and not arriver
+    one_call = not return_parts and stage_events is None and not (atomic or lds_tile or arriver)
     cols = 0
     if narrow:
         # the one-call path takes activations at the true width as they are (bf16 ones only in its 16-row blocks): whole
@@ -307,18 +320,31 @@ def fused_moe(
         # from a graph)
         x = hidden_states
         # the kernels read 16-byte pieces of a row: views with an odd row stride or base (a column slice) are copied
-        if x.stride(1) != 1 or (w4a16 and not cols and x.stride(0) != H) or x.stride(0) % 8 != 0 or x.data_ptr() % 16 != 0:
+        rows, step = x.stride()
+        at = x.data_ptr()
+        if step != 1 or (w4a16 and not cols and rows != H) or rows % 8 != 0 or at % 16 != 0:
             x = x.contiguous()
+            rows, at = x.stride(0), x.data_ptr()
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-        out = torch.empty(T, H, dtype=out_dtype, device=dev)
+        out = torch.empty((T, H), dtype=out_dtype, device=dev)
         p = _lib.address
         rc = lib.pyhip_layer_forward(
-            _LAYER_CALL.pack(x.data_ptr(), w1u.data_ptr(), w1s.data_ptr(), w2u.data_ptr(), w2s.data_ptr(), p(bias1), p(bias2), 0,
+            _LAYER_CALL.pack(at, w1u.data_ptr(), w1s.data_ptr(), w2u.data_ptr(), w2s.data_ptr(), p(bias1), p(bias2), 0,
                              topk_ids.data_ptr(), topk_weight.data_ptr(), p(expert_mask), p(num_local_tokens), out.data_ptr(),
-                             ws.data_ptr(), x.stride(0), ws_bytes, cols, out_dtype == torch.float32, T, k, global_E, H, I,
+                             ws.data_ptr(), rows, ws_bytes, cols, out_dtype == torch.float32, T, k, global_E, H, I,
                              hidden_pad, intermediate_pad, bm, w4a16, splitk, act, 0, 0, 0, limit), _lib.stream_handle())
-        _lib.check(rc, "moe_forward")
-        return out[:, : H - hidden_pad] if narrow else out
+        if rc:
+            _lib.check(rc, "moe_forward")
+        return out.narrow(1, 0, H - hidden_pad) if narrow else out
+
+    def _mark(name, start=None):
+        if stage_events is None:
+            return None
+        ev = torch.cuda.Event(enable_timing=True)
+        ev.record()
+        if start is not None:
+            stage_events.append((name, start, ev))
+        return ev
 
     ev = _mark("start")
     # MXFP4-activation path: the input quantisation rides in the sort's launches (independent work, one dispatch less)
@@ -455,26 +481,26 @@ def fused_moe_routed(hidden_states, w1, w2, gating_output, topk, renormalize=Tru
     T, H = hidden_states.shape
     E, N1, Hb = w1u.shape
     I = N1 // 2
-    _require(Hb * 2 == H and tuple(w2u.shape) == (E, H, I // 2), "shapes do not fit")
+    _require(Hb * 2 == H and w2u.shape == (E, H, I // 2), "shapes do not fit")
     global_E = E if expert_mask is None else expert_mask.numel()
-    _require(gating_output.is_cuda and tuple(gating_output.shape) == (T, global_E) and global_E % 64 == 0,
+    _require(gating_output.is_cuda and gating_output.shape == (T, global_E) and global_E % 64 == 0,
              "gating_output must be [tokens, experts] on the GPU with experts a multiple of 64")
-    g = gating_output.float().contiguous()
+    g = _plain(gating_output, torch.float32)
     dev = hidden_states.device
     if expert_mask is not None:
-        expert_mask = expert_mask.to(device=dev, dtype=torch.int32).contiguous()
+        expert_mask = _plain(expert_mask, torch.int32, dev)
     w4a16, bm, ws_bytes = _plan(T, topk, global_E, H, I, method, block_size_M, E)
     if bias1 is not None:
-        bias1 = bias1.to(torch.bfloat16).contiguous()
+        bias1 = _plain(bias1, torch.bfloat16)
     if bias2 is not None:
-        bias2 = bias2.to(torch.bfloat16).contiguous()
+        bias2 = _plain(bias2, torch.bfloat16)
     x = hidden_states
     if x.stride(1) != 1 or (w4a16 and x.stride(0) != H) or x.stride(0) % 8 != 0 or x.data_ptr() % 16 != 0:
         x = x.contiguous()
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-    out = torch.empty(T, H, dtype=out_dtype, device=dev)
-    tw = torch.empty(T, topk, dtype=torch.float32, device=dev)
-    ti = torch.empty(T, topk, dtype=torch.int32, device=dev)
+    out = torch.empty((T, H), dtype=out_dtype, device=dev)
+    tw = torch.empty((T, topk), dtype=torch.float32, device=dev)
+    ti = torch.empty((T, topk), dtype=torch.int32, device=dev)
     p = _lib.address
     rc = lib.pyhip_layer_forward(
         _LAYER_CALL.pack(x.data_ptr(), w1u.data_ptr(), w1s.data_ptr(), w2u.data_ptr(), w2s.data_ptr(), p(bias1), p(bias2),
@@ -482,5 +508,6 @@ def fused_moe_routed(hidden_states, w1, w2, gating_output, topk, renormalize=Tru
                          ws.data_ptr(), x.stride(0), ws_bytes, 0, out_dtype == torch.float32, T, topk, global_E, H, I,
                          int(hidden_pad), int(intermediate_pad), bm, w4a16, splitk, act, int(num_expert_group), int(topk_group),
                          bool(renormalize), limit), _lib.stream_handle())
-    _lib.check(rc, "moe_forward_routed")
+    if rc:
+        _lib.check(rc, "moe_forward_routed")
     return (out, tw, ti) if return_routing else out
