@@ -4,6 +4,7 @@
 // and launches its kernels one by one from Python); the choice of kernel family and row block stays with the caller.
 #include "common.h"
 #include "moe_gemm_pairs.h"
+#include "quant_device.h"
 #include <math.h>
 
 extern "C" {
@@ -266,14 +267,22 @@ struct Router
 };
 }   // namespace
 
-// Whether forward_pairs below serves the call
+// Whether forward_pairs below serves the call.  MXFP4 activations: without a sort, or while experts have at most four rows on average,
+// so that even a busy one has few blocks.  With more rows per expert the persistent kernel, in which workgroups take the tiles of an
+// expert's blocks together, wins.  Layer, us, 16-row blocks, persistent kernel / this, by rows per expert: DeepSeek-V3 shape 0.5: 374.8 /
+// 353.4, 1.9: 758.7 / 727.4, 4: 887.1 / 868.6, 6.3: 911.0 / 908.4, 12.5: 1044 / 1085; Qwen3 shape 0.75: 63.6 / 56.4, 3.75: 119.5 / 106.9,
+// 8: 169.8 / 160.8, 31: 327 / 395; gpt-oss shape 1: 173.1 / 166.2, 3.4: 252.2 / 239.4, 9.4: 283.1 / 288.5; 96 experts, top-4, Zipf router,
+// 6272 x 1920, 1.7: 95.5 / 92.5, 3.8: 132.6 / 128.3, 8.3: 195.5 / 214.5
 static bool takes_pairs(int64_t tokens, int topk, int experts, int hidden, int inter, int block_m, int w4a16, int split_k)
 {
-    return w4a16 && block_m == 16 && hidden % 512 == 0 && inter % 512 == 0 && topk > 0 && experts <= 2048 &&
-           pyhip_pairs_served(tokens, topk, experts, hidden, inter, pyhip_moe_sorting_max_blocks(tokens, topk, experts, 16), split_k);
+    const int64_t pairs = tokens * topk;
+    if(!w4a16 && pairs > PAIRS_UNSORTED_MAX && pairs > 4ll * experts)
+        return false;
+    return block_m == 16 && hidden % 512 == 0 && inter % 512 == 0 && topk > 0 && experts <= 2048 &&
+           pyhip_pairs_served(tokens, topk, experts, hidden, inter, pyhip_moe_sorting_max_blocks(tokens, topk, experts, 16), !w4a16, split_k);
 }
 
-// The layer with bf16 activations and 16-row blocks (moe_gemm_pairs.hip).  Up to 64 pairs the kernels find their rows themselves
+// The layer in 16-row blocks by the kernels of moe_gemm_pairs.hip.  Up to 64 pairs the kernels find their rows themselves
 // and the sort is left out; where pairs rarely share an expert the down GEMM sums the slots and the reduction is left out too: two
 // launches (with the router three) instead of four.  What that saves is the launch on the host (3.3 us each) and the latency chain of the stage
 // on the device (sort 4.5-5.5, reduction 3-5 us).
@@ -281,14 +290,23 @@ static int forward_pairs(const void* hidden_bf16, int64_t row_stride, int hidden
                          const uint8_t* w2, const uint8_t* w2_scale, const void* bias1_bf16, const void* bias2_bf16,
                          const Router& router, int32_t* topk_ids, float* topk_weights, const int32_t* expert_mask,
                          const int32_t* num_local_tokens, void* out, int out_is_f32, int tokens, int topk, int experts,
-                         int hidden, int inter, int hidden_pad, int inter_pad, int split_k, int activation, float swiglu_limit,
-                         const Layout& l, uint8_t* ws, hipStream_t stream)
+                         int hidden, int inter, int hidden_pad, int inter_pad, int w4a16, int split_k, int activation,
+                         float swiglu_limit, const Layout& l, uint8_t* ws, hipStream_t stream)
 {
+    uint8_t* a2         = ws + (w4a16 ? l.a2 : l.a2_q);      // a row for every pair
     const bool unsorted = (int64_t)tokens * topk <= PAIRS_UNSORTED_MAX;
     uint32_t* s_ids     = (uint32_t*)(ws + l.sorted_ids);
     float* s_w          = (float*)(ws + l.sorted_w);
     uint32_t *s_e = (uint32_t*)(ws + l.sorted_e), *n_valid = (uint32_t*)(ws + l.num_valid), *sched = (uint32_t*)(ws + l.sched);
     int rc = PYHIP_OK;
+    if(!w4a16 && unsorted)
+    {
+        // (what the launch that quantises them asks of the hidden states)
+        QuantArgs q;
+        rc = pyhip_make_quant_args("moe_forward", hidden_bf16, row_stride, tokens, hidden, ws + l.a1_q, ws + l.a1_s, nullptr, &q, hidden_cols);
+        if(rc)
+            return rc;
+    }
     if(router.gating && unsorted)
         rc = router.n_group > 0 ? pyhip_moe_topk_grouped_sigmoid(router.gating, tokens, experts, topk, router.n_group, router.topk_group,
                                                                  router.renormalize, topk_weights, topk_ids, stream)
@@ -296,7 +314,12 @@ static int forward_pairs(const void* hidden_bf16, int64_t row_stride, int hidden
     else if(router.gating)
         rc = pyhip_moe_route_sorting(router.gating, tokens, topk, experts, router.n_group, router.topk_group, router.renormalize, 16,
                                      expert_mask, num_local_tokens, topk_weights, topk_ids, s_ids, s_w, s_e, n_valid, sched,
-                                     ws + l.sort_ws, l.sort_ws_bytes, nullptr, 0, tokens, hidden, nullptr, nullptr, stream);
+                                     ws + l.sort_ws, l.sort_ws_bytes, w4a16 ? nullptr : hidden_bf16, row_stride, tokens, hidden,
+                                     w4a16 ? nullptr : ws + l.a1_q, w4a16 ? nullptr : ws + l.a1_s, stream);
+    else if(!unsorted && !w4a16)
+        rc = pyhip_sorting_quant_cols(topk_ids, topk_weights, tokens, topk, experts, 16, expert_mask, num_local_tokens, s_ids, s_w, s_e,
+                                      n_valid, sched, ws + l.sort_ws, l.sort_ws_bytes, hidden_bf16, row_stride, tokens, hidden,
+                                      ws + l.a1_q, ws + l.a1_s, hidden_cols, stream);
     else if(!unsorted)
         rc = pyhip_moe_sorting(topk_ids, topk_weights, tokens, topk, experts, 16, expert_mask, num_local_tokens, s_ids, s_w, s_e,
                                n_valid, sched, nullptr, 0, ws + l.sort_ws, l.sort_ws_bytes, stream);
@@ -313,15 +336,25 @@ static int forward_pairs(const void* hidden_bf16, int64_t row_stride, int hidden
     }
     g.T = tokens; g.topk = topk; g.experts = experts;
     PairArgs up = g, down = g;
-    up.a = (const uint16_t*)hidden_bf16; up.w = w1; up.w_s = w1_scale; up.bias = (const uint16_t*)bias1_bf16;
-    up.out = ws + l.a2; up.K = hidden; up.N = 2 * inter;
+    up.a = hidden_bf16; up.w = w1; up.w_s = w1_scale; up.bias = (const uint16_t*)bias1_bf16;
+    up.out = a2; up.K = hidden; up.N = 2 * inter;
     up.a_pitch = (int)row_stride; up.k_real = hidden_cols ? hidden_cols : hidden - hidden_pad; up.n_pad = inter_pad;
-    down.a = (const uint16_t*)(ws + l.a2); down.w = w2; down.w_s = w2_scale; down.bias = (const uint16_t*)bias2_bf16;
+    down.a = a2; down.w = w2; down.w_s = w2_scale; down.bias = (const uint16_t*)bias2_bf16;
     down.out = out; down.out_f32 = out_is_f32; down.K = inter; down.N = hidden;
     down.a_pitch = inter; down.k_real = inter - inter_pad; down.n_pad = hidden_pad;
+    up.fp4 = down.fp4 = !w4a16;
+    if(!w4a16)
+    {
+        up.out_s = ws + l.a2_s; down.a_s = ws + l.a2_s;
+        if(!unsorted)
+        {
+            // (the sort's launch has quantised the tokens)
+            up.a = ws + l.a1_q; up.a_s = ws + l.a1_s; up.a_pitch = hidden;
+        }
+    }
     // (the kernels that sum a top-2 token's slots read the rows of a2 where the single-token entry points put them, and all of their
     // columns)
-    const bool top2 = tokens == 1 && topk == 2;
+    const bool top2 = w4a16 && tokens == 1 && topk == 2;
     up.row_step = down.row_step = top2 ? 16 : 1;
     up.all_channels             = top2;
     rc = pyhip_pairs_gate_up(up, tokens, l.n_blk, split_k, activation, swiglu_limit, stream);
@@ -329,16 +362,17 @@ static int forward_pairs(const void* hidden_bf16, int64_t row_stride, int hidden
         return rc;
     if(top2)
     {
-        rc = pyhip_w4a16_token_top2(ws + l.a2, w2, w2_scale, bias2_bf16, topk_ids, topk_weights, expert_mask, num_local_tokens,
+        rc = pyhip_w4a16_token_top2(a2, w2, w2_scale, bias2_bf16, topk_ids, topk_weights, expert_mask, num_local_tokens,
                                     out, out_is_f32, topk, experts, hidden, inter, split_k, stream);
         if(rc >= 0)
             return rc;
     }
-    rc = pyhip_pairs_down_sum(down, l.rows2, l.n_blk, split_k, stream);
+    const int64_t a2_rows = w4a16 ? l.rows2 : (int64_t)tokens * topk;
+    rc                    = pyhip_pairs_down_sum(down, a2_rows, l.n_blk, split_k, stream);
     if(rc >= 0)
         return rc;
     down.out = ws + l.out3;
-    rc       = pyhip_pairs_down(down, l.rows2, l.n_blk, split_k, stream);
+    rc       = pyhip_pairs_down(down, a2_rows, l.n_blk, split_k, stream);
     if(rc)
         return rc;
     return pyhip_moe_topk_reduce_routed(ws + l.out3, out, tokens, topk, hidden, out_is_f32, topk_ids, experts, expert_mask,
@@ -361,7 +395,8 @@ static int forward_impl(const void* hidden_bf16, int64_t hidden_row_stride, int 
     PYHIP_REQUIRE(block_m == 16 || block_m == 32 || block_m == 64 ||
                       ((block_m == 128 || block_m == 160 || block_m == 192 || block_m == 256 || block_m == 288) && !w4a16),
                   "moe_forward: block_m=%d (16/32/64, and 128/160/192/256/288 with MXFP4 activations)", block_m);
-    const bool pairs = takes_pairs(tokens, topk, experts, hidden, inter, block_m, w4a16, split_k);
+    // (32-bit offsets into the hidden states)
+    const bool pairs = takes_pairs(tokens, topk, experts, hidden, inter, block_m, w4a16, split_k) && tokens * hidden_row_stride < (1 << 30);
     bf16_cols        = bf16_cols && pairs && hidden_cols > 0 && hidden_row_stride >= hidden_cols && hidden_row_stride % 8 == 0 &&
                 hidden_row_stride < (1 << 24);
     PYHIP_REQUIRE(!w4a16 || hidden_row_stride == hidden || bf16_cols, "moe_forward: the bf16-activation kernels need contiguous rows");
@@ -382,7 +417,7 @@ static int forward_impl(const void* hidden_bf16, int64_t hidden_row_stride, int 
     if(pairs)
         return forward_pairs(hidden_bf16, hidden_row_stride, hidden_cols, w1, w1_scale, w2, w2_scale, bias1_bf16, bias2_bf16, router,
                              topk_ids, topk_weights, expert_mask, num_local_tokens, out, out_is_f32, tokens, topk, experts, hidden,
-                             inter, hidden_pad, inter_pad, split_k, activation, swiglu_limit, l, ws, stream);
+                             inter, hidden_pad, inter_pad, w4a16, split_k, activation, swiglu_limit, l, ws, stream);
     if(w4a16 && tokens == 1 && !router.gating)
     {
         // a single token with bf16 activations: no sort; the GEMMs read the routing themselves, one block per slot

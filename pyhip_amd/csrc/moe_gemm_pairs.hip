@@ -1,16 +1,20 @@
-// The layer call's GEMMs with bf16 activations and 16-row blocks: few tokens, so the call is a weight stream and a chain of
-// launches.  The arithmetic (and with it every bit of the result) is that of moe_gemm_w4a16.hip, whose entry points serve callers
-// that run the stages one by one; what is different is what a call of 20-100 us spends beside its weights:
+// The layer call's GEMMs in 16-row blocks: few tokens, so the call is a weight stream and a chain of launches.  With bf16
+// activations the arithmetic (and with it every bit of the result) is that of moe_gemm_w4a16.hip, with MXFP4 ones that of
+// moe_gemm_mxfp4.hip; their entry points serve callers that run the stages one by one.  What is different is what a call of 20-100 us spends beside its weights:
 //   * Up to 64 pairs (token, slot) there is no sort: every wave reads the routing, a pair to a lane, and finds its block's
 //     expert and rows with a few ballots (find_block).
 //   * Activations come at their own row pitch and width, and neither the padding rows nor the padding columns of the weights
 //     are fetched (raw buffer loads: a lane or a row group that has nothing to fetch is out of its descriptor's range).
 //   * Where nearly every pair has an expert of its own, the down GEMM goes by token instead of by expert: a workgroup holds
-//     all of a token's slots for 16 to 64 output channels, so it sums them and no reduction follows.
+//     all of a token's slots for 16 to 64 output channels, so it sums them and no reduction follows (bf16 activations).
+//   * With MXFP4 activations a workgroup is one tile of 64 weight rows, not a persistent loop over tiles that meets a barrier
+//     for each K-step, and its waves hold three K-steps in flight without LDS between them and the matrix cores.
 // Bound: the weight stream from about 40 us on, the launches and their latency chains below.  Layer call, us, sort + moe_gemm_w4a16
 // kernels + reduction (padded layers: after a widening of the activations) / this: gpt-oss shape, 2 tokens 39.5 / 28.7, 5 tokens
 // 67.0 / 51.3 (bound at 6.9 TB/s: 38); 32 experts, top-1, 2144 x 3040, 3 tokens 36.7 / 18.4; 1024 x 512, 8 experts, 10 tokens 25.0 / 17.6;
-// Mixtral shape, 5 tokens 100.6 / 94.5, 29 tokens 129.9 / 124.1 (5.75 -> 6.0 TB/s).
+// Mixtral shape, 5 tokens 100.6 / 94.5, 29 tokens 129.9 / 124.1 (5.75 -> 6.0 TB/s).  MXFP4 activations, sort with quantisation + persistent
+// kernels + reduction / this: gpt-oss shape, 16 tokens 121.5 / 108.8 (bound 97.7); Qwen3 shape, 5 tokens 57.7 / 43.0, 30 tokens 87.9 / 77.6;
+// DeepSeek-V3 shape, 16 tokens 374.8 / 353.4, 100 tokens 863.9 / 834.9 (6.7 -> 6.95 TB/s).
 #include "w4a16_device.h"
 #include "moe_gemm_pairs.h"
 
@@ -89,14 +93,44 @@ __device__ __forceinline__ v4f add_bias4(v4f v, uint2 b)
     return v;
 }
 
+// 32 bf16 of a row (a lane's K-elements of a K-step, which are one MX block) as the quantiser gives them (quant_device.h): eight e2m1
+// codes to a dword, and the block's scale byte
+__device__ __forceinline__ void quantise32(const v4i (&x)[4], v4i& q, int& e8)
+{
+    u32 am = 0;
+#pragma unroll
+    for(int i = 0; i < 4; i++)
+#pragma unroll
+        for(int c = 0; c < 4; c++)
+            am = amax15x2(am, (u32)x[i][c]);
+    const u32 s = mx_scale_byte(amax15_fold(am));
+#pragma unroll
+    for(int i = 0; i < 4; i++)
+        q[i] = (int)cvt8(__builtin_bit_cast(uint4, x[i]), s);
+    e8 = (int)s;
+}
+// acc += W(16 rows x 128 K, e2m1) * A(128 K x 16 rows, e2m1), scales in the low bytes
+__device__ __forceinline__ v4f mfma_fp4(const v4i& w, int ws, const v4i& a, int as, const v4f& acc)
+{
+    const v8i w8 = {w.x, w.y, w.z, w.w, 0, 0, 0, 0}, a8 = {a.x, a.y, a.z, a.w, 0, 0, 0, 0};
+    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w8, a8, acc, 4, 4, 0, ws, 0, as);
+}
+
 // STAGE 1 = gate_up (+ the gated activation), 2 = down (* routing weight).  SPLIT 0: a wave owns 64 weight rows over the whole K;
 // 4: the four waves share 64 weight rows, wave w takes K-steps w, w + 4, .. and the partial sums meet in LDS.
-// Three K-steps of operands are in flight; a register set is refilled as soon as its MFMAs are issued.
-template <int STAGE, int SPLIT>
+// NB K-steps of operands are in flight; a register set is refilled as soon as its MFMAs are issued.
+// ACT: the activations are BF16 (their products with the weights expanded to bf16), or MXFP4, quantised by whoever wrote them (QUANTISED)
+// or on the way to the matrix cores (TO_FP4: 40 instructions a K-step, where expanding the weights takes 64).  With MXFP4 the products are
+// multiples of powers of two, which 32-bit sums hold exactly in whatever order: the bits of moe_gemm_mxfp4.hip.  Its gate_up GEMM
+// quantises its result as that one does: a workgroup's 32 channels are one MX block of a row, which wave 0 finishes.
+enum { BF16, TO_FP4, QUANTISED };
+template <int STAGE, int SPLIT, int ACT>
 __global__ void __launch_bounds__(W4A16_THREADS) moe_gemm_pairs_kernel(PairArgs g)
 {
     constexpr bool SPLITK = SPLIT != 0;
+    static_assert(SPLITK || ACT == BF16, "MXFP4 activations: the four waves split K");
     constexpr int NB = 3, KSTRIDE = SPLITK ? 4 : 1;
+    constexpr int NA = ACT == QUANTISED ? 1 : 4;                  // 16-byte pieces of a row in a lane's K-step
     __shared__ float red[SPLITK ? 4 * 4 * WAVE * 4 : 1];          // [wave][row group][lane][4]
     const int tid = threadIdx.x, lane = tid % WAVE;
     const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
@@ -136,8 +170,9 @@ __global__ void __launch_bounds__(W4A16_THREADS) moe_gemm_pairs_kernel(PairArgs 
         const int tok = (int)(id & 0xFFFFFFu), slot = (int)(id >> 24);
         if(slot < g.topk && tok < g.T)
         {
-            arow = STAGE == 1 ? tok : p;
-            orow = STAGE == 1 ? p : tok * g.topk + slot;
+            const int pair = tok * g.topk + slot;
+            arow           = STAGE == 1 ? tok : pair;
+            orow           = pair;
         }
     }
     // row group j = 0..3 (stage 1: 0, 1 gate rows, 2, 3 the matching up rows); two of them share a scale tile of 32 rows
@@ -155,68 +190,93 @@ __global__ void __launch_bounds__(W4A16_THREADS) moe_gemm_pairs_kernel(PairArgs 
 #pragma unroll
     for(int h = 0; h < 2; h++)
         sb[h] = buffer_of(g.w_s + (size_t)(row_of(2 * h) / 32) * sc_tile, sc_tile);
-    const rsrc_t ab = buffer_of(g.a, g.a_bytes);
-    const int a_off = arow >= 0 ? arow * g.a_pitch * 2 + kb * 64 : NOWHERE;
+    const rsrc_t ab = buffer_of(g.a, g.a_bytes), asb = buffer_of(g.a_s, g.as_bytes);
+    const int SK     = (g.K + 511) / 512 * 16;      // bytes of a row's scales (moe_quant.hip)
+    const int a_off  = arow < 0 ? NOWHERE : ACT == QUANTISED ? arow * Kb + kb * 16 : arow * g.a_pitch * 2 + kb * 64;
+    const int as_off = arow < 0 ? NOWHERE : arow * SK + kb * 4;
 
     v4f acc[4];
 #pragma unroll
     for(int j = 0; j < 4; j++)
         acc[j] = (v4f){0.f, 0.f, 0.f, 0.f};
     const int KT = (g.k_real + 127) / 128;
-    v4i wf[NB][4], af[NB][4];
-    u32 wsc[NB][2];
+    v4i wf[NB][4], af[NB][NA];
+    u32 wsc[NB][2], asc[NB];
     auto load_step = [&](auto BB, int kt) __attribute__((always_inline)) {
         constexpr int b = decltype(BB)::value;
         const int away  = kt * 128 + kb * 32 >= g.k_real ? NOWHERE : 0;
 #pragma unroll
         for(int h = 0; h < 2; h++)
-            wsc[b][h] = load4(sb[h], lane * 4, (kt >> 1) * 256);
+            wsc[b][h] = load4(sb[h], lane * 4 | away, (kt >> 1) * 256);
 #pragma unroll
         for(int j = 0; j < 4; j++)
             wf[b][j] = load16_nt(wb[j], lane * 16 | away, kt * 1024);
 #pragma unroll
-        for(int i = 0; i < 4; i++)
-            af[b][i] = load16(ab, (a_off + i * 16) | away, kt * 256);
+        for(int i = 0; i < NA; i++)
+            af[b][i] = load16(ab, (a_off + i * 16) | away, kt * (64 * NA));
+        if constexpr(ACT == QUANTISED)
+            asc[b] = load4(asb, as_off | away, (kt >> 2) * 16);
     };
     auto step = [&](auto BB, int kt) __attribute__((always_inline)) {
         constexpr int b = decltype(BB)::value;
+        v4i aq;
+        int as;
+        if constexpr(ACT == TO_FP4)
+            quantise32(af[b], aq, as);
+        else if constexpr(ACT == QUANTISED)
+        {
+            aq = af[b][0];
+            as = (int)(asc[b] >> (8 * (kt & 3)));
+        }
 #pragma unroll
         for(int j = 0; j < 4; j++)
         {
-            v8bf wq[4];
-            expand_fp4(wf[b][j], (wsc[b][j >> 1] >> (8 * ((kt & 1) * 2 + (j & 1)))) & 0xFFu, wq);
+            const u32 ws = wsc[b][j >> 1] >> (8 * ((kt & 1) * 2 + (j & 1)));
+            if constexpr(ACT != BF16)
+                acc[j] = mfma_fp4(wf[b][j], (int)ws, aq, as, acc[j]);
+            else
+            {
+                v8bf wq[4];
+                expand_fp4(wf[b][j], ws & 0xFFu, wq);
 #pragma unroll
-            for(int i = 0; i < 4; i++)
-                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wq[i], __builtin_bit_cast(v8bf, af[b][i]), acc[j], 0, 0, 0);
+                for(int i = 0; i < 4; i++)
+                    acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wq[i], __builtin_bit_cast(v8bf, af[b][i]), acc[j], 0, 0, 0);
+            }
         }
-        if(kt + NB * KSTRIDE < KT)
-            load_step(BB, kt + NB * KSTRIDE);
     };
+    // (the loads carry no condition: K-steps past the last one are out of range.  A branch around them costs the loop its prefetch
+    // distance: the register sets then meet in copies, which wait for what is in flight.  So does a scheduler that moves a K-step's
+    // loads behind the next one's waits: gpt-oss shape, 16 tokens, MXFP4, 132.7 us with both, 108.2 without.)
     const int kt0 = SPLITK ? wave : 0;
     static_for<NB>([&](auto BB) __attribute__((always_inline)) {
-        const int kt = kt0 + decltype(BB)::value * KSTRIDE;
-        if(kt < KT)
-            load_step(BB, kt);
+        load_step(BB, kt0 + decltype(BB)::value * KSTRIDE);
+        __builtin_amdgcn_sched_barrier(0);
     });
-    for(int kb0 = kt0; kb0 < KT; kb0 += NB * KSTRIDE)
+    int kt = kt0;
+    for(; kt + NB * KSTRIDE < KT; kt += NB * KSTRIDE)
         static_for<NB>([&](auto BB) __attribute__((always_inline)) {
-            const int kt = kb0 + decltype(BB)::value * KSTRIDE;
-            if(kt < KT)
-                step(BB, kt);
+            step(BB, kt + decltype(BB)::value * KSTRIDE);
+            __builtin_amdgcn_sched_barrier(0);
+            load_step(BB, kt + (decltype(BB)::value + NB) * KSTRIDE);
+            __builtin_amdgcn_sched_barrier(0);
         });
+    static_for<NB>([&](auto BB) __attribute__((always_inline)) {
+        if(kt + decltype(BB)::value * KSTRIDE < KT)
+            step(BB, kt + decltype(BB)::value * KSTRIDE);
+    });
 
     // ---- epilogue: lane (r, kb) holds channels kb*4 .. + 3 of row group j for row r.  Under the K split wave w finishes row
-    // group w (stage 1: gate group w and its up group, waves 0 and 1)
+    // group w (stage 1: gate group w and its up group, waves 0 and 1; where the result is quantised wave 0 finishes both)
     auto channel = [&](int j) __attribute__((always_inline)) -> int {
         return (STAGE == 1 ? (j >> 1) * I + chbase + (j & 1) * 16 : chbase + j * 16) + kb * 4;
     };
+    auto with_bias = [&](int j, v4f v) __attribute__((always_inline)) -> v4f {
+        return g.bias ? add_bias4(v, load_bias4(g.bias + (size_t)e * g.N + channel(j))) : v;
+    };
     auto finish = [&](int j, v4f lo, v4f hi) __attribute__((always_inline)) {      // hi: stage 1, the up group
-        if(g.bias)
-        {
-            lo = add_bias4(lo, load_bias4(g.bias + (size_t)e * g.N + channel(j)));
-            if(STAGE == 1)
-                hi = add_bias4(hi, load_bias4(g.bias + (size_t)e * g.N + channel(j + 2)));
-        }
+        lo = with_bias(j, lo);
+        if(STAGE == 1)
+            hi = with_bias(j + 2, hi);
         if(arow < 0)
             return;
         float v[4];
@@ -232,7 +292,7 @@ __global__ void __launch_bounds__(W4A16_THREADS) moe_gemm_pairs_kernel(PairArgs 
         for(int j = 0; j < 4; j++)
             *(v4f*)&red[((wave * 4 + j) * WAVE + lane) * 4] = acc[j];
         __syncthreads();
-        if(STAGE == 1 && wave >= 2)
+        if(STAGE == 1 && wave >= (ACT == BF16 ? 2 : 1))
             return;
         auto sum_of = [&](int j) __attribute__((always_inline)) -> v4f {
             v4f sum = {0.f, 0.f, 0.f, 0.f};
@@ -241,7 +301,42 @@ __global__ void __launch_bounds__(W4A16_THREADS) moe_gemm_pairs_kernel(PairArgs 
                 sum += *(const v4f*)&red[((w * 4 + j) * WAVE + lane) * 4];
             return sum;
         };
-        finish(wave, sum_of(wave), STAGE == 1 ? sum_of(wave + 2) : (v4f){0.f, 0.f, 0.f, 0.f});
+        if constexpr(STAGE == 1 && ACT != BF16)
+        {
+            // the steps of moe_gemm_mxfp4.hip's epilogue (gemm_device.h): round to bf16, eight consecutive channels to a lane, the
+            // block's maximum over the lane rows, e2m1 codes and the scale byte
+            u32 d[2][2];
+#pragma unroll
+            for(int j = 0; j < 2; j++)
+            {
+                const v4f lo = with_bias(j, sum_of(j)), hi = with_bias(j + 2, sum_of(j + 2));
+                float v[4];
+#pragma unroll
+                for(int i = 0; i < 4; i++)
+                    v[i] = g.swiglu ? swiglu_f32(lo[i], hi[i], g.act.limit) : silu_f32(lo[i]) * hi[i];
+                d[j][0] = pack_bf16x2(v[0], v[1]);
+                d[j][1] = pack_bf16x2(v[2], v[3]);
+            }
+            typedef unsigned v2u __attribute__((ext_vector_type(2)));
+            const v2u t0  = __builtin_amdgcn_permlane16_swap(d[0][0], d[1][0], false, false);
+            const v2u t1  = __builtin_amdgcn_permlane16_swap(d[0][1], d[1][1], false, false);
+            const uint4 o = make_uint4(t0.x, t1.x, t0.y, t1.y);
+            u32 am        = amax15_fold(amax15x2(amax15x2(o.x, o.y), amax15x2(o.z, o.w)));
+            const v2u s16 = __builtin_amdgcn_permlane16_swap(am, am, false, false);
+            am            = s16.x > s16.y ? s16.x : s16.y;
+            const v2u s32 = __builtin_amdgcn_permlane32_swap(am, am, false, false);
+            am            = s32.x > s32.y ? s32.x : s32.y;
+            const u32 e8  = mx_scale_byte(am);
+            if(arow >= 0)
+            {
+                const int ch = chbase + (kb & 1) * 16 + (kb >> 1) * 8, blk = chbase / 32;
+                *(u32*)((uint8_t*)g.out + (size_t)orow * (I / 2) + ch / 2) = cvt8(o, e8);
+                if(kb == 0)
+                    g.out_s[(size_t)orow * ((I + 511) / 512 * 16) + (blk & ~15) + (blk & 3) * 4 + ((blk & 15) >> 2)] = (uint8_t)e8;
+            }
+        }
+        else
+            finish(wave, sum_of(wave), STAGE == 1 ? sum_of(wave + 2) : (v4f){0.f, 0.f, 0.f, 0.f});
     }
     else
 #pragma unroll
@@ -309,12 +404,11 @@ __global__ void __launch_bounds__(512) moe_pairs_down_sum_kernel(PairArgs g)
     u32 wsc[NB][NS];
     auto load_next = [&](auto BB) __attribute__((always_inline)) {
         constexpr int b = decltype(BB)::value;
-        if(!to_load)
-            return;
-        const int away = lk * 128 + kb * 32 >= g.k_real ? NOWHERE : 0;
+        // (no condition around the loads, see moe_gemm_pairs_kernel)
+        const int away = !to_load || lk * 128 + kb * 32 >= g.k_real ? NOWHERE : 0;
 #pragma unroll
         for(int h = 0; h < NS; h++)
-            wsc[b][h] = load4(sb[h], lane * 4, (lk >> 1) * 256);
+            wsc[b][h] = load4(sb[h], lane * 4 | away, (lk >> 1) * 256);
 #pragma unroll
         for(int j = 0; j < NR; j++)
             wf[b][j] = load16_nt(wb[j], lane * 16 | away, lk * 1024);
@@ -322,7 +416,7 @@ __global__ void __launch_bounds__(512) moe_pairs_down_sum_kernel(PairArgs g)
         for(int c = 0; c < 4; c++)
             af[b][c] = load16(ab, (a_off + c * 16) | away, lk * 256);
         lk += 4;
-        if(lk >= KT)
+        if(lk >= KT && to_load)
         {
             lk = w;
             to_load &= to_load - 1u;
@@ -333,39 +427,50 @@ __global__ void __launch_bounds__(512) moe_pairs_down_sum_kernel(PairArgs g)
     if(turn && steps > 0)
     {
         take_slot();
-        static_for<NB>([&](auto BB) __attribute__((always_inline)) { load_next(BB); });
+        static_for<NB>([&](auto BB) __attribute__((always_inline)) {
+            load_next(BB);
+            __builtin_amdgcn_sched_barrier(0);
+        });
         u32 mine = turn;
         int kt = w;
-        while(mine)
-            static_for<NB>([&](auto BB) __attribute__((always_inline)) {
-                constexpr int b = decltype(BB)::value;
-                if(!mine)
-                    return;
+        auto step = [&](auto BB) __attribute__((always_inline)) {
+            constexpr int b = decltype(BB)::value;
+#pragma unroll
+            for(int j = 0; j < NR; j++)
+            {
+                v8bf wq[4];
+                expand_fp4(wf[b][j], (wsc[b][j / 2] >> (8 * ((kt & 1) * 2 + half + (j & 1)))) & 0xFFu, wq);
+#pragma unroll
+                for(int c = 0; c < 4; c++)
+                    acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wq[c], __builtin_bit_cast(v8bf, af[b][c]), acc[j], 0, 0, 0);
+            }
+            kt += 4;
+            if(kt >= KT)
+            {
+                kt = w;
+                const int s = __builtin_ctz(mine);
+                mine &= mine - 1u;
 #pragma unroll
                 for(int j = 0; j < NR; j++)
                 {
-                    v8bf wq[4];
-                    expand_fp4(wf[b][j], (wsc[b][j / 2] >> (8 * ((kt & 1) * 2 + half + (j & 1)))) & 0xFFu, wq);
-#pragma unroll
-                    for(int c = 0; c < 4; c++)
-                        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wq[c], __builtin_bit_cast(v8bf, af[b][c]), acc[j], 0, 0, 0);
+                    if(r == 0)
+                        *(v4f*)&red[s][w][j * 16 + kb * 4] = acc[j];
+                    acc[j] = (v4f){0.f, 0.f, 0.f, 0.f};
                 }
+            }
+        };
+        int left = __builtin_popcount(turn) * steps;
+        for(; left > NB; left -= NB)
+            static_for<NB>([&](auto BB) __attribute__((always_inline)) {
+                step(BB);
+                __builtin_amdgcn_sched_barrier(0);
                 load_next(BB);
-                kt += 4;
-                if(kt >= KT)
-                {
-                    kt = w;
-                    const int s = __builtin_ctz(mine);
-                    mine &= mine - 1u;
-#pragma unroll
-                    for(int j = 0; j < NR; j++)
-                    {
-                        if(r == 0)
-                            *(v4f*)&red[s][w][j * 16 + kb * 4] = acc[j];
-                        acc[j] = (v4f){0.f, 0.f, 0.f, 0.f};
-                    }
-                }
+                __builtin_amdgcn_sched_barrier(0);
             });
+        static_for<NB>([&](auto BB) __attribute__((always_inline)) {
+            if(left > decltype(BB)::value)
+                step(BB);
+        });
     }
     else if(turn)
         for(u32 m = turn; m; m &= m - 1u)      // (fewer K-steps than waves)
@@ -416,10 +521,17 @@ static int64_t block_bound(int64_t rows, int64_t n_blk, int experts)
     return experts + rows / 16 < b ? experts + rows / 16 : b;
 }
 
-bool pyhip_pairs_served(int64_t tokens, int topk, int experts, int hidden, int inter, int64_t n_blk, int split_k)
+// bf16 activations: the K split of the sorted entry points, so that the sums are theirs.  MXFP4 ones, whose sums have no order: always
+// four waves to a tile (without a split, DeepSeek-V3 shape, 16 tokens 372.7 / 354.4 us, 60 tokens 767 / 736)
+static int pairs_split(int fp4, int stage, int64_t tiles, int K, int split_k)
+{
+    return fp4 ? 4 : w4a16_split(stage, 16, tiles, K, split_k);
+}
+
+bool pyhip_pairs_served(int64_t tokens, int topk, int experts, int hidden, int inter, int64_t n_blk, int fp4, int split_k)
 {
     const int64_t blocks = block_bound(tokens * topk, n_blk, experts);
-    const int s1 = w4a16_split(1, 16, blocks * (inter / 128), hidden, split_k), s2 = w4a16_split(2, 16, blocks * (hidden / 256), inter, split_k);
+    const int s1 = pairs_split(fp4, 1, blocks * (inter / 128), hidden, split_k), s2 = pairs_split(fp4, 2, blocks * (hidden / 256), inter, split_k);
     // (offsets into the activations are 32-bit and signed)
     return (s1 == 0 || s1 == 4) && (s2 == 0 || s2 == 4 || (s2 == 32 && tokens == 1 && topk == 2 && inter >= 2048 && inter <= 16384)) &&      // (pyhip_w4a16_token_top2)
           
@@ -439,7 +551,26 @@ static int prepare(const char* name, PairArgs& g, int64_t rows, int64_t blocks, 
     g.SC      = (g.K / 32 + 7) / 8 * 8;
     // (the last row need not be a whole pitch long)
     g.a_bytes = (u32)(((rows - 1) * g.a_pitch + (g.k_real + 31) / 32 * 32) * 2);
+    if(g.a_s)
+    {
+        PYHIP_REQUIRE(g.fp4 && ((uintptr_t)g.a_s % 4) == 0, "%s: scales", name);
+        g.a_bytes  = (u32)(rows * (g.K / 2));
+        g.as_bytes = (u32)(rows * ((g.K + 511) / 512 * 16));
+    }
     return PYHIP_OK;
+}
+
+template <int STAGE>
+static void launch_pairs(const PairArgs& g, int split, dim3 grid, hipStream_t stream)
+{
+    if(g.fp4 && g.a_s)
+        hipLaunchKernelGGL((moe_gemm_pairs_kernel<STAGE, 4, QUANTISED>), grid, dim3(W4A16_THREADS), 0, stream, g);
+    else if(STAGE == 1 && g.fp4)
+        hipLaunchKernelGGL((moe_gemm_pairs_kernel<1, 4, TO_FP4>), grid, dim3(W4A16_THREADS), 0, stream, g);
+    else if(split)
+        hipLaunchKernelGGL((moe_gemm_pairs_kernel<STAGE, 4, BF16>), grid, dim3(W4A16_THREADS), 0, stream, g);
+    else
+        hipLaunchKernelGGL((moe_gemm_pairs_kernel<STAGE, 0, BF16>), grid, dim3(W4A16_THREADS), 0, stream, g);
 }
 
 int pyhip_pairs_gate_up(PairArgs g, int64_t rows, int64_t n_blk, int split_k, int activation, float swiglu_limit, hipStream_t stream)
@@ -448,20 +579,19 @@ int pyhip_pairs_gate_up(PairArgs g, int64_t rows, int64_t n_blk, int split_k, in
                   "moe_pairs_gate_up: activation=%d (0 SiLU, 1 SwiGLU with a positive limit)", activation);
     const int64_t blocks = block_bound((int64_t)g.T * g.topk, n_blk, g.experts);
     g.n_tiles            = g.N / 256;
-    const int split      = w4a16_split(1, 16, blocks * g.n_tiles, g.K, split_k);
+    const int split      = pairs_split(g.fp4, 1, blocks * g.n_tiles, g.K, split_k);
     const int rc         = prepare("moe_pairs_gate_up", g, rows, blocks, g.n_tiles);
     if(rc)
         return rc;
     PYHIP_REQUIRE(split == 0 || split == 4, "moe_pairs_gate_up: split_k=%d", split_k);
-    g.act = make_gated_act(activation, swiglu_limit);
+    PYHIP_REQUIRE(!g.fp4 || (g.out_s && g.N % 1024 == 0), "moe_pairs_gate_up: quantised output");
+    g.act    = make_gated_act(activation, swiglu_limit);
+    g.swiglu = activation;
     // (tiles whose channels are all padding are not launched)
     const int tile = split ? 32 : 128;
     g.n_tiles      = (g.N / 2 - (g.all_channels ? 0 : g.n_pad) + tile - 1) / tile;
     const dim3 grid((unsigned)(blocks * g.n_tiles));
-    if(split)
-        hipLaunchKernelGGL((moe_gemm_pairs_kernel<1, 4>), grid, dim3(W4A16_THREADS), 0, stream, g);
-    else
-        hipLaunchKernelGGL((moe_gemm_pairs_kernel<1, 0>), grid, dim3(W4A16_THREADS), 0, stream, g);
+    launch_pairs<1>(g, split, grid, stream);
     PYHIP_CHECK_LAUNCH("moe_gemm_pairs_kernel");
     return PYHIP_OK;
 }
@@ -470,7 +600,7 @@ int pyhip_pairs_down(PairArgs g, int64_t rows, int64_t n_blk, int split_k, hipSt
 {
     const int64_t blocks = block_bound((int64_t)g.T * g.topk, n_blk, g.experts);
     g.n_tiles            = g.N / 256;
-    const int split      = w4a16_split(2, 16, blocks * g.n_tiles, g.K, split_k);
+    const int split      = pairs_split(g.fp4, 2, blocks * g.n_tiles, g.K, split_k);
     const int rc         = prepare("moe_pairs_down", g, rows, blocks, g.n_tiles);
     if(rc)
         return rc;
@@ -478,10 +608,7 @@ int pyhip_pairs_down(PairArgs g, int64_t rows, int64_t n_blk, int split_k, hipSt
     if(split)
         g.n_tiles *= 4;
     const dim3 grid((unsigned)(blocks * g.n_tiles));
-    if(split)
-        hipLaunchKernelGGL((moe_gemm_pairs_kernel<2, 4>), grid, dim3(W4A16_THREADS), 0, stream, g);
-    else
-        hipLaunchKernelGGL((moe_gemm_pairs_kernel<2, 0>), grid, dim3(W4A16_THREADS), 0, stream, g);
+    launch_pairs<2>(g, split, grid, stream);
     PYHIP_CHECK_LAUNCH("moe_gemm_pairs_kernel");
     return PYHIP_OK;
 }
@@ -491,7 +618,7 @@ int pyhip_pairs_down_sum(PairArgs g, int64_t rows, int64_t n_blk, int split_k, h
     const int64_t pairs  = (int64_t)g.T * g.topk;
     const int64_t blocks = block_bound(pairs, n_blk, g.experts);
     // by token the weights of an expert are fetched for each of its pairs: only where pairs rarely share one
-    if(!g.ids || g.topk > 8 || (g.T > 1 && 8 * pairs > g.experts) || w4a16_split(2, 16, blocks * (g.N / 256), g.K, split_k) != 4)
+    if(!g.ids || g.fp4 || g.topk > 8 || (g.T > 1 && 8 * pairs > g.experts) || w4a16_split(2, 16, blocks * (g.N / 256), g.K, split_k) != 4)
         return -1;
     PYHIP_REQUIRE(((uintptr_t)g.out % 16) == 0, "moe_pairs_down_sum: unaligned pointer");
     const int rc = prepare("moe_pairs_down_sum", g, rows, blocks, g.N / 64);
