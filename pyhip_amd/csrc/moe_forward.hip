@@ -204,10 +204,16 @@ static const TileCost tile_costs[] = {{16, 1.2, 1.37, 1e9, 0.35}, {32, 1.5, 1.39
 // even routers and cost 6-18 % under Zipf ones.)
 extern "C" int pyhip_layer_block_m(int64_t tokens, int topk, int experts, int local_experts, int hidden, int inter)
 {
-    const int ladder = pyhip_moe_pick_block_m(tokens, topk, experts, hidden, 0);
+    int ladder = pyhip_moe_pick_block_m(tokens, topk, experts, hidden, 0);
     if(tokens <= 0 || topk <= 0 || experts <= 0 || local_experts <= 0)
         return ladder;
     const double est = (double)tokens * topk / experts;
+    // The ladder's lowest line is that of the persistent kernels.  In those of moe_gemm_pairs.hip, 32 rows cost next to nothing where 16
+    // would do, and hold the busy experts of an uneven router in a block.  Layer, us, 16 / 32 rows: DeepSeek-V3 shape, 80 tokens (2.5 rows per
+    // expert) 771 / 775; 64 experts, top-6, 2048 x 1408, 40 tokens (3.8) 54.7 / 55.4; Qwen3 shape, 45 tokens (2.8) 88.5 / 86.4; under Zipf
+    // routers 256 experts, top-8, 2048 x 512, 100 tokens (3.1) 41.0 / 37.7; 96, top-4, 6272 x 1920, 90 tokens (3.8) 123 / 108.
+    if(ladder == 16 && experts >= 32 && est >= 2.0 && tokens * topk > PAIRS_UNSORTED_MAX)
+        ladder = 32;
     if(local_experts * expected_blocks(est, ladder) * (inter / 128) >= 256.0)
         return ladder;
     auto estimate = [&](const TileCost& c) {
@@ -267,22 +273,28 @@ struct Router
 };
 }   // namespace
 
-// Whether forward_pairs below serves the call.  MXFP4 activations: without a sort, or while experts have at most four rows on average,
-// so that even a busy one has few blocks.  With more rows per expert the persistent kernel, in which workgroups take the tiles of an
-// expert's blocks together, wins.  Layer, us, 16-row blocks, persistent kernel / this, by rows per expert: DeepSeek-V3 shape 0.5: 374.8 /
-// 353.4, 1.9: 758.7 / 727.4, 4: 887.1 / 868.6, 6.3: 911.0 / 908.4, 12.5: 1044 / 1085; Qwen3 shape 0.75: 63.6 / 56.4, 3.75: 119.5 / 106.9,
-// 8: 169.8 / 160.8, 31: 327 / 395; gpt-oss shape 1: 173.1 / 166.2, 3.4: 252.2 / 239.4, 9.4: 283.1 / 288.5; 96 experts, top-4, Zipf router,
-// 6272 x 1920, 1.7: 95.5 / 92.5, 3.8: 132.6 / 128.3, 8.3: 195.5 / 214.5
+// Whether forward_pairs below serves the call.  MXFP4 activations: without a sort, or while experts have few rows on average, so that
+// even a busy one has few blocks: a quarter of a block, or with a handful of experts, whose loads are even in relative terms, half of
+// one.  With more, blocks that fetch the weights of their expert again cost more than the persistent kernels, in which one workgroup's rows
+// share what it fetched (with 64 rows a block this way is the slower one at any load).  Layer, us, persistent kernel / this, by rows
+// per expert; 16-row blocks: DeepSeek-V3 shape 0.5: 374.8 / 355.6, 3.1: 868 / 821; Qwen3 shape 1.9: 88.7 / 77.1, 4: 121 / 107; gpt-oss shape 2:
+// 220 / 214; 96 experts, top-4, Zipf router, 6272 x 1920 1.7: 95.9 / 91.4, 3.8: 133 / 123, 6.3: 166 / 166, 10: 231 / 244.
+// 32-row blocks: DeepSeek-V3 shape 4: 906 / 855, 9.4: 941 / 913, 16: 962 / 985; Qwen3 shape 4: 102.7 / 101.5, 8: 139.0 / 137.2; gpt-oss shape 4: 263 /
+// 244, 9.4: 277 / 269, 16: 284 / 290; 96 experts 3.8: 124 / 108, 6.3: 143 / 141, 10: 189 / 195; 8 experts, 4096 x 14336, 10: 136 / 121, 16, Zipf: 154 /
+// 146, 25: 152 / 145, 40: 167 / 217; 28 experts, top-6, 2048 x 4096, 15: 78.5 / 71.7
 static bool takes_pairs(int64_t tokens, int topk, int experts, int hidden, int inter, int block_m, int w4a16, int split_k)
 {
     const int64_t pairs = tokens * topk;
-    if(!w4a16 && pairs > PAIRS_UNSORTED_MAX && pairs > 4ll * experts)
+    if(block_m != 16 && (block_m != 32 || w4a16))
         return false;
-    return block_m == 16 && hidden % 512 == 0 && inter % 512 == 0 && topk > 0 && experts <= 2048 &&
-           pyhip_pairs_served(tokens, topk, experts, hidden, inter, pyhip_moe_sorting_max_blocks(tokens, topk, experts, 16), !w4a16, split_k);
+    if(!w4a16 && (block_m != 16 || pairs > PAIRS_UNSORTED_MAX) && pairs > (int64_t)experts * (experts < 32 ? block_m / 2 : block_m / 4))
+        return false;
+    return hidden % 512 == 0 && inter % 512 == 0 && topk > 0 && experts <= 2048 &&
+           pyhip_pairs_served(tokens, topk, experts, hidden, inter, pyhip_moe_sorting_max_blocks(tokens, topk, experts, block_m) * (block_m / 16),
+                              !w4a16, split_k);
 }
 
-// The layer in 16-row blocks by the kernels of moe_gemm_pairs.hip.  Up to 64 pairs the kernels find their rows themselves
+// The layer by the kernels of moe_gemm_pairs.hip.  Up to 64 pairs the kernels find their rows themselves
 // and the sort is left out; where pairs rarely share an expert the down GEMM sums the slots and the reduction is left out too: two
 // launches (with the router three) instead of four.  What that saves is the launch on the host (3.3 us each) and the latency chain of the stage
 // on the device (sort 4.5-5.5, reduction 3-5 us).
@@ -290,11 +302,11 @@ static int forward_pairs(const void* hidden_bf16, int64_t row_stride, int hidden
                          const uint8_t* w2, const uint8_t* w2_scale, const void* bias1_bf16, const void* bias2_bf16,
                          const Router& router, int32_t* topk_ids, float* topk_weights, const int32_t* expert_mask,
                          const int32_t* num_local_tokens, void* out, int out_is_f32, int tokens, int topk, int experts,
-                         int hidden, int inter, int hidden_pad, int inter_pad, int w4a16, int split_k, int activation,
-                         float swiglu_limit, const Layout& l, uint8_t* ws, hipStream_t stream)
+                         int hidden, int inter, int hidden_pad, int inter_pad, int block_m, int w4a16, int split_k, int activation,
+                         float swiglu_limit, int held, const Layout& l, uint8_t* ws, hipStream_t stream)
 {
     uint8_t* a2         = ws + (w4a16 ? l.a2 : l.a2_q);      // a row for every pair
-    const bool unsorted = (int64_t)tokens * topk <= PAIRS_UNSORTED_MAX;
+    const bool unsorted = block_m == 16 && (int64_t)tokens * topk <= PAIRS_UNSORTED_MAX;
     uint32_t* s_ids     = (uint32_t*)(ws + l.sorted_ids);
     float* s_w          = (float*)(ws + l.sorted_w);
     uint32_t *s_e = (uint32_t*)(ws + l.sorted_e), *n_valid = (uint32_t*)(ws + l.num_valid), *sched = (uint32_t*)(ws + l.sched);
@@ -312,16 +324,16 @@ static int forward_pairs(const void* hidden_bf16, int64_t row_stride, int hidden
                                                                  router.renormalize, topk_weights, topk_ids, stream)
                                 : pyhip_moe_topk_softmax(router.gating, tokens, experts, topk, router.renormalize, topk_weights, topk_ids, stream);
     else if(router.gating)
-        rc = pyhip_moe_route_sorting(router.gating, tokens, topk, experts, router.n_group, router.topk_group, router.renormalize, 16,
+        rc = pyhip_moe_route_sorting(router.gating, tokens, topk, experts, router.n_group, router.topk_group, router.renormalize, block_m,
                                      expert_mask, num_local_tokens, topk_weights, topk_ids, s_ids, s_w, s_e, n_valid, sched,
                                      ws + l.sort_ws, l.sort_ws_bytes, w4a16 ? nullptr : hidden_bf16, row_stride, tokens, hidden,
                                      w4a16 ? nullptr : ws + l.a1_q, w4a16 ? nullptr : ws + l.a1_s, stream);
     else if(!unsorted && !w4a16)
-        rc = pyhip_sorting_quant_cols(topk_ids, topk_weights, tokens, topk, experts, 16, expert_mask, num_local_tokens, s_ids, s_w, s_e,
+        rc = pyhip_sorting_quant_cols(topk_ids, topk_weights, tokens, topk, experts, block_m, expert_mask, num_local_tokens, s_ids, s_w, s_e,
                                       n_valid, sched, ws + l.sort_ws, l.sort_ws_bytes, hidden_bf16, row_stride, tokens, hidden,
                                       ws + l.a1_q, ws + l.a1_s, hidden_cols, stream);
     else if(!unsorted)
-        rc = pyhip_moe_sorting(topk_ids, topk_weights, tokens, topk, experts, 16, expert_mask, num_local_tokens, s_ids, s_w, s_e,
+        rc = pyhip_moe_sorting(topk_ids, topk_weights, tokens, topk, experts, block_m, expert_mask, num_local_tokens, s_ids, s_w, s_e,
                                n_valid, sched, nullptr, 0, ws + l.sort_ws, l.sort_ws_bytes, stream);
     if(rc)
         return rc;
@@ -334,7 +346,7 @@ static int forward_pairs(const void* hidden_bf16, int64_t row_stride, int hidden
     {
         g.sorted_ids = s_ids; g.sorted_w = s_w; g.sorted_e = s_e; g.num_valid = n_valid;
     }
-    g.T = tokens; g.topk = topk; g.experts = experts;
+    g.T = tokens; g.topk = topk; g.experts = experts; g.rows = block_m; g.held = held;
     PairArgs up = g, down = g;
     up.a = hidden_bf16; up.w = w1; up.w_s = w1_scale; up.bias = (const uint16_t*)bias1_bf16;
     up.out = a2; up.K = hidden; up.N = 2 * inter;
@@ -367,12 +379,11 @@ static int forward_pairs(const void* hidden_bf16, int64_t row_stride, int hidden
         if(rc >= 0)
             return rc;
     }
-    const int64_t a2_rows = w4a16 ? l.rows2 : (int64_t)tokens * topk;
-    rc                    = pyhip_pairs_down_sum(down, a2_rows, l.n_blk, split_k, stream);
+    rc = pyhip_pairs_down_sum(down, l.rows2, l.n_blk, split_k, stream);
     if(rc >= 0)
         return rc;
     down.out = ws + l.out3;
-    rc       = pyhip_pairs_down(down, a2_rows, l.n_blk, split_k, stream);
+    rc       = pyhip_pairs_down(down, l.rows2, l.n_blk, split_k, stream);
     if(rc)
         return rc;
     return pyhip_moe_topk_reduce_routed(ws + l.out3, out, tokens, topk, hidden, out_is_f32, topk_ids, experts, expert_mask,
@@ -387,7 +398,7 @@ static int forward_impl(const void* hidden_bf16, int64_t hidden_row_stride, int 
                         const int32_t* num_local_tokens, void* out, int out_is_f32, int tokens, int topk, int experts,
                         int hidden, int inter, int hidden_pad, int inter_pad, int block_m, int w4a16, int split_k,
                         int activation, float swiglu_limit, void* workspace, int64_t workspace_bytes, hipStream_t stream,
-                        bool bf16_cols = false)
+                        bool bf16_cols = false, int local_experts = 0)
 {
     PYHIP_REQUIRE(hidden_bf16 && w1 && w1_scale && w2 && w2_scale && topk_ids && topk_weights && out,
                   "moe_forward: null pointer");
@@ -417,7 +428,8 @@ static int forward_impl(const void* hidden_bf16, int64_t hidden_row_stride, int 
     if(pairs)
         return forward_pairs(hidden_bf16, hidden_row_stride, hidden_cols, w1, w1_scale, w2, w2_scale, bias1_bf16, bias2_bf16, router,
                              topk_ids, topk_weights, expert_mask, num_local_tokens, out, out_is_f32, tokens, topk, experts, hidden,
-                             inter, hidden_pad, inter_pad, w4a16, split_k, activation, swiglu_limit, l, ws, stream);
+                             inter, hidden_pad, inter_pad, block_m, w4a16, split_k, activation, swiglu_limit,
+                             expert_mask && local_experts > 0 && local_experts < experts ? local_experts : experts, l, ws, stream);
     if(w4a16 && tokens == 1 && !router.gating)
     {
         // a single token with bf16 activations: no sort; the GEMMs read the routing themselves, one block per slot
@@ -547,6 +559,7 @@ struct LayerCall
     int cols, out_f32, tokens, topk, experts, hidden, inter, hidden_pad, inter_pad, block_m, w4a16, split_k, activation;
     int n_group, topk_group, renormalize;
     float swiglu_limit;
+    int local_experts;      // matrices in w1 and w2 (under a mask: the experts that it has), or 0: not told
 };
 static_assert(sizeof(LayerCall) == 200, "packed by pyhip_amd/fused_moe.py");
 
@@ -558,7 +571,7 @@ extern "C" int pyhip_layer_forward(const LayerCall* c, hipStream_t stream)
                         (const uint8_t*)c->w2_scale, c->bias1, c->bias2, r, (int32_t*)c->topk_ids, (float*)c->topk_weights,
                         (const int32_t*)c->expert_mask, (const int32_t*)c->num_local_tokens, c->out, c->out_f32, c->tokens, c->topk,
                         c->experts, c->hidden, c->inter, c->hidden_pad, c->inter_pad, c->block_m, c->w4a16, c->split_k, c->activation,
-                        c->swiglu_limit, c->workspace, c->workspace_bytes, stream, true);
+                        c->swiglu_limit, c->workspace, c->workspace_bytes, stream, true, c->local_experts);
 }
 
 extern "C" int pyhip_layer_takes_cols(int64_t tokens, int topk, int experts, int hidden, int inter, int block_m, int w4a16, int split_k)

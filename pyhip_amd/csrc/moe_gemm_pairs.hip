@@ -1,4 +1,4 @@
-// The layer call's GEMMs in 16-row blocks: few tokens, so the call is a weight stream and a chain of launches.  With bf16
+// The layer call's GEMMs in blocks of 16 rows (MXFP4 activations: or 32): few tokens, so the call is a weight stream and a chain of launches.  With bf16
 // activations the arithmetic (and with it every bit of the result) is that of moe_gemm_w4a16.hip, with MXFP4 ones that of
 // moe_gemm_mxfp4.hip; their entry points serve callers that run the stages one by one.  What is different is what a call of 20-100 us spends beside its weights:
 //   * Up to 64 pairs (token, slot) there is no sort: every wave reads the routing, a pair to a lane, and finds its block's
@@ -8,13 +8,14 @@
 //   * Where nearly every pair has an expert of its own, the down GEMM goes by token instead of by expert: a workgroup holds
 //     all of a token's slots for 16 to 64 output channels, so it sums them and no reduction follows (bf16 activations).
 //   * With MXFP4 activations a workgroup is one tile of 64 weight rows, not a persistent loop over tiles that meets a barrier
-//     for each K-step, and its waves hold three K-steps in flight without LDS between them and the matrix cores.
+//     for each K-step, and its waves hold two or three K-steps in flight without LDS between them and the matrix cores.  What is
+//     left to save is the vector cache's time for the activations: where a block is full, a gather of its rows costs it more than the weights.
 // Bound: the weight stream from about 40 us on, the launches and their latency chains below.  Layer call, us, sort + moe_gemm_w4a16
 // kernels + reduction (padded layers: after a widening of the activations) / this: gpt-oss shape, 2 tokens 39.5 / 28.7, 5 tokens
 // 67.0 / 51.3 (bound at 6.9 TB/s: 38); 32 experts, top-1, 2144 x 3040, 3 tokens 36.7 / 18.4; 1024 x 512, 8 experts, 10 tokens 25.0 / 17.6;
 // Mixtral shape, 5 tokens 100.6 / 94.5, 29 tokens 129.9 / 124.1 (5.75 -> 6.0 TB/s).  MXFP4 activations, sort with quantisation + persistent
-// kernels + reduction / this: gpt-oss shape, 16 tokens 121.5 / 108.8 (bound 97.7); Qwen3 shape, 5 tokens 57.7 / 43.0, 30 tokens 87.9 / 77.6;
-// DeepSeek-V3 shape, 16 tokens 374.8 / 353.4, 100 tokens 863.9 / 834.9 (6.7 -> 6.95 TB/s).
+// kernels + reduction / this: gpt-oss shape, 16 tokens 121.5 / 108.8 (bound 97.7); Qwen3 shape, 5 tokens 57.7 / 43.0, 30 tokens 88.7 / 77.1;
+// DeepSeek-V3 shape, 16 tokens 374.8 / 355.6, 100 tokens 868 / 821 (6.7 -> 7.1 TB/s), 128 tokens, 32-row blocks, 906 / 855.
 #include "w4a16_device.h"
 #include "moe_gemm_pairs.h"
 
@@ -124,14 +125,15 @@ __device__ __forceinline__ v4f mfma_fp4(const v4i& w, int ws, const v4i& a, int 
 // multiples of powers of two, which 32-bit sums hold exactly in whatever order: the bits of moe_gemm_mxfp4.hip.  Its gate_up GEMM
 // quantises its result as that one does: a workgroup's 32 channels are one MX block of a row, which wave 0 finishes.
 enum { BF16, TO_FP4, QUANTISED };
-template <int STAGE, int SPLIT, int ACT>
-__global__ void __launch_bounds__(W4A16_THREADS) moe_gemm_pairs_kernel(PairArgs g)
+template <int STAGE, int SPLIT, int ACT, int MT = 1>
+__global__ void __launch_bounds__(W4A16_THREADS, MT == 1 ? 1 : 3) moe_gemm_pairs_kernel(PairArgs g)
 {
     constexpr bool SPLITK = SPLIT != 0;
     static_assert(SPLITK || ACT == BF16, "MXFP4 activations: the four waves split K");
-    constexpr int NB = 3, KSTRIDE = SPLITK ? 4 : 1;
+    static_assert(MT == 1 || ACT == QUANTISED, "several groups of rows: activations that take few registers");
+    constexpr int NB = MT > 1 ? 2 : 3, KSTRIDE = SPLITK ? 4 : 1;
     constexpr int NA = ACT == QUANTISED ? 1 : 4;                  // 16-byte pieces of a row in a lane's K-step
-    __shared__ float red[SPLITK ? 4 * 4 * WAVE * 4 : 1];          // [wave][row group][lane][4]
+    __shared__ float red[SPLITK ? 4 * 4 * MT * WAVE * 4 : 1];     // [wave][row group][row tile][lane][4]
     const int tid = threadIdx.x, lane = tid % WAVE;
     const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int r = lane & 15, kb = lane >> 4;
@@ -142,37 +144,54 @@ __global__ void __launch_bounds__(W4A16_THREADS) moe_gemm_pairs_kernel(PairArgs 
     if(STAGE == 1 && chbase >= I - g.n_pad && !g.all_channels)      // (channels of padding: the down GEMM does not read them)
         return;
     // the block's expert, and for row r: the activation row, the output row, the routing weight
-    int e, arow = -1, orow = 0;
-    float rw = 0.f;
-    if(g.ids)
+    int e, arow[MT], orow[MT];
+    float rw[MT];
+#pragma unroll
+    for(int m = 0; m < MT; m++)
+    {
+        arow[m] = -1;
+        orow[m] = 0;
+        rw[m]   = 0.f;
+    }
+    if(MT == 1 && g.ids)
     {
         int pair;
         if(!find_block(g, m_blk, lane, e, pair))
             return;
         if(pair >= 0)
         {
-            arow = STAGE == 1 ? (int)((u32)pair / (u32)g.topk) : pair * g.row_step;
-            orow = STAGE == 1 ? pair * g.row_step : pair;
+            arow[0] = STAGE == 1 ? (int)((u32)pair / (u32)g.topk) : pair * g.row_step;
+            orow[0] = STAGE == 1 ? pair * g.row_step : pair;
             if(STAGE == 2)
-                rw = g.weights[pair];
+                rw[0] = g.weights[pair];
         }
     }
     else
     {
         // (all read together: the arrays are there for every block that is launched, whether or not it holds rows)
-        const int p  = m_blk * 16 + r;
-        const u32 id = g.sorted_ids[p], last = g.num_valid[0];
-        e            = __builtin_amdgcn_readfirstlane((int)g.sorted_e[m_blk]);
-        if(STAGE == 2)
-            rw = g.sorted_w[p];
-        if((u32)(m_blk * 16) >= last)
-            return;
-        const int tok = (int)(id & 0xFFFFFFu), slot = (int)(id >> 24);
-        if(slot < g.topk && tok < g.T)
+        const u32 last = g.num_valid[0];
+        e              = __builtin_amdgcn_readfirstlane((int)g.sorted_e[m_blk]);
+        u32 id[MT];
+#pragma unroll
+        for(int m = 0; m < MT; m++)
         {
-            const int pair = tok * g.topk + slot;
-            arow           = STAGE == 1 ? tok : pair;
-            orow           = pair;
+            const int p = (m_blk * MT + m) * 16 + r;
+            id[m]       = g.sorted_ids[p];
+            if(STAGE == 2)
+                rw[m] = g.sorted_w[p];
+        }
+        if((u32)(m_blk * MT * 16) >= last)
+            return;
+#pragma unroll
+        for(int m = 0; m < MT; m++)
+        {
+            const int tok = (int)(id[m] & 0xFFFFFFu), slot = (int)(id[m] >> 24);
+            if(slot < g.topk && tok < g.T)
+            {
+                const int pair = tok * g.topk + slot;
+                arow[m]        = STAGE == 1 ? tok : pair;
+                orow[m]        = pair;
+            }
         }
     }
     // row group j = 0..3 (stage 1: 0, 1 gate rows, 2, 3 the matching up rows); two of them share a scale tile of 32 rows
@@ -192,19 +211,35 @@ __global__ void __launch_bounds__(W4A16_THREADS) moe_gemm_pairs_kernel(PairArgs 
         sb[h] = buffer_of(g.w_s + (size_t)(row_of(2 * h) / 32) * sc_tile, sc_tile);
     const rsrc_t ab = buffer_of(g.a, g.a_bytes), asb = buffer_of(g.a_s, g.as_bytes);
     const int SK     = (g.K + 511) / 512 * 16;      // bytes of a row's scales (moe_quant.hip)
-    const int a_off  = arow < 0 ? NOWHERE : ACT == QUANTISED ? arow * Kb + kb * 16 : arow * g.a_pitch * 2 + kb * 64;
-    const int as_off = arow < 0 ? NOWHERE : arow * SK + kb * 4;
+    // gate_up: quantised tokens are fetched with a row's four groups of 32 in adjacent lanes, and change places on their way to the
+    // matrix cores: 64 bytes to four lanes are one access of the vector cache, 16 bytes of four rows are four.  The down GEMM's
+    // operand lies as its lanes read it: [16-row tile][K-step][lane][16 bytes], and scales [tile][4 K-steps][lane][a byte for each].
+    // Qwen3 shape, 128 tokens in 16-row blocks, rows fetched as they lie / the first / both: 160.9 / 156.8 / 151.8 us; DeepSeek-V3 shape,
+    // 200 tokens: 909.5 / 903.6 / 879.3.
+    constexpr bool SWAP = ACT == QUANTISED && STAGE == 1, TILES = ACT == QUANTISED && STAGE == 2;
+    const int lk = SWAP ? lane & 3 : kb, from = (r * 4 + kb) * 4;
+    int a_off[MT], as_off[MT];
+#pragma unroll
+    for(int m = 0; m < MT; m++)
+    {
+        const int row = SWAP ? __builtin_amdgcn_ds_bpermute((lane >> 2) * 4, arow[m]) : arow[m], tile = m_blk * MT + m;
+        a_off[m]      = row < 0 ? NOWHERE : TILES ? tile * 16 * Kb + lane * 16 : SWAP ? row * Kb + lk * 16 : row * g.a_pitch * 2 + kb * 64;
+        as_off[m]     = row < 0 ? NOWHERE : TILES ? tile * 16 * SK + lane * 4 : row * SK + lk * 4;
+    }
 
-    v4f acc[4];
+    v4f acc[4][MT];
 #pragma unroll
     for(int j = 0; j < 4; j++)
-        acc[j] = (v4f){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for(int m = 0; m < MT; m++)
+            acc[j][m] = (v4f){0.f, 0.f, 0.f, 0.f};
     const int KT = (g.k_real + 127) / 128;
-    v4i wf[NB][4], af[NB][NA];
-    u32 wsc[NB][2], asc[NB];
+    v4i wf[NB][4], af[NB][MT][NA];
+    u32 wsc[NB][2], asc[NB][MT];
     auto load_step = [&](auto BB, int kt) __attribute__((always_inline)) {
         constexpr int b = decltype(BB)::value;
         const int away  = kt * 128 + kb * 32 >= g.k_real ? NOWHERE : 0;
+        const int aaway = kt * 128 + lk * 32 >= g.k_real ? NOWHERE : 0;
 #pragma unroll
         for(int h = 0; h < 2; h++)
             wsc[b][h] = load4(sb[h], lane * 4 | away, (kt >> 1) * 256);
@@ -212,35 +247,51 @@ __global__ void __launch_bounds__(W4A16_THREADS) moe_gemm_pairs_kernel(PairArgs 
         for(int j = 0; j < 4; j++)
             wf[b][j] = load16_nt(wb[j], lane * 16 | away, kt * 1024);
 #pragma unroll
-        for(int i = 0; i < NA; i++)
-            af[b][i] = load16(ab, (a_off + i * 16) | away, kt * (64 * NA));
-        if constexpr(ACT == QUANTISED)
-            asc[b] = load4(asb, as_off | away, (kt >> 2) * 16);
+        for(int m = 0; m < MT; m++)
+        {
+#pragma unroll
+            for(int i = 0; i < NA; i++)
+                af[b][m][i] = load16(ab, (a_off[m] + i * 16) | aaway, kt * (TILES ? 1024 : 64 * NA));
+            if constexpr(ACT == QUANTISED)
+                asc[b][m] = load4(asb, as_off[m] | aaway, (kt >> 2) * (TILES ? 256 : 16));
+        }
     };
     auto step = [&](auto BB, int kt) __attribute__((always_inline)) {
         constexpr int b = decltype(BB)::value;
-        v4i aq;
-        int as;
-        if constexpr(ACT == TO_FP4)
-            quantise32(af[b], aq, as);
-        else if constexpr(ACT == QUANTISED)
-        {
-            aq = af[b][0];
-            as = (int)(asc[b] >> (8 * (kt & 3)));
-        }
 #pragma unroll
-        for(int j = 0; j < 4; j++)
+        for(int m = 0; m < MT; m++)
         {
-            const u32 ws = wsc[b][j >> 1] >> (8 * ((kt & 1) * 2 + (j & 1)));
-            if constexpr(ACT != BF16)
-                acc[j] = mfma_fp4(wf[b][j], (int)ws, aq, as, acc[j]);
-            else
+            v4i aq;
+            int as;
+            if constexpr(ACT == TO_FP4)
+                quantise32(af[b][m], aq, as);
+            else if constexpr(ACT == QUANTISED)
             {
-                v8bf wq[4];
-                expand_fp4(wf[b][j], ws & 0xFFu, wq);
+                aq = af[b][m][0];
+                as = (int)asc[b][m];
+                if constexpr(SWAP)
+                {
 #pragma unroll
-                for(int i = 0; i < 4; i++)
-                    acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wq[i], __builtin_bit_cast(v8bf, af[b][i]), acc[j], 0, 0, 0);
+                    for(int i = 0; i < 4; i++)
+                        aq[i] = __builtin_amdgcn_ds_bpermute(from, aq[i]);
+                    as = __builtin_amdgcn_ds_bpermute(from, as);
+                }
+                as >>= 8 * (kt & 3);
+            }
+#pragma unroll
+            for(int j = 0; j < 4; j++)
+            {
+                const u32 ws = wsc[b][j >> 1] >> (8 * ((kt & 1) * 2 + (j & 1)));
+                if constexpr(ACT != BF16)
+                    acc[j][m] = mfma_fp4(wf[b][j], (int)ws, aq, as, acc[j][m]);
+                else
+                {
+                    v8bf wq[4];
+                    expand_fp4(wf[b][j], ws & 0xFFu, wq);
+#pragma unroll
+                    for(int i = 0; i < 4; i++)
+                        acc[j][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wq[i], __builtin_bit_cast(v8bf, af[b][m][i]), acc[j][m], 0, 0, 0);
+                }
             }
         }
     };
@@ -266,39 +317,41 @@ __global__ void __launch_bounds__(W4A16_THREADS) moe_gemm_pairs_kernel(PairArgs 
     });
 
     // ---- epilogue: lane (r, kb) holds channels kb*4 .. + 3 of row group j for row r.  Under the K split wave w finishes row
-    // group w (stage 1: gate group w and its up group, waves 0 and 1; where the result is quantised wave 0 finishes both)
+    // group w (stage 1: gate group w and its up group, waves 0 and 1; where the result is quantised wave m finishes row tile m)
     auto channel = [&](int j) __attribute__((always_inline)) -> int {
         return (STAGE == 1 ? (j >> 1) * I + chbase + (j & 1) * 16 : chbase + j * 16) + kb * 4;
     };
     auto with_bias = [&](int j, v4f v) __attribute__((always_inline)) -> v4f {
         return g.bias ? add_bias4(v, load_bias4(g.bias + (size_t)e * g.N + channel(j))) : v;
     };
-    auto finish = [&](int j, v4f lo, v4f hi) __attribute__((always_inline)) {      // hi: stage 1, the up group
+    auto finish = [&](int j, int m, v4f lo, v4f hi) __attribute__((always_inline)) {      // hi: stage 1, the up group
         lo = with_bias(j, lo);
         if(STAGE == 1)
             hi = with_bias(j + 2, hi);
-        if(arow < 0)
+        if(arow[m] < 0)
             return;
         float v[4];
 #pragma unroll
         for(int i = 0; i < 4; i++)
-            v[i] = STAGE == 1 ? gated_act_f32(g.act, lo[i], hi[i]) : lo[i] * rw;
-        *(uint2*)((uint16_t*)g.out + (size_t)orow * (STAGE == 1 ? I : g.N) + channel(j)) =
+            v[i] = STAGE == 1 ? gated_act_f32(g.act, lo[i], hi[i]) : lo[i] * rw[m];
+        *(uint2*)((uint16_t*)g.out + (size_t)orow[m] * (STAGE == 1 ? I : g.N) + channel(j)) =
             make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
     };
     if constexpr(SPLITK)
     {
 #pragma unroll
         for(int j = 0; j < 4; j++)
-            *(v4f*)&red[((wave * 4 + j) * WAVE + lane) * 4] = acc[j];
+#pragma unroll
+            for(int m = 0; m < MT; m++)
+                *(v4f*)&red[(((wave * 4 + j) * MT + m) * WAVE + lane) * 4] = acc[j][m];
         __syncthreads();
-        if(STAGE == 1 && wave >= (ACT == BF16 ? 2 : 1))
+        if(STAGE == 1 && wave >= (ACT == BF16 ? 2 : MT))
             return;
-        auto sum_of = [&](int j) __attribute__((always_inline)) -> v4f {
+        auto sum_of = [&](int j, int m) __attribute__((always_inline)) -> v4f {
             v4f sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for(int w = 0; w < 4; w++)
-                sum += *(const v4f*)&red[((w * 4 + j) * WAVE + lane) * 4];
+                sum += *(const v4f*)&red[(((w * 4 + j) * MT + m) * WAVE + lane) * 4];
             return sum;
         };
         if constexpr(STAGE == 1 && ACT != BF16)
@@ -309,7 +362,7 @@ __global__ void __launch_bounds__(W4A16_THREADS) moe_gemm_pairs_kernel(PairArgs 
 #pragma unroll
             for(int j = 0; j < 2; j++)
             {
-                const v4f lo = with_bias(j, sum_of(j)), hi = with_bias(j + 2, sum_of(j + 2));
+                const v4f lo = with_bias(j, sum_of(j, wave)), hi = with_bias(j + 2, sum_of(j + 2, wave));
                 float v[4];
 #pragma unroll
                 for(int i = 0; i < 4; i++)
@@ -327,21 +380,28 @@ __global__ void __launch_bounds__(W4A16_THREADS) moe_gemm_pairs_kernel(PairArgs 
             const v2u s32 = __builtin_amdgcn_permlane32_swap(am, am, false, false);
             am            = s32.x > s32.y ? s32.x : s32.y;
             const u32 e8  = mx_scale_byte(am);
-            if(arow >= 0)
+            bool here = arow[0] >= 0;
+#pragma unroll
+            for(int m = 1; m < MT; m++)
+                here = wave == m ? arow[m] >= 0 : here;
+            if(here)
             {
-                const int ch = chbase + (kb & 1) * 16 + (kb >> 1) * 8, blk = chbase / 32;
-                *(u32*)((uint8_t*)g.out + (size_t)orow * (I / 2) + ch / 2) = cvt8(o, e8);
+                const int blk = chbase / 32, kt = blk / 4;
+                const size_t at = (size_t)(m_blk * MT + wave) * (I / 128) + kt, lane2 = (blk & 3) * 16 + r;
+                *(u32*)((uint8_t*)g.out + (at * WAVE + lane2) * 16 + (kb & 1) * 8 + (kb >> 1) * 4) = cvt8(o, e8);
                 if(kb == 0)
-                    g.out_s[(size_t)orow * ((I + 511) / 512 * 16) + (blk & ~15) + (blk & 3) * 4 + ((blk & 15) >> 2)] = (uint8_t)e8;
+                    g.out_s[((at / 4) * WAVE + lane2) * 4 + (kt & 3)] = (uint8_t)e8;
             }
         }
         else
-            finish(wave, sum_of(wave), STAGE == 1 ? sum_of(wave + 2) : (v4f){0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+            for(int m = 0; m < MT; m++)
+                finish(wave, m, sum_of(wave, m), STAGE == 1 ? sum_of(wave + 2, m) : (v4f){0.f, 0.f, 0.f, 0.f});
     }
     else
 #pragma unroll
         for(int j = 0; j < (STAGE == 1 ? 2 : 4); j++)
-            finish(j, acc[j], acc[STAGE == 1 ? j + 2 : j]);
+            finish(j, 0, acc[j][0], acc[STAGE == 1 ? j + 2 : j][0]);
 }
 
 // The down GEMM by token, with the sum over the token's slots.  A workgroup owns NR groups of 16 output channels of one token: groups
@@ -528,6 +588,14 @@ static int pairs_split(int fp4, int stage, int64_t tiles, int K, int split_k)
     return fp4 ? 4 : w4a16_split(stage, 16, tiles, K, split_k);
 }
 
+// the row blocks to launch: those of the experts that are here
+static int64_t launched_blocks(const PairArgs& g, int64_t n_blk)
+{
+    const int64_t pairs = (int64_t)g.T * g.topk, b = g.held + pairs / g.rows;
+    const int64_t most  = pairs < n_blk ? pairs : n_blk;
+    return b < most ? b : most;
+}
+
 bool pyhip_pairs_served(int64_t tokens, int topk, int experts, int hidden, int inter, int64_t n_blk, int fp4, int split_k)
 {
     const int64_t blocks = block_bound(tokens * topk, n_blk, experts);
@@ -542,6 +610,7 @@ static int prepare(const char* name, PairArgs& g, int64_t rows, int64_t blocks, 
 {
     PYHIP_REQUIRE(g.a && g.w && g.w_s && g.out && (g.ids || (g.sorted_ids && g.sorted_e && g.num_valid)), "%s: null pointer", name);
     PYHIP_REQUIRE(g.K > 0 && g.K % 512 == 0 && g.N > 0 && g.N % 256 == 0, "%s: K=%d must be a multiple of 512, N=%d of 256", name, g.K, g.N);
+    PYHIP_REQUIRE(g.held > 0 && g.held <= g.experts && (g.rows == 16 || (g.rows == 32 && g.fp4 && !g.ids && g.a_s)), "%s: bad blocks", name);
     PYHIP_REQUIRE(g.T > 0 && g.topk > 0 && g.experts > 0 && (!g.ids || (int64_t)g.T * g.topk <= PAIRS_UNSORTED_MAX), "%s: bad sizes", name);
     PYHIP_REQUIRE(g.k_real > 0 && g.k_real <= g.K && g.a_pitch >= (g.k_real + 31) / 32 * 32 && g.a_pitch % 8 == 0,
                   "%s: %d of %d columns, rows of %d", name, g.k_real, g.K, g.a_pitch);
@@ -563,7 +632,9 @@ static int prepare(const char* name, PairArgs& g, int64_t rows, int64_t blocks, 
 template <int STAGE>
 static void launch_pairs(const PairArgs& g, int split, dim3 grid, hipStream_t stream)
 {
-    if(g.fp4 && g.a_s)
+    if(g.rows == 32)
+        hipLaunchKernelGGL((moe_gemm_pairs_kernel<STAGE, 4, QUANTISED, 2>), grid, dim3(W4A16_THREADS), 0, stream, g);
+    else if(g.fp4 && g.a_s)
         hipLaunchKernelGGL((moe_gemm_pairs_kernel<STAGE, 4, QUANTISED>), grid, dim3(W4A16_THREADS), 0, stream, g);
     else if(STAGE == 1 && g.fp4)
         hipLaunchKernelGGL((moe_gemm_pairs_kernel<1, 4, TO_FP4>), grid, dim3(W4A16_THREADS), 0, stream, g);
@@ -590,7 +661,7 @@ int pyhip_pairs_gate_up(PairArgs g, int64_t rows, int64_t n_blk, int split_k, in
     // (tiles whose channels are all padding are not launched)
     const int tile = split ? 32 : 128;
     g.n_tiles      = (g.N / 2 - (g.all_channels ? 0 : g.n_pad) + tile - 1) / tile;
-    const dim3 grid((unsigned)(blocks * g.n_tiles));
+    const dim3 grid((unsigned)(launched_blocks(g, n_blk) * g.n_tiles));
     launch_pairs<1>(g, split, grid, stream);
     PYHIP_CHECK_LAUNCH("moe_gemm_pairs_kernel");
     return PYHIP_OK;
@@ -607,7 +678,7 @@ int pyhip_pairs_down(PairArgs g, int64_t rows, int64_t n_blk, int split_k, hipSt
     PYHIP_REQUIRE(split == 0 || split == 4, "moe_pairs_down: split_k=%d", split_k);
     if(split)
         g.n_tiles *= 4;
-    const dim3 grid((unsigned)(blocks * g.n_tiles));
+    const dim3 grid((unsigned)(launched_blocks(g, n_blk) * g.n_tiles));
     launch_pairs<2>(g, split, grid, stream);
     PYHIP_CHECK_LAUNCH("moe_gemm_pairs_kernel");
     return PYHIP_OK;

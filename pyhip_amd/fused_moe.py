@@ -141,7 +141,7 @@ _remembered_plan = functools.lru_cache(maxsize=512)(_ask_plan)
 
 
 #: struct LayerCall of csrc/moe_forward.hip: pointers, row stride and workspace bytes, sizes and options, the SwiGLU limit
-_LAYER_CALL = struct.Struct("<14Q2q16if")
+_LAYER_CALL = struct.Struct("<14Q2q16ifi")
 
 
 @functools.lru_cache(maxsize=512)
@@ -332,7 +332,7 @@ def fused_moe(
             _LAYER_CALL.pack(at, w1u.data_ptr(), w1s.data_ptr(), w2u.data_ptr(), w2s.data_ptr(), p(bias1), p(bias2), 0,
                              topk_ids.data_ptr(), topk_weight.data_ptr(), p(expert_mask), p(num_local_tokens), out.data_ptr(),
                              ws.data_ptr(), rows, ws_bytes, cols, out_dtype == torch.float32, T, k, global_E, H, I,
-                             hidden_pad, intermediate_pad, bm, w4a16, splitk, act, 0, 0, 0, limit), _lib.stream_handle())
+                             hidden_pad, intermediate_pad, bm, w4a16, splitk, act, 0, 0, 0, limit, E), _lib.stream_handle())
         if rc:
             _lib.check(rc, "moe_forward")
         return out.narrow(1, 0, H - hidden_pad) if narrow else out
@@ -507,7 +507,7 @@ def fused_moe_routed(hidden_states, w1, w2, gating_output, topk, renormalize=Tru
                          g.data_ptr(), ti.data_ptr(), tw.data_ptr(), p(expert_mask), p(num_local_tokens), out.data_ptr(),
                          ws.data_ptr(), x.stride(0), ws_bytes, 0, out_dtype == torch.float32, T, topk, global_E, H, I,
                          int(hidden_pad), int(intermediate_pad), bm, w4a16, splitk, act, int(num_expert_group), int(topk_group),
-                         bool(renormalize), limit), _lib.stream_handle())
+                         bool(renormalize), limit, E), _lib.stream_handle())
     if rc:
         _lib.check(rc, "moe_forward_routed")
     return (out, tw, ti) if return_routing else out

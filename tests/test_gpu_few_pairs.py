@@ -1,4 +1,4 @@
-"""The layer call in 16-row blocks with bf16 activations, or with MXFP4 ones up to 64 pairs or four rows per expert (kernels of its own, without a sort up to 64
+"""The layer call in 16-row blocks with bf16 activations, or with MXFP4 ones and few rows per expert (kernels of its own, without a sort up to 64
 pairs and without a reduction where pairs rarely share an expert), against the step-by-step path.  With bf16 activations the arithmetic
 and its order are the same; with MXFP4 ones the sums are exact in any order: the same bits."""
 import pytest
@@ -9,11 +9,11 @@ import cases
 pytestmark = pytest.mark.gpu
 
 
-def _poison(T, k, E, H, I, method):
+def _poison(T, k, E, H, I, method, rows=16):
     """the memory that the next call of these (padded) sizes gets as its workspace holds NaNs, in bf16 and in fp32"""
     import sys
     plan = sys.modules["pyhip_amd.fused_moe"]._plan
-    x = torch.empty(plan(T, k, E, H, I, method, 16)[2], dtype=torch.uint8, device="cuda")
+    x = torch.empty(plan(T, k, E, H, I, method, rows)[2], dtype=torch.uint8, device="cuda")
     x.fill_(255)
 
 
@@ -41,6 +41,24 @@ def _poison(T, k, E, H, I, method):
 ])
 @pytest.mark.parametrize("method", ["w4a16", "a4w4"])
 def test_few_pairs_equal_the_stages(T, k, E, H, I, splitk, method):
+    _equal_the_stages(T, k, E, H, I, splitk, method, 16)
+
+
+@pytest.mark.parametrize("T,k,E,H,I", [
+    (1, 1, 8, 512, 512),             # one row
+    (64, 2, 8, 1024, 1536),          # sixteen rows per expert: the most in fewer experts
+    (65, 2, 8, 512, 512),            # more
+    (40, 8, 40, 1536, 1024),
+    (100, 6, 75, 512, 512),          # eight rows per expert: the most in 32 experts and more
+    (90, 8, 192, 2560, 512),         # an uneven share of K-steps
+    (128, 1, 8, 512, 512),           # one K-step for each wave
+])
+def test_two_row_tiles_equal_the_stages(T, k, E, H, I):
+    _equal_the_stages(T, k, E, H, I, 0, "a4w4", 32)
+
+
+def _equal_the_stages(T, k, E, H, I, splitk, method, rows):
+    """plain routing, holes in it, no bias, an expert mask, a local token count; SiLU to bf16 and SwiGLU to fp32"""
     from pyhip_amd import fused_moe
     from pyhip_amd.enums import ActivationType
     L = cases.make_layer("", T, seed=T * 7 + k, bias=True, E=E, k=min(k, E), H=H, I=I, router="softmax")
@@ -68,25 +86,25 @@ def test_few_pairs_equal_the_stages(T, k, E, H, I, splitk, method):
                                 ("mask", ma, mb, ids, rank), ("local", w1, w2, ids, dict(whole, num_local_tokens=local))):
         for more in (dict(), dict(dtype=torch.float32, activation=ActivationType.Swiglu)):
             print(f"few pairs T={T} k={L.k} E={E} H={H} I={I} {name} {sorted(more)}", flush=True)
-            kw2 = dict(kw, method=method, block_size_M=16, splitk=splitk, **more)
+            kw2 = dict(kw, method=method, block_size_M=rows, splitk=splitk, **more)
             want = fused_moe(hidden, wa, wb, tw, t.cuda(), return_parts=True, **kw2)[0]
             for _ in range(2):
-                _poison(T, L.k, E, H, I, method)
+                _poison(T, L.k, E, H, I, method, rows)
                 got = fused_moe(hidden, wa, wb, tw, t.cuda(), **kw2)
                 assert torch.equal(got, want)
 
 
 @pytest.mark.parametrize("T,H,I", [(1, 544, 544), (1, 544, 8224), (3, 1440, 1440), (1, 992, 32 * 47), (20, 1440, 1056), (30, 576, 1440), (50, 1440, 1056)])
 @pytest.mark.parametrize("wide", [False, True])
-@pytest.mark.parametrize("method", ["w4a16", "a4w4"])
-def test_few_pairs_leave_padding_alone(T, H, I, wide, method):
+@pytest.mark.parametrize("method,rows", [("w4a16", 16), ("a4w4", 16), ("a4w4", 32)])
+def test_few_pairs_leave_padding_alone(T, H, I, wide, method, rows):
     """Padded layers, activations at the true or the padded width.  The weights' padding is told, so it is not read: its rows and
     columns are filled with ones here, and what the padded columns of the activations hold does not matter either."""
     from pyhip_amd import fused_moe
     L = cases.make_layer("", T, seed=H, bias=True, E=32, k=2, H=H, I=I, router="softmax")
     w1, w1s, w2, w2s, b1, b2, hp, ip = cases.padded_device_weights(L)
     tw, ti = torch.from_numpy(L.topk_w).cuda(), torch.from_numpy(L.topk_ids).cuda()
-    kw = dict(bias1=b1, bias2=b2, method=method, block_size_M=16)
+    kw = dict(bias1=b1, bias2=b2, method=method, block_size_M=rows)
     x = torch.nn.functional.pad(L.hidden.cuda(), (0, hp))
     want = fused_moe(x, w1, w2, tw, ti, w1_scale=w1s, w2_scale=w2s, return_parts=True, **kw)[0]
     # ones (code 2) in the padding rows of w2, in whole row groups of 16, and in the padding columns of both, in whole 1 KB blocks' groups of 32
@@ -103,20 +121,20 @@ def test_few_pairs_leave_padding_alone(T, H, I, wide, method):
         x = x[:, :H]
         x = torch.nn.functional.pad(x, (0, 8), value=float("nan"))[:, :H]
     print("few pairs, padded", T, H, I, wide, flush=True)
-    _poison(T, 2, 32, H + hp, I + ip, method)
+    _poison(T, 2, 32, H + hp, I + ip, method, rows)
     got = fused_moe(x, f1, f2, tw, ti, w1_scale=w1s, w2_scale=w2s, hidden_pad=hp, intermediate_pad=ip, **kw)
     assert torch.equal(got[:, :H], want[:, :H]) and (not wide or (got[:, H:] == 0).all())
 
 
 @pytest.mark.parametrize("T", [1, 4, 8, 9, 40])
 @pytest.mark.parametrize("grouped", [False, True])
-@pytest.mark.parametrize("method", ["w4a16", "a4w4"])
-def test_few_pairs_with_the_router(T, grouped, method):
+@pytest.mark.parametrize("method,rows", [("w4a16", 16), ("a4w4", 16), ("a4w4", 32)])
+def test_few_pairs_with_the_router(T, grouped, method, rows):
     from pyhip_amd import fused_moe, fused_moe_routed
     L = cases.make_layer("", T, seed=T, E=256, k=8, H=512, I=512, router="softmax")
     w1, w1s, w2, w2s = cases.device_weights(L)
     logits = torch.randn(T, 256, generator=torch.Generator().manual_seed(T)).cuda()
-    kw = dict(w1_scale=w1s, w2_scale=w2s, method=method, block_size_M=16)
+    kw = dict(w1_scale=w1s, w2_scale=w2s, method=method, block_size_M=rows)
     print("few pairs, routed", T, grouped, flush=True)
     out, tw, ti = fused_moe_routed(L.hidden.cuda(), w1, w2, logits, 8, return_routing=True,
                                    **(dict(num_expert_group=8, topk_group=4) if grouped else {}), **kw)

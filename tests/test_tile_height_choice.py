@@ -14,6 +14,9 @@ from pyhip_amd import _lib
     (4096, 2, 8, 8, 4096, 14336, 128), (4096, 4, 128, 128, 3072, 3072, 160), (2048, 8, 128, 128, 4096, 1536, 160),
     (4001, 8, 256, 32, 7168, 2048, 160), (8192, 8, 256, 256, 7168, 2048, 288), (128, 8, 256, 256, 7168, 2048, 32),
     (16, 4, 128, 128, 3072, 3072, 16), (64, 2, 8, 8, 1024, 512, 32),
+    # two rows per expert and more, in 32 experts and more: 32 rows (the ladder: 16)
+    (80, 8, 256, 256, 7168, 2048, 32), (63, 8, 256, 256, 7168, 2048, 16), (17, 4, 32, 32, 4096, 4096, 32), (16, 4, 32, 32, 4096, 4096, 16),
+    (20, 4, 31, 31, 4096, 4096, 16),
 ])
 def test_known_choices(tokens, topk, experts, local, hidden, inter, want):
     assert _lib.load().pyhip_layer_block_m(tokens, topk, experts, local, hidden, inter) == want
