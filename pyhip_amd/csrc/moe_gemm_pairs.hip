@@ -125,15 +125,16 @@ __device__ __forceinline__ v4f mfma_fp4(const v4i& w, int ws, const v4i& a, int 
 // multiples of powers of two, which 32-bit sums hold exactly in whatever order: the bits of moe_gemm_mxfp4.hip.  Its gate_up GEMM
 // quantises its result as that one does: a workgroup's 32 channels are one MX block of a row, which wave 0 finishes.
 enum { BF16, TO_FP4, QUANTISED };
-template <int STAGE, int SPLIT, int ACT, int MT = 1>
+template <int STAGE, int SPLIT, int ACT, int MT = 1, bool STAGED = false>
 __global__ void __launch_bounds__(W4A16_THREADS, MT == 1 ? 1 : 3) moe_gemm_pairs_kernel(PairArgs g)
 {
     constexpr bool SPLITK = SPLIT != 0;
     static_assert(SPLITK || ACT == BF16, "MXFP4 activations: the four waves split K");
+    static_assert(!STAGED || (ACT == BF16 && MT == 1), "staged: bf16 rows");
     static_assert(MT == 1 || ACT == QUANTISED, "several groups of rows: activations that take few registers");
     constexpr int NB = MT > 1 ? 2 : 3, KSTRIDE = SPLITK ? 4 : 1;
     constexpr int NA = ACT == QUANTISED ? 1 : 4;                  // 16-byte pieces of a row in a lane's K-step
-    __shared__ float red[SPLITK ? 4 * 4 * MT * WAVE * 4 : 1];     // [wave][row group][row tile][lane][4]
+    __shared__ __attribute__((aligned(16))) float red[SPLITK || STAGED ? 4 * 4 * MT * WAVE * 4 : 1];     // [wave][row group][row tile][lane][4]
     const int tid = threadIdx.x, lane = tid % WAVE;
     const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int r = lane & 15, kb = lane >> 4;
@@ -227,6 +228,18 @@ __global__ void __launch_bounds__(W4A16_THREADS, MT == 1 ? 1 : 3) moe_gemm_pairs
         as_off[m]     = row < 0 ? NOWHERE : TILES ? tile * 16 * SK + lane * 4 : row * SK + lk * 4;
     }
 
+    // Staged bf16 rows: a load fetches 256 bytes of each of four rows, 16 lanes to a row; a K-step's four loads are written to the wave's own
+    // 4 KB of LDS and read back as the matrix cores want them, piece p of row r at r * 16 + (p ^ r) (no two of eight lanes in a bank).
+    // As the rows lie, a load is 64 accesses of the vector cache, four times what the weights of a K-step cost it.
+    int st_off[4];
+    v4i* const mine = (v4i*)red + wave * 256;
+    if constexpr(STAGED)
+#pragma unroll
+        for(int i = 0; i < 4; i++)
+        {
+            const int row = __builtin_amdgcn_ds_bpermute((i * 4 + kb) * 4, arow[0]);
+            st_off[i]     = row < 0 ? NOWHERE : row * g.a_pitch * 2 + r * 16;
+        }
     v4f acc[4][MT];
 #pragma unroll
     for(int j = 0; j < 4; j++)
@@ -239,7 +252,7 @@ __global__ void __launch_bounds__(W4A16_THREADS, MT == 1 ? 1 : 3) moe_gemm_pairs
     auto load_step = [&](auto BB, int kt) __attribute__((always_inline)) {
         constexpr int b = decltype(BB)::value;
         const int away  = kt * 128 + kb * 32 >= g.k_real ? NOWHERE : 0;
-        const int aaway = kt * 128 + lk * 32 >= g.k_real ? NOWHERE : 0;
+        const int aaway = kt * 128 + (STAGED ? r >> 2 : lk) * 32 >= g.k_real ? NOWHERE : 0;
 #pragma unroll
         for(int h = 0; h < 2; h++)
             wsc[b][h] = load4(sb[h], lane * 4 | away, (kt >> 1) * 256);
@@ -251,13 +264,24 @@ __global__ void __launch_bounds__(W4A16_THREADS, MT == 1 ? 1 : 3) moe_gemm_pairs
         {
 #pragma unroll
             for(int i = 0; i < NA; i++)
-                af[b][m][i] = load16(ab, (a_off[m] + i * 16) | aaway, kt * (TILES ? 1024 : 64 * NA));
+                af[b][m][i] = STAGED ? load16(ab, st_off[i] | aaway, kt * 256) : load16(ab, (a_off[m] + i * 16) | aaway, kt * (TILES ? 1024 : 64 * NA));
             if constexpr(ACT == QUANTISED)
                 asc[b][m] = load4(asb, as_off[m] | aaway, (kt >> 2) * (TILES ? 256 : 16));
         }
     };
     auto step = [&](auto BB, int kt) __attribute__((always_inline)) {
         constexpr int b = decltype(BB)::value;
+        if constexpr(STAGED)
+        {
+#pragma unroll
+            for(int i = 0; i < 4; i++)
+                mine[(i * 4 + kb) * 16 + (r ^ (i * 4 + kb))] = af[b][0][i];
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for(int i = 0; i < 4; i++)
+                af[b][0][i] = mine[r * 16 + ((kb * 4 + i) ^ r)];
+            __builtin_amdgcn_wave_barrier();
+        }
 #pragma unroll
         for(int m = 0; m < MT; m++)
         {
@@ -632,16 +656,25 @@ static int prepare(const char* name, PairArgs& g, int64_t rows, int64_t blocks, 
 template <int STAGE>
 static void launch_pairs(const PairArgs& g, int split, dim3 grid, hipStream_t stream)
 {
+    // bf16 rows go through LDS where a block has several.  Layer, us, not / staged, by rows per expert: Mixtral shape 1.3: 93.5 / 95.3,
+    // 5: 120.2 / 119.8, 7.3: 125.5 / 121.9; 16 experts, 4096 x 4096 5: 78.3 / 79.5; 32 experts, 2880 x 2880 5: 78.1 / 79.1; 28, 2048 x 4096
+    // 6.4: 79.1 / 76.8; 60, 2048 x 1408 3.3: 57.4 / 58.2, 6.7: 63.5 / 61.8, with a Zipf router 51.1 / 48.0
+    const bool staged = (int64_t)g.T * g.topk >= 6ll * g.experts;
+    const dim3 block(W4A16_THREADS);
     if(g.rows == 32)
-        hipLaunchKernelGGL((moe_gemm_pairs_kernel<STAGE, 4, QUANTISED, 2>), grid, dim3(W4A16_THREADS), 0, stream, g);
+        hipLaunchKernelGGL((moe_gemm_pairs_kernel<STAGE, 4, QUANTISED, 2>), grid, block, 0, stream, g);
     else if(g.fp4 && g.a_s)
-        hipLaunchKernelGGL((moe_gemm_pairs_kernel<STAGE, 4, QUANTISED>), grid, dim3(W4A16_THREADS), 0, stream, g);
+        hipLaunchKernelGGL((moe_gemm_pairs_kernel<STAGE, 4, QUANTISED>), grid, block, 0, stream, g);
     else if(STAGE == 1 && g.fp4)
-        hipLaunchKernelGGL((moe_gemm_pairs_kernel<1, 4, TO_FP4>), grid, dim3(W4A16_THREADS), 0, stream, g);
+        hipLaunchKernelGGL((moe_gemm_pairs_kernel<1, 4, TO_FP4>), grid, block, 0, stream, g);
+    else if(split && staged)
+        hipLaunchKernelGGL((moe_gemm_pairs_kernel<STAGE, 4, BF16, 1, true>), grid, block, 0, stream, g);
     else if(split)
-        hipLaunchKernelGGL((moe_gemm_pairs_kernel<STAGE, 4, BF16>), grid, dim3(W4A16_THREADS), 0, stream, g);
+        hipLaunchKernelGGL((moe_gemm_pairs_kernel<STAGE, 4, BF16>), grid, block, 0, stream, g);
+    else if(staged)
+        hipLaunchKernelGGL((moe_gemm_pairs_kernel<STAGE, 0, BF16, 1, true>), grid, block, 0, stream, g);
     else
-        hipLaunchKernelGGL((moe_gemm_pairs_kernel<STAGE, 0, BF16>), grid, dim3(W4A16_THREADS), 0, stream, g);
+        hipLaunchKernelGGL((moe_gemm_pairs_kernel<STAGE, 0, BF16>), grid, block, 0, stream, g);
 }
 
 int pyhip_pairs_gate_up(PairArgs g, int64_t rows, int64_t n_blk, int split_k, int activation, float swiglu_limit, hipStream_t stream)
