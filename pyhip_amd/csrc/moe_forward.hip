@@ -208,12 +208,17 @@ extern "C" int pyhip_layer_block_m(int64_t tokens, int topk, int experts, int lo
     if(tokens <= 0 || topk <= 0 || experts <= 0 || local_experts <= 0)
         return ladder;
     const double est = (double)tokens * topk / experts;
-    // The ladder's lowest line is that of the persistent kernels.  In those of moe_gemm_pairs.hip, 32 rows cost next to nothing where 16
-    // would do, and hold the busy experts of an uneven router in a block.  Layer, us, 16 / 32 rows: DeepSeek-V3 shape, 80 tokens (2.5 rows per
-    // expert) 771 / 775; 64 experts, top-6, 2048 x 1408, 40 tokens (3.8) 54.7 / 55.4; Qwen3 shape, 45 tokens (2.8) 88.5 / 86.4; under Zipf
-    // routers 256 experts, top-8, 2048 x 512, 100 tokens (3.1) 41.0 / 37.7; 96, top-4, 6272 x 1920, 90 tokens (3.8) 123 / 108.
+    // The ladder's lower lines are those of the persistent kernels.  In those of moe_gemm_pairs.hip, which compute the row tiles that have
+    // rows, a higher block costs next to nothing and holds the busy experts of an uneven router.  Layer, us, 16 / 32 rows: DeepSeek-V3 shape, 80
+    // tokens (2.5 rows per expert) 771 / 775; 64 experts, top-6, 2048 x 1408, 40 tokens (3.8) 54.7 / 55.4; Qwen3 shape, 45 tokens (2.8) 88.5 / 86.4;
+    // under Zipf routers 256 experts, top-8, 2048 x 512, 100 tokens (3.1) 41.0 / 37.7; 96, top-4, 6272 x 1920, 90 tokens (3.8) 123 / 108.
+    // 32 / 64 rows (three waves per SIMD instead of four, which a short K loop feels): DeepSeek-V3 shape 6.3: 881 / 887, 9.4: 913 / 917; gpt-oss shape
+    // 6.3: 257 / 257, 11.6: 272 / 277; Qwen3 shape 6.3: 120 / 118, 11: 155 / 147; 96 experts, Zipf, 5: 121 / 114, 7.5: 152 / 143, 11.7: 211 / 189; hidden
+    // 2048: 256 experts, top-1 9.8: 338 / 355; 128, top-8, 11: 70.7 / 74.2; 60, top-4, 10: 56.4 / 58.7
     if(ladder == 16 && experts >= 32 && est >= 2.0 && tokens * topk > PAIRS_UNSORTED_MAX)
         ladder = 32;
+    else if(ladder == 32 && experts >= 32 && est >= 5.0 && hidden >= 3072 && inter % 512 == 0)
+        ladder = 64;
     if(local_experts * expected_blocks(est, ladder) * (inter / 128) >= 256.0)
         return ladder;
     auto estimate = [&](const TileCost& c) {
@@ -274,20 +279,24 @@ struct Router
 }   // namespace
 
 // Whether forward_pairs below serves the call.  MXFP4 activations: without a sort, or while experts have few rows on average, so that
-// even a busy one has few blocks: a quarter of a block, or with a handful of experts, whose loads are even in relative terms, half of
-// one.  With more, blocks that fetch the weights of their expert again cost more than the persistent kernels, in which one workgroup's rows
-// share what it fetched (with 64 rows a block this way is the slower one at any load).  Layer, us, persistent kernel / this, by rows
-// per expert; 16-row blocks: DeepSeek-V3 shape 0.5: 374.8 / 355.6, 3.1: 868 / 821; Qwen3 shape 1.9: 88.7 / 77.1, 4: 121 / 107; gpt-oss shape 2:
-// 220 / 214; 96 experts, top-4, Zipf router, 6272 x 1920 1.7: 95.9 / 91.4, 3.8: 133 / 123, 6.3: 166 / 166, 10: 231 / 244.
-// 32-row blocks: DeepSeek-V3 shape 4: 906 / 855, 9.4: 941 / 913, 16: 962 / 985; Qwen3 shape 4: 102.7 / 101.5, 8: 139.0 / 137.2; gpt-oss shape 4: 263 /
-// 244, 9.4: 277 / 269, 16: 284 / 290; 96 experts 3.8: 124 / 108, 6.3: 143 / 141, 10: 189 / 195; 8 experts, 4096 x 14336, 10: 136 / 121, 16, Zipf: 154 /
-// 146, 25: 152 / 145, 40: 167 / 217; 28 experts, top-6, 2048 x 4096, 15: 78.5 / 71.7
+// a busy one has few blocks, and few blocks are full.  With more, blocks that fetch the weights of their expert again, and activations that
+// every 64 weight rows fetch again, cost more than the persistent kernels, whose workgroups have 256.  With a handful of experts loads are
+// even in relative terms and the lines lie higher.  Layer, us, persistent kernel / this, by rows per expert:
+//   16 rows: DeepSeek-V3 shape 0.5: 374.8 / 355.6, 3.1: 868 / 821; Qwen3 shape 1.9: 88.7 / 77.1, 4: 121 / 107; gpt-oss shape 2: 220 / 214; 96
+//     experts, top-4, Zipf router, 6272 x 1920 1.7: 95.9 / 91.4, 3.8: 133 / 123, 6.3: 166 / 166, 10: 231 / 243
+//   32 rows: DeepSeek-V3 shape 4: 906 / 852, 6.3: 928 / 881, 11.6: 949 / 935, 16: 964 / 984; Qwen3 shape 4: 103.7 / 99.8, 11: 158 / 155; gpt-oss shape
+//     6.3: 273 / 257, 11.6: 280 / 272, 16: 284 / 288; 64 experts, top-6, 2048 x 1408 9.4: 62.2 / 58.4; 96 experts 7.5: 150 / 152, 11.7: 212 / 211;
+//     8 experts, 4096 x 14336, 10: 136 / 121, 16, Zipf: 154 / 146, 25: 152 / 147, 40: 166 / 218; 28 experts, top-6, 2048 x 4096, 15: 78.5 / 71.7
+//   64 rows (against the persistent kernel of the better height): Qwen3 shape 6.3: 128 / 118, 11: 158 / 147; gpt-oss shape 9.4: 277 / 268, 11.6: 280 /
+//     277, 31: 323 / 357; DeepSeek-V3 shape 11.6: 949 / 939, 16: 964 / 981; 96 experts 5: 128 / 114, 11.7: 212 / 189; 8 experts 17.5: 140 / 123, 25: 142 /
+//     129, 40: 147 / 149; 16, top-2, 4096 x 4096 25: 84.3 / 83.0, 31: 85.0 / 88.4; 12, 5120 x 2048 22: 46.8 / 47.4, 28: 47.6 / 51.2
 static bool takes_pairs(int64_t tokens, int topk, int experts, int hidden, int inter, int block_m, int w4a16, int split_k)
 {
     const int64_t pairs = tokens * topk;
-    if(block_m != 16 && (block_m != 32 || w4a16))
+    if(block_m != 16 && ((block_m != 32 && block_m != 64) || w4a16))
         return false;
-    if(!w4a16 && (block_m != 16 || pairs > PAIRS_UNSORTED_MAX) && pairs > (int64_t)experts * (experts < 32 ? block_m / 2 : block_m / 4))
+    const int rows_per_expert = experts < 32 ? (block_m == 16 ? 8 : block_m == 32 ? 16 : 24) : (block_m == 16 ? 4 : 12);
+    if(!w4a16 && (block_m != 16 || pairs > PAIRS_UNSORTED_MAX) && pairs > (int64_t)experts * rows_per_expert)
         return false;
     return hidden % 512 == 0 && inter % 512 == 0 && topk > 0 && experts <= 2048 &&
            pyhip_pairs_served(tokens, topk, experts, hidden, inter, pyhip_moe_sorting_max_blocks(tokens, topk, experts, block_m) * (block_m / 16),

@@ -22,7 +22,7 @@ struct PairArgs
     const u32* num_valid  = nullptr;
     void* out = nullptr;              // gate_up: a2 bf16 [.., N/2], or (fp4) e2m1 pairs, in tiles; down: out3 bf16 [T, topk, N]; down that sums: [T, N]
     uint8_t* out_s = nullptr;         // gate_up, fp4: the scales of a2
-    int rows = 16;                    // of a block; 32: sorted, activations quantised
+    int rows = 16;                    // of a block; 32, 64: sorted, activations quantised
     int T = 0, topk = 0, experts = 0, K = 0, N = 0;
     int held = 0;                     // experts that are here (mask: how many it has)
     int a_pitch = 0, row_step = 1;

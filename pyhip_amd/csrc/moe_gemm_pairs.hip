@@ -1,4 +1,4 @@
-// The layer call's GEMMs in blocks of 16 rows (MXFP4 activations: or 32): few tokens, so the call is a weight stream and a chain of launches.  With bf16
+// The layer call's GEMMs in blocks of 16 rows (MXFP4 activations: or 32 or 64): few tokens, so the call is a weight stream and a chain of launches.  With bf16
 // activations the arithmetic (and with it every bit of the result) is that of moe_gemm_w4a16.hip, with MXFP4 ones that of
 // moe_gemm_mxfp4.hip; their entry points serve callers that run the stages one by one.  What is different is what a call of 20-100 us spends beside its weights:
 //   * Up to 64 pairs (token, slot) there is no sort: every wave reads the routing, a pair to a lane, and finds its block's
@@ -15,7 +15,8 @@
 // 67.0 / 51.3 (bound at 6.9 TB/s: 38); 32 experts, top-1, 2144 x 3040, 3 tokens 36.7 / 18.4; 1024 x 512, 8 experts, 10 tokens 25.0 / 17.6;
 // Mixtral shape, 5 tokens 100.6 / 94.5, 29 tokens 129.9 / 124.1 (5.75 -> 6.0 TB/s).  MXFP4 activations, sort with quantisation + persistent
 // kernels + reduction / this: gpt-oss shape, 16 tokens 121.5 / 108.8 (bound 97.7); Qwen3 shape, 5 tokens 57.7 / 43.0, 30 tokens 88.7 / 77.1;
-// DeepSeek-V3 shape, 16 tokens 374.8 / 355.6, 100 tokens 868 / 821 (6.7 -> 7.1 TB/s), 128 tokens, 32-row blocks, 906 / 855.
+// DeepSeek-V3 shape, 16 tokens 374.8 / 355.6, 100 tokens 868 / 821 (6.7 -> 7.1 TB/s), 128 tokens, 32-row blocks, 906 / 852; Qwen3
+// shape, 180 tokens, 64-row blocks, 158 / 147.
 #include "w4a16_device.h"
 #include "moe_gemm_pairs.h"
 
@@ -125,76 +126,22 @@ __device__ __forceinline__ v4f mfma_fp4(const v4i& w, int ws, const v4i& a, int 
 // multiples of powers of two, which 32-bit sums hold exactly in whatever order: the bits of moe_gemm_mxfp4.hip.  Its gate_up GEMM
 // quantises its result as that one does: a workgroup's 32 channels are one MX block of a row, which wave 0 finishes.
 enum { BF16, TO_FP4, QUANTISED };
-template <int STAGE, int SPLIT, int ACT, int MT = 1, bool STAGED = false>
-__global__ void __launch_bounds__(W4A16_THREADS, MT == 1 ? 1 : 3) moe_gemm_pairs_kernel(PairArgs g)
+template <int STAGE, int SPLIT, int ACT, bool STAGED, int BT, int MT>
+__device__ __forceinline__ void pairs_tile(const PairArgs& g, float* red, int lane, int wave, int m_blk, int nt, int e,
+                                           const int* arow, const int* orow, const float* rw)
 {
     constexpr bool SPLITK = SPLIT != 0;
     static_assert(SPLITK || ACT == BF16, "MXFP4 activations: the four waves split K");
     static_assert(!STAGED || (ACT == BF16 && MT == 1), "staged: bf16 rows");
-    static_assert(MT == 1 || ACT == QUANTISED, "several groups of rows: activations that take few registers");
-    constexpr int NB = MT > 1 ? 2 : 3, KSTRIDE = SPLITK ? 4 : 1;
+    static_assert(BT == 1 || ACT == QUANTISED, "several row tiles: activations that take few registers");
+    constexpr int NB = BT == 1 || MT == 1 ? 3 : 2, KSTRIDE = SPLITK ? 4 : 1;
     constexpr int NA = ACT == QUANTISED ? 1 : 4;                  // 16-byte pieces of a row in a lane's K-step
-    __shared__ __attribute__((aligned(16))) float red[SPLITK || STAGED ? 4 * 4 * MT * WAVE * 4 : 1];     // [wave][row group][row tile][lane][4]
-    const int tid = threadIdx.x, lane = tid % WAVE;
-    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int r = lane & 15, kb = lane >> 4;
-    const int m_blk = blockIdx.x / g.n_tiles, nt = blockIdx.x - m_blk * g.n_tiles;
     const int Kb = g.K / 2, I = g.N / 2;
     // first output channel of this wave's rows (stage 1: within the gate half; the up half is I further)
     const int chbase = STAGE == 1 ? (SPLITK ? nt * 32 : nt * 128 + wave * 32) : (SPLITK ? nt * 64 : nt * 256 + wave * 64);
     if(STAGE == 1 && chbase >= I - g.n_pad && !g.all_channels)      // (channels of padding: the down GEMM does not read them)
         return;
-    // the block's expert, and for row r: the activation row, the output row, the routing weight
-    int e, arow[MT], orow[MT];
-    float rw[MT];
-#pragma unroll
-    for(int m = 0; m < MT; m++)
-    {
-        arow[m] = -1;
-        orow[m] = 0;
-        rw[m]   = 0.f;
-    }
-    if(MT == 1 && g.ids)
-    {
-        int pair;
-        if(!find_block(g, m_blk, lane, e, pair))
-            return;
-        if(pair >= 0)
-        {
-            arow[0] = STAGE == 1 ? (int)((u32)pair / (u32)g.topk) : pair * g.row_step;
-            orow[0] = STAGE == 1 ? pair * g.row_step : pair;
-            if(STAGE == 2)
-                rw[0] = g.weights[pair];
-        }
-    }
-    else
-    {
-        // (all read together: the arrays are there for every block that is launched, whether or not it holds rows)
-        const u32 last = g.num_valid[0];
-        e              = __builtin_amdgcn_readfirstlane((int)g.sorted_e[m_blk]);
-        u32 id[MT];
-#pragma unroll
-        for(int m = 0; m < MT; m++)
-        {
-            const int p = (m_blk * MT + m) * 16 + r;
-            id[m]       = g.sorted_ids[p];
-            if(STAGE == 2)
-                rw[m] = g.sorted_w[p];
-        }
-        if((u32)(m_blk * MT * 16) >= last)
-            return;
-#pragma unroll
-        for(int m = 0; m < MT; m++)
-        {
-            const int tok = (int)(id[m] & 0xFFFFFFu), slot = (int)(id[m] >> 24);
-            if(slot < g.topk && tok < g.T)
-            {
-                const int pair = tok * g.topk + slot;
-                arow[m]        = STAGE == 1 ? tok : pair;
-                orow[m]        = pair;
-            }
-        }
-    }
     // row group j = 0..3 (stage 1: 0, 1 gate rows, 2, 3 the matching up rows); two of them share a scale tile of 32 rows
     const u32 sc_tile = (u32)(g.SC / 8) * 256u;
     rsrc_t wb[4], sb[2];
@@ -223,7 +170,7 @@ __global__ void __launch_bounds__(W4A16_THREADS, MT == 1 ? 1 : 3) moe_gemm_pairs
 #pragma unroll
     for(int m = 0; m < MT; m++)
     {
-        const int row = SWAP ? __builtin_amdgcn_ds_bpermute((lane >> 2) * 4, arow[m]) : arow[m], tile = m_blk * MT + m;
+        const int row = SWAP ? __builtin_amdgcn_ds_bpermute((lane >> 2) * 4, arow[m]) : arow[m], tile = m_blk * BT + m;
         a_off[m]      = row < 0 ? NOWHERE : TILES ? tile * 16 * Kb + lane * 16 : SWAP ? row * Kb + lk * 16 : row * g.a_pitch * 2 + kb * 64;
         as_off[m]     = row < 0 ? NOWHERE : TILES ? tile * 16 * SK + lane * 4 : row * SK + lk * 4;
     }
@@ -361,71 +308,165 @@ __global__ void __launch_bounds__(W4A16_THREADS, MT == 1 ? 1 : 3) moe_gemm_pairs
         *(uint2*)((uint16_t*)g.out + (size_t)orow[m] * (STAGE == 1 ? I : g.N) + channel(j)) =
             make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
     };
+    // the steps of moe_gemm_mxfp4.hip's epilogue (gemm_device.h): round to bf16, eight consecutive channels to a lane, the block's maximum
+    // over the lane rows, e2m1 codes and the scale byte.  x: the sums of row tile m, a row group each
+    auto quantise_row = [&](const v4f (&x)[4], int m, bool here) __attribute__((always_inline)) {
+        u32 d[2][2];
+#pragma unroll
+        for(int j = 0; j < 2; j++)
+        {
+            const v4f lo = with_bias(j, x[j]), hi = with_bias(j + 2, x[j + 2]);
+            float v[4];
+#pragma unroll
+            for(int i = 0; i < 4; i++)
+                v[i] = g.swiglu ? swiglu_f32(lo[i], hi[i], g.act.limit) : silu_f32(lo[i]) * hi[i];
+            d[j][0] = pack_bf16x2(v[0], v[1]);
+            d[j][1] = pack_bf16x2(v[2], v[3]);
+        }
+        typedef unsigned v2u __attribute__((ext_vector_type(2)));
+        const v2u t0  = __builtin_amdgcn_permlane16_swap(d[0][0], d[1][0], false, false);
+        const v2u t1  = __builtin_amdgcn_permlane16_swap(d[0][1], d[1][1], false, false);
+        const uint4 o = make_uint4(t0.x, t1.x, t0.y, t1.y);
+        u32 am        = amax15_fold(amax15x2(amax15x2(o.x, o.y), amax15x2(o.z, o.w)));
+        const v2u s16 = __builtin_amdgcn_permlane16_swap(am, am, false, false);
+        am            = s16.x > s16.y ? s16.x : s16.y;
+        const v2u s32 = __builtin_amdgcn_permlane32_swap(am, am, false, false);
+        am            = s32.x > s32.y ? s32.x : s32.y;
+        const u32 e8  = mx_scale_byte(am);
+        if(here)
+        {
+            const int blk = chbase / 32, kt = blk / 4;
+            const size_t at = (size_t)(m_blk * BT + m) * (I / 128) + kt, lane2 = (blk & 3) * 16 + r;
+            *(u32*)((uint8_t*)g.out + (at * WAVE + lane2) * 16 + (kb & 1) * 8 + (kb >> 1) * 4) = cvt8(o, e8);
+            if(kb == 0)
+                g.out_s[((at / 4) * WAVE + lane2) * 4 + (kt & 3)] = (uint8_t)e8;
+        }
+    };
     if constexpr(SPLITK)
     {
+        // (two row tiles at a time, in 32 KB)
+        constexpr int MR = MT < 2 ? MT : 2;
 #pragma unroll
-        for(int j = 0; j < 4; j++)
-#pragma unroll
-            for(int m = 0; m < MT; m++)
-                *(v4f*)&red[(((wave * 4 + j) * MT + m) * WAVE + lane) * 4] = acc[j][m];
-        __syncthreads();
-        if(STAGE == 1 && wave >= (ACT == BF16 ? 2 : MT))
-            return;
-        auto sum_of = [&](int j, int m) __attribute__((always_inline)) -> v4f {
-            v4f sum = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for(int w = 0; w < 4; w++)
-                sum += *(const v4f*)&red[(((w * 4 + j) * MT + m) * WAVE + lane) * 4];
-            return sum;
-        };
-        if constexpr(STAGE == 1 && ACT != BF16)
+        for(int m0 = 0; m0 < MT; m0 += MR)
         {
-            // the steps of moe_gemm_mxfp4.hip's epilogue (gemm_device.h): round to bf16, eight consecutive channels to a lane, the
-            // block's maximum over the lane rows, e2m1 codes and the scale byte
-            u32 d[2][2];
+            if(m0)
+                __syncthreads();
 #pragma unroll
-            for(int j = 0; j < 2; j++)
+            for(int j = 0; j < 4; j++)
+#pragma unroll
+                for(int m = 0; m < MR; m++)
+                    if(m0 + m < MT)
+                        *(v4f*)&red[(((wave * 4 + j) * MR + m) * WAVE + lane) * 4] = acc[j][m0 + m];
+            __syncthreads();
+            auto sum_of = [&](int j, int m) __attribute__((always_inline)) -> v4f {
+                v4f sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for(int w = 0; w < 4; w++)
+                    sum += *(const v4f*)&red[(((w * 4 + j) * MR + m) * WAVE + lane) * 4];
+                return sum;
+            };
+            if constexpr(STAGE == 1 && ACT != BF16)
             {
-                const v4f lo = with_bias(j, sum_of(j, wave)), hi = with_bias(j + 2, sum_of(j + 2, wave));
-                float v[4];
-#pragma unroll
-                for(int i = 0; i < 4; i++)
-                    v[i] = g.swiglu ? swiglu_f32(lo[i], hi[i], g.act.limit) : silu_f32(lo[i]) * hi[i];
-                d[j][0] = pack_bf16x2(v[0], v[1]);
-                d[j][1] = pack_bf16x2(v[2], v[3]);
+                if(wave < MR && m0 + wave < MT)
+                {
+                    const v4f x[4] = {sum_of(0, wave), sum_of(1, wave), sum_of(2, wave), sum_of(3, wave)};
+                    bool here      = arow[m0] >= 0;
+                    if(MR == 2 && m0 + 1 < MT && wave == 1)
+                        here = arow[m0 + 1] >= 0;
+                    quantise_row(x, m0 + wave, here);
+                }
             }
-            typedef unsigned v2u __attribute__((ext_vector_type(2)));
-            const v2u t0  = __builtin_amdgcn_permlane16_swap(d[0][0], d[1][0], false, false);
-            const v2u t1  = __builtin_amdgcn_permlane16_swap(d[0][1], d[1][1], false, false);
-            const uint4 o = make_uint4(t0.x, t1.x, t0.y, t1.y);
-            u32 am        = amax15_fold(amax15x2(amax15x2(o.x, o.y), amax15x2(o.z, o.w)));
-            const v2u s16 = __builtin_amdgcn_permlane16_swap(am, am, false, false);
-            am            = s16.x > s16.y ? s16.x : s16.y;
-            const v2u s32 = __builtin_amdgcn_permlane32_swap(am, am, false, false);
-            am            = s32.x > s32.y ? s32.x : s32.y;
-            const u32 e8  = mx_scale_byte(am);
-            bool here = arow[0] >= 0;
+            else if(STAGE == 2 || wave < 2)
 #pragma unroll
-            for(int m = 1; m < MT; m++)
-                here = wave == m ? arow[m] >= 0 : here;
-            if(here)
-            {
-                const int blk = chbase / 32, kt = blk / 4;
-                const size_t at = (size_t)(m_blk * MT + wave) * (I / 128) + kt, lane2 = (blk & 3) * 16 + r;
-                *(u32*)((uint8_t*)g.out + (at * WAVE + lane2) * 16 + (kb & 1) * 8 + (kb >> 1) * 4) = cvt8(o, e8);
-                if(kb == 0)
-                    g.out_s[((at / 4) * WAVE + lane2) * 4 + (kt & 3)] = (uint8_t)e8;
-            }
+                for(int m = 0; m < MR; m++)
+                    if(m0 + m < MT)
+                        finish(wave, m0 + m, sum_of(wave, m), STAGE == 1 ? sum_of(wave + 2, m) : (v4f){0.f, 0.f, 0.f, 0.f});
         }
-        else
-#pragma unroll
-            for(int m = 0; m < MT; m++)
-                finish(wave, m, sum_of(wave, m), STAGE == 1 ? sum_of(wave + 2, m) : (v4f){0.f, 0.f, 0.f, 0.f});
     }
     else
 #pragma unroll
         for(int j = 0; j < (STAGE == 1 ? 2 : 4); j++)
             finish(j, 0, acc[j][0], acc[STAGE == 1 ? j + 2 : j][0]);
+}
+
+// BT: 16-row tiles of a block.  The real rows of a block come first; what a block computes are the row tiles that have any.
+template <int STAGE, int SPLIT, int ACT, int BT = 1, bool STAGED = false>
+__global__ void __launch_bounds__(W4A16_THREADS, BT == 1 ? 1 : 3) moe_gemm_pairs_kernel(PairArgs g)
+{
+    // [wave][row group][row tile][lane][4]; staged rows: [wave][row][16 pieces of 16 bytes]
+    __shared__ __attribute__((aligned(16))) float red[SPLIT || STAGED ? 4 * 4 * (BT < 2 ? 1 : 2) * WAVE * 4 : 1];
+    const int tid = threadIdx.x, lane = tid % WAVE;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    const int r = lane & 15;
+    const int m_blk = blockIdx.x / g.n_tiles, nt = blockIdx.x - m_blk * g.n_tiles;
+    // the block's expert, and for row r: the activation row, the output row, the routing weight
+    int e, arow[BT], orow[BT];
+    float rw[BT];
+#pragma unroll
+    for(int m = 0; m < BT; m++)
+    {
+        arow[m] = -1;
+        orow[m] = 0;
+        rw[m]   = 0.f;
+    }
+    if(BT == 1 && g.ids)
+    {
+        int pair;
+        if(!find_block(g, m_blk, lane, e, pair))
+            return;
+        if(pair >= 0)
+        {
+            arow[0] = STAGE == 1 ? (int)((u32)pair / (u32)g.topk) : pair * g.row_step;
+            orow[0] = STAGE == 1 ? pair * g.row_step : pair;
+            if(STAGE == 2)
+                rw[0] = g.weights[pair];
+        }
+    }
+    else
+    {
+        // (all read together: the arrays are there for every block that is launched, whether or not it holds rows)
+        const u32 last = g.num_valid[0];
+        e              = __builtin_amdgcn_readfirstlane((int)g.sorted_e[m_blk]);
+        u32 id[BT];
+#pragma unroll
+        for(int m = 0; m < BT; m++)
+        {
+            const int p = (m_blk * BT + m) * 16 + r;
+            id[m]       = g.sorted_ids[p];
+            if(STAGE == 2)
+                rw[m] = g.sorted_w[p];
+        }
+        if((u32)(m_blk * BT * 16) >= last)
+            return;
+#pragma unroll
+        for(int m = 0; m < BT; m++)
+        {
+            const int tok = (int)(id[m] & 0xFFFFFFu), slot = (int)(id[m] >> 24);
+            if(slot < g.topk && tok < g.T)
+            {
+                const int pair = tok * g.topk + slot;
+                arow[m]        = STAGE == 1 ? tok : pair;
+                orow[m]        = pair;
+            }
+        }
+    }
+    if constexpr(BT == 1)
+        pairs_tile<STAGE, SPLIT, ACT, STAGED, 1, 1>(g, red, lane, wave, m_blk, nt, e, arow, orow, rw);
+    else
+    {
+        int tiles = 1;
+#pragma unroll
+        for(int m = 1; m < BT; m++)
+            tiles = __ballot(arow[m] >= 0) ? m + 1 : tiles;
+        if(tiles == 1)
+            pairs_tile<STAGE, SPLIT, ACT, STAGED, BT, 1>(g, red, lane, wave, m_blk, nt, e, arow, orow, rw);
+        else if(BT == 2 || tiles == 2)
+            pairs_tile<STAGE, SPLIT, ACT, STAGED, BT, 2>(g, red, lane, wave, m_blk, nt, e, arow, orow, rw);
+        else if(BT == 4 && tiles == 3)
+            pairs_tile<STAGE, SPLIT, ACT, STAGED, BT, BT == 4 ? 3 : 2>(g, red, lane, wave, m_blk, nt, e, arow, orow, rw);
+        else
+            pairs_tile<STAGE, SPLIT, ACT, STAGED, BT, BT>(g, red, lane, wave, m_blk, nt, e, arow, orow, rw);
+    }
 }
 
 // The down GEMM by token, with the sum over the token's slots.  A workgroup owns NR groups of 16 output channels of one token: groups
@@ -634,7 +675,7 @@ static int prepare(const char* name, PairArgs& g, int64_t rows, int64_t blocks, 
 {
     PYHIP_REQUIRE(g.a && g.w && g.w_s && g.out && (g.ids || (g.sorted_ids && g.sorted_e && g.num_valid)), "%s: null pointer", name);
     PYHIP_REQUIRE(g.K > 0 && g.K % 512 == 0 && g.N > 0 && g.N % 256 == 0, "%s: K=%d must be a multiple of 512, N=%d of 256", name, g.K, g.N);
-    PYHIP_REQUIRE(g.held > 0 && g.held <= g.experts && (g.rows == 16 || (g.rows == 32 && g.fp4 && !g.ids && g.a_s)), "%s: bad blocks", name);
+    PYHIP_REQUIRE(g.held > 0 && g.held <= g.experts && (g.rows == 16 || ((g.rows == 32 || g.rows == 64) && g.fp4 && !g.ids && g.a_s)), "%s: bad blocks", name);
     PYHIP_REQUIRE(g.T > 0 && g.topk > 0 && g.experts > 0 && (!g.ids || (int64_t)g.T * g.topk <= PAIRS_UNSORTED_MAX), "%s: bad sizes", name);
     PYHIP_REQUIRE(g.k_real > 0 && g.k_real <= g.K && g.a_pitch >= (g.k_real + 31) / 32 * 32 && g.a_pitch % 8 == 0,
                   "%s: %d of %d columns, rows of %d", name, g.k_real, g.K, g.a_pitch);
@@ -661,7 +702,9 @@ static void launch_pairs(const PairArgs& g, int split, dim3 grid, hipStream_t st
     // 6.4: 79.1 / 76.8; 60, 2048 x 1408 3.3: 57.4 / 58.2, 6.7: 63.5 / 61.8, with a Zipf router 51.1 / 48.0
     const bool staged = (int64_t)g.T * g.topk >= 6ll * g.experts;
     const dim3 block(W4A16_THREADS);
-    if(g.rows == 32)
+    if(g.rows == 64)
+        hipLaunchKernelGGL((moe_gemm_pairs_kernel<STAGE, 4, QUANTISED, 4>), grid, block, 0, stream, g);
+    else if(g.rows == 32)
         hipLaunchKernelGGL((moe_gemm_pairs_kernel<STAGE, 4, QUANTISED, 2>), grid, block, 0, stream, g);
     else if(g.fp4 && g.a_s)
         hipLaunchKernelGGL((moe_gemm_pairs_kernel<STAGE, 4, QUANTISED>), grid, block, 0, stream, g);

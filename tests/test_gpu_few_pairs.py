@@ -44,21 +44,25 @@ def test_few_pairs_equal_the_stages(T, k, E, H, I, splitk, method):
     _equal_the_stages(T, k, E, H, I, splitk, method, 16)
 
 
-@pytest.mark.parametrize("T,k,E,H,I", [
-    (1, 1, 8, 512, 512),             # one row
-    (64, 2, 8, 1024, 1536),          # sixteen rows per expert: the most in fewer experts
-    (65, 2, 8, 512, 512),            # more
-    (40, 8, 40, 1536, 1024),
-    (100, 6, 75, 512, 512),          # eight rows per expert: the most in 32 experts and more
-    (90, 8, 192, 2560, 512),         # an uneven share of K-steps
-    (128, 1, 8, 512, 512),           # one K-step for each wave
+@pytest.mark.parametrize("T,k,E,H,I,rows", [
+    (1, 1, 8, 512, 512, 32),             # one row
+    (64, 2, 8, 1024, 1536, 32),          # sixteen rows per expert: the most in fewer than 32
+    (65, 2, 8, 512, 512, 32),            # more
+    (40, 8, 40, 1536, 1024, 32),
+    (150, 6, 75, 512, 512, 32),          # twelve: the most in 32 experts and more
+    (90, 8, 192, 2560, 512, 32),         # an uneven share of K-steps
+    (128, 1, 8, 512, 512, 32),           # one K-step for each wave
+    (72, 1, 3, 1024, 1536, 64),          # 24: the most in fewer than 32
+    (49, 2, 4, 512, 512, 64),            # more
+    (120, 3, 30, 1536, 512, 64),
+    (96, 8, 64, 512, 1024, 64),          # twelve
 ])
-def test_two_row_tiles_equal_the_stages(T, k, E, H, I):
-    _equal_the_stages(T, k, E, H, I, 0, "a4w4", 32)
+def test_several_row_tiles_equal_the_stages(T, k, E, H, I, rows):
+    _equal_the_stages(T, k, E, H, I, 0, "a4w4", rows)
 
 
 def _equal_the_stages(T, k, E, H, I, splitk, method, rows):
-    """plain routing, holes in it, no bias, an expert mask, a local token count; SiLU to bf16 and SwiGLU to fp32"""
+    """plain routing, holes in it, no bias, an expert mask, a local token count, one expert; SiLU to bf16 and SwiGLU to fp32"""
     from pyhip_amd import fused_moe
     from pyhip_amd.enums import ActivationType
     L = cases.make_layer("", T, seed=T * 7 + k, bias=True, E=E, k=min(k, E), H=H, I=I, router="softmax")
@@ -83,7 +87,8 @@ def _equal_the_stages(T, k, E, H, I, splitk, method, rows):
     hidden, tw = L.hidden.cuda(), torch.from_numpy(L.topk_w).cuda()
     for name, wa, wb, t, kw in (("plain", w1, w2, ids, whole), ("holes", w1, w2, hole, whole),
                                 ("no bias", w1, w2, ids, dict(whole, bias1=None, bias2=None)),
-                                ("mask", ma, mb, ids, rank), ("local", w1, w2, ids, dict(whole, num_local_tokens=local))):
+                                ("mask", ma, mb, ids, rank), ("local", w1, w2, ids, dict(whole, num_local_tokens=local)),
+                                ("one expert", w1, w2, torch.full_like(ids, E - 1), whole)):      # full blocks, and one of 1 to 4 row tiles
         for more in (dict(), dict(dtype=torch.float32, activation=ActivationType.Swiglu)):
             print(f"few pairs T={T} k={L.k} E={E} H={H} I={I} {name} {sorted(more)}", flush=True)
             kw2 = dict(kw, method=method, block_size_M=rows, splitk=splitk, **more)
@@ -96,7 +101,7 @@ def _equal_the_stages(T, k, E, H, I, splitk, method, rows):
 
 @pytest.mark.parametrize("T,H,I", [(1, 544, 544), (1, 544, 8224), (3, 1440, 1440), (1, 992, 32 * 47), (20, 1440, 1056), (30, 576, 1440), (50, 1440, 1056)])
 @pytest.mark.parametrize("wide", [False, True])
-@pytest.mark.parametrize("method,rows", [("w4a16", 16), ("a4w4", 16), ("a4w4", 32)])
+@pytest.mark.parametrize("method,rows", [("w4a16", 16), ("a4w4", 16), ("a4w4", 32), ("a4w4", 64)])
 def test_few_pairs_leave_padding_alone(T, H, I, wide, method, rows):
     """Padded layers, activations at the true or the padded width.  The weights' padding is told, so it is not read: its rows and
     columns are filled with ones here, and what the padded columns of the activations hold does not matter either."""
@@ -128,7 +133,7 @@ def test_few_pairs_leave_padding_alone(T, H, I, wide, method, rows):
 
 @pytest.mark.parametrize("T", [1, 4, 8, 9, 40])
 @pytest.mark.parametrize("grouped", [False, True])
-@pytest.mark.parametrize("method,rows", [("w4a16", 16), ("a4w4", 16), ("a4w4", 32)])
+@pytest.mark.parametrize("method,rows", [("w4a16", 16), ("a4w4", 16), ("a4w4", 32), ("a4w4", 64)])
 def test_few_pairs_with_the_router(T, grouped, method, rows):
     from pyhip_amd import fused_moe, fused_moe_routed
     L = cases.make_layer("", T, seed=T, E=256, k=8, H=512, I=512, router="softmax")

@@ -17,6 +17,8 @@ from pyhip_amd import _lib
     # two rows per expert and more, in 32 experts and more: 32 rows (the ladder: 16)
     (80, 8, 256, 256, 7168, 2048, 32), (63, 8, 256, 256, 7168, 2048, 16), (17, 4, 32, 32, 4096, 4096, 32), (16, 4, 32, 32, 4096, 4096, 16),
     (20, 4, 31, 31, 4096, 4096, 16),
+    # five and more, hidden 3072 and more: 64 (32)
+    (300, 8, 256, 256, 7168, 2048, 64), (160, 4, 128, 128, 3072, 3072, 64), (159, 4, 128, 128, 3072, 3072, 32), (150, 4, 60, 60, 2048, 1536, 32),
 ])
 def test_known_choices(tokens, topk, experts, local, hidden, inter, want):
     assert _lib.load().pyhip_layer_block_m(tokens, topk, experts, local, hidden, inter) == want
