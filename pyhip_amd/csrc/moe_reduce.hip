@@ -16,7 +16,7 @@ struct ReduceRouting
     int experts;
 };
 
-// One wave per (token, 64 pieces of 16 bytes): everything about the routing is then the same for the whole wave.  Lanes
+// One wave per (token, 64 * PIECES pieces of 16 bytes): everything about the routing is then the same for the whole wave.  Lanes
 // 0..7 fetch the ids of eight slots, one ballot says which of them count, and the loop over slots branches on scalar
 // bits, so a slot that was dropped costs neither a load nor an addition.  (One thread per piece that read its token's
 // ids and mask entries for itself issued sixteen loads, one after the other, for every eight of data.)
@@ -34,10 +34,9 @@ struct ReduceRouting
 //     512 tokens: all kept 5.42 / 4.58 / 5.04; 4001 tokens 21.4 / 18.2 / 19.7
 // In the layer, where the ids come from memory rather than a cache, asking first costs decode sizes 0.1-0.35 us.
 #define ALONG_PIECES (1 << 18)
-template <bool OUT_F32, bool ROUTED>
-__global__ void __launch_bounds__(256)
-    moe_topk_reduce_kernel(const uint4* __restrict__ in, void* __restrict__ out, long long T, int k, int H8,
-                           const u32* __restrict__ tokens_limit, ReduceRouting rt)
+template <bool OUT_F32, bool ROUTED, int PIECES>
+__device__ __forceinline__ void topk_reduce(const uint4* __restrict__ in, void* __restrict__ out, long long T, int k, int H8,
+                                            const u32* __restrict__ tokens_limit, const ReduceRouting& rt)
 {
     if(tokens_limit)
     {
@@ -46,7 +45,7 @@ __global__ void __launch_bounds__(256)
     }
     const int lane   = lane_id();
     const u32 wave   = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    const u32 chunks = ((u32)H8 + WAVE - 1) / WAVE;
+    const u32 pieces = WAVE * PIECES, chunks = ((u32)H8 + pieces - 1) / pieces;
     // this wave's first (token, chunk) and the step to its next one: no 64-bit division
     const u32 first = blockIdx.x * 4u + wave, step = gridDim.x * 4u;
     const u32 step_t = step / chunks, step_c = step - step_t * chunks;
@@ -61,11 +60,16 @@ __global__ void __launch_bounds__(256)
     }
     while(t < T)
     {
-        const int c  = (int)(ch * WAVE) + lane;
-        const int cc = c < H8 ? c : H8 - 1;         // lanes past the row read its last piece and store nothing
-        float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        const uint4* p = in + (t * k) * H8 + cc;
-        for(int s0 = 0; s0 < k; s0 += 8)            // up to 8 independent loads in flight, added in slot order
+        int c[PIECES];
+        const uint4* p[PIECES];
+        float acc[PIECES][8] = {};
+#pragma unroll
+        for(int q = 0; q < PIECES; q++)
+        {
+            c[q] = (int)(ch * pieces) + q * WAVE + lane;
+            p[q] = in + (t * k) * H8 + (c[q] < H8 ? c[q] : H8 - 1);      // (lanes past the row read its last piece and store nothing)
+        }
+        for(int s0 = 0; s0 < k; s0 += 8)            // up to 8 independent loads in flight for each piece, added in slot order
         {
             const int n = k - s0 < 8 ? k - s0 : 8;
             u32 on      = (1u << n) - 1u;           // slots that count, the same in every lane
@@ -74,11 +78,13 @@ __global__ void __launch_bounds__(256)
                 e = rt.topk_ids[t * k + s0 + lane];
             if(ROUTED && ask_first)
                 on = (u32)__ballot(moe_pair_is_kept(e, rt.experts, rt.expert_mask));
-            v4i v[8];
+            v4i v[PIECES][8];
 #pragma unroll
             for(int j = 0; j < 8; j++)
                 if((on >> j) & 1u)
-                    v[j] = __builtin_nontemporal_load((const v4i*)(p + (long long)(s0 + j) * H8));
+#pragma unroll
+                    for(int q = 0; q < PIECES; q++)
+                        v[q][j] = __builtin_nontemporal_load((const v4i*)(p[q] + (long long)(s0 + j) * H8));
             if(ROUTED && !ask_first)
                 on = (u32)__ballot(moe_pair_is_kept(e, rt.experts, nullptr));
 #pragma unroll
@@ -87,31 +93,37 @@ __global__ void __launch_bounds__(256)
                 // (leaving a slot out is adding +0.0: the sums start at +0.0 and can never become -0.0)
                 if(!((on >> j) & 1u))
                     continue;
-                acc[0] += bf16_bits_to_f32((u32)v[j][0] & 0xFFFFu); acc[1] += bf16_bits_to_f32((u32)v[j][0] >> 16);
-                acc[2] += bf16_bits_to_f32((u32)v[j][1] & 0xFFFFu); acc[3] += bf16_bits_to_f32((u32)v[j][1] >> 16);
-                acc[4] += bf16_bits_to_f32((u32)v[j][2] & 0xFFFFu); acc[5] += bf16_bits_to_f32((u32)v[j][2] >> 16);
-                acc[6] += bf16_bits_to_f32((u32)v[j][3] & 0xFFFFu); acc[7] += bf16_bits_to_f32((u32)v[j][3] >> 16);
+#pragma unroll
+                for(int q = 0; q < PIECES; q++)
+#pragma unroll
+                    for(int i = 0; i < 4; i++)
+                    {
+                        acc[q][2 * i] += bf16_bits_to_f32((u32)v[q][j][i] & 0xFFFFu);
+                        acc[q][2 * i + 1] += bf16_bits_to_f32((u32)v[q][j][i] >> 16);
+                    }
             }
         }
-        if(c < H8)
-        {
-            const long long id = t * H8 + c;
-            if(OUT_F32)
+#pragma unroll
+        for(int q = 0; q < PIECES; q++)
+            if(c[q] < H8)
             {
-                float4* o = (float4*)out + id * 2;
-                o[0]      = make_float4(acc[0], acc[1], acc[2], acc[3]);
-                o[1]      = make_float4(acc[4], acc[5], acc[6], acc[7]);
+                const long long id = t * H8 + c[q];
+                if(OUT_F32)
+                {
+                    float4* o = (float4*)out + id * 2;
+                    o[0]      = make_float4(acc[q][0], acc[q][1], acc[q][2], acc[q][3]);
+                    o[1]      = make_float4(acc[q][4], acc[q][5], acc[q][6], acc[q][7]);
+                }
+                else
+                {
+                    uint4 o;
+                    o.x = pack_bf16x2(acc[q][0], acc[q][1]);
+                    o.y = pack_bf16x2(acc[q][2], acc[q][3]);
+                    o.z = pack_bf16x2(acc[q][4], acc[q][5]);
+                    o.w = pack_bf16x2(acc[q][6], acc[q][7]);
+                    ((uint4*)out)[id] = o;
+                }
             }
-            else
-            {
-                uint4 o;
-                o.x = pack_bf16x2(acc[0], acc[1]);
-                o.y = pack_bf16x2(acc[2], acc[3]);
-                o.z = pack_bf16x2(acc[4], acc[5]);
-                o.w = pack_bf16x2(acc[6], acc[7]);
-                ((uint4*)out)[id] = o;
-            }
-        }
         t += step_t;
         ch += step_c;
         if(ch >= chunks)
@@ -120,6 +132,25 @@ __global__ void __launch_bounds__(256)
             t++;
         }
     }
+}
+
+template <bool OUT_F32, bool ROUTED>
+__global__ void __launch_bounds__(256)
+    moe_topk_reduce_kernel(const uint4* __restrict__ in, void* __restrict__ out, long long T, int k, int H8,
+                           const u32* __restrict__ tokens_limit, ReduceRouting rt)
+{
+    topk_reduce<OUT_F32, ROUTED, 1>(in, out, T, k, H8, tokens_limit, rt);
+}
+
+// Under an expert mask a wave waits for ids, mask and data one after the other and fetches little: two pieces to a lane share the
+// chain.  Layer, us, one / two / four: one of 8 ranks of the DeepSeek-V3 shape, 4001 tokens 209.5 / 206.9 / 209.1, 2000 tokens 166.6 / 164.2 /
+// 165.2; one of 4 of the Qwen3 shape, 2000 tokens 93.2 / 91.7 / 92.3.  Without a mask (8192 tokens, 1875 / 1882) and in small calls, whose
+// waves are all resident at once (0.2-0.6 us), one is the faster.
+template <bool OUT_F32>
+__global__ void __launch_bounds__(256)
+    moe_topk_reduce_masked_kernel(const uint4* __restrict__ in, void* __restrict__ out, long long T, int k, int H8, ReduceRouting rt)
+{
+    topk_reduce<OUT_F32, true, 2>(in, out, T, k, H8, nullptr, rt);
 }
 
 static int launch_reduce(const char* name, const void* in_bf16, void* out, int64_t tokens, int topk, int hidden,
@@ -131,15 +162,26 @@ static int launch_reduce(const char* name, const void* in_bf16, void* out, int64
     PYHIP_REQUIRE(((uintptr_t)in_bf16 % 16) == 0 && ((uintptr_t)out % 16) == 0, "%s: unaligned pointer", name);
     if(tokens <= 0)
         return PYHIP_OK;
-    // a wave for every (token, 64 pieces of 16 bytes), four to a workgroup; a launch past 65536 workgroups strides
-    const long long waves = (long long)tokens * ((hidden / 8 + WAVE - 1) / WAVE);
+    // a wave for every (token, 64 or 128 pieces of 16 bytes), four to a workgroup; a launch past 65536 workgroups strides
+    const bool masked     = rt && rt->expert_mask && (long long)tokens * topk * (hidden / 8) > ALONG_PIECES;
+    const int pieces      = WAVE * (masked ? 2 : 1);
+    const long long waves = (long long)tokens * ((hidden / 8 + pieces - 1) / pieces);
     long long grid        = (waves + 3) / 4;
     grid                  = grid > 65536 ? 65536 : grid;
     const ReduceRouting none = {nullptr, nullptr, nullptr, 0};
 #define REDUCE_LAUNCH(F32, ROUTED)                                                                                  \
     hipLaunchKernelGGL((moe_topk_reduce_kernel<F32, ROUTED>), dim3((unsigned)grid), dim3(256), 0, stream,           \
                        (const uint4*)in_bf16, out, (long long)tokens, topk, hidden / 8, num_valid_ids, rt ? *rt : none)
-    if(rt)
+    if(masked)
+    {
+        if(out_is_f32)
+            hipLaunchKernelGGL((moe_topk_reduce_masked_kernel<true>), dim3((unsigned)grid), dim3(256), 0, stream, (const uint4*)in_bf16, out,
+                               (long long)tokens, topk, hidden / 8, *rt);
+        else
+            hipLaunchKernelGGL((moe_topk_reduce_masked_kernel<false>), dim3((unsigned)grid), dim3(256), 0, stream, (const uint4*)in_bf16, out,
+                               (long long)tokens, topk, hidden / 8, *rt);
+    }
+    else if(rt)
     {
         if(out_is_f32)
             REDUCE_LAUNCH(true, true);
