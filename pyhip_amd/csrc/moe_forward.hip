@@ -215,7 +215,7 @@ extern "C" int pyhip_layer_block_m(int64_t tokens, int topk, int experts, int lo
     // 32 / 64 rows (three waves per SIMD instead of four, which a short K loop feels): DeepSeek-V3 shape 6.3: 881 / 887, 9.4: 913 / 917; gpt-oss shape
     // 6.3: 257 / 257, 11.6: 272 / 277; Qwen3 shape 6.3: 120 / 118, 11: 155 / 147; 96 experts, Zipf, 5: 121 / 114, 7.5: 152 / 143, 11.7: 211 / 189; hidden
     // 2048: 256 experts, top-1 9.8: 338 / 355; 128, top-8, 11: 70.7 / 74.2; 60, top-4, 10: 56.4 / 58.7
-    if(ladder == 16 && experts >= 32 && est >= 2.0 && tokens * topk > PAIRS_UNSORTED_MAX)
+    if(ladder == 16 && experts >= 32 && est >= 2.0 && tokens * topk > WAVE)
         ladder = 32;
     else if(ladder == 32 && experts >= 32 && est >= 5.0 && hidden >= 3072 && inter % 512 == 0)
         ladder = 64;
@@ -290,20 +290,34 @@ struct Router
 //   64 rows (against the persistent kernel of the better height): Qwen3 shape 6.3: 128 / 118, 11: 158 / 147; gpt-oss shape 9.4: 277 / 268, 11.6: 280 /
 //     277, 31: 323 / 357; DeepSeek-V3 shape 11.6: 949 / 939, 16: 964 / 981; 96 experts 5: 128 / 114, 11.7: 212 / 189; 8 experts 17.5: 140 / 123, 25: 142 /
 //     129, 40: 147 / 149; 16, top-2, 4096 x 4096 25: 84.3 / 83.0, 31: 85.0 / 88.4; 12, 5120 x 2048 22: 46.8 / 47.4, 28: 47.6 / 51.2
+static int rows_per_expert_max(int experts, int block_m)
+{
+    return experts < 32 ? (block_m == 16 ? 8 : block_m == 32 ? 16 : 24) : (block_m == 16 ? 4 : 12);
+}
+// Whether they find their rows themselves, in blocks of 16: up to a pair to a lane; with two, where that costs every workgroup of the gate_up
+// GEMM a microsecond more, if all of its workgroups run at once (and the list of blocks fits where a sort into 32 rows would put its own).
+// Layer, us, sorted / this: 8 experts, 1024 x 512, top-2, 40 tokens 22.0 / 16.8, 64 tokens 20.0 / 17.8; 12, 1024 x 1024, 50 tokens 22.1 / 18.2.
+static bool leaves_sort_out(int64_t tokens, int topk, int experts, int inter, int block_m, int w4a16)
+{
+    const int64_t pairs = tokens * topk, blocks = pairs < experts + pairs / 16 ? pairs : experts + pairs / 16;
+    if(block_m > 32 || (w4a16 && block_m > 16) || pairs > PAIRS_UNSORTED_MAX)
+        return false;
+    return (block_m == 16 && pairs <= WAVE) || (blocks * (inter / 32) <= 768 && blocks <= 64 && pairs <= 16ll * experts);
+}
 static bool takes_pairs(int64_t tokens, int topk, int experts, int hidden, int inter, int block_m, int w4a16, int split_k)
 {
     const int64_t pairs = tokens * topk;
     if(block_m != 16 && ((block_m != 32 && block_m != 64) || w4a16))
         return false;
-    const int rows_per_expert = experts < 32 ? (block_m == 16 ? 8 : block_m == 32 ? 16 : 24) : (block_m == 16 ? 4 : 12);
-    if(!w4a16 && (block_m != 16 || pairs > PAIRS_UNSORTED_MAX) && pairs > (int64_t)experts * rows_per_expert)
+    if(!w4a16 && !leaves_sort_out(tokens, topk, experts, inter, block_m, w4a16) &&
+       pairs > (int64_t)experts * rows_per_expert_max(experts, block_m))
         return false;
     return hidden % 512 == 0 && inter % 512 == 0 && topk > 0 && experts <= 2048 &&
            pyhip_pairs_served(tokens, topk, experts, hidden, inter, pyhip_moe_sorting_max_blocks(tokens, topk, experts, block_m) * (block_m / 16),
                               !w4a16, split_k);
 }
 
-// The layer by the kernels of moe_gemm_pairs.hip.  Up to 64 pairs the kernels find their rows themselves
+// The layer by the kernels of moe_gemm_pairs.hip.  Up to 128 pairs the kernels find their rows themselves
 // and the sort is left out; where pairs rarely share an expert the down GEMM sums the slots and the reduction is left out too: two
 // launches (with the router three) instead of four.  What that saves is the launch on the host (3.3 us each) and the latency chain of the stage
 // on the device (sort 4.5-5.5, reduction 3-5 us).
@@ -315,7 +329,7 @@ static int forward_pairs(const void* hidden_bf16, int64_t row_stride, int hidden
                          float swiglu_limit, int held, const Layout& l, uint8_t* ws, hipStream_t stream)
 {
     uint8_t* a2         = ws + (w4a16 ? l.a2 : l.a2_q);      // a row for every pair
-    const bool unsorted = block_m == 16 && (int64_t)tokens * topk <= PAIRS_UNSORTED_MAX;
+    const bool unsorted = leaves_sort_out(tokens, topk, experts, inter, block_m, w4a16);
     uint32_t* s_ids     = (uint32_t*)(ws + l.sorted_ids);
     float* s_w          = (float*)(ws + l.sorted_w);
     uint32_t *s_e = (uint32_t*)(ws + l.sorted_e), *n_valid = (uint32_t*)(ws + l.num_valid), *sched = (uint32_t*)(ws + l.sched);
@@ -355,7 +369,7 @@ static int forward_pairs(const void* hidden_bf16, int64_t row_stride, int hidden
     {
         g.sorted_ids = s_ids; g.sorted_w = s_w; g.sorted_e = s_e; g.num_valid = n_valid;
     }
-    g.T = tokens; g.topk = topk; g.experts = experts; g.rows = block_m; g.held = held;
+    g.T = tokens; g.topk = topk; g.experts = experts; g.rows = unsorted ? 16 : block_m; g.held = held;
     PairArgs up = g, down = g;
     up.a = hidden_bf16; up.w = w1; up.w_s = w1_scale; up.bias = (const uint16_t*)bias1_bf16;
     up.out = a2; up.K = hidden; up.N = 2 * inter;
@@ -378,7 +392,13 @@ static int forward_pairs(const void* hidden_bf16, int64_t row_stride, int hidden
     const bool top2 = w4a16 && tokens == 1 && topk == 2;
     up.row_step = down.row_step = top2 ? 16 : 1;
     up.all_channels             = top2;
-    rc = pyhip_pairs_gate_up(up, tokens, l.n_blk, split_k, activation, swiglu_limit, stream);
+    if(unsorted && !top2)
+    {
+        up.tab_ids = s_ids; up.tab_w = s_w; up.tab_e = s_e; up.tab_valid = n_valid;
+    }
+    // (unsorted 32-row blocks are two of 16)
+    const int64_t n_blk = unsorted ? l.n_blk * (block_m / 16) : l.n_blk;
+    rc = pyhip_pairs_gate_up(up, tokens, n_blk, split_k, activation, swiglu_limit, stream);
     if(rc)
         return rc;
     if(top2)
@@ -388,11 +408,16 @@ static int forward_pairs(const void* hidden_bf16, int64_t row_stride, int hidden
         if(rc >= 0)
             return rc;
     }
-    rc = pyhip_pairs_down_sum(down, l.rows2, l.n_blk, split_k, stream);
+    rc = pyhip_pairs_down_sum(down, l.rows2, n_blk, split_k, stream);
     if(rc >= 0)
         return rc;
     down.out = ws + l.out3;
-    rc       = pyhip_pairs_down(down, l.rows2, l.n_blk, split_k, stream);
+    if(up.tab_ids)
+    {
+        down.ids = nullptr;
+        down.sorted_ids = s_ids; down.sorted_w = s_w; down.sorted_e = s_e; down.num_valid = n_valid;
+    }
+    rc = pyhip_pairs_down(down, l.rows2, n_blk, split_k, stream);
     if(rc)
         return rc;
     return pyhip_moe_topk_reduce_routed(ws + l.out3, out, tokens, topk, hidden, out_is_f32, topk_ids, experts, expert_mask,

@@ -10,7 +10,7 @@ struct PairArgs
     const uint8_t* w_s = nullptr;   // weight scales, shuffled  [E*N (padded to 256), SC]
     const uint16_t* bias = nullptr; // bf16 [E, N] or null
     // bf16 a2 has a row for every pair, pair t * topk + slot in row pair * row_step; quantised a2 one for each row of the blocks.
-    // The routing as the caller gave it, read by the kernels themselves (at most 64 pairs) ...
+    // The routing as the caller gave it, read by the kernels themselves (at most PAIRS_UNSORTED_MAX pairs) ...
     const int* ids       = nullptr;   // [T, topk], or null: the sort's output below (row_step 1)
     const float* weights = nullptr;   // [T, topk] (down)
     const int* mask      = nullptr;   // [experts] or null
@@ -20,6 +20,11 @@ struct PairArgs
     const float* sorted_w = nullptr;
     const u32* sorted_e   = nullptr;
     const u32* num_valid  = nullptr;
+    // gate_up, unsorted: where it leaves the blocks that it has found, in that form, or null
+    u32* tab_ids   = nullptr;
+    float* tab_w   = nullptr;
+    u32* tab_e     = nullptr;
+    u32* tab_valid = nullptr;
     void* out = nullptr;              // gate_up: a2 bf16 [.., N/2], or (fp4) e2m1 pairs, in tiles; down: out3 bf16 [T, topk, N]; down that sums: [T, N]
     uint8_t* out_s = nullptr;         // gate_up, fp4: the scales of a2
     int rows = 16;                    // of a block; 32, 64: sorted, activations quantised
@@ -38,7 +43,7 @@ struct PairArgs
     GatedAct act = {};
 };
 
-#define PAIRS_UNSORTED_MAX 64
+#define PAIRS_UNSORTED_MAX 128
 
 // Whether these kernels have the K splits that the sorted entry points take for such a call (split_k as there)
 bool pyhip_pairs_served(int64_t tokens, int topk, int experts, int hidden, int inter, int64_t n_blk, int fp4, int split_k);

@@ -1,7 +1,7 @@
 // The layer call's GEMMs in blocks of 16 rows (MXFP4 activations: or 32 or 64): few tokens, so the call is a weight stream and a chain of launches.  With bf16
 // activations the arithmetic (and with it every bit of the result) is that of moe_gemm_w4a16.hip, with MXFP4 ones that of
 // moe_gemm_mxfp4.hip; their entry points serve callers that run the stages one by one.  What is different is what a call of 20-100 us spends beside its weights:
-//   * Up to 64 pairs (token, slot) there is no sort: every wave reads the routing, a pair to a lane, and finds its block's
+//   * Up to 128 pairs (token, slot) there is no sort: every wave reads the routing, one or two pairs to a lane, and finds its block's
 //     expert and rows with a few ballots (find_block).
 //   * Activations come at their own row pitch and width, and neither the padding rows nor the padding columns of the weights
 //     are fetched (raw buffer loads: a lane or a row group that has nothing to fetch is out of its descriptor's range).
@@ -43,40 +43,100 @@ __device__ __forceinline__ int local_expert(int e, const int* mask, int lane)
     return __builtin_amdgcn_readfirstlane(n);
 }
 
-// Block m_blk of the unsorted call, or false.  Lane p holds pair p; lanes whose pairs share an expert are found by a ballot for each
+// Block m_blk of the unsorted call, or false.  Lane p holds pairs p and p + 64; pairs that share an expert are found by a ballot for each
 // bit of the expert number; every 16th of them, in pair order, starts a block, and blocks are numbered by the pair that starts them.
 // -> expert (local id) and, in lane r of each 16, the pair of the block's row r (-1: no row)
-__device__ __forceinline__ bool find_block(const PairArgs& g, int m_blk, int lane, int& e, int& pair)
+// blocks: how many there are.  TWO: more than 64 pairs.  (The sort's launch in front of the GEMMs costs the host 3.3 us and the device 5-7.  This
+// costs every workgroup 0.3 us, and 1.2 us with two pairs to a lane: 128 pairs in both GEMMs of the DeepSeek-V3 shape 356 -> 426 us, of
+// the tiny layer 20.9 -> 18.1.  So gate_up leaves what it has found to the down GEMM: Qwen3 shape, 8 tokens, 47.3 -> 46.7; Mixtral shape, 29 tokens,
+// 121.2 -> 119.9; 96 experts, top-4, 16 tokens 61.7 -> 60.0.)
+template <bool TWO>
+__device__ __forceinline__ bool find_block(const PairArgs& g, int m_blk, int lane, int& e, int& pair, int& blocks)
 {
+    constexpr int H = TWO ? 2 : 1;
     int n = g.T * g.topk;
     if(g.local_tok)
     {
         const int lim = *g.local_tok;
         n             = lim < 0 ? 0 : lim < g.T ? lim * g.topk : n;
     }
-    const int id    = lane < n ? g.ids[lane] : -1;
-    const bool kept = moe_pair_is_kept(id, g.experts, g.mask);
-    u64 same        = __ballot(kept);
+    int id[H];
+    bool kept[H];
+    u64 same[H][H];      // [of the lane's pair h][among pairs 64 * i ..]
+#pragma unroll
+    for(int h = 0; h < H; h++)
+        id[h] = h * WAVE + lane < n ? g.ids[h * WAVE + lane] : -1;
+#pragma unroll
+    for(int h = 0; h < H; h++)
+        kept[h] = moe_pair_is_kept(id[h], g.experts, g.mask);
+#pragma unroll
+    for(int h = 0; h < H; h++)
+#pragma unroll
+        for(int i = 0; i < H; i++)
+            same[h][i] = __ballot(kept[i]);
     for(int b = 0; (g.experts - 1) >> b; b++)
     {
-        const bool bit = (id >> b) & 1;
-        const u64 s    = __ballot(bit);
-        same &= bit ? s : ~s;
+        u64 s[H];
+#pragma unroll
+        for(int i = 0; i < H; i++)
+            s[i] = __ballot((id[i] >> b) & 1);
+#pragma unroll
+        for(int h = 0; h < H; h++)
+#pragma unroll
+            for(int i = 0; i < H; i++)
+                same[h][i] &= (id[h] >> b) & 1 ? s[i] : ~s[i];
     }
-    const u64 below  = (1ull << lane) - 1ull;
-    const bool start = kept && (__builtin_popcountll(same & below) & 15) == 0;
-    const u64 starts = __ballot(start);
-    const u64 hit    = __ballot(start && __builtin_popcountll(starts & below) == m_blk);
-    if(!hit)
-        return false;
-    const int lead = __builtin_ctzll(hit);
-    u64 rows = (u64)(u32)__builtin_amdgcn_readlane((int)same, lead) | (u64)(u32)__builtin_amdgcn_readlane((int)(same >> 32), lead) << 32;
-    rows &= ~((1ull << lead) - 1ull);
-    e    = local_expert(__builtin_amdgcn_readlane(id, lead), g.mask, lane);
-    pair = -1;
-    for(int i = 0; i < 16 && rows; i++, rows &= rows - 1ull)
-        pair = (lane & 15) == i ? __builtin_ctzll(rows) : pair;
-    return true;
+    const u64 below = (1ull << lane) - 1ull;
+    u64 hits[H];
+    blocks = 0;
+#pragma unroll
+    for(int h = 0; h < H; h++)
+    {
+        const int rank   = (h ? __builtin_popcountll(same[h][0]) : 0) + __builtin_popcountll(same[h][h] & below);
+        const bool start = kept[h] && (rank & 15) == 0;
+        const u64 starts = __ballot(start);
+        hits[h]          = __ballot(start && blocks + __builtin_popcountll(starts & below) == m_blk);
+        blocks += __builtin_popcountll(starts);
+    }
+#pragma unroll
+    for(int h = 0; h < H; h++)
+    {
+        const u64 hit = hits[h];
+        if(!hit)
+            continue;
+        const int lead = __builtin_ctzll(hit);
+        u64 rows[H];
+#pragma unroll
+        for(int i = 0; i < H; i++)
+        {
+            rows[i] = i < h ? 0ull
+                            : (u64)(u32)__builtin_amdgcn_readlane((int)same[h][i], lead) |
+                                  (u64)(u32)__builtin_amdgcn_readlane((int)(same[h][i] >> 32), lead) << 32;
+            if(i == h)
+                rows[i] &= ~((1ull << lead) - 1ull);
+        }
+        e    = local_expert(__builtin_amdgcn_readlane(id[h], lead), g.mask, lane);
+        pair = -1;
+        for(int r = 0; r < 16; r++)
+        {
+            int p = -1;
+            if(rows[0])
+            {
+                p = __builtin_ctzll(rows[0]);
+                rows[0] &= rows[0] - 1ull;
+            }
+            else if(TWO && rows[H - 1])
+            {
+                p = WAVE + __builtin_ctzll(rows[H - 1]);
+                rows[H - 1] &= rows[H - 1] - 1ull;
+            }
+            if(p < 0)
+                break;
+            pair = (lane & 15) == r ? p : pair;
+        }
+        return true;
+    }
+    return false;
 }
 
 // the lane's four biases of channels c .. c + 3 (element-aligned tensors: one by one)
@@ -391,7 +451,7 @@ __device__ __forceinline__ void pairs_tile(const PairArgs& g, float* red, int la
 
 // BT: 16-row tiles of a block.  The real rows of a block come first; what a block computes are the row tiles that have any.
 template <int STAGE, int SPLIT, int ACT, int BT = 1, bool STAGED = false>
-__global__ void __launch_bounds__(W4A16_THREADS, BT == 1 ? 1 : 3) moe_gemm_pairs_kernel(PairArgs g)
+__global__ void __launch_bounds__(W4A16_THREADS, BT == 1 && !STAGED ? 1 : 3) moe_gemm_pairs_kernel(PairArgs g)
 {
     // [wave][row group][row tile][lane][4]; staged rows: [wave][row][16 pieces of 16 bytes]
     __shared__ __attribute__((aligned(16))) float red[SPLIT || STAGED ? 4 * 4 * (BT < 2 ? 1 : 2) * WAVE * 4 : 1];
@@ -411,8 +471,23 @@ __global__ void __launch_bounds__(W4A16_THREADS, BT == 1 ? 1 : 3) moe_gemm_pairs
     }
     if(BT == 1 && g.ids)
     {
-        int pair;
-        if(!find_block(g, m_blk, lane, e, pair))
+        int pair, blocks;
+        const bool found = g.T * g.topk > WAVE ? find_block<true>(g, m_blk, lane, e, pair, blocks) : find_block<false>(g, m_blk, lane, e, pair, blocks);
+        if(STAGE == 1 && nt == 0 && wave == 0 && g.tab_ids)
+        {
+            // for the down GEMM, as the sort would have written it
+            if(m_blk == 0 && lane == 0)
+                g.tab_valid[0] = (u32)(blocks * 16);
+            if(found && lane < 16)
+            {
+                const int tok              = (int)((u32)pair / (u32)g.topk);
+                g.tab_ids[m_blk * 16 + lane] = pair < 0 ? ~0u : (u32)tok | (u32)(pair - tok * g.topk) << 24;
+                g.tab_w[m_blk * 16 + lane]   = pair < 0 ? 0.f : g.weights[pair];
+                if(lane == 0)
+                    g.tab_e[m_blk] = (u32)e;
+            }
+        }
+        if(!found)
             return;
         if(pair >= 0)
         {

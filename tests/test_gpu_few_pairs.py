@@ -1,4 +1,4 @@
-"""The layer call in 16-row blocks with bf16 activations, or with MXFP4 ones and few rows per expert (kernels of its own, without a sort up to 64
+"""The layer call in 16-row blocks with bf16 activations, or with MXFP4 ones and few rows per expert (kernels of its own, without a sort up to 64 or 128
 pairs and without a reduction where pairs rarely share an expert), against the step-by-step path.  With bf16 activations the arithmetic
 and its order are the same; with MXFP4 ones the sums are exact in any order: the same bits."""
 import pytest
@@ -31,8 +31,14 @@ def _poison(T, k, E, H, I, method, rows=16):
     (63, 1, 3, 512, 1024, 0),        # more than a block for an expert; an expert count that is no power of two
     (64, 1, 1, 512, 512, 1),         # one expert, four full blocks, no K split
     (8, 8, 16, 1024, 1536, 1),
-    (65, 1, 8, 512, 512, 0),         # one pair more: sorted
-    (13, 5, 8, 1536, 512, 0),        # sorted, an odd top-k
+    (65, 1, 8, 512, 512, 0),         # one pair more: two to a lane
+    (13, 5, 8, 1536, 512, 0),        # an odd top-k
+    (64, 2, 8, 1024, 512, 0),        # 128 pairs
+    (128, 1, 12, 512, 1024, 1),
+    (16, 8, 40, 512, 512, 0),        # as many workgroups as run at once
+    (16, 8, 41, 512, 512, 0),        # more: sorted
+    (129, 1, 33, 512, 512, 0),       # a pair more: sorted
+    (10, 8, 640, 512, 512, 0),       # summed by token, more than 64 pairs
     (40, 4, 16, 512, 1536, 1),       # sorted, no K split
     (17, 4, 17, 1024, 1536, 0),      # sorted, four rows per expert
     (23, 3, 17, 512, 512, 0),        # one pair more
@@ -46,12 +52,13 @@ def test_few_pairs_equal_the_stages(T, k, E, H, I, splitk, method):
 
 @pytest.mark.parametrize("T,k,E,H,I,rows", [
     (1, 1, 8, 512, 512, 32),             # one row
-    (64, 2, 8, 1024, 1536, 32),          # sixteen rows per expert: the most in fewer than 32
-    (65, 2, 8, 512, 512, 32),            # more
+    (72, 2, 9, 1024, 1536, 32),          # sixteen rows per expert: the most in fewer than 32
+    (73, 2, 9, 512, 512, 32),            # more
     (40, 8, 40, 1536, 1024, 32),
     (150, 6, 75, 512, 512, 32),          # twelve: the most in 32 experts and more
     (90, 8, 192, 2560, 512, 32),         # an uneven share of K-steps
-    (128, 1, 8, 512, 512, 32),           # one K-step for each wave
+    (128, 1, 8, 512, 512, 32),           # 32 rows asked for, blocks of 16 found without a sort
+    (140, 1, 9, 512, 512, 32),           # one K-step for each wave
     (72, 1, 3, 1024, 1536, 64),          # 24: the most in fewer than 32
     (49, 2, 4, 512, 512, 64),            # more
     (120, 3, 30, 1536, 512, 64),
