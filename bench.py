@@ -107,7 +107,7 @@ def time_point(torch, fused_moe, W, shape, tokens, steps, warmup, block_m, metho
     """-> dict with wall-clock ms over exactly `steps` calls, and median / IQR over event-timed batches; only the
     one-call product path runs inside the timed regions"""
     from pyhip_amd import workloads
-    from pyhip_amd.fused_moe import pick_block_m, pick_w4a16
+    from pyhip_amd.fused_moe import _plan
     hidden, topk_w, topk_ids = workloads.make_inputs(shape, tokens)
     if W["hidden_pad"]:      # padded shapes (gpt-oss): activations at the padded width, as the reference passes them
         hidden = torch.nn.functional.pad(hidden, (0, W["hidden_pad"]))
@@ -154,11 +154,11 @@ def time_point(torch, fused_moe, W, shape, tokens, steps, warmup, block_m, metho
     q = lambda f: per[min(batches - 1, int(f * batches))]
     cfg = workloads.SHAPES[shape]
     Hp = cfg["H"] + W["hidden_pad"]
-    w4a16 = method == "w4a16" or (method != "a4w4" and pick_w4a16(tokens, cfg["k"], cfg["E"], Hp))
-    bm = block_m or pick_block_m(tokens, cfg["k"], cfg["E"], Hp, w4a16)
+    # (what the call itself chooses)
+    w4a16, bm, _ = _plan(tokens, cfg["k"], cfg["E"], Hp, cfg["I"] + W["intermediate_pad"], method, block_m or None)
     return dict(wall_ms=wall_ms, median_ms=q(0.5), q1_ms=q(0.25), q3_ms=q(0.75), work=work, hidden=hidden,
                 topk_w=topk_w, topk_ids=topk_ids, out=out, method="w4a16" if w4a16 else "a4w4",
-                block_m=min(bm, 64) if w4a16 else bm, weight_copies=len(sets), calls_per_batch=reps)
+                block_m=bm, weight_copies=len(sets), calls_per_batch=reps)
 
 
 def stage_pass(torch, fused_moe, W, res, block_m, method, passes=8):
