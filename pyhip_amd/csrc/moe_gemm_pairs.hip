@@ -194,7 +194,10 @@ __device__ __forceinline__ void pairs_tile(const PairArgs& g, float* red, int la
     static_assert(SPLITK || ACT == BF16, "MXFP4 activations: the four waves split K");
     static_assert(!STAGED || (ACT == BF16 && MT == 1), "staged: bf16 rows");
     static_assert(BT == 1 || ACT == QUANTISED, "several row tiles: activations that take few registers");
-    constexpr int NB = BT == 1 || MT == 1 ? 3 : 2, KSTRIDE = SPLITK ? 4 : 1;
+    // (bf16 activations take 16 registers a K-step: two K-steps in flight and four waves per SIMD, not three and three.  Layer, us, three / two: 60
+    // experts, 2048 x 1408, 10 tokens 31.8 / 29.4, 50 tokens 57.7 / 53.4; 28, 2048 x 4096, 20 tokens 75.9 / 71.4; 24, 2048 x 2048, 12 tokens 33.2 / 29.8;
+    // Mixtral shape, 20 tokens 118.5 / 117.5; 32, 2880 x 2880, 10 tokens 54.5 / 55.1.  Staged, four waves do not fit without spilling.)
+    constexpr int NB = (ACT == BF16 && !STAGED) || (BT > 1 && MT > 1) ? 2 : 3, KSTRIDE = SPLITK ? 4 : 1;
     constexpr int NA = ACT == QUANTISED ? 1 : 4;                  // 16-byte pieces of a row in a lane's K-step
     const int r = lane & 15, kb = lane >> 4;
     const int Kb = g.K / 2, I = g.N / 2;
@@ -451,7 +454,7 @@ __device__ __forceinline__ void pairs_tile(const PairArgs& g, float* red, int la
 
 // BT: 16-row tiles of a block.  The real rows of a block come first; what a block computes are the row tiles that have any.
 template <int STAGE, int SPLIT, int ACT, int BT = 1, bool STAGED = false>
-__global__ void __launch_bounds__(W4A16_THREADS, BT == 1 && !STAGED ? 1 : 3) moe_gemm_pairs_kernel(PairArgs g)
+__global__ void __launch_bounds__(W4A16_THREADS, ACT == BF16 && !STAGED ? 4 : BT > 1 || STAGED ? 3 : 1) moe_gemm_pairs_kernel(PairArgs g)
 {
     // [wave][row group][row tile][lane][4]; staged rows: [wave][row][16 pieces of 16 bytes]
     __shared__ __attribute__((aligned(16))) float red[SPLIT || STAGED ? 4 * 4 * (BT < 2 ? 1 : 2) * WAVE * 4 : 1];
@@ -772,10 +775,10 @@ static int prepare(const char* name, PairArgs& g, int64_t rows, int64_t blocks, 
 template <int STAGE>
 static void launch_pairs(const PairArgs& g, int split, dim3 grid, hipStream_t stream)
 {
-    // bf16 rows go through LDS where a block has several.  Layer, us, not / staged, by rows per expert: Mixtral shape 1.3: 93.5 / 95.3,
-    // 5: 120.2 / 119.8, 7.3: 125.5 / 121.9; 16 experts, 4096 x 4096 5: 78.3 / 79.5; 32 experts, 2880 x 2880 5: 78.1 / 79.1; 28, 2048 x 4096
-    // 6.4: 79.1 / 76.8; 60, 2048 x 1408 3.3: 57.4 / 58.2, 6.7: 63.5 / 61.8, with a Zipf router 51.1 / 48.0
-    const bool staged = (int64_t)g.T * g.topk >= 6ll * g.experts;
+    // bf16 rows go through LDS where blocks are half full.  Layer, us, not / staged, by rows per expert: 24 experts, 2048 x 2048 6.7: 38.9 / 41.1, 7.8:
+    // 39.9 / 41.3; 60, 2048 x 1408 6.3: 58.3 / 61.3, 6.7 with a Zipf router 49.0 / 47.8; 28, 2048 x 4096 6.4: 74.3 / 77.3, 7.7: 78.1 / 78.6; Mixtral
+    // shape 6: 118.6 / 119.5, 7.3: 122.3 / 120.8, 8: 124.5 / 121.7; 32, 2880 x 2880 7.5: 85.7 / 81.7; 16, 4096 x 4096 7.5 with a Zipf router 75.0 / 70.5
+    const bool staged = (int64_t)g.T * g.topk >= 7ll * g.experts;
     const dim3 block(W4A16_THREADS);
     if(g.rows == 64)
         hipLaunchKernelGGL((moe_gemm_pairs_kernel<STAGE, 4, QUANTISED, 4>), grid, block, 0, stream, g);
