@@ -155,15 +155,15 @@ def time_point(torch, fused_moe, W, shape, tokens, steps, warmup, block_m, metho
     cfg = workloads.SHAPES[shape]
     Hp = cfg["H"] + W["hidden_pad"]
     # (what the call itself chooses)
-    w4a16, bm, _ = _plan(tokens, cfg["k"], cfg["E"], Hp, cfg["I"] + W["intermediate_pad"], method, block_m or None)
+    w4a16, bm, _ = _plan(tokens, cfg["k"], cfg["E"], Hp, cfg["I"] + W["intermediate_pad"], method, block_m or None, cfg["E"])
     return dict(wall_ms=wall_ms, median_ms=q(0.5), q1_ms=q(0.25), q3_ms=q(0.75), work=work, hidden=hidden,
                 topk_w=topk_w, topk_ids=topk_ids, out=out, method="w4a16" if w4a16 else "a4w4",
                 block_m=bm, weight_copies=len(sets), calls_per_batch=reps)
 
 
 def stage_pass(torch, fused_moe, W, res, block_m, method, passes=8):
-    """average duration of each launch group of the step-by-step path, from events on the launch stream; untimed
-    (not part of any ms_per_step)"""
+    """average duration of each launch group of the step-by-step path in blocks of block_m rows, from events on the launch
+    stream; untimed (not part of any ms_per_step)"""
     kw = call_kwargs(W, block_m, method)
     events = []
     for _ in range(2):
@@ -423,15 +423,15 @@ def main():
             if rec["method"] == "a4w4" and rec["block_m"] >= 64:
                 # how evenly the persistent GEMMs' tiles spread over the 8 XCDs for this routing
                 rec["gate_up_tiles_per_xcd"] = workloads.xcd_tile_counts(s, r["topk_ids"], rec["block_m"], W["intermediate_pad"])
-            rec["stage_ms_untimed_pass"] = {k: round(v, 4) for k, v in stage_pass(torch, fused_moe, W, r, 0, "auto", 4).items()}
+            rec["stage_ms_untimed_pass"] = {k: round(v, 4) for k, v in stage_pass(torch, fused_moe, W, r, r["block_m"], "auto", 4).items()}
             configs.append(rec)
             del r
         if shape == a.shape:
             # headline: exactly --steps timed calls after --warmup untimed ones
             main_res = time_point(torch, fused_moe, W, a.shape, a.tokens, a.steps, a.warmup, a.block_m, a.method)
-            main_stage = stage_pass(torch, fused_moe, W, main_res, a.block_m, a.method)
+            main_stage = stage_pass(torch, fused_moe, W, main_res, main_res["block_m"], a.method)
             dec = time_point(torch, fused_moe, W, a.shape, a.decode_tokens, max(a.steps, 50), max(a.warmup, 10), a.block_m)
-            dec_stage = stage_pass(torch, fused_moe, W, dec, a.block_m, "auto")
+            dec_stage = stage_pass(torch, fused_moe, W, dec, dec["block_m"], "auto")
             other = "a4w4" if dec["method"] == "w4a16" else "w4a16"
             dec4 = time_point(torch, fused_moe, W, a.shape, a.decode_tokens, max(a.steps, 50), max(a.warmup, 10), a.block_m, other)
             dec_graph_ms = graph_replay_ms(torch, fused_moe, W, dec, max(a.steps, 50), a.block_m)

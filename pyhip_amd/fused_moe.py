@@ -116,7 +116,8 @@ def pick_w4a16(tokens, topk, experts, hidden):
 def _plan(tokens, topk, experts, hidden, inter, method, block_m, local_experts=None):
     """(bf16 activations?, row block, workspace bytes) of a layer call: a function of its sizes and options alone, so a
     program's few call shapes ask the library once each instead of three times a call (``method`` and ``block_m`` as
-    given by the caller).  Only plain integers are remembered: whatever else converts to one may not be hashable (a numpy
+    given by the caller; ``local_experts``: the matrices here, for the call that runs the whole layer, whose kernels have
+    heights of their own; ``None``: stage by stage, the ladder's height).  Only plain integers are remembered: whatever else converts to one may not be hashable (a numpy
     array) or may change its value and stay the same key (a tensor is hashed by identity).
     With this, checks whose messages are put together only when they fail, and raw stream and data pointers, the
     tiny layer at 64 tokens went from 29.1 to 22.7 us a call."""
@@ -128,10 +129,10 @@ def _ask_plan(tokens, topk, experts, hidden, inter, method, block_m, local_exper
     w4a16 = method == "w4a16" or (method != "a4w4" and pick_w4a16(tokens, topk, experts, hidden))
     if block_m is not None:
         bm = block_m
-    elif w4a16:
-        bm = pick_block_m(tokens, topk, experts, hidden, True)
+    elif w4a16 or local_experts is None:
+        bm = pick_block_m(tokens, topk, experts, hidden, w4a16)
     else:
-        bm = _lib.load().pyhip_layer_block_m(tokens, topk, experts, local_experts or experts, hidden, inter)
+        bm = _lib.load().pyhip_layer_block_m(tokens, topk, experts, local_experts, hidden, inter)
     if w4a16:
         bm = min(bm, 64)
     return w4a16, bm, _lib.load().pyhip_moe_forward_workspace_bytes(tokens, topk, experts, hidden, inter, bm, 1 if w4a16 else 0)
@@ -276,8 +277,9 @@ def fused_moe(
         return torch.zeros(0, H, dtype=out_dtype, device=dev)
 
     topk_ids, topk_weight = _plain(topk_ids, torch.int32), _plain(topk_weight, torch.float32)
+    one_call = not return_parts and stage_events is None and topk_reduce == "store" and operand_staging == "registers"
     # "auto" (and the reference's "jit" / "gluon", which name its own back ends): see pick_w4a16
-    w4a16, bm, ws_bytes = _plan(T, k, global_E, H, I, method, block_size_M, E)
+    w4a16, bm, ws_bytes = _plan(T, k, global_E, H, I, method, block_size_M, E if one_call else None)
     if bias1 is not None:
         bias1 = _plain(bias1, torch.bfloat16)
         _require(bias1.shape == (E, N1), "bias1 must be [E, 2*inter]")
@@ -302,7 +304,6 @@ def fused_moe(
                  "topk_reduce='atomic' needs the MXFP4-activation path, a row block of 16 or 128 and bf16 output")
         _require(not arriver or (not w4a16 and bm in (16, 128, 288) and not lds_tile),
                  "topk_reduce='last_arriver' needs the MXFP4-activation path and a row block of 16, 128 or 288")
-    one_call = not return_parts and stage_events is None and not (atomic or lds_tile or arriver)
     cols = 0
     if narrow:
         # the one-call path takes activations at the true width as they are (bf16 ones only in its 16-row blocks): whole
