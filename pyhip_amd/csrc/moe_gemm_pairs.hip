@@ -528,6 +528,9 @@ __global__ void __launch_bounds__(W4A16_THREADS, ACT == BF16 && !STAGED ? 4 : BT
             }
         }
     }
+    // (a mask with more entries than there are matrices, one that is still being written for instance: no weights past their tensor)
+    if((u32)e >= (u32)g.held)
+        return;
     if constexpr(BT == 1)
         pairs_tile<STAGE, SPLIT, ACT, STAGED, 1, 1>(g, red, lane, wave, m_blk, nt, e, arow, orow, rw);
     else
@@ -571,7 +574,11 @@ __global__ void __launch_bounds__(512) moe_pairs_down_sum_kernel(PairArgs g)
     // lane s: slot s's expert
     const bool here = !(g.local_tok && t >= *g.local_tok);
     const int id    = here && lane < g.topk ? g.ids[t * g.topk + lane] : -1;
-    const u32 on    = (u32)__ballot(moe_pair_is_kept(id, g.experts, g.mask));
+    u32 on          = (u32)__ballot(moe_pair_is_kept(id, g.experts, g.mask));
+    if(g.mask)      // (no weights past their tensor, see moe_gemm_pairs_kernel)
+        for(u32 rest = on; rest; rest &= rest - 1u)
+            if(local_expert(__builtin_amdgcn_readlane(id, __builtin_ctz(rest)), g.mask, lane) >= g.held)
+                on &= ~(rest & -rest);
     u32 turn = 0;                         // this group's slots: in turns, of those that count
     {
         int i = 0;

@@ -152,3 +152,29 @@ def test_few_pairs_with_the_router(T, grouped, method, rows):
                                    **(dict(num_expert_group=8, topk_group=4) if grouped else {}), **kw)
     want = fused_moe(L.hidden.cuda(), w1, w2, tw, ti, return_parts=True, **kw)[0]
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("T,k,method,rows", [(2, 1, "w4a16", 16), (1, 3, "w4a16", 16), (12, 1, "w4a16", 16), (12, 1, "a4w4", 16), (100, 1, "a4w4", 32),
+                                             (100, 1, "a4w4", 64)])
+def test_mask_with_more_entries_than_matrices(T, k, method, rows):
+    """Not a call that means anything, but one that reads nothing past the weights: pairs whose number among the mask's entries is no matrix
+    are left out, and the tokens of the others have their results."""
+    from pyhip_amd import fused_moe
+    E, here = 48, 24
+    L = cases.make_layer("", T, seed=T, E=E, k=k, H=512, I=512, router="softmax")
+    w1, w1s, w2, w2s = cases.device_weights(L)
+    g = torch.Generator().manual_seed(T)
+    ids = torch.randint(0, here, (T, k), generator=g, dtype=torch.int32)
+    ids[0] = torch.arange(E - k, E)                     # a token whose experts are all past the matrices
+    if T > 2:
+        ids[T - 1] = here                               # the first of them
+    tw = torch.rand(T, k, generator=g).cuda()
+    want = fused_moe(L.hidden.cuda(), w1, w2, tw, ids.cuda(), w1_scale=w1s, w2_scale=w2s, method=method, block_size_M=rows)
+    half = lambda w: w.view(E, -1)[:here].reshape(-1, w.shape[-1]).contiguous()
+    ma, mb = w1[:here].contiguous(), w2[:here].contiguous()
+    ma.is_shuffled = mb.is_shuffled = True
+    print("few pairs, wide mask", T, k, method, rows, flush=True)
+    got = fused_moe(L.hidden.cuda(), ma, mb, tw, ids.cuda(), w1_scale=half(w1s), w2_scale=half(w2s), method=method, block_size_M=rows,
+                    expert_mask=torch.ones(E, dtype=torch.int32, device="cuda"))
+    held = (ids < here).all(dim=1).cuda()
+    assert held.sum() == T - (1 if T <= 2 else 2) and torch.equal(got[held], want[held])
