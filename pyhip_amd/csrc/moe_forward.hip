@@ -342,6 +342,8 @@ static int forward_pairs(const void* hidden_bf16, int64_t row_stride, int hidden
         if(rc)
             return rc;
     }
+    // (the launch that routes and sorts refuses it as well)
+    PYHIP_REQUIRE(!router.gating || router.n_group >= 0, "moe_forward: n_group=%d (0 groups = softmax router)", router.n_group);
     if(router.gating && unsorted)
         rc = router.n_group > 0 ? pyhip_moe_topk_grouped_sigmoid(router.gating, tokens, experts, topk, router.n_group, router.topk_group,
                                                                  router.renormalize, topk_weights, topk_ids, stream)

@@ -1,0 +1,25 @@
+"""What the layer call refuses, and that it does so before it launches anything: the pointers here are no memory."""
+import sys
+
+import pytest
+import torch
+
+from pyhip_amd import _lib, fused_moe  # noqa: F401
+
+pytestmark = pytest.mark.skipif(torch.cuda.is_available(), reason="no pointers like these where a launch could follow")
+
+
+def _call(T, k, E, H, I, rows, w4a16, stride=None, cols=0, pad=0, gating=0, n_group=0, topk_group=0):
+    lib, P = _lib.load(), 1 << 20
+    ws = lib.pyhip_moe_forward_workspace_bytes(T, k, E, H, I, rows, w4a16)
+    block = sys.modules["pyhip_amd.fused_moe"]._LAYER_CALL.pack(P, P, P, P, P, 0, 0, gating, P, P, 0, 0, P, P, H if stride is None else stride, ws, cols, 0,
+                                                                T, k, E, H, I, pad, 0, rows, w4a16, 0, 0, n_group, topk_group, 1, 7.0, E)
+    return lib.pyhip_layer_forward(block, None)
+
+
+@pytest.mark.parametrize("T", [1, 8, 200])
+@pytest.mark.parametrize("w4a16", [0, 1])
+def test_negative_group_counts(T, w4a16):
+    """with and without a sort in front of the GEMMs"""
+    with pytest.raises(RuntimeError, match="n_group=-1"):
+        _lib.check(_call(T, 2, 64, 512, 512, 16, w4a16, gating=1 << 20, n_group=-1, topk_group=1), "layer")
