@@ -317,6 +317,14 @@ static bool takes_pairs(int64_t tokens, int topk, int experts, int hidden, int i
                               !w4a16, split_k);
 }
 
+// the rows of hidden states that they take: offsets into them are 32-bit and signed, in bytes
+static bool takes_rows(int64_t tokens, int64_t row_stride) { return row_stride < (1 << 30) && tokens * row_stride < (1 << 30); }
+// ... and with bf16 activations at the true width of a padded layer
+static bool takes_bf16_cols(int64_t tokens, int64_t row_stride, int cols)
+{
+    return takes_rows(tokens, row_stride) && row_stride >= cols && row_stride % 8 == 0 && row_stride < (1 << 24);
+}
+
 // The layer by the kernels of moe_gemm_pairs.hip.  Up to 128 pairs the kernels find their rows themselves
 // and the sort is left out; where pairs rarely share an expert the down GEMM sums the slots and the reduction is left out too: two
 // launches (with the router three) instead of four.  What that saves is the launch on the host (3.3 us each) and the latency chain of the stage
@@ -442,10 +450,8 @@ static int forward_impl(const void* hidden_bf16, int64_t hidden_row_stride, int 
     PYHIP_REQUIRE(block_m == 16 || block_m == 32 || block_m == 64 ||
                       ((block_m == 128 || block_m == 160 || block_m == 192 || block_m == 256 || block_m == 288) && !w4a16),
                   "moe_forward: block_m=%d (16/32/64, and 128/160/192/256/288 with MXFP4 activations)", block_m);
-    // (32-bit offsets into the hidden states)
-    const bool pairs = takes_pairs(tokens, topk, experts, hidden, inter, block_m, w4a16, split_k) && tokens * hidden_row_stride < (1 << 30);
-    bf16_cols        = bf16_cols && pairs && hidden_cols > 0 && hidden_row_stride >= hidden_cols && hidden_row_stride % 8 == 0 &&
-                hidden_row_stride < (1 << 24);
+    const bool pairs = takes_pairs(tokens, topk, experts, hidden, inter, block_m, w4a16, split_k) && takes_rows(tokens, hidden_row_stride);
+    bf16_cols        = bf16_cols && pairs && hidden_cols > 0 && takes_bf16_cols(tokens, hidden_row_stride, hidden_cols);
     PYHIP_REQUIRE(!w4a16 || hidden_row_stride == hidden || bf16_cols, "moe_forward: the bf16-activation kernels need contiguous rows");
     PYHIP_REQUIRE(hidden_cols == 0 || ((!w4a16 || bf16_cols) && !router.gating && hidden_cols == hidden - hidden_pad && hidden_cols % 32 == 0),
                   "moe_forward: hidden_cols=%d (0, or hidden - hidden_pad, a multiple of 32, with MXFP4 activations)", hidden_cols);
@@ -610,7 +616,9 @@ extern "C" int pyhip_layer_forward(const LayerCall* c, hipStream_t stream)
                         c->swiglu_limit, c->workspace, c->workspace_bytes, stream, true, c->local_experts);
 }
 
-extern "C" int pyhip_layer_takes_cols(int64_t tokens, int topk, int experts, int hidden, int inter, int block_m, int w4a16, int split_k)
+// Whether hidden states at the true width of a padded layer, rows row_stride apart, are taken as they are
+extern "C" int pyhip_layer_takes_cols(int64_t tokens, int topk, int experts, int hidden, int inter, int block_m, int w4a16, int split_k,
+                                      int64_t row_stride)
 {
-    return !w4a16 || takes_pairs(tokens, topk, experts, hidden, inter, block_m, w4a16, split_k);
+    return !w4a16 || (takes_pairs(tokens, topk, experts, hidden, inter, block_m, w4a16, split_k) && takes_bf16_cols(tokens, row_stride, 0));
 }

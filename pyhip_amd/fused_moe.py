@@ -146,8 +146,8 @@ _LAYER_CALL = struct.Struct("<14Q2q16ifi")
 
 
 @functools.lru_cache(maxsize=512)
-def _w4a16_takes_cols(tokens, topk, experts, hidden, inter, block_m, splitk):
-    return bool(_lib.load().pyhip_layer_takes_cols(tokens, topk, experts, hidden, inter, block_m, 1, splitk))
+def _w4a16_takes_cols(tokens, topk, experts, hidden, inter, block_m, splitk, row_stride):
+    return bool(_lib.load().pyhip_layer_takes_cols(tokens, topk, experts, hidden, inter, block_m, 1, splitk, row_stride))
 
 
 def act_quant_mxfp4(x, rows_limit=None):
@@ -312,7 +312,7 @@ def fused_moe(
         cols = H - hidden_pad
         if not (one_call and cols % 32 == 0 and hidden_states.stride(1) == 1 and hidden_states.stride(0) >= cols
                 and hidden_states.stride(0) % 8 == 0 and hidden_states.data_ptr() % 16 == 0
-                and (not w4a16 or (hidden_states.stride(0) < 1 << 24 and _w4a16_takes_cols(T, k, global_E, H, I, int(bm), int(splitk))))):
+                and (not w4a16 or _w4a16_takes_cols(T, k, global_E, H, I, int(bm), int(splitk), hidden_states.stride(0)))):
             cols = 0
             hidden_states = torch.nn.functional.pad(hidden_states, (0, hidden_pad))
     if one_call:

@@ -23,3 +23,13 @@ def test_negative_group_counts(T, w4a16):
     """with and without a sort in front of the GEMMs"""
     with pytest.raises(RuntimeError, match="n_group=-1"):
         _lib.check(_call(T, 2, 64, 512, 512, 16, w4a16, gating=1 << 20, n_group=-1, topk_group=1), "layer")
+
+
+@pytest.mark.parametrize("T,stride", [(64, 2 ** 24 - 8), (65, 2 ** 24 - 8), (64, 2 ** 24), (127, 2 ** 23 + 65536), (128, 2 ** 23), (1, 2 ** 24), (1, 960)])
+def test_rows_at_the_true_width_are_asked_for_where_they_are_taken(T, stride):
+    """bf16 activations of a padded layer: what the host is told about a row stride is what the call does with it"""
+    sizes = (T, 1, 8, 1024, 512, 16, 1, 0)
+    told = _lib.load().pyhip_layer_takes_cols(*sizes, stride)
+    with pytest.raises(RuntimeError) as e:
+        _lib.check(_call(T, 1, 8, 1024, 512, 16, 1, stride=stride, cols=960, pad=64), "layer")
+    assert told == ("launch failed" in str(e.value)) != ("contiguous rows" in str(e.value))
