@@ -13,6 +13,7 @@ Pipeline (all launches on the current torch stream, no host synchronisation):
 reference runs for few tokens (src/contrib/moe.py:362-787); ``method="a4w4"`` forces the MXFP4-activation path;
 ``method="auto"`` takes w4a16 for the very smallest calls (see ``pick_w4a16``) and a4w4 above.
 """
+import ctypes
 import functools
 import struct
 
@@ -141,6 +142,11 @@ def _ask_plan(tokens, topk, experts, hidden, inter, method, block_m, local_exper
 _remembered_plan = functools.lru_cache(maxsize=512)(_ask_plan)
 
 
+def _swiglu_limit(limit):
+    """as the kernels get it: a limit past float32 (no limit, in a caller's mind) is infinite, where ``struct`` would refuse it"""
+    return ctypes.c_float(limit).value if limit else 7.0
+
+
 #: struct LayerCall of csrc/moe_forward.hip: pointers, row stride and workspace bytes, sizes and options, the SwiGLU limit
 _LAYER_CALL = struct.Struct("<14Q2q16ifi")
 
@@ -246,7 +252,7 @@ def fused_moe(
         _refuse_options(hidden_states, activation, quant_type, doweight_stage1, w1_scale, w2_scale, a1_scale, a2_scale, splitk, out_dtype,
                         method, topk_reduce, operand_staging)
     act = 1 if activation == ActivationType.Swiglu else 0
-    limit = float(swiglu_limit) if swiglu_limit else 7.0
+    limit = _swiglu_limit(swiglu_limit)
 
     # weights in the plain layout (no ``is_shuffled`` mark) are re-tiled once; the scales always come e8m0-shuffled,
     # as the reference passes them (tests/contrib/moe/test_moe.py:167-189)
@@ -471,7 +477,7 @@ def fused_moe_routed(hidden_states, w1, w2, gating_output, topk, renormalize=Tru
     lib = _lib.load()
     _require(activation in (ActivationType.Silu, ActivationType.Swiglu), "SiLU- or SwiGLU-gated experts only")
     act = 1 if activation == ActivationType.Swiglu else 0
-    limit = float(swiglu_limit) if swiglu_limit else 7.0
+    limit = _swiglu_limit(swiglu_limit)
     _require(w1_scale is not None and w2_scale is not None, "w1_scale and w2_scale (e8m0, shuffled) are required")
     _require(hidden_states.is_cuda and hidden_states.dtype == torch.bfloat16 and hidden_states.dim() == 2,
              "hidden_states must be a bf16 matrix on the GPU", TypeError)

@@ -41,3 +41,14 @@ def test_row_block_of_any_integer_type(method):
     for v in (32.0, "32"):
         with pytest.raises((TypeError, ctypes.ArgumentError)):
             plan(*sizes, v)
+
+
+@pytest.mark.parametrize("limit,want", [(None, 7.0), (0, 7.0), (3, 3.0), (0.1, np.float32(0.1)), (1e39, float("inf")), (sys.float_info.max, float("inf")),
+                                        (float("inf"), float("inf")), (np.float32(2.5), 2.5), (torch.tensor(5.0), 5.0)])
+def test_swiglu_limit_of_any_size(limit, want):
+    """limits past float32 are taken, as infinity, also where the call goes over as one packed block"""
+    import pyhip_amd.fused_moe  # noqa: F401
+    m = sys.modules["pyhip_amd.fused_moe"]
+    got = m._swiglu_limit(limit)
+    assert got == want
+    assert m._LAYER_CALL.unpack(m._LAYER_CALL.pack(*[0] * 32, got, 8))[-2] == want
