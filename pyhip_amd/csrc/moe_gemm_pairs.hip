@@ -1,6 +1,6 @@
 // The layer call's GEMMs in blocks of 16 rows (MXFP4 activations: or 32 or 64): few tokens, so the call is a weight stream and a chain of launches.  With bf16
 // activations the arithmetic (and with it every bit of the result) is that of moe_gemm_w4a16.hip, with MXFP4 ones that of
-// moe_gemm_mxfp4.hip; their entry points serve callers that run the stages one by one.  What is different is what a call of 20-100 us spends beside its weights:
+// moe_gemm_mxfp4.hip but for the order of the sums (see pairs_tile); their entry points serve callers that run the stages one by one.  What is different is what a call of 20-100 us spends beside its weights:
 //   * Up to 128 pairs (token, slot) there is no sort: every wave reads the routing, one or two pairs to a lane, and finds its block's
 //     expert and rows with a few ballots (find_block).
 //   * Activations come at their own row pitch and width, and neither the padding rows nor the padding columns of the weights
@@ -183,7 +183,9 @@ __device__ __forceinline__ v4f mfma_fp4(const v4i& w, int ws, const v4i& a, int 
 // NB K-steps of operands are in flight; a register set is refilled as soon as its MFMAs are issued.
 // ACT: the activations are BF16 (their products with the weights expanded to bf16), or MXFP4, quantised by whoever wrote them (QUANTISED)
 // or on the way to the matrix cores (TO_FP4: 40 instructions a K-step, where expanding the weights takes 64).  With MXFP4 the products are
-// multiples of powers of two, which 32-bit sums hold exactly in whatever order: the bits of moe_gemm_mxfp4.hip.  Its gate_up GEMM
+// multiples of powers of two.  While the block scales along a row span a few bits, as those of N(0, 1) data do, 32-bit sums hold them exactly
+// in whatever order, and the bits are those of moe_gemm_mxfp4.hip; with channels that stand far out (factors of 1000 between blocks) four
+// partial sums and one chain are rounded at different places, and differ in the last bits.  The gate_up GEMM
 // quantises its result as that one does: a workgroup's 32 channels are one MX block of a row, which wave 0 finishes.
 enum { BF16, TO_FP4, QUANTISED };
 template <int STAGE, int SPLIT, int ACT, bool STAGED, int BT, int MT>
@@ -731,8 +733,8 @@ static int64_t block_bound(int64_t rows, int64_t n_blk, int experts)
     return experts + rows / 16 < b ? experts + rows / 16 : b;
 }
 
-// bf16 activations: the K split of the sorted entry points, so that the sums are theirs.  MXFP4 ones, whose sums have no order: always
-// four waves to a tile (without a split, DeepSeek-V3 shape, 16 tokens 372.7 / 354.4 us, 60 tokens 767 / 736)
+// bf16 activations: the K split of the sorted entry points, so that the sums are theirs.  MXFP4 ones, whose sums are exact or as good in either
+// order: always four waves to a tile (without a split, DeepSeek-V3 shape, 16 tokens 372.7 / 354.4 us, 60 tokens 767 / 736)
 static int pairs_split(int fp4, int stage, int64_t tiles, int K, int split_k)
 {
     return fp4 ? 4 : w4a16_split(stage, 16, tiles, K, split_k);

@@ -1,6 +1,7 @@
 """The layer call in 16-row blocks with bf16 activations, or with MXFP4 ones and few rows per expert (kernels of its own, without a sort up to 64 or 128
 pairs and without a reduction where pairs rarely share an expert), against the step-by-step path.  With bf16 activations the arithmetic
-and its order are the same; with MXFP4 ones the sums are exact in any order: the same bits."""
+and its order are the same; with MXFP4 ones the sums of such data are exact in any order: the same bits.  Data whose block scales lie far
+apart are compared within the rounding of two orders of summation."""
 import pytest
 import torch
 
@@ -178,3 +179,44 @@ def test_mask_with_more_entries_than_matrices(T, k, method, rows):
                     expert_mask=torch.ones(E, dtype=torch.int32, device="cuda"))
     held = (ids < here).all(dim=1).cuda()
     assert held.sum() == T - (1 if T <= 2 else 2) and torch.equal(got[held], want[held])
+
+
+@pytest.mark.parametrize("T,E,rows", [
+    (6, 4, 16),          # unsorted
+    (36, 10, 16),        # sorted
+    (40, 9, 32),
+    (40, 4, 64),
+])
+def test_wide_block_scales_equal_the_stages_within_rounding(T, E, rows):
+    """MXFP4 activations whose block scales lie 2^20 apart along a row of the down GEMM (rows of w1 scaled by 2^-10, 1 and 2^10, 32 at a time;
+    the gate_up GEMM's sums stay exact, so both paths have the same intermediate).  There n = K / 32 partial sums of a magnitude of at
+    most S = sum |a2 * w2| are added in two orders: at most 2 n 2^-24 S between them, the routing weight and the bf16 rounding of the
+    slot on top (half an ulp, 2^-9 of the value, on either side)."""
+    import numpy as np
+    from oracle import mxfp4
+    from pyhip_amd import fused_moe
+    H, I, k = 512, 2048, 2
+    L = cases.make_layer("", T, seed=T, E=E, k=k, H=H, I=I, router="softmax")
+    up = L.w1s.reshape(E, 2, I // 32, 32, H // 32)[:, 1]           # (a view: the up halves' scale bytes)
+    up[:, 0::3] -= 10
+    up[:, 2::3] += 10
+    w1, w1s, w2, w2s = cases.device_weights(L)
+    args = (L.hidden.cuda(), w1, w2, torch.from_numpy(L.topk_w).cuda(), torch.from_numpy(L.topk_ids).cuda())
+    kw = dict(w1_scale=w1s, w2_scale=w2s, method="a4w4", block_size_M=rows, dtype=torch.float32)
+    print("few pairs, wide scales", T, E, rows, flush=True)
+    want, parts = fused_moe(*args, return_parts=True, **kw)
+    _poison(T, k, E, H, I, "a4w4", rows)
+    got = fused_moe(*args, **kw)
+    a2_q, a2_s = parts["a2_q"].cpu().numpy(), cases.untranspose_act_scales(parts["a2_s"].cpu().numpy(), I)
+    ids = parts["sorted_ids"].cpu().numpy().astype(np.int64)[:int(parts["num_valid_ids"][0])] & 0xFFFFFFFF
+    bound = np.zeros((T, H))
+    for p, (tok, slot) in enumerate(zip(ids & 0xFFFFFF, ids >> 24)):
+        if tok < T and slot < k:
+            e, a2 = L.topk_ids[tok, slot], mxfp4.dequantize_mxfp4(a2_q[p], a2_s[p])
+            S = np.abs(mxfp4.dequantize_mxfp4(L.w2q[e], L.w2s[e])).astype(np.float64) @ np.abs(a2).astype(np.float64)
+            bound[tok] += 2 * (I // 32) * 2.0 ** -24 * S * L.topk_w[tok, slot]
+    bound += 2.0 ** -8 * parts["out3"].float().abs().sum(dim=1).cpu().numpy()
+    diff = (got - want).abs().cpu().numpy()
+    print("  differ:", (diff > 0).mean(), "largest share of the bound:", (diff / bound).max(), flush=True)
+    assert np.isfinite(diff).all() and (diff <= bound).all(), (diff / bound).max()
+    assert want.abs().mean() > 100 * bound.mean()                  # (the bound says something)
