@@ -294,9 +294,12 @@ static int rows_per_expert_max(int experts, int block_m)
 {
     return experts < 32 ? (block_m == 16 ? 8 : block_m == 32 ? 16 : 24) : (block_m == 16 ? 4 : 12);
 }
-// Whether they find their rows themselves, in blocks of 16: up to a pair to a lane; with two, where that costs every workgroup of the gate_up
-// GEMM a microsecond more, if all of its workgroups run at once (and the list of blocks fits where a sort into 32 rows would put its own).
-// Layer, us, sorted / this: 8 experts, 1024 x 512, top-2, 40 tokens 22.0 / 16.8, 64 tokens 20.0 / 17.8; 12, 1024 x 1024, 50 tokens 22.1 / 18.2.
+// Whether they find their rows themselves, in blocks of 16: up to a pair to a lane; with two, which costs every workgroup of the gate_up
+// GEMM more, if all of its workgroups run at once (and the list of blocks fits where a sort into 32 rows would put its own).
+// Layer, us, sorted / this: 8 experts, 1024 x 512, top-2, 40 tokens 21.3 / 17.9, 64 tokens 21.2 / 17.7; 12, 1024 x 1024, top-1, 100 tokens 22.9 /
+// 19.0.  With more workgroups it goes either way: DeepSeek-V3 shape, 16 tokens 356.0 / 347.5; 96 experts, top-4, 6272 x 1920, 30 tokens 204.6 / 198.2;
+// 60, 2048 x 1408, 32 tokens 49.2 / 47.0; gpt-oss shape, 32 tokens 167.9 / 170.6; Qwen3 shape, 16 tokens 65.9 / 68.3; Mixtral shape, 50 tokens, bf16
+// activations 121.4 / 131.4: left to the sort.
 static bool leaves_sort_out(int64_t tokens, int topk, int experts, int inter, int block_m, int w4a16)
 {
     const int64_t pairs = tokens * topk, blocks = pairs < experts + pairs / 16 ? pairs : experts + pairs / 16;

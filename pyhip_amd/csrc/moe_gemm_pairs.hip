@@ -47,9 +47,9 @@ __device__ __forceinline__ int local_expert(int e, const int* mask, int lane)
 // bit of the expert number; every 16th of them, in pair order, starts a block, and blocks are numbered by the pair that starts them.
 // -> expert (local id) and, in lane r of each 16, the pair of the block's row r (-1: no row)
 // blocks: how many there are.  TWO: more than 64 pairs.  (The sort's launch in front of the GEMMs costs the host 3.3 us and the device 5-7.  This
-// costs every workgroup 0.3 us, and 1.2 us with two pairs to a lane: 128 pairs in both GEMMs of the DeepSeek-V3 shape 356 -> 426 us, of
-// the tiny layer 20.9 -> 18.1.  So gate_up leaves what it has found to the down GEMM: Qwen3 shape, 8 tokens, 47.3 -> 46.7; Mixtral shape, 29 tokens,
-// 121.2 -> 119.9; 96 experts, top-4, 16 tokens 61.7 -> 60.0.)
+// costs every workgroup a few hundred ns, more with two pairs to a lane: see leaves_sort_out in moe_forward.hip for where that pays.  So
+// gate_up leaves what it has found to the down GEMM: Qwen3 shape, 8 tokens, 47.3 -> 46.7; Mixtral shape, 29 tokens, 121.2 -> 119.9; 96 experts, top-4, 16
+// tokens 61.7 -> 60.0.)
 template <bool TWO>
 __device__ __forceinline__ bool find_block(const PairArgs& g, int m_blk, int lane, int& e, int& pair, int& blocks)
 {
@@ -98,45 +98,39 @@ __device__ __forceinline__ bool find_block(const PairArgs& g, int m_blk, int lan
         hits[h]          = __ballot(start && blocks + __builtin_popcountll(starts & below) == m_blk);
         blocks += __builtin_popcountll(starts);
     }
-#pragma unroll
-    for(int h = 0; h < H; h++)
+    // (straight on from here: a loop over h with a way out in it is left a loop, and same[][] then lies in scratch memory to be indexed)
+    const bool second = TWO && !hits[0];      // which word the pair that starts the block is in
+    const u64 hit     = second ? hits[H - 1] : hits[0];
+    if(!hit)
+        return false;
+    const int lead = __builtin_ctzll(hit);
+    auto of_lead = [&](u64 v) __attribute__((always_inline)) -> u64 {
+        return (u64)(u32)__builtin_amdgcn_readlane((int)v, lead) | (u64)(u32)__builtin_amdgcn_readlane((int)(v >> 32), lead) << 32;
+    };
+    // the pairs of its expert from that one on
+    const u64 from = ~((1ull << lead) - 1ull);
+    u64 row0 = second ? 0ull : of_lead(same[0][0]) & from;
+    u64 row1 = !TWO ? 0ull : second ? of_lead(same[H - 1][H - 1]) & from : of_lead(same[0][H - 1]);
+    e    = local_expert(__builtin_amdgcn_readlane(second ? id[H - 1] : id[0], lead), g.mask, lane);
+    pair = -1;
+    for(int r = 0; r < 16; r++)
     {
-        const u64 hit = hits[h];
-        if(!hit)
-            continue;
-        const int lead = __builtin_ctzll(hit);
-        u64 rows[H];
-#pragma unroll
-        for(int i = 0; i < H; i++)
+        int p = -1;
+        if(row0)
         {
-            rows[i] = i < h ? 0ull
-                            : (u64)(u32)__builtin_amdgcn_readlane((int)same[h][i], lead) |
-                                  (u64)(u32)__builtin_amdgcn_readlane((int)(same[h][i] >> 32), lead) << 32;
-            if(i == h)
-                rows[i] &= ~((1ull << lead) - 1ull);
+            p = __builtin_ctzll(row0);
+            row0 &= row0 - 1ull;
         }
-        e    = local_expert(__builtin_amdgcn_readlane(id[h], lead), g.mask, lane);
-        pair = -1;
-        for(int r = 0; r < 16; r++)
+        else if(row1)
         {
-            int p = -1;
-            if(rows[0])
-            {
-                p = __builtin_ctzll(rows[0]);
-                rows[0] &= rows[0] - 1ull;
-            }
-            else if(TWO && rows[H - 1])
-            {
-                p = WAVE + __builtin_ctzll(rows[H - 1]);
-                rows[H - 1] &= rows[H - 1] - 1ull;
-            }
-            if(p < 0)
-                break;
-            pair = (lane & 15) == r ? p : pair;
+            p = WAVE + __builtin_ctzll(row1);
+            row1 &= row1 - 1ull;
         }
-        return true;
+        if(p < 0)
+            break;
+        pair = (lane & 15) == r ? p : pair;
     }
-    return false;
+    return true;
 }
 
 // the lane's four biases of channels c .. c + 3 (element-aligned tensors: one by one)
@@ -471,7 +465,7 @@ __global__ void __launch_bounds__(W4A16_THREADS, ACT == BF16 && !STAGED ? 4 : BT
     for(int m = 0; m < BT; m++)
     {
         arow[m] = -1;
-        orow[m] = 0;
+        orow[m] = -1;      // (as arow: the same registers in the sorted down GEMM, whose 64-row blocks would spill two otherwise)
         rw[m]   = 0.f;
     }
     if(BT == 1 && g.ids)

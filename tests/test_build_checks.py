@@ -72,6 +72,15 @@ def test_compiler_never_touches_accumulation_registers_of_fixed_tiles(gemm_asm):
         assert m and int(m.group(1)) == 0, (name, "spills")
 
 
+def test_pairs_kernels_use_no_scratch(tmp_path_factory):
+    """neither for spilled registers nor for arrays: a private segment costs every workgroup its set-up, also where nothing is stored"""
+    text, kernels = _device_asm(tmp_path_factory, os.path.join(ROOT, "pyhip_amd", "csrc", "moe_gemm_pairs.hip"),
+                                r"^(_Z\w*(?:moe_gemm_pairs_kernel|moe_pairs_down_sum_kernel)\w*):[^\n]*\n(.*?)\.end_amdhsa_kernel")
+    assert len(kernels) == 18
+    for name, body in kernels:
+        assert re.search(r"\.amdhsa_private_segment_fixed_size 0\n", body) and not re.search(r"^\s*scratch_", body, re.M), name
+
+
 def test_compiler_never_uses_m0(gemm_asm):
     """The LDS-DMA helpers set M0 by hand inside inline assembly.  M0 is reserved for the compiler (a clobber on it
     is not honoured), so the helpers are only sound while no instruction of the compiler's own reads or writes M0
