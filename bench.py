@@ -75,7 +75,7 @@ def parse():
                     help="only run the MFMA / HBM-stream probe (six variants of the 288-row GEMM's inner loop) and print "
                          "matrix-pipeline duty and TB/s of each")
     ap.add_argument("--print-kernel-sources-digest", action="store_true",
-                    help="print the digest that profiles/fused_moe_dsv3_hbm_traffic.txt records next to its counters, and exit")
+                    help="print the digests that profiles/fused_moe_dsv3_hbm_traffic.txt records next to its counters, and exit")
     return ap.parse_args()
 
 
@@ -106,7 +106,7 @@ def weight_copies(torch, W, work):
 def time_point(torch, fused_moe, W, shape, tokens, steps, warmup, block_m, method="auto"):
     """-> dict with wall-clock ms over exactly `steps` calls, and median / IQR over event-timed batches; only the
     one-call product path runs inside the timed regions"""
-    from pyhip_amd import workloads
+    from pyhip_amd import _lib, workloads
     from pyhip_amd.fused_moe import _plan
     hidden, topk_w, topk_ids = workloads.make_inputs(shape, tokens)
     if W["hidden_pad"]:      # padded shapes (gpt-oss): activations at the padded width, as the reference passes them
@@ -155,15 +155,18 @@ def time_point(torch, fused_moe, W, shape, tokens, steps, warmup, block_m, metho
     cfg = workloads.SHAPES[shape]
     Hp = cfg["H"] + W["hidden_pad"]
     # (what the call itself chooses)
-    w4a16, bm, _ = _plan(tokens, cfg["k"], cfg["E"], Hp, cfg["I"] + W["intermediate_pad"], method, block_m or None, cfg["E"])
+    Ip = cfg["I"] + W["intermediate_pad"]
+    w4a16, bm, _ = _plan(tokens, cfg["k"], cfg["E"], Hp, Ip, method, block_m or None, cfg["E"])
+    pairs = bool(_lib.load().pyhip_layer_takes_pairs(tokens, cfg["k"], cfg["E"], Hp, Ip, bm, w4a16, 0))
     return dict(wall_ms=wall_ms, median_ms=q(0.5), q1_ms=q(0.25), q3_ms=q(0.75), work=work, hidden=hidden,
                 topk_w=topk_w, topk_ids=topk_ids, out=out, method="w4a16" if w4a16 else "a4w4",
-                block_m=bm, weight_copies=len(sets), calls_per_batch=reps)
+                block_m=bm, kernels="few tokens" if pairs else "step by step", weight_copies=len(sets), calls_per_batch=reps)
 
 
 def stage_pass(torch, fused_moe, W, res, block_m, method, passes=8):
     """average duration of each launch group of the step-by-step path in blocks of block_m rows, from events on the launch
-    stream; untimed (not part of any ms_per_step)"""
+    stream; untimed (not part of any ms_per_step).  Calls of few tokens run other GEMM kernels than these: the record of a point says
+    which the timed call runs ("kernels")"""
     kw = call_kwargs(W, block_m, method)
     events = []
     for _ in range(2):
@@ -293,23 +296,25 @@ def graph_replay_ms(torch, fused_moe, W, res, steps, block_m, method="auto"):
     return (time.perf_counter() - t0) * 1e3 / steps
 
 
-KERNEL_SOURCES = ("moe_gemm_mxfp4.hip", "gemm_device.h", "common.h", "quant_device.h")
+#: by the line of the counter summary that holds their digest: the sources of the persistent GEMMs, and of the layer call's for few tokens
+KERNEL_SOURCES = {"kernel_sources_sha256": ("moe_gemm_mxfp4.hip", "gemm_device.h", "common.h", "quant_device.h"),
+                  "pairs_kernel_sources_sha256": ("moe_gemm_pairs.hip", "moe_gemm_pairs.h", "w4a16_device.h", "common.h", "quant_device.h")}
 
 
-def kernel_sources_digest():
+def kernel_sources_digest(line="kernel_sources_sha256"):
     """sha256 over the sources the measured GEMM kernels are compiled from"""
     import hashlib
     h = hashlib.sha256()
-    for name in KERNEL_SOURCES:
+    for name in KERNEL_SOURCES[line]:
         with open(os.path.join(ROOT, "pyhip_amd", "csrc", name), "rb") as f:
             h.update(f.read())
     return h.hexdigest()
 
 
-def measured_traffic(kernel_key):
+def measured_traffic(kernel_key, line="kernel_sources_sha256"):
     """HBM-side bytes per launch of a kernel from the committed counter summary (lines of the form
     `traffic_bytes_per_launch <key> <bytes>`, written when the counters were collected, next to a line
-    `kernel_sources_sha256 <digest>` of the kernel sources they were collected with).  None when the summary has no
+    `kernel_sources_sha256 <digest>` (`line`) of the kernel sources they were collected with).  None when the summary has no
     such line, or when the kernel sources have changed since: a counter reading of other code is not reported."""
     try:
         text = open(TRAFFIC_FILE).read()
@@ -317,8 +322,8 @@ def measured_traffic(kernel_key):
         return None, None
     m = re.search(r"^traffic_bytes_per_launch\s+%s\s+([0-9.eE+]+)" % re.escape(kernel_key), text, re.M)
     c = re.search(r"^collected_at\s+(.+)$", text, re.M)
-    d = re.search(r"^kernel_sources_sha256\s+([0-9a-f]{64})", text, re.M)
-    if m is None or d is None or d.group(1) != kernel_sources_digest():
+    d = re.search(r"^%s\s+([0-9a-f]{64})" % line, text, re.M)
+    if m is None or d is None or d.group(1) != kernel_sources_digest(line):
         return None, None
     return float(m.group(1)), (c.group(1).strip() if c else None)
 
@@ -374,7 +379,7 @@ def point_record(shape, tokens, r):
     w, ms = r["work"], r["median_ms"]
     tfl = w["flops"] / (ms * 1e-3) / 1e12
     gbs = w["bytes"] / (ms * 1e-3) / 1e9
-    return {"shape": shape, "tokens": tokens, "method": r["method"], "block_m": r["block_m"], "experts_hit": w["e_hit"],
+    return {"shape": shape, "tokens": tokens, "method": r["method"], "block_m": r["block_m"], "kernels": r["kernels"], "experts_hit": w["e_hit"],
             "ms_median": round(ms, 4), "ms_iqr": [round(r["q1_ms"], 4), round(r["q3_ms"], 4)],
             "ms_wall_mean": round(r["wall_ms"], 4), "tflops": round(tfl, 1),
             "frac_of_mfma_peak": round(tfl / PEAK_MFMA_FP4_TFLOPS, 4), "hbm_gbps": round(gbs, 1),
@@ -384,7 +389,8 @@ def point_record(shape, tokens, r):
 def main():
     a = parse()
     if a.print_kernel_sources_digest:
-        print(kernel_sources_digest())
+        for line in KERNEL_SOURCES:
+            print(line, kernel_sources_digest(line))
         return
     if a.frontier:
         import torch
@@ -462,7 +468,20 @@ def main():
     dec_gbps = dw["bytes"] / (dec["median_ms"] * 1e-3) / 1e9
     dg1_ms = dec_stage["gemm1"]
     traffic, collected = measured_traffic("gate_up_%s_T%d" % (a.shape, a.tokens))
-    dtraffic, _ = measured_traffic("gate_up_%s_T%d" % (a.shape, a.decode_tokens))
+    if dec["kernels"] == "few tokens":
+        # what the call runs is not what the stage pass times: the whole call against its bytes
+        both = [measured_traffic("%s_pairs_%s_T%d" % (k, a.shape, a.decode_tokens), "pairs_kernel_sources_sha256")[0] for k in ("gate_up", "down")]
+        droof = {"kernel": "whole call: moe_gemm_pairs_kernel<1,..> (gate_up) and <2,..> (down, %s activations), sort and reduction"
+                 % ("bf16" if dec["method"] == "w4a16" else "MXFP4"), "bound": "hbm", "achieved": round(dec_gbps, 1), "peak": PEAK_HBM_GBPS,
+                 "unit": "GB/s", "frac": round(dec_gbps / PEAK_HBM_GBPS, 4),
+                 "traffic": sum(both) if None not in both else None, "traffic_of": "both GEMM launches", "avg_call_ms": round(dec["median_ms"], 4)}
+    else:
+        dtraffic, _ = measured_traffic("gate_up_%s_T%d" % (a.shape, a.decode_tokens))
+        droof = {"kernel": "moe_gemm_w4a16_kernel<1,1> (gate_up, bf16 activations)" if dec["method"] == "w4a16"
+                 else "moe_gemm_mxfp4_kernel<1,*> (gate_up, MXFP4 activations)", "bound": "hbm",
+                 "achieved": round(dw["bytes_stage1"] / (dg1_ms * 1e-3) / 1e9, 1), "peak": PEAK_HBM_GBPS, "unit": "GB/s",
+                 "frac": round(dw["bytes_stage1"] / (dg1_ms * 1e-3) / 1e9 / PEAK_HBM_GBPS, 4),
+                 "traffic": dtraffic, "avg_launch_ms": round(dg1_ms, 4)}
     out = {
         "metric": "MXFP4 fused-MoE TFLOP/s (DeepSeek-V3 routed-expert layer, %d tokens); decode-size HBM GB/s in 'decode'"
                   % a.tokens if a.shape == "dsv3" else "MXFP4 fused-MoE TFLOP/s (%s, %d tokens)" % (a.shape, a.tokens),
@@ -491,12 +510,7 @@ def main():
                    "tflops": round(dw["flops"] / (dec["median_ms"] * 1e-3) / 1e12, 2),
                    "stage_ms_untimed_pass": {k: round(v, 4) for k, v in dec_stage.items()},
                    "graph_replay_ms_per_step": round(dec_graph_ms, 4),
-                   "roofline": {"kernel": "moe_gemm_w4a16_kernel<1,1> (gate_up, bf16 activations)" if dec["method"] == "w4a16"
-                                else "moe_gemm_mxfp4_kernel<1,1,0,true> (gate_up, MXFP4 activations)", "bound": "hbm",
-                                "achieved": round(dw["bytes_stage1"] / (dg1_ms * 1e-3) / 1e9, 1), "peak": PEAK_HBM_GBPS,
-                                "unit": "GB/s",
-                                "frac": round(dw["bytes_stage1"] / (dg1_ms * 1e-3) / 1e9 / PEAK_HBM_GBPS, 4),
-                                "traffic": dtraffic, "avg_launch_ms": round(dg1_ms, 4)}},
+                   "kernels": dec["kernels"], "roofline": droof},
         "decode_other_method": {"tokens": a.decode_tokens, "method": dec4["method"], "ms_per_step": round(dec4["median_ms"], 4),
                         "hbm_gbps": round(dw["bytes"] / (dec4["median_ms"] * 1e-3) / 1e9, 1),
                         "frac_of_hbm_peak": round(dw["bytes"] / (dec4["median_ms"] * 1e-3) / 1e9 / PEAK_HBM_GBPS, 4)},

@@ -619,6 +619,12 @@ extern "C" int pyhip_layer_forward(const LayerCall* c, hipStream_t stream)
                         c->swiglu_limit, c->workspace, c->workspace_bytes, stream, true, c->local_experts);
 }
 
+// Whether a call of these sizes runs the kernels of moe_gemm_pairs.hip (for whoever reports on it)
+extern "C" int pyhip_layer_takes_pairs(int64_t tokens, int topk, int experts, int hidden, int inter, int block_m, int w4a16, int split_k)
+{
+    return takes_pairs(tokens, topk, experts, hidden, inter, block_m, w4a16, split_k);
+}
+
 // Whether hidden states at the true width of a padded layer, rows row_stride apart, are taken as they are
 extern "C" int pyhip_layer_takes_cols(int64_t tokens, int topk, int experts, int hidden, int inter, int block_m, int w4a16, int split_k,
                                       int64_t row_stride)
