@@ -553,7 +553,7 @@ __global__ void __launch_bounds__(W4A16_THREADS, ACT == BF16 && !STAGED ? 4 : BT
 // Bound: the weight stream, less well fed than by expert (a wave brings the activations of one row for 1, 2 or 4 KB of weights),
 // against the reduction's launch.  Layer, us, down by expert + reduction / NR = 1 / 2 / 4: gpt-oss shape, 1 token 21.9 / 19.3 / 20.8 /
 // 24.0, 2 tokens 26.8 / 28.2 / 25.1 / 28.3, 4 tokens 41.7 / 50.3 / 43.1 / 40.5; DeepSeek-V3 shape, 1 token 37.2 / 39.8 / 35.3 / 38.7, 2 tokens
-// 61.2 / 71.0 / 61.9 / 58.9, 3 tokens 87.7 / 102 / 89.4 / 91.8, 4 tokens 111.5 / 128 / 115.6 / 111.2; 256 experts, top-1, 5120 x 1536,
+// 61.2 / 71.0 / 61.9 / 58.9, 3 tokens 87.7 / 104.5 / 89.8 / 89.9, 4 tokens 111.5 / 128 / 115.6 / 111.2; 256 experts, top-1, 5120 x 1536,
 // 30 tokens 62.1 / 67.0 / 59.9 / 56.7.  (Sixteen waves, every slot on waves of its own: 113 us at 3 tokens of the DeepSeek-V3 shape.)
 template <int NR>
 __global__ void __launch_bounds__(512) moe_pairs_down_sum_kernel(PairArgs g)
@@ -852,9 +852,11 @@ int pyhip_pairs_down_sum(PairArgs g, int64_t rows, int64_t n_blk, int split_k, h
     const int rc = prepare("moe_pairs_down_sum", g, rows, blocks, g.N / 64);
     if(rc)
         return rc;
-    // as wide a tile as still gives half of the CUs a workgroup (and not, where a workgroup has many slots, every third CU a second one)
+    // As wide a tile as still gives half of the CUs a workgroup.  Layer, us, NR = 2 / 4, by at4: 256 experts, top-8, 7168 x 2048 224: 62.9 / 58.9, 336: 89.8 /
+    // 89.9, 448: 118.1 / 110.4; 3584 x 1024 224: 35.6 / 33.4; top-6, 3584 x 2048 280: 59.5 / 60.3, 4608 x 1024 360: 42.7 / 40.1; 512, top-8, 2560 x 1024 320:
+    // 49.8 / 48.5; 256, top-8, 6144 x 1536 288: 65.3 / 65.8
     const int64_t at4 = (int64_t)g.T * (g.N / 64);
-    const int nr      = at4 >= 140 && !(g.topk > 4 && at4 > 256 && at4 < 400) ? 4 : at4 >= 80 ? 2 : 1;
+    const int nr      = at4 >= 140 ? 4 : at4 >= 80 ? 2 : 1;
     g.n_tiles         = g.N / (16 * nr);
     const dim3 grid((unsigned)(g.T * g.n_tiles)), block((g.topk > 1 ? 2 : 1) * 4 * WAVE);
     if(nr == 4)
