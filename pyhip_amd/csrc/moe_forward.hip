@@ -194,11 +194,19 @@ static const TileCost tile_costs[] = {{16, 1.2, 1.37, 1e9, 0.35}, {32, 1.5, 1.39
                                       {128, 4.5, 2.10, 307, 0.33}, {160, 5.8, 2.27, 284, 0.75}, {192, 6.8, 2.38, 271, 1.05},
                                       {256, 8.6, 2.84, 276, 1.6},  {288, 9.8, 3.15, 273, 2.0}};
 
+static bool takes_pairs(int64_t tokens, int topk, int experts, int hidden, int inter, int block_m, int w4a16, int split_k);
+
 // The tile height of an MXFP4-activation layer call whose sizes are known: the one of pyhip_moe_pick_block_m, which looks at the rows
 // per expert alone, unless that has fewer tiles in the gate_up GEMM than the chip has CUs and 64, 32 or 16 rows are estimated to
 // take 5 % less: lower tiles are more of them, and each is done sooner.  Layer, us: 8 experts, 1024 x 512, top-2, 493 tokens, 160 / 16 rows:
 // 30.2 / 23.7; 1024 tokens, 128 / 32: 30.2 / 27.1; 2208 x 1792, top-1, 446 tokens, 128 / 32: 36.5 / 27.2; 6176 x 512, Zipf, 371 tokens, 128 / 32:
-// 52.3 / 37.1.  Of 556 layers it moves 88, which take 16 % less then; two take more, by 2 and 3 %.
+// 52.3 / 37.1.  The estimate is trusted where lower tiles cannot lose much, else the ladder stays: with few enough of them that all run at
+// once also under a router that makes more (64 rows: 96 in the gate_up GEMM, 160 up to hidden 2048; 16 and 32: 128), or with a short K loop (16 and 32
+// rows: hidden up to 2048, or 2560 where an expert has two blocks and few are here; 64: 1024).  Beyond that it was wrong by up to 40 % (8 experts, 128 / 64
+// rows: 6720 x 2944, Zipf, 216 tokens 68.2 / 95.4; 4576 x 2304, 348 tokens 52.6 / 64.7; 5888 x 2528, 466 tokens, 160 / 64: 66.6 / 80.0; 24 experts, 128 / 32: 4960 x
+// 512, 1153 tokens 57.8 / 67.0; 64 / 32: 1856 x 1024, Zipf, 162 tokens 30.2 / 37.1).  Of 1400 other
+// layers that the rule moves, each under an even and a Zipf router, the calls take 16 % less (geometric mean), and one of 2800 takes more than 3 % more (11:
+// 28 experts, 1920 x 512, top-1, Zipf, 4114 tokens).
 // (With as many tiles as CUs and more the estimate would find other heights too, and is not good enough for it, nor does it know the
 // router: 64 rows instead of 128 cost up to 20 % between 33 and 60 rows per expert, 192 to 288 rows at hidden below 6144 save 14-23 % under
 // even routers and cost 6-18 % under Zipf ones.)
@@ -219,7 +227,8 @@ extern "C" int pyhip_layer_block_m(int64_t tokens, int topk, int experts, int lo
         ladder = 32;
     else if(ladder == 32 && experts >= 32 && est >= 5.0 && hidden >= 3072 && inter % 512 == 0)
         ladder = 64;
-    if(local_experts * expected_blocks(est, ladder) * (inter / 128) >= 256.0)
+    // (the estimate is of the persistent kernels)
+    if(local_experts * expected_blocks(est, ladder) * (inter / 128) >= 256.0 || takes_pairs(tokens, topk, experts, hidden, inter, ladder, 0, 0))
         return ladder;
     auto estimate = [&](const TileCost& c) {
         const double hit = local_experts * (1.0 - exp(-est)), nb = local_experts * expected_blocks(est, c.rows);
@@ -245,7 +254,11 @@ extern "C" int pyhip_layer_block_m(int64_t tokens, int topk, int experts, int lo
             best = estimate(c);
             rows = c.rows;
         }
-    return rows;
+    const double tiles = local_experts * expected_blocks(est, rows) * (inter / 128);
+    const bool short_k = hidden <= 2048 || (hidden <= 2560 && est <= 2.0 * rows && local_experts <= 12);
+    const bool trusted = rows == 64 ? hidden <= 1024 || tiles <= (hidden <= 2048 ? 160.0 : 96.0)
+                                    : tiles <= 128.0 || (short_k && (ladder > 64 || tiles <= 192.0));
+    return trusted ? rows : ladder;
 }
 
 extern "C" int pyhip_moe_pick_w4a16(int64_t tokens, int topk, int experts, int hidden)

@@ -34,3 +34,16 @@ def test_any_sizes_get_a_served_height():
         assert lib.pyhip_layer_block_m(*a) in served, a
     for a in ((0, 2, 8, 8, 1024, 512), (64, 0, 8, 8, 1024, 512), (64, 2, 8, 0, 1024, 512)):
         assert lib.pyhip_layer_block_m(*a) == lib.pyhip_moe_pick_block_m(a[0], a[1], a[2], a[4], 0)
+
+
+@pytest.mark.parametrize("tokens,topk,experts,local,hidden,inter,want", [
+    # fewer tiles than CUs, but a long K loop and more lower tiles than run at once: measured slower by 12 to 40 %
+    (216, 2, 8, 8, 7168, 3072, 128), (377, 2, 12, 12, 4096, 2048, 128), (348, 2, 8, 8, 4608, 2560, 128), (466, 2, 8, 8, 6144, 2560, 160),
+    (193, 2, 8, 8, 4608, 3072, 128), (1153, 2, 24, 24, 5120, 512, 128), (1016, 2, 8, 8, 2560, 1024, 128),
+    # few enough of them
+    (371, 1, 8, 8, 6656, 512, 32),
+    # the few-token kernels serve the ladder's height: the estimate is not of them
+    (83, 2, 8, 8, 1536, 3584, 64), (135, 1, 8, 8, 4096, 1536, 64), (324, 1, 16, 16, 2048, 1024, 64),
+])
+def test_lower_tiles_only_where_they_cannot_lose_much(tokens, topk, experts, local, hidden, inter, want):
+    assert _lib.load().pyhip_layer_block_m(tokens, topk, experts, local, hidden, inter) == want
