@@ -145,6 +145,28 @@ __device__ __forceinline__ u32 mx_scale_byte(u32 am)
     u32 e8 = (u32)(ex > 2 ? ex - 2 : 0);
     return e8 > 254u ? 254u : e8;
 }
+// The gate_up GEMMs' results, packed in pairs as their lanes hold them: lane (r, kb) has channels j * 16 + kb * 4 .. + 3 (j = 0, 1) of row r in
+// d[j].  -> eight consecutive channels of that row, from 0, 16, 8, 24 on in lane rows kb = 0 .. 3: even lane rows then have channels
+// of kb, kb + 1 at j = 0, odd ones those of kb - 1, kb at j = 1
+__device__ __forceinline__ uint4 join_channels8(const u32 (&d)[2][2])
+{
+    typedef unsigned v2u __attribute__((ext_vector_type(2)));
+    const v2u t0 = __builtin_amdgcn_permlane16_swap(d[0][0], d[1][0], false, false);
+    const v2u t1 = __builtin_amdgcn_permlane16_swap(d[0][1], d[1][1], false, false);
+    return make_uint4(t0.x, t1.x, t0.y, t1.y);
+}
+// ... whose 32 channels are one MX block, eight of them in each of the four lane rows: the block's scale byte, by the same steps as in
+// the stand-alone quantiser
+__device__ __forceinline__ u32 mx_scale_of_row(uint4 o)
+{
+    typedef unsigned v2u __attribute__((ext_vector_type(2)));
+    u32 am        = amax15_fold(amax15x2(amax15x2(o.x, o.y), amax15x2(o.z, o.w)));
+    const v2u s16 = __builtin_amdgcn_permlane16_swap(am, am, false, false);
+    am            = s16.x > s16.y ? s16.x : s16.y;
+    const v2u s32 = __builtin_amdgcn_permlane32_swap(am, am, false, false);
+    am            = s32.x > s32.y ? s32.x : s32.y;
+    return mx_scale_byte(am);
+}
 __device__ __forceinline__ int lane_id() { return threadIdx.x & (WAVE - 1); }
 
 // compile-time loop: f(std::integral_constant<int, 0>{}), ..., f(std::integral_constant<int, N-1>{})

@@ -395,7 +395,6 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, int nt, int row
     {
         // lane (r, kb) holds channels j*16 + kb*4 .. +3 (j = 0, 1) of row r.  After one permlane16 swap per
         // packed dword a lane holds 8 consecutive channels: one 16 B store, 64 B contiguous per row and wave.
-        typedef unsigned v2u __attribute__((ext_vector_type(2)));
         uint16_t* out = (uint16_t*)g.out;
         const int chw = nt * 128 + wcol * 32;
         // after the swap: lane rows 0..3 hold channel offsets 0, 16, 8, 24
@@ -433,10 +432,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, int nt, int row
                         d[j][0] = pack_bf16x2(v[0], v[1]);
                         d[j][1] = pack_bf16x2(v[2], v[3]);
                     }
-                    v2u t0 = __builtin_amdgcn_permlane16_swap(d[0][0], d[1][0], false, false);
-                    v2u t1 = __builtin_amdgcn_permlane16_swap(d[0][1], d[1][1], false, false);
-                    // even lane rows: x = (kb, j0), y = (kb+1, j0); odd lane rows: x = (kb-1, j1), y = (kb, j1)
-                    o[q] = make_uint4(t0.x, t1.x, t0.y, t1.y);
+                    o[q] = join_channels8(d);
                 });
             }
             // the wave's 32 channels of a row are exactly one MX block (8 channels in each of the four lane rows): block
@@ -447,14 +443,9 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, int nt, int row
 #pragma unroll
                 for(int q = 0; q < NP; q++)
                 {
-                    u32 am  = amax15_fold(amax15x2(amax15x2(o[q].x, o[q].y), amax15x2(o[q].z, o[q].w)));
-                    v2u s16 = __builtin_amdgcn_permlane16_swap(am, am, false, false);
-                    am      = s16.x > s16.y ? s16.x : s16.y;
-                    v2u s32 = __builtin_amdgcn_permlane32_swap(am, am, false, false);
-                    am      = s32.x > s32.y ? s32.x : s32.y;
-                    e8[q]   = mx_scale_byte(am);
-                    q4[q]   = ok[q] ? cvt8(o[q], e8[q]) : 0u;
-                    e8[q]   = ok[q] ? e8[q] : 0u;
+                    e8[q] = mx_scale_of_row(o[q]);
+                    q4[q] = ok[q] ? cvt8(o[q], e8[q]) : 0u;
+                    e8[q] = ok[q] ? e8[q] : 0u;
                 }
 #pragma unroll
                 for(int q = 0; q < NP; q++)

@@ -194,7 +194,7 @@ static const TileCost tile_costs[] = {{16, 1.2, 1.37, 1e9, 0.35}, {32, 1.5, 1.39
                                       {128, 4.5, 2.10, 307, 0.33}, {160, 5.8, 2.27, 284, 0.75}, {192, 6.8, 2.38, 271, 1.05},
                                       {256, 8.6, 2.84, 276, 1.6},  {288, 9.8, 3.15, 273, 2.0}};
 
-static bool takes_pairs(int64_t tokens, int topk, int experts, int hidden, int inter, int block_m, int w4a16, int split_k);
+static bool takes_pairs(int64_t tokens, int topk, int experts, int local_experts, int hidden, int inter, int block_m, int w4a16, int split_k);
 
 // The tile height of an MXFP4-activation layer call whose sizes are known: the one of pyhip_moe_pick_block_m, which looks at the rows
 // per expert alone, unless that has fewer tiles in the gate_up GEMM than the chip has CUs and 64, 32 or 16 rows are estimated to
@@ -223,12 +223,15 @@ extern "C" int pyhip_layer_block_m(int64_t tokens, int topk, int experts, int lo
     // 32 / 64 rows (three waves per SIMD instead of four, which a short K loop feels): DeepSeek-V3 shape 6.3: 881 / 887, 9.4: 913 / 917; gpt-oss shape
     // 6.3: 257 / 257, 11.6: 272 / 277; Qwen3 shape 6.3: 120 / 118, 11: 155 / 147; 96 experts, Zipf, 5: 121 / 114, 7.5: 152 / 143, 11.7: 211 / 189; hidden
     // 2048: 256 experts, top-1 9.8: 338 / 355; 128, top-8, 11: 70.7 / 74.2; 60, top-4, 10: 56.4 / 58.7
-    if(ladder == 16 && experts >= 32 && est >= 2.0 && tokens * topk > WAVE)
+    // 64 rows with a K loop of 1024 columns in the down GEMM cost 2-4 % (3072 x 1024, 512 experts, 8 rows per expert, 32 / 64 rows 417.9 / 423.0, the persistent
+    // kernels 412.5).  And only where those kernels serve the higher block
+    auto served = [&](int rows) { return takes_pairs(tokens, topk, experts, local_experts, hidden, inter, rows, 0, 0); };
+    if(ladder == 16 && experts >= 32 && est >= 2.0 && tokens * topk > WAVE && served(32))
         ladder = 32;
-    else if(ladder == 32 && experts >= 32 && est >= 5.0 && hidden >= 3072 && inter % 512 == 0)
+    else if(ladder == 32 && experts >= 32 && est >= 5.0 && hidden >= 3072 && inter > 1024 && served(64))
         ladder = 64;
     // (the estimate is of the persistent kernels)
-    if(local_experts * expected_blocks(est, ladder) * (inter / 128) >= 256.0 || takes_pairs(tokens, topk, experts, hidden, inter, ladder, 0, 0))
+    if(local_experts * expected_blocks(est, ladder) * (inter / 128) >= 256.0 || served(ladder))
         return ladder;
     auto estimate = [&](const TileCost& c) {
         const double hit = local_experts * (1.0 - exp(-est)), nb = local_experts * expected_blocks(est, c.rows);
@@ -320,7 +323,25 @@ static bool leaves_sort_out(int64_t tokens, int topk, int experts, int inter, in
         return false;
     return (block_m == 16 && pairs <= WAVE) || (blocks * (inter / 32) <= 768 && blocks <= 64 && pairs <= 16ll * experts);
 }
-static bool takes_pairs(int64_t tokens, int topk, int experts, int hidden, int inter, int block_m, int w4a16, int split_k)
+// A workgroup's start and end against its K loop, of which 512 columns are a single K-step to each of its four waves.  With MXFP4 activations
+// such layers are served only while few workgroups follow one another on a CU, or in 16-row blocks with hidden between 1024 and 2048.  Layer, us,
+// persistent kernels / this, by the workgroups of both GEMMs: 512 x 512, 16-row blocks, 160 experts, top-6 1300: 22.3 / 19.3, 2280: 22.3 / 24.6, 3420: 27.1 / 29.1; 384
+// experts, top-8 8200: 42.8 / 50.9; 512 x 1536 19100: 93.5 / 108.9; 1024 x 512, 128 experts, top-8 2040: 22.8 / 21.9, 3180: 29.7 / 30.5, 32-row blocks 4070: 33.5 /
+// 34.8; 3072 x 512, 64 experts, top-6 3260: 35.3 / 36.5; 4096 x 512, 512 experts, top-8 31800: 236.0 / 250.8; between, 16-row blocks: 1536 x 512, 160
+// experts 5700: 47.2 / 45.1; 2048 x 512, 256 experts, top-8 6110: 59.8 / 54.3, 11700: 86.0 / 85.2, 64-row blocks 90.3 / 93.0.  With 1024 columns it is
+// no matter any more (512 experts, 3072 x 1024 38900: 381.8 / 375.2; 384, 1024 x 1024 10900: 80.6 / 75.5).  bf16 activations, whose K-steps
+// take longer: only where full blocks pass through LDS first (512 x 1024, 160 experts, 9.5 rows per expert 55.4 / 59.1, 6 rows 0.95).
+static bool too_short_for_pairs(int64_t pairs, int experts, int local_experts, int hidden, int inter, int block_m, int w4a16)
+{
+    if(w4a16)
+        return hidden < 1024 && experts >= 32 && pairs >= 7ll * experts;
+    if(hidden >= 1024 && inter >= 1024)
+        return false;
+    if(block_m == 16 && hidden > 1024 && hidden <= 2048)
+        return false;
+    return local_experts * expected_blocks((double)pairs / experts, block_m) * (inter / 32 + hidden / 64) > 2048.0;
+}
+static bool takes_pairs(int64_t tokens, int topk, int experts, int local_experts, int hidden, int inter, int block_m, int w4a16, int split_k)
 {
     const int64_t pairs = tokens * topk;
     if(block_m != 16 && ((block_m != 32 && block_m != 64) || w4a16))
@@ -328,7 +349,10 @@ static bool takes_pairs(int64_t tokens, int topk, int experts, int hidden, int i
     if(!w4a16 && !leaves_sort_out(tokens, topk, experts, inter, block_m, w4a16) &&
        pairs > (int64_t)experts * rows_per_expert_max(experts, block_m))
         return false;
-    return hidden % 512 == 0 && inter % 512 == 0 && topk > 0 && experts <= 2048 &&
+    if(topk <= 0 || ((w4a16 || !leaves_sort_out(tokens, topk, experts, inter, block_m, w4a16)) &&
+                     too_short_for_pairs(pairs, experts, local_experts > 0 && local_experts < experts ? local_experts : experts, hidden, inter, block_m, w4a16)))
+        return false;
+    return hidden % 512 == 0 && inter % 512 == 0 && experts <= 2048 &&
            pyhip_pairs_served(tokens, topk, experts, hidden, inter, pyhip_moe_sorting_max_blocks(tokens, topk, experts, block_m) * (block_m / 16),
                               !w4a16, split_k);
 }
@@ -470,7 +494,8 @@ static int forward_impl(const void* hidden_bf16, int64_t hidden_row_stride, int 
     const bool pads_fit = hidden_pad >= 0 && hidden_pad < hidden && inter_pad >= 0 && inter_pad < inter;
     PYHIP_REQUIRE(w4a16 || pads_fit, "moe_forward: hidden_pad=%d / inter_pad=%d outside [0, hidden=%d) / [0, inter=%d)", hidden_pad, inter_pad, hidden,
                   inter);
-    const bool pairs = pads_fit && takes_pairs(tokens, topk, experts, hidden, inter, block_m, w4a16, split_k) && takes_rows(tokens, hidden_row_stride);
+    const bool pairs = pads_fit && takes_pairs(tokens, topk, experts, expert_mask ? local_experts : experts, hidden, inter, block_m, w4a16, split_k) &&
+                       takes_rows(tokens, hidden_row_stride);
     bf16_cols        = bf16_cols && pairs && hidden_cols > 0 && takes_bf16_cols(tokens, hidden_row_stride, hidden_cols);
     PYHIP_REQUIRE(!w4a16 || hidden_row_stride == hidden || bf16_cols, "moe_forward: the bf16-activation kernels need contiguous rows");
     PYHIP_REQUIRE(hidden_cols == 0 || ((!w4a16 || bf16_cols) && !router.gating && hidden_cols == hidden - hidden_pad && hidden_cols % 32 == 0),
@@ -639,12 +664,12 @@ extern "C" int pyhip_layer_forward(const LayerCall* c, hipStream_t stream)
 // Whether a call of these sizes runs the kernels of moe_gemm_pairs.hip (for whoever reports on it)
 extern "C" int pyhip_layer_takes_pairs(int64_t tokens, int topk, int experts, int hidden, int inter, int block_m, int w4a16, int split_k)
 {
-    return takes_pairs(tokens, topk, experts, hidden, inter, block_m, w4a16, split_k);
+    return takes_pairs(tokens, topk, experts, experts, hidden, inter, block_m, w4a16, split_k);
 }
 
 // Whether hidden states at the true width of a padded layer, rows row_stride apart, are taken as they are
 extern "C" int pyhip_layer_takes_cols(int64_t tokens, int topk, int experts, int hidden, int inter, int block_m, int w4a16, int split_k,
                                       int64_t row_stride)
 {
-    return !w4a16 || (takes_pairs(tokens, topk, experts, hidden, inter, block_m, w4a16, split_k) && takes_bf16_cols(tokens, row_stride, 0));
+    return !w4a16 || (takes_pairs(tokens, topk, experts, experts, hidden, inter, block_m, w4a16, split_k) && takes_bf16_cols(tokens, row_stride, 0));
 }

@@ -382,16 +382,8 @@ __device__ __forceinline__ void pairs_tile(const PairArgs& g, float* red, int la
             d[j][0] = pack_bf16x2(v[0], v[1]);
             d[j][1] = pack_bf16x2(v[2], v[3]);
         }
-        typedef unsigned v2u __attribute__((ext_vector_type(2)));
-        const v2u t0  = __builtin_amdgcn_permlane16_swap(d[0][0], d[1][0], false, false);
-        const v2u t1  = __builtin_amdgcn_permlane16_swap(d[0][1], d[1][1], false, false);
-        const uint4 o = make_uint4(t0.x, t1.x, t0.y, t1.y);
-        u32 am        = amax15_fold(amax15x2(amax15x2(o.x, o.y), amax15x2(o.z, o.w)));
-        const v2u s16 = __builtin_amdgcn_permlane16_swap(am, am, false, false);
-        am            = s16.x > s16.y ? s16.x : s16.y;
-        const v2u s32 = __builtin_amdgcn_permlane32_swap(am, am, false, false);
-        am            = s32.x > s32.y ? s32.x : s32.y;
-        const u32 e8  = mx_scale_byte(am);
+        const uint4 o = join_channels8(d);
+        const u32 e8  = mx_scale_of_row(o);
         if(here)
         {
             const int blk = chbase / 32, kt = blk / 4;

@@ -36,12 +36,12 @@ def test_rows_at_the_true_width_are_asked_for_where_they_are_taken(T, stride):
 
 
 @pytest.mark.parametrize("pad,inter_pad", [(-32, 0), (0, -512), (512, 0), (0, 1024), (544, 0), (0, 1056), (-512, -1024)])
-@pytest.mark.parametrize("T", [3, 100])
+@pytest.mark.parametrize("T", [3, 60])
 def test_padding_outside_of_the_matrices(T, pad, inter_pad):
     """refused with MXFP4 activations; with bf16 ones taken by the kernels that look at no padding, as channels past an expert's matrix would be
     read and written by those that do"""
-    assert _lib.load().pyhip_layer_takes_pairs(T, 2, 64, 512, 1024, 16, 0, 0) and _lib.load().pyhip_layer_takes_pairs(T, 2, 64, 512, 1024, 16, 1, 0)
+    assert _lib.load().pyhip_layer_takes_pairs(T, 2, 32, 512, 1024, 16, 0, 0) and _lib.load().pyhip_layer_takes_pairs(T, 2, 32, 512, 1024, 16, 1, 0)
     with pytest.raises(RuntimeError, match="hidden_pad=%d / inter_pad=%d" % (pad, inter_pad)):
-        _lib.check(_call(T, 2, 64, 512, 1024, 16, 0, pad=pad, inter_pad=inter_pad), "layer")
+        _lib.check(_call(T, 2, 32, 512, 1024, 16, 0, pad=pad, inter_pad=inter_pad), "layer")
     with pytest.raises(RuntimeError, match="moe_sort.* launch failed"):
-        _lib.check(_call(T, 2, 64, 512, 1024, 16, 1, pad=pad, inter_pad=inter_pad), "layer")
+        _lib.check(_call(T, 2, 32, 512, 1024, 16, 1, pad=pad, inter_pad=inter_pad), "layer")

@@ -47,3 +47,27 @@ def test_any_sizes_get_a_served_height():
 ])
 def test_lower_tiles_only_where_they_cannot_lose_much(tokens, topk, experts, local, hidden, inter, want):
     assert _lib.load().pyhip_layer_block_m(tokens, topk, experts, local, hidden, inter) == want
+
+
+@pytest.mark.parametrize("tokens,topk,experts,hidden,inter,rows,w4a16,want", [
+    # a GEMM of 512 columns, more workgroups than few follow one another on a CU: measured slower by 2 to 20 % with MXFP4 activations
+    (192, 8, 384, 512, 512, 16, 0, 0), (106, 8, 384, 512, 1536, 16, 0, 0), (107, 6, 160, 512, 512, 32, 0, 0), (80, 8, 128, 1024, 512, 32, 0, 0),
+    (96, 8, 512, 4096, 512, 16, 0, 0), (96, 8, 256, 2048, 512, 64, 0, 0),
+    # few of them, no sort, 16-row blocks of the middle sizes, or 1024 columns
+    (11, 6, 160, 512, 512, 16, 0, 1), (8, 8, 384, 512, 512, 16, 0, 1), (96, 8, 256, 2048, 512, 16, 0, 1), (16, 4, 8, 512, 512, 32, 0, 1),
+    (192, 8, 384, 1024, 1024, 32, 0, 1), (192, 8, 512, 3072, 1024, 32, 0, 1),
+    # bf16 activations: only blocks that pass through LDS
+    (253, 6, 160, 512, 1024, 16, 1, 0), (160, 6, 160, 512, 1024, 16, 1, 1), (253, 6, 160, 1024, 512, 16, 1, 1),
+])
+def test_few_token_kernels_only_where_their_k_loop_is_long_enough(tokens, topk, experts, hidden, inter, rows, w4a16, want):
+    assert _lib.load().pyhip_layer_takes_pairs(tokens, topk, experts, hidden, inter, rows, w4a16, 0) == want
+
+
+@pytest.mark.parametrize("tokens,topk,experts,hidden,inter,want", [
+    # where they do not serve the higher block the ladder's height stays
+    (192, 8, 512, 512, 512, 16), (96, 8, 256, 2048, 512, 16), (320, 8, 512, 4096, 512, 32),
+    # 64 rows not with 1024 columns in the down GEMM
+    (512, 8, 512, 3072, 1024, 32), (180, 8, 128, 4096, 1536, 64),
+])
+def test_higher_blocks_only_where_the_few_token_kernels_serve_them(tokens, topk, experts, hidden, inter, want):
+    assert _lib.load().pyhip_layer_block_m(tokens, topk, experts, experts, hidden, inter) == want
