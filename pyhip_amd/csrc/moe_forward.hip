@@ -230,8 +230,8 @@ extern "C" int pyhip_layer_block_m(int64_t tokens, int topk, int experts, int lo
         ladder = 32;
     else if(ladder == 32 && experts >= 32 && est >= 5.0 && hidden >= 3072 && inter > 1024 && served(64))
         ladder = 64;
-    // (the estimate is of the persistent kernels)
-    if(local_experts * expected_blocks(est, ladder) * (inter / 128) >= 256.0 || served(ladder))
+    // (the estimate is of the persistent kernels; 16 rows instead of 32 were not measured)
+    if(local_experts * expected_blocks(est, ladder) * (inter / 128) >= 256.0 || ladder <= 32 || served(ladder))
         return ladder;
     auto estimate = [&](const TileCost& c) {
         const double hit = local_experts * (1.0 - exp(-est)), nb = local_experts * expected_blocks(est, c.rows);
@@ -306,22 +306,33 @@ struct Router
 //   64 rows (against the persistent kernel of the better height): Qwen3 shape 6.3: 128 / 118, 11: 158 / 147; gpt-oss shape 9.4: 277 / 268, 11.6: 280 /
 //     277, 31: 323 / 357; DeepSeek-V3 shape 11.6: 949 / 939, 16: 964 / 981; 96 experts 5: 128 / 114, 11.7: 212 / 189; 8 experts 17.5: 140 / 123, 25: 142 /
 //     129, 40: 147 / 149; 16, top-2, 4096 x 4096 25: 84.3 / 83.0, 31: 85.0 / 88.4; 12, 5120 x 2048 22: 46.8 / 47.4, 28: 47.6 / 51.2
-static int rows_per_expert_max(int experts, int block_m)
+// With a handful of experts, 12 to 24 rows: not where the persistent kernels' tiles of the gate_up GEMM are one full round (up to 256; `tiles`), nor,
+// with a long K loop, where they are less than half of one.  Layer, us, 64-row blocks: 28 experts, top-2, 7168 x 1024, 23 rows (224 tiles) 71.9 / 79.4, 4096 x
+// 1024 47.4 / 51.3, 16 rows 45.2 / 45.7; 4096 x 3072 (672) 19 rows 103.9 / 103.8; 20, 4096 x 2048, 19 (320) 67.3 / 59.2, 5120 x 1536, 23 (240) 55.9 / 60.7;
+// 8, 4096 x 2048, 19 (128) 34.6 / 30.4; 7168 x 2048, 23 under a Zipf router (128) 49.4 / 56.4.
+static bool few_enough_rows(int64_t pairs, int experts, int local_experts, int hidden, int inter, int block_m)
 {
-    return experts < 32 ? (block_m == 16 ? 8 : block_m == 32 ? 16 : 24) : (block_m == 16 ? 4 : 12);
+    if(experts >= 32 || block_m == 16)
+        return pairs <= (int64_t)experts * (experts < 32 ? 8 : block_m == 16 ? 4 : 12);
+    const double tiles = local_experts * expected_blocks((double)pairs / experts, block_m) * (inter / 128);
+    const bool round = tiles > 256.0, half = tiles <= 128.0 && hidden < 5120;
+    return pairs <= (int64_t)experts * (!round && !half ? 12 : block_m == 32 ? 16 : round ? 21 : 24);
 }
 // Whether they find their rows themselves, in blocks of 16: up to a pair to a lane; with two, which costs every workgroup of the gate_up
 // GEMM more, if all of its workgroups run at once (and the list of blocks fits where a sort into 32 rows would put its own).
 // Layer, us, sorted / this: 8 experts, 1024 x 512, top-2, 40 tokens 21.3 / 17.9, 64 tokens 21.2 / 17.7; 12, 1024 x 1024, top-1, 100 tokens 22.9 /
 // 19.0.  With more workgroups it goes either way: DeepSeek-V3 shape, 16 tokens 356.0 / 347.5; 96 experts, top-4, 6272 x 1920, 30 tokens 204.6 / 198.2;
 // 60, 2048 x 1408, 32 tokens 49.2 / 47.0; gpt-oss shape, 32 tokens 167.9 / 170.6; Qwen3 shape, 16 tokens 65.9 / 68.3; Mixtral shape, 50 tokens, bf16
-// activations 121.4 / 131.4: left to the sort.
-static bool leaves_sort_out(int64_t tokens, int topk, int experts, int inter, int block_m, int w4a16)
+// activations 121.4 / 131.4: left to the sort.  Nor with more than 8 rows per expert in wide layers: 8 experts, top-2, 64 tokens, by the layer, persistent
+// kernels / this: 2560 x 1536 27.8 / 23.9, 3584 x 1024 28.1 / 23.6, 3072 x 1536 28.8 / 27.4, 5120 x 1536 36.2 / 39.7, 7168 x 1536 43.8 / 52.0.
+static bool leaves_sort_out(int64_t tokens, int topk, int experts, int hidden, int inter, int block_m, int w4a16)
 {
     const int64_t pairs = tokens * topk, blocks = pairs < experts + pairs / 16 ? pairs : experts + pairs / 16;
     if(block_m > 32 || (w4a16 && block_m > 16) || pairs > PAIRS_UNSORTED_MAX)
         return false;
-    return (block_m == 16 && pairs <= WAVE) || (blocks * (inter / 32) <= 768 && blocks <= 64 && pairs <= 16ll * experts);
+    // (with more than one block of 16 to an expert its weights are fetched again)
+    return (block_m == 16 && pairs <= WAVE) || (blocks * (inter / 32) <= 768 && blocks <= 64 &&
+                                                pairs <= (w4a16 || (int64_t)hidden * inter <= 4 << 20 ? 16ll : 8ll) * experts);
 }
 // A workgroup's start and end against its K loop, of which 512 columns are a single K-step to each of its four waves.  With MXFP4 activations
 // such layers are served only while few workgroups follow one another on a CU, or in 16-row blocks with hidden between 1024 and 2048.  Layer, us,
@@ -346,11 +357,12 @@ static bool takes_pairs(int64_t tokens, int topk, int experts, int local_experts
     const int64_t pairs = tokens * topk;
     if(block_m != 16 && ((block_m != 32 && block_m != 64) || w4a16))
         return false;
-    if(!w4a16 && !leaves_sort_out(tokens, topk, experts, inter, block_m, w4a16) &&
-       pairs > (int64_t)experts * rows_per_expert_max(experts, block_m))
+    const int here = local_experts > 0 && local_experts < experts ? local_experts : experts;
+    if(topk <= 0)
         return false;
-    if(topk <= 0 || ((w4a16 || !leaves_sort_out(tokens, topk, experts, inter, block_m, w4a16)) &&
-                     too_short_for_pairs(pairs, experts, local_experts > 0 && local_experts < experts ? local_experts : experts, hidden, inter, block_m, w4a16)))
+    if(w4a16 ? too_short_for_pairs(pairs, experts, here, hidden, inter, block_m, w4a16)
+             : !leaves_sort_out(tokens, topk, experts, hidden, inter, block_m, w4a16) &&
+                   (!few_enough_rows(pairs, experts, here, hidden, inter, block_m) || too_short_for_pairs(pairs, experts, here, hidden, inter, block_m, w4a16)))
         return false;
     return hidden % 512 == 0 && inter % 512 == 0 && experts <= 2048 &&
            pyhip_pairs_served(tokens, topk, experts, hidden, inter, pyhip_moe_sorting_max_blocks(tokens, topk, experts, block_m) * (block_m / 16),
@@ -377,7 +389,7 @@ static int forward_pairs(const void* hidden_bf16, int64_t row_stride, int hidden
                          float swiglu_limit, int held, const Layout& l, uint8_t* ws, hipStream_t stream)
 {
     uint8_t* a2         = ws + (w4a16 ? l.a2 : l.a2_q);      // a row for every pair
-    const bool unsorted = leaves_sort_out(tokens, topk, experts, inter, block_m, w4a16);
+    const bool unsorted = leaves_sort_out(tokens, topk, experts, hidden, inter, block_m, w4a16);
     uint32_t* s_ids     = (uint32_t*)(ws + l.sorted_ids);
     float* s_w          = (float*)(ws + l.sorted_w);
     uint32_t *s_e = (uint32_t*)(ws + l.sorted_e), *n_valid = (uint32_t*)(ws + l.num_valid), *sched = (uint32_t*)(ws + l.sched);
