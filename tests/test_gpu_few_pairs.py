@@ -220,3 +220,25 @@ def test_wide_block_scales_equal_the_stages_within_rounding(T, E, rows):
     print("  differ:", (diff > 0).mean(), "largest share of the bound:", (diff / bound).max(), flush=True)
     assert np.isfinite(diff).all() and (diff <= bound).all(), (diff / bound).max()
     assert want.abs().mean() > 100 * bound.mean()                  # (the bound says something)
+
+
+@pytest.mark.parametrize("T,k,E,H,I,method,rows", [
+    (1, 8, 16, 512, 1536, "w4a16", 16),      # a token's slots of 12288 columns together: summed in the down GEMM
+    (1, 8, 16, 512, 2048, "w4a16", 16),      # of more: by expert, and reduced
+    (2, 5, 80, 512, 2560, "w4a16", 16),
+    (64, 8, 128, 512, 512, "a4w4", 16),      # four rows per expert, but too many workgroups of one K-step
+    (80, 2, 40, 512, 512, "a4w4", 16),       # sorted, four rows per expert, few workgroups
+    (72, 2, 32, 2560, 512, "a4w4", 32),      # the same in 32 rows, an uneven share of K-steps
+    (70, 1, 5, 5120, 512, "a4w4", 32),       # a handful of experts, twelve rows and more, a long K loop
+])
+def test_lines_of_the_few_token_kernels(T, k, E, H, I, method, rows):
+    """on both sides of the lines by the length of the K loops: the bits of the stages one by one"""
+    from pyhip_amd import fused_moe
+    L = cases.make_layer("", T, seed=T, E=E, k=k, H=H, I=I, router="softmax")
+    w1, w1s, w2, w2s = cases.device_weights(L)
+    args = (L.hidden.cuda(), w1, w2, torch.from_numpy(L.topk_w).cuda(), torch.from_numpy(L.topk_ids).cuda())
+    kw = dict(w1_scale=w1s, w2_scale=w2s, method=method, block_size_M=rows)
+    print("few pairs, lines", T, k, E, H, I, method, rows, flush=True)
+    want = fused_moe(*args, return_parts=True, **kw)[0]
+    _poison(T, k, E, H, I, method, rows)
+    assert torch.equal(fused_moe(*args, **kw), want)
