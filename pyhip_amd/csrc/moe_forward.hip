@@ -306,17 +306,18 @@ struct Router
 //   64 rows (against the persistent kernel of the better height): Qwen3 shape 6.3: 128 / 118, 11: 158 / 147; gpt-oss shape 9.4: 277 / 268, 11.6: 280 /
 //     277, 31: 323 / 357; DeepSeek-V3 shape 11.6: 949 / 939, 16: 964 / 981; 96 experts 5: 128 / 114, 11.7: 212 / 189; 8 experts 17.5: 140 / 123, 25: 142 /
 //     129, 40: 147 / 149; 16, top-2, 4096 x 4096 25: 84.3 / 83.0, 31: 85.0 / 88.4; 12, 5120 x 2048 22: 46.8 / 47.4, 28: 47.6 / 51.2
-// With a handful of experts, 12 to 24 rows: not where the persistent kernels' tiles of the gate_up GEMM are one full round (up to 256; `tiles`), nor,
+// With a handful of experts, from 12 rows (with a long K loop 9) to 24: not where the persistent kernels' tiles of the gate_up GEMM are one full round (up to 256; `tiles`), nor,
 // with a long K loop, where they are less than half of one.  Layer, us, 64-row blocks: 28 experts, top-2, 7168 x 1024, 23 rows (224 tiles) 71.9 / 79.4, 4096 x
 // 1024 47.4 / 51.3, 16 rows 45.2 / 45.7; 4096 x 3072 (672) 19 rows 103.9 / 103.8; 20, 4096 x 2048, 19 (320) 67.3 / 59.2, 5120 x 1536, 23 (240) 55.9 / 60.7;
-// 8, 4096 x 2048, 19 (128) 34.6 / 30.4; 7168 x 2048, 23 under a Zipf router (128) 49.4 / 56.4.
+// 8, 4096 x 2048, 19 (128) 34.6 / 30.4; 7168 x 2048, 23 under a Zipf router (128) 49.4 / 56.4. 32-row blocks under Zipf
+// routers: 24, top-4, 7168 x 1024, 10 (192) 58.6 / 63.5, 16, 7168 x 1536, 13 (192) 57.4 / 64.3; 8, top-2, 5120 x 3072, 13 (192) 45.4 / 48.8.
 static bool few_enough_rows(int64_t pairs, int experts, int local_experts, int hidden, int inter, int block_m)
 {
     if(experts >= 32 || block_m == 16)
         return pairs <= (int64_t)experts * (experts < 32 ? 8 : block_m == 16 ? 4 : 12);
     const double tiles = local_experts * expected_blocks((double)pairs / experts, block_m) * (inter / 128);
     const bool round = tiles > 256.0, half = tiles <= 128.0 && hidden < 5120;
-    return pairs <= (int64_t)experts * (!round && !half ? 12 : block_m == 32 ? 16 : round ? 21 : 24);
+    return pairs <= (int64_t)experts * (!round && !half ? (hidden < 5120 ? 12 : 9) : block_m == 32 ? 16 : round ? 21 : 24);
 }
 // Whether they find their rows themselves, in blocks of 16: up to a pair to a lane; with two, which costs every workgroup of the gate_up
 // GEMM more, if all of its workgroups run at once (and the list of blocks fits where a sort into 32 rows would put its own).

@@ -76,8 +76,9 @@ def test_higher_blocks_only_where_the_few_token_kernels_serve_them(tokens, topk,
 @pytest.mark.parametrize("tokens,topk,experts,hidden,inter,rows,want", [
     # a handful of experts: the persistent kernels' tiles are one full round of the chip, or a long K loop and less than half of one
     (322, 2, 28, 7168, 1024, 64, 0), (322, 2, 28, 4096, 1024, 64, 0), (92, 2, 8, 7168, 2048, 64, 0), (230, 2, 20, 5120, 1536, 64, 0), (70, 4, 20, 4096, 1536, 32, 0),
+    (140, 2, 28, 7168, 1024, 32, 0),
     # several rounds, or few tiles and a shorter loop, or few rows
-    (190, 2, 20, 4096, 2048, 64, 1), (76, 2, 8, 4096, 2048, 64, 1), (114, 2, 12, 4096, 1024, 64, 1), (140, 2, 28, 7168, 1024, 32, 1), (266, 2, 28, 4096, 3072, 64, 1),
+    (190, 2, 20, 4096, 2048, 64, 1), (76, 2, 8, 4096, 2048, 64, 1), (114, 2, 12, 4096, 1024, 64, 1), (140, 2, 28, 4096, 1024, 32, 1), (112, 2, 28, 7168, 1024, 32, 1), (266, 2, 28, 4096, 3072, 64, 1),
     # without a sort, more than a block of 16 to an expert: not in wide layers
     (64, 2, 8, 7168, 1536, 32, 0), (64, 2, 8, 3072, 1536, 32, 1), (64, 2, 8, 1024, 512, 32, 1), (64, 2, 8, 7168, 1536, 16, 0),
 ])
