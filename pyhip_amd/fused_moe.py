@@ -144,7 +144,7 @@ _remembered_plan = functools.lru_cache(maxsize=512)(_ask_plan)
 
 def _swiglu_limit(limit):
     """as the kernels get it: a limit past float32 (no limit, in a caller's mind) is infinite, where ``struct`` would refuse it"""
-    return ctypes.c_float(limit).value if limit else 7.0
+    return ctypes.c_float(float(limit)).value if limit else 7.0
 
 
 #: struct LayerCall of csrc/moe_forward.hip: pointers, row stride and workspace bytes, sizes and options, the SwiGLU limit

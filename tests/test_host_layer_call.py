@@ -52,3 +52,12 @@ def test_swiglu_limit_of_any_size(limit, want):
     got = m._swiglu_limit(limit)
     assert got == want
     assert m._LAYER_CALL.unpack(m._LAYER_CALL.pack(*[0] * 32, got, 8))[-2] == want
+
+
+def test_swiglu_limit_of_whatever_float_takes():
+    import decimal
+    import pyhip_amd.fused_moe  # noqa: F401
+    limit = sys.modules["pyhip_amd.fused_moe"]._swiglu_limit
+    assert limit("2.5") == limit(decimal.Decimal("2.5")) == limit(torch.tensor([2.5])) == 2.5
+    with pytest.raises((TypeError, ValueError)):
+        limit("none")
