@@ -367,7 +367,7 @@ __device__ __forceinline__ void pairs_tile(const PairArgs& g, float* red, int la
         *(uint2*)((uint16_t*)g.out + (size_t)orow[m] * (STAGE == 1 ? I : g.N) + channel(j)) =
             make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
     };
-    // the steps of moe_gemm_mxfp4.hip's epilogue (gemm_device.h): round to bf16, eight consecutive channels to a lane, the block's maximum
+    // as the epilogue of the persistent kernels (gemm_device.h), with the same functions: round to bf16, eight consecutive channels to a lane, the block's maximum
     // over the lane rows, e2m1 codes and the scale byte.  x: the sums of row tile m, a row group each
     auto quantise_row = [&](const v4f (&x)[4], int m, bool here) __attribute__((always_inline)) {
         u32 d[2][2];
@@ -740,7 +740,6 @@ bool pyhip_pairs_served(int64_t tokens, int topk, int experts, int hidden, int i
     const int s1 = pairs_split(fp4, 1, blocks * (inter / 128), hidden, split_k), s2 = pairs_split(fp4, 2, blocks * (hidden / 256), inter, split_k);
     // (offsets into the activations are 32-bit and signed)
     return (s1 == 0 || s1 == 4) && (s2 == 0 || s2 == 4 || (s2 == 32 && tokens == 1 && topk == 2 && inter >= 2048 && inter <= 16384)) &&      // (pyhip_w4a16_token_top2)
-          
            (n_blk * 16 + tokens) * (int64_t)(hidden > inter ? hidden : inter) * 2 < (1ll << 31);
 }
 
