@@ -504,9 +504,10 @@ static int forward_impl(const void* hidden_bf16, int64_t hidden_row_stride, int 
                       ((block_m == 128 || block_m == 160 || block_m == 192 || block_m == 256 || block_m == 288) && !w4a16),
                   "moe_forward: block_m=%d (16/32/64, and 128/160/192/256/288 with MXFP4 activations)", block_m);
     // (the bf16-activation kernels of the step-by-step path look at no padding and take any; those of the pairs would leave their matrices)
-    const bool pads_fit = hidden_pad >= 0 && hidden_pad < hidden && inter_pad >= 0 && inter_pad < inter;
-    PYHIP_REQUIRE(w4a16 || pads_fit, "moe_forward: hidden_pad=%d / inter_pad=%d outside [0, hidden=%d) / [0, inter=%d)", hidden_pad, inter_pad, hidden,
-                  inter);
+    const bool h_fits = hidden_pad >= 0 && hidden_pad < hidden, i_fits = inter_pad >= 0 && inter_pad < inter, pads_fit = h_fits && i_fits;
+    // (columns that do not fit are refused with the hidden states)
+    PYHIP_REQUIRE(w4a16 || (i_fits && (h_fits || hidden_cols)), "moe_forward: hidden_pad=%d / inter_pad=%d outside [0, hidden=%d) / [0, inter=%d)",
+                  hidden_pad, inter_pad, hidden, inter);
     const bool pairs = pads_fit && takes_pairs(tokens, topk, experts, expert_mask ? local_experts : experts, hidden, inter, block_m, w4a16, split_k) &&
                        takes_rows(tokens, hidden_row_stride);
     bf16_cols        = bf16_cols && pairs && hidden_cols > 0 && takes_bf16_cols(tokens, hidden_row_stride, hidden_cols);
