@@ -341,17 +341,17 @@ static bool leaves_sort_out(int64_t tokens, int topk, int experts, int hidden, i
 // experts, top-8 8200: 42.8 / 50.9; 512 x 1536 19100: 93.5 / 108.9; 1024 x 512, 128 experts, top-8 2040: 22.8 / 21.9, 3180: 29.7 / 30.5, 32-row blocks 4070: 33.5 /
 // 34.8; 3072 x 512, 64 experts, top-6 3260: 35.3 / 36.5; 4096 x 512, 512 experts, top-8 31800: 236.0 / 250.8; between, 16-row blocks: 1536 x 512, 160
 // experts 5700: 47.2 / 45.1; 2048 x 512, 256 experts, top-8 6110: 59.8 / 54.3, 11700: 86.0 / 85.2, 64-row blocks 90.3 / 93.0.  With 1024 columns it is
-// no matter any more (512 experts, 3072 x 1024 38900: 381.8 / 375.2; 384, 1024 x 1024 10900: 80.6 / 75.5).  bf16 activations, whose K-steps
+// no matter any more (512 experts, 3072 x 1024 38900: 381.8 / 375.2; 384, 1024 x 1024 10900: 80.6 / 75.5) but for 64-row blocks with hidden 1024 (160
+// experts, 1024 x 1024, 7700: 1.10).  bf16 activations, whose K-steps
 // take longer: only where full blocks pass through LDS first (512 x 1024, 160 experts, 9.5 rows per expert 55.4 / 59.1, 6 rows 0.95).
 static bool too_short_for_pairs(int64_t pairs, int experts, int local_experts, int hidden, int inter, int block_m, int w4a16)
 {
     if(w4a16)
         return hidden < 1024 && experts >= 32 && pairs >= 7ll * experts;
-    if(hidden >= 1024 && inter >= 1024)
+    const bool loops_of_two = hidden >= 1024 && inter >= 1024;
+    if(loops_of_two ? hidden > 1024 || block_m != 64 : block_m == 16 && hidden > 1024 && hidden <= 2048)
         return false;
-    if(block_m == 16 && hidden > 1024 && hidden <= 2048)
-        return false;
-    return local_experts * expected_blocks((double)pairs / experts, block_m) * (inter / 32 + hidden / 64) > 2048.0;
+    return local_experts * expected_blocks((double)pairs / experts, block_m) * (inter / 32 + hidden / 64) > (loops_of_two ? 4096.0 : 2048.0);
 }
 static bool takes_pairs(int64_t tokens, int topk, int experts, int local_experts, int hidden, int inter, int block_m, int w4a16, int split_k)
 {

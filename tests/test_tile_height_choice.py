@@ -53,7 +53,9 @@ def test_lower_tiles_only_where_they_cannot_lose_much(tokens, topk, experts, loc
     # a GEMM of 512 columns, more workgroups than few follow one another on a CU: measured slower by 2 to 20 % with MXFP4 activations
     (192, 8, 384, 512, 512, 16, 0, 0), (106, 8, 384, 512, 1536, 16, 0, 0), (107, 6, 160, 512, 512, 32, 0, 0), (80, 8, 128, 1024, 512, 32, 0, 0),
     (96, 8, 512, 4096, 512, 16, 0, 0), (96, 8, 256, 2048, 512, 64, 0, 0),
+    (253, 6, 160, 1024, 1024, 64, 0, 0),
     # few of them, no sort, 16-row blocks of the middle sizes, or 1024 columns
+    (253, 6, 160, 1024, 1024, 32, 0, 1), (60, 4, 32, 1024, 1024, 64, 0, 1),
     (11, 6, 160, 512, 512, 16, 0, 1), (8, 8, 384, 512, 512, 16, 0, 1), (96, 8, 256, 2048, 512, 16, 0, 1), (16, 4, 8, 512, 512, 32, 0, 1),
     (192, 8, 384, 1024, 1024, 32, 0, 1), (192, 8, 512, 3072, 1024, 32, 0, 1),
     # bf16 activations: only blocks that pass through LDS
