@@ -306,18 +306,19 @@ struct Router
 //   64 rows (against the persistent kernel of the better height): Qwen3 shape 6.3: 128 / 118, 11: 158 / 147; gpt-oss shape 9.4: 277 / 268, 11.6: 280 /
 //     277, 31: 323 / 357; DeepSeek-V3 shape 11.6: 949 / 939, 16: 964 / 981; 96 experts 5: 128 / 114, 11.7: 212 / 189; 8 experts 17.5: 140 / 123, 25: 142 /
 //     129, 40: 147 / 149; 16, top-2, 4096 x 4096 25: 84.3 / 83.0, 31: 85.0 / 88.4; 12, 5120 x 2048 22: 46.8 / 47.4, 28: 47.6 / 51.2
-// With a handful of experts, from 12 rows (with a long K loop 9) to 24: not where the persistent kernels' tiles of the gate_up GEMM are one full round (up to 256; `tiles`), nor,
-// with a long K loop, where they are less than half of one.  Layer, us, 64-row blocks: 28 experts, top-2, 7168 x 1024, 23 rows (224 tiles) 71.9 / 79.4, 4096 x
-// 1024 47.4 / 51.3, 16 rows 45.2 / 45.7; 4096 x 3072 (672) 19 rows 103.9 / 103.8; 20, 4096 x 2048, 19 (320) 67.3 / 59.2, 5120 x 1536, 23 (240) 55.9 / 60.7;
-// 8, 4096 x 2048, 19 (128) 34.6 / 30.4; 7168 x 2048, 23 under a Zipf router (128) 49.4 / 56.4. 32-row blocks under Zipf
-// routers: 24, top-4, 7168 x 1024, 10 (192) 58.6 / 63.5, 16, 7168 x 1536, 13 (192) 57.4 / 64.3; 8, top-2, 5120 x 3072, 13 (192) 45.4 / 48.8.
+// With a handful of experts and hidden 2560 and more the line lies lower where the persistent kernels' tiles of the gate_up GEMM (`tiles`) make most of one
+// round of the chip: from there to 256 an uneven router takes them into a second round, which costs them up to 25 %.  Layer, us, by rows per expert:
+// 28 experts, top-2, 224 tiles, 7168 x 1024 23: 71.9 / 79.4, 16 under a Zipf router 0.87; 4096 x 1024 23: 47.4 / 51.3, 13: 43.6 / 45.3; 192 tiles, 24, top-4, 7168 x 1024 23
+// under a Zipf router 64.2 / 72.0, 10: 58.6 / 63.5 and 0.98 under an even one; 20, 240 tiles, 3072 x 1536 13: 0.95, under a Zipf router 0.77; 64, 8, 5120 x 1024 10: 0.69;
+// 320, 20, 4096 x 2048 19: 67.3 / 59.2.
 static bool few_enough_rows(int64_t pairs, int experts, int local_experts, int hidden, int inter, int block_m)
 {
     if(experts >= 32 || block_m == 16)
         return pairs <= (int64_t)experts * (experts < 32 ? 8 : block_m == 16 ? 4 : 12);
     const double tiles = local_experts * expected_blocks((double)pairs / experts, block_m) * (inter / 128);
-    const bool round = tiles > 256.0, half = tiles <= 128.0 && hidden < 5120;
-    return pairs <= (int64_t)experts * (!round && !half ? (hidden < 5120 ? 12 : 9) : block_m == 32 ? 16 : round ? 21 : 24);
+    const bool full = tiles > 136.0 && tiles <= 232.0 && hidden >= 2560;
+    const int most = block_m == 32 ? 16 : 24, most_full = hidden < 5120 ? 21 : tiles <= 216.0 ? 14 : 17;
+    return pairs <= (int64_t)experts * (full && most_full < most ? most_full : most);
 }
 // Whether they find their rows themselves, in blocks of 16: up to a pair to a lane; with two, which costs every workgroup of the gate_up
 // GEMM more, if all of its workgroups run at once (and the list of blocks fits where a sort into 32 rows would put its own).
@@ -336,10 +337,10 @@ static bool leaves_sort_out(int64_t tokens, int topk, int experts, int hidden, i
                                                 pairs <= (w4a16 || (int64_t)hidden * inter <= 4 << 20 ? 16ll : 8ll) * experts);
 }
 // A workgroup's start and end against its K loop, of which 512 columns are a single K-step to each of its four waves.  With MXFP4 activations
-// such layers are served only while few workgroups follow one another on a CU, or in 16-row blocks with hidden between 1024 and 2048.  Layer, us,
+// such layers are served only while few workgroups follow one another on a CU, or in 16-row blocks with hidden between 1024 and 2048 or few pairs.  Layer, us,
 // persistent kernels / this, by the workgroups of both GEMMs: 512 x 512, 16-row blocks, 160 experts, top-6 1300: 22.3 / 19.3, 2280: 22.3 / 24.6, 3420: 27.1 / 29.1; 384
 // experts, top-8 8200: 42.8 / 50.9; 512 x 1536 19100: 93.5 / 108.9; 1024 x 512, 128 experts, top-8 2040: 22.8 / 21.9, 3180: 29.7 / 30.5, 32-row blocks 4070: 33.5 /
-// 34.8; 3072 x 512, 64 experts, top-6 3260: 35.3 / 36.5; 4096 x 512, 512 experts, top-8 31800: 236.0 / 250.8; between, 16-row blocks: 1536 x 512, 160
+// 34.8; 3072 x 512, 64 experts, top-6 3260: 35.3 / 36.5, 128, 0.7 rows per expert: 49.4 / 42.8; 4096 x 512, 512 experts, top-8 31800: 236.0 / 250.8; between, 16-row blocks: 1536 x 512, 160
 // experts 5700: 47.2 / 45.1; 2048 x 512, 256 experts, top-8 6110: 59.8 / 54.3, 11700: 86.0 / 85.2, 64-row blocks 90.3 / 93.0.  With 1024 columns it is
 // no matter any more (512 experts, 3072 x 1024 38900: 381.8 / 375.2; 384, 1024 x 1024 10900: 80.6 / 75.5) but for 64-row blocks with hidden 1024 (160
 // experts, 1024 x 1024, 7700: 1.10).  bf16 activations, whose K-steps
@@ -348,10 +349,12 @@ static bool too_short_for_pairs(int64_t pairs, int experts, int local_experts, i
 {
     if(w4a16)
         return hidden < 1024 && experts >= 32 && pairs >= 7ll * experts;
-    const bool loops_of_two = hidden >= 1024 && inter >= 1024;
-    if(loops_of_two ? hidden > 1024 || block_m != 64 : block_m == 16 && hidden > 1024 && hidden <= 2048)
-        return false;
-    return local_experts * expected_blocks((double)pairs / experts, block_m) * (inter / 32 + hidden / 64) > (loops_of_two ? 4096.0 : 2048.0);
+    const double est = (double)pairs / experts, workgroups = local_experts * expected_blocks(est, block_m) * (inter / 32 + hidden / 64);
+    if(hidden < 1024)
+        return workgroups > 2048.0;
+    if(inter < 1024)
+        return workgroups > 3000.0 && !(block_m == 16 && ((hidden > 1024 && hidden <= 2048) || (est <= 1.6 && workgroups <= 8192.0)));
+    return block_m == 64 && hidden == 1024 && workgroups > 4096.0;
 }
 static bool takes_pairs(int64_t tokens, int topk, int experts, int local_experts, int hidden, int inter, int block_m, int w4a16, int split_k)
 {

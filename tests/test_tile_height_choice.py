@@ -76,22 +76,22 @@ def test_higher_blocks_only_where_the_few_token_kernels_serve_them(tokens, topk,
 
 
 @pytest.mark.parametrize("tokens,topk,experts,hidden,inter,rows,want", [
-    # a handful of experts: the persistent kernels' tiles are one full round of the chip, or a long K loop and less than half of one
-    (322, 2, 28, 7168, 1024, 64, 0), (322, 2, 28, 4096, 1024, 64, 0), (92, 2, 8, 7168, 2048, 64, 0), (230, 2, 20, 5120, 1536, 64, 0), (70, 4, 20, 4096, 1536, 32, 0),
-    (140, 2, 28, 7168, 1024, 32, 0),
-    # several rounds, or few tiles and a shorter loop, or few rows
-    (190, 2, 20, 4096, 2048, 64, 1), (76, 2, 8, 4096, 2048, 64, 1), (114, 2, 12, 4096, 1024, 64, 1), (140, 2, 28, 4096, 1024, 32, 1), (112, 2, 28, 7168, 1024, 32, 1), (266, 2, 28, 4096, 3072, 64, 1),
-    # without a sort, more than a block of 16 to an expert: not in wide layers
-    (64, 2, 8, 7168, 1536, 32, 0), (64, 2, 8, 3072, 1536, 32, 1), (64, 2, 8, 1024, 512, 32, 1), (64, 2, 8, 7168, 1536, 16, 0),
+    # a handful of experts: the persistent kernels' tiles make most of one round of the chip
+    (322, 2, 28, 7168, 1024, 64, 0), (322, 2, 28, 4096, 1024, 64, 0), (92, 4, 24, 7168, 1024, 64, 0), (96, 4, 24, 5120, 1024, 32, 0),
+    # too few of them, as many as an uneven router takes into a second round, or few rows
+    (92, 2, 8, 7168, 2048, 64, 1), (230, 2, 20, 5120, 1536, 64, 1), (190, 2, 20, 4096, 2048, 64, 1), (76, 2, 8, 4096, 2048, 64, 1), (140, 2, 28, 7168, 1024, 32, 1),
+    (280, 2, 28, 4096, 1024, 64, 1), (322, 2, 28, 2048, 1024, 64, 1),
+    # with or without a sort
+    (64, 2, 8, 7168, 1536, 32, 1), (64, 2, 8, 1024, 512, 32, 1), (64, 2, 8, 7168, 1536, 16, 0),
 ])
 def test_few_token_kernels_against_full_rounds_of_tiles(tokens, topk, experts, hidden, inter, rows, want):
     assert _lib.load().pyhip_layer_takes_pairs(tokens, topk, experts, hidden, inter, rows, 0, 0) == want
 
 
-@pytest.mark.parametrize("topk,hidden,inter,want", [
-    (8, 1536, 1536, 1), (4, 3072, 3072, 1), (8, 7168, 2048, 1), (8, 7168, 4096, 1), (1, 512, 4096, 1), (6, 2560, 2048, 1),
+@pytest.mark.parametrize("tokens,topk,hidden,inter,want", [
+    (1, 8, 1536, 1536, 1), (1, 4, 3072, 3072, 1), (1, 8, 7168, 2048, 1), (1, 8, 7168, 4096, 1), (1, 1, 512, 4096, 1), (1, 6, 2560, 2048, 1), (2, 8, 4096, 4096, 1),
     # a token's slots one after the other take longer than the reduction does: up to 31 % more of the layer call than before these kernels
-    (8, 1536, 3584, 0), (8, 2048, 2048, 0), (6, 1536, 3072, 0), (4, 2048, 4096, 0), (8, 3072, 4096, 0),
+    (1, 8, 1536, 3584, 0), (1, 8, 2048, 2048, 0), (1, 6, 1536, 3072, 0), (1, 4, 2048, 4096, 0), (1, 8, 3072, 4096, 0), (2, 6, 1024, 3072, 0),
 ])
-def test_slots_are_summed_in_the_down_gemm_only_where_they_are_short(topk, hidden, inter, want):
-    assert _lib.load().pyhip_layer_sums(topk, hidden, inter) == want
+def test_slots_are_summed_in_the_down_gemm_only_where_they_are_short(tokens, topk, hidden, inter, want):
+    assert _lib.load().pyhip_layer_sums(tokens, topk, hidden, inter) == want
