@@ -64,7 +64,7 @@ INTERNAL = {
     "pyhip_layer_forward": (_I, [_c.c_char_p, _P]),
     "pyhip_layer_block_m": (_I, [_L, _I, _I, _I, _I, _I]),
     "pyhip_layer_takes_pairs": (_I, [_L, _I, _I, _I, _I, _I, _I, _I]),
-    "pyhip_layer_sums": (_I, [_L, _I, _I, _I]),
+    "pyhip_layer_sums": (_I, [_L, _I, _I, _I, _I, _I]),
     "pyhip_layer_takes_cols": (_I, [_L, _I, _I, _I, _I, _I, _I, _I, _L]),
 }
 

@@ -200,7 +200,9 @@ static bool takes_pairs(int64_t tokens, int topk, int experts, int local_experts
 // per expert alone, unless that has fewer tiles in the gate_up GEMM than the chip has CUs and 64, 32 or 16 rows are estimated to
 // take 5 % less: lower tiles are more of them, and each is done sooner.  Layer, us: 8 experts, 1024 x 512, top-2, 493 tokens, 160 / 16 rows:
 // 30.2 / 23.7; 1024 tokens, 128 / 32: 30.2 / 27.1; 2208 x 1792, top-1, 446 tokens, 128 / 32: 36.5 / 27.2; 6176 x 512, Zipf, 371 tokens, 128 / 32:
-// 52.3 / 37.1.  The estimate is trusted where lower tiles cannot lose much, else the ladder stays: with few enough of them that all run at
+// 52.3 / 37.1.  The estimate is trusted where lower tiles cannot lose much, else the ladder stays: where the
+// ladder, at 128 rows and more, leaves nearly half of the CUs without a tile (388 calls of random layers take 21 % less, the slowest 8 % more; beyond, up to 44 %
+// more: 8 experts, 6656 x 3584, 60 rows per expert, 224 tiles of 128 rows), with few enough of them that all run at
 // once also under a router that makes more (64 rows: 96 in the gate_up GEMM, 160 up to hidden 2048; 16 and 32: 128), or with a short K loop (16 and 32
 // rows: hidden up to 2048, or 2560 where an expert has two blocks and few are here; 64: 1024).  Beyond that it was wrong by up to 40 % (8 experts, 128 / 64
 // rows: 6720 x 2944, Zipf, 216 tokens 68.2 / 95.4; 4576 x 2304, 348 tokens 52.6 / 64.7; 5888 x 2528, 466 tokens, 160 / 64: 66.6 / 80.0; 24 experts, 128 / 32: 4960 x
@@ -257,6 +259,9 @@ extern "C" int pyhip_layer_block_m(int64_t tokens, int topk, int experts, int lo
             best = estimate(c);
             rows = c.rows;
         }
+    const double at_ladder = local_experts * expected_blocks(est, ladder) * (inter / 128);
+    if(ladder >= 128 && at_ladder <= 145.0 && (rows == 64 || local_experts * expected_blocks(est, rows) * (inter / 128) <= 280.0))
+        return rows;
     const double tiles = local_experts * expected_blocks(est, rows) * (inter / 128);
     const bool short_k = hidden <= 2048 || (hidden <= 2560 && est <= 2.0 * rows && local_experts <= 12);
     const bool trusted = rows == 64 ? hidden <= 1024 || tiles <= (hidden <= 2048 ? 160.0 : 96.0)
@@ -325,7 +330,8 @@ static bool few_enough_rows(int64_t pairs, int experts, int local_experts, int h
 // Layer, us, sorted / this: 8 experts, 1024 x 512, top-2, 40 tokens 21.3 / 17.9, 64 tokens 21.2 / 17.7; 12, 1024 x 1024, top-1, 100 tokens 22.9 /
 // 19.0.  With more workgroups it goes either way: DeepSeek-V3 shape, 16 tokens 356.0 / 347.5; 96 experts, top-4, 6272 x 1920, 30 tokens 204.6 / 198.2;
 // 60, 2048 x 1408, 32 tokens 49.2 / 47.0; gpt-oss shape, 32 tokens 167.9 / 170.6; Qwen3 shape, 16 tokens 65.9 / 68.3; Mixtral shape, 50 tokens, bf16
-// activations 121.4 / 131.4: left to the sort.  Nor with more than 8 rows per expert in wide layers: 8 experts, top-2, 64 tokens, by the layer, persistent
+// activations 121.4 / 131.4: left to the sort.  Nor with more than 8 rows per expert in wide layers: 8 experts, top-2, 40 tokens, 7168 x
+// 1024 0.69, 64 tokens, by the layer, persistent
 // kernels / this: 2560 x 1536 27.8 / 23.9, 3584 x 1024 28.1 / 23.6, 3072 x 1536 28.8 / 27.4, 5120 x 1536 36.2 / 39.7, 7168 x 1536 43.8 / 52.0.
 static bool leaves_sort_out(int64_t tokens, int topk, int experts, int hidden, int inter, int block_m, int w4a16)
 {
@@ -334,7 +340,7 @@ static bool leaves_sort_out(int64_t tokens, int topk, int experts, int hidden, i
         return false;
     // (with more than one block of 16 to an expert its weights are fetched again)
     return (block_m == 16 && pairs <= WAVE) || (blocks * (inter / 32) <= 768 && blocks <= 64 &&
-                                                pairs <= (w4a16 || (int64_t)hidden * inter <= 4 << 20 ? 16ll : 8ll) * experts);
+                                                pairs <= 16ll * experts && (w4a16 || pairs <= 8ll * experts || pairs * hidden * inter <= (80ll << 20) * experts));
 }
 // A workgroup's start and end against its K loop, of which 512 columns are a single K-step to each of its four waves.  With MXFP4 activations
 // such layers are served only while few workgroups follow one another on a CU, or in 16-row blocks with hidden between 1024 and 2048 or few pairs.  Layer, us,

@@ -833,17 +833,21 @@ int pyhip_pairs_down(PairArgs g, int64_t rows, int64_t n_blk, int split_k, hipSt
 }
 
 // Whether a token's slots are few and short enough for a workgroup of the summing GEMM to take them in turns: it streams topk x inter columns.  Layer,
-// us, by expert + reduction / summed, 128 experts, one token: top-8, 1536 x 1536 16.9 / 16.2, 2048 x 2048 17.0 / 19.7, 1536 x 3072 18.5 / 23.4, 4096 x
+// us, by expert + reduction / summed, 128 experts, one token: top-8, 1024 x 2048 0.99 (16 experts 16.6 / 14.6), 1536 x 1536 16.9 / 16.2, 2048 x 2048 17.0 / 19.7, 1536 x 3072 18.5 / 23.4, 4096 x
 // 4096 40.0 / 42.9; top-4, 3072 x 3072 19.4 / 18.4, 3072 x 4096 20.4 / 21.3; two tokens, top-6, 1024 x 3072 19.4 / 21.5.  With 7168 channels over
 // the tokens there are workgroups enough: top-8, one token, hidden 7168, inter 2048 35.8 / 34.7, 4096 62.0 / 60.7; two, 4096 x 4096 0.97; top-4, three, 2560 x 4096 0.96.
-extern "C" int pyhip_layer_sums(int64_t tokens, int topk, int hidden, int inter) { return (int64_t)topk * inter <= 12288 || tokens * hidden >= 7168; }
+// (Under an expert mask a token has topk * held / experts slots here: 32 experts, top-8, 4096 x 4096, one of 8 ranks 17.8 / 14.1.)
+extern "C" int pyhip_layer_sums(int64_t tokens, int topk, int experts, int held, int hidden, int inter)
+{
+    return (int64_t)topk * inter * held <= (hidden <= 1024 ? 16384ll : 12288ll) * experts || tokens * hidden >= 7168;
+}
 
 int pyhip_pairs_down_sum(PairArgs g, int64_t rows, int64_t n_blk, int split_k, hipStream_t stream)
 {
     const int64_t pairs  = (int64_t)g.T * g.topk;
     const int64_t blocks = block_bound(pairs, n_blk, g.experts);
     // by token the weights of an expert are fetched for each of its pairs: only where pairs rarely share one
-    if(!g.ids || g.fp4 || g.topk > 8 || !pyhip_layer_sums(g.T, g.topk, g.N, g.K) || (g.T > 1 && 8 * pairs > g.experts) || w4a16_split(2, 16, blocks * (g.N / 256), g.K, split_k) != 4)
+    if(!g.ids || g.fp4 || g.topk > 8 || !pyhip_layer_sums(g.T, g.topk, g.experts, g.held, g.N, g.K) || (g.T > 1 && 8 * pairs > g.experts) || w4a16_split(2, 16, blocks * (g.N / 256), g.K, split_k) != 4)
         return -1;
     PYHIP_REQUIRE(((uintptr_t)g.out % 16) == 0, "moe_pairs_down_sum: unaligned pointer");
     const int rc = prepare("moe_pairs_down_sum", g, rows, blocks, g.N / 64);

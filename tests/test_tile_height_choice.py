@@ -88,10 +88,21 @@ def test_few_token_kernels_against_full_rounds_of_tiles(tokens, topk, experts, h
     assert _lib.load().pyhip_layer_takes_pairs(tokens, topk, experts, hidden, inter, rows, 0, 0) == want
 
 
-@pytest.mark.parametrize("tokens,topk,hidden,inter,want", [
-    (1, 8, 1536, 1536, 1), (1, 4, 3072, 3072, 1), (1, 8, 7168, 2048, 1), (1, 8, 7168, 4096, 1), (1, 1, 512, 4096, 1), (1, 6, 2560, 2048, 1), (2, 8, 4096, 4096, 1),
+@pytest.mark.parametrize("tokens,topk,experts,held,hidden,inter,want", [
+    (1, 8, 64, 64, 1536, 1536, 1), (1, 4, 64, 64, 3072, 3072, 1), (1, 8, 64, 64, 7168, 2048, 1), (1, 1, 64, 64, 512, 4096, 1), (1, 8, 16, 16, 1024, 2048, 1),
+    (2, 8, 128, 128, 4096, 4096, 1), (1, 8, 32, 4, 4096, 4096, 1),
     # a token's slots one after the other take longer than the reduction does: up to 31 % more of the layer call than before these kernels
-    (1, 8, 1536, 3584, 0), (1, 8, 2048, 2048, 0), (1, 6, 1536, 3072, 0), (1, 4, 2048, 4096, 0), (1, 8, 3072, 4096, 0), (2, 6, 1024, 3072, 0),
+    (1, 8, 60, 60, 1536, 3584, 0), (1, 8, 64, 64, 2048, 2048, 0), (1, 4, 64, 64, 2048, 4096, 0), (2, 6, 96, 96, 1024, 3072, 0), (1, 8, 32, 32, 4096, 4096, 0),
 ])
-def test_slots_are_summed_in_the_down_gemm_only_where_they_are_short(tokens, topk, hidden, inter, want):
-    assert _lib.load().pyhip_layer_sums(tokens, topk, hidden, inter) == want
+def test_slots_are_summed_in_the_down_gemm_only_where_they_are_short(tokens, topk, experts, held, hidden, inter, want):
+    assert _lib.load().pyhip_layer_sums(tokens, topk, experts, held, hidden, inter) == want
+
+
+@pytest.mark.parametrize("tokens,topk,experts,local,hidden,inter,want", [
+    # the ladder's height leaves nearly half of the CUs without a tile: 20 to 35 % less with lower ones
+    (930, 1, 28, 28, 5120, 512, 32), (419, 2, 8, 8, 6144, 1024, 64), (289, 2, 8, 8, 5120, 1024, 32), (1130, 1, 8, 8, 6656, 1536, 64), (710, 1, 8, 8, 6656, 1024, 64),
+    # more tiles than that
+    (484, 1, 8, 8, 6656, 3584, 128), (200, 2, 8, 8, 6656, 3072, 128), (1009, 8, 128, 16, 4096, 1536, 128),
+])
+def test_lower_tiles_where_the_ladder_leaves_half_of_the_chip(tokens, topk, experts, local, hidden, inter, want):
+    assert _lib.load().pyhip_layer_block_m(tokens, topk, experts, local, hidden, inter) == want
