@@ -312,10 +312,11 @@ struct Router
 //     277, 31: 323 / 357; DeepSeek-V3 shape 11.6: 949 / 939, 16: 964 / 981; 96 experts 5: 128 / 114, 11.7: 212 / 189; 8 experts 17.5: 140 / 123, 25: 142 /
 //     129, 40: 147 / 149; 16, top-2, 4096 x 4096 25: 84.3 / 83.0, 31: 85.0 / 88.4; 12, 5120 x 2048 22: 46.8 / 47.4, 28: 47.6 / 51.2
 // With a handful of experts and hidden 2560 and more the line lies lower where the persistent kernels' tiles of the gate_up GEMM (`tiles`) make most of one
-// round of the chip: from there to 256 an uneven router takes them into a second round, which costs them up to 25 %.  Layer, us, by rows per expert:
-// 28 experts, top-2, 224 tiles, 7168 x 1024 23: 71.9 / 79.4, 16 under a Zipf router 0.87; 4096 x 1024 23: 47.4 / 51.3, 13: 43.6 / 45.3; 192 tiles, 24, top-4, 7168 x 1024 23
-// under a Zipf router 64.2 / 72.0, 10: 58.6 / 63.5 and 0.98 under an even one; 20, 240 tiles, 3072 x 1536 13: 0.95, under a Zipf router 0.77; 64, 8, 5120 x 1024 10: 0.69;
-// 320, 20, 4096 x 2048 19: 67.3 / 59.2.
+// round of the chip.  (From 232 to 256 an uneven router takes them into a second round, which costs them up to 25 %.)  Layer, us, persistent kernels / this, or the
+// ratio, by rows per expert:
+//   192 tiles, 24 experts, top-4, 7168 x 1024 under a Zipf router 10: 58.6 / 63.5, 23: 64.2 / 72.0, under an even one 10: 0.98
+//   224, 28 experts, top-2, 7168 x 1024 23: 71.9 / 79.4; 4096 x 1024 13: 43.6 / 45.3, 23: 47.4 / 51.3
+//   240, 20 experts, 3072 x 1536 13: 0.95, under a Zipf router 0.77; 64, 8 experts, 5120 x 1024 10: 0.69; 320, 20 experts, 4096 x 2048 19: 67.3 / 59.2
 static bool few_enough_rows(int64_t pairs, int experts, int local_experts, int hidden, int inter, int block_m)
 {
     if(experts >= 32 || block_m == 16)
@@ -330,15 +331,14 @@ static bool few_enough_rows(int64_t pairs, int experts, int local_experts, int h
 // Layer, us, sorted / this: 8 experts, 1024 x 512, top-2, 40 tokens 21.3 / 17.9, 64 tokens 21.2 / 17.7; 12, 1024 x 1024, top-1, 100 tokens 22.9 /
 // 19.0.  With more workgroups it goes either way: DeepSeek-V3 shape, 16 tokens 356.0 / 347.5; 96 experts, top-4, 6272 x 1920, 30 tokens 204.6 / 198.2;
 // 60, 2048 x 1408, 32 tokens 49.2 / 47.0; gpt-oss shape, 32 tokens 167.9 / 170.6; Qwen3 shape, 16 tokens 65.9 / 68.3; Mixtral shape, 50 tokens, bf16
-// activations 121.4 / 131.4: left to the sort.  Nor with more than 8 rows per expert in wide layers: 8 experts, top-2, 40 tokens, 7168 x
-// 1024 0.69, 64 tokens, by the layer, persistent
-// kernels / this: 2560 x 1536 27.8 / 23.9, 3584 x 1024 28.1 / 23.6, 3072 x 1536 28.8 / 27.4, 5120 x 1536 36.2 / 39.7, 7168 x 1536 43.8 / 52.0.
+// activations 121.4 / 131.4: left to the sort.  Nor, with more than 8 rows per expert, in large layers, which fetch the weights of their
+// second blocks again.  Layer, us, persistent kernels / this, 8 experts, top-2, 64 tokens: 2560 x 1536 27.8 / 23.9, 3584 x 1024 28.1 / 23.6, 3072 x 1536 28.8 / 27.4, 5120 x
+// 1536 36.2 / 39.7, 7168 x 1536 43.8 / 52.0; 40 tokens, 7168 x 1024 0.69.
 static bool leaves_sort_out(int64_t tokens, int topk, int experts, int hidden, int inter, int block_m, int w4a16)
 {
     const int64_t pairs = tokens * topk, blocks = pairs < experts + pairs / 16 ? pairs : experts + pairs / 16;
     if(block_m > 32 || (w4a16 && block_m > 16) || pairs > PAIRS_UNSORTED_MAX)
         return false;
-    // (with more than one block of 16 to an expert its weights are fetched again)
     return (block_m == 16 && pairs <= WAVE) || (blocks * (inter / 32) <= 768 && blocks <= 64 &&
                                                 pairs <= 16ll * experts && (w4a16 || pairs <= 8ll * experts || pairs * hidden * inter <= (80ll << 20) * experts));
 }
